@@ -621,7 +621,7 @@ void compute_norm(dcrf_model& m, Term& t) {
     if (tiled)
         launch_splat_tiled(ts, ent.get(), ones.get(), vals0.get(), 1, 1, m.lds_cap, s);
     else
-        launch_splat(ch.get(), (int)hch.size(), ent.get(), ones.get(), 1, vals0.get(), 1, 1, s);
+        launch_splat(ch.get(), (int)hch.size(), ent.get(), ones.get(), N, 1, vals0.get(), 1, 1, s);
     launch_combine(cb.get(), (int)hcb.size(), vals0.get(), 1, 1, s);
     BlurTable bt{};
     bt.nterms = 1;
@@ -885,7 +885,7 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
     DevBuf<float> in1;
     in1.reserve((size_t)P.parts.size() * N);
     launch_fill(in1.get(), 1.f, (size_t)P.parts.size() * N, s);
-    launch_splat(P.ch2.get(), P.nch, P.ent.get(), in1.get(), 1, P.ones[0].get(), 1, 1, s);
+    launch_splat(P.ch2.get(), P.nch, P.ent.get(), in1.get(), P.parts.size() * (size_t)N, 1, P.ones[0].get(), 1, 1, s);
     launch_combine(P.cb2.get(), P.ncb, P.ones[0].get(), 1, 1, s);
     float* const obuf[2] = {P.ones[1].get(), P.ones[2].get()};
     kg_blur(P, false, P.ones[0].get(), obuf, 1, s);
@@ -956,7 +956,7 @@ void kernel_grad_group(dcrf_model& m, const KgPlan& P, const float* b, const flo
         launch_kg_prepare(Qt, b, t.norm.get(), N, L, st, t.ntype, need_fa ? lbl + i * NL : nullptr,
                           pk + (size_t)i * 2 * NL, s);
     }
-    launch_splat(P.ch2.get(), P.nch, P.ent.get(), pk, L2, P.S2.get(), L2, L2, s);
+    launch_splat(P.ch2.get(), P.nch, P.ent.get(), pk, (size_t)T * N, L2, P.S2.get(), L2, L2, s);
     launch_combine(P.cb2.get(), P.ncb, P.S2.get(), L2, L2, s);
     float* const pbuf[2] = {P.X2[0].get(), P.X2[1].get()};
     kg_blur(P, false, P.S2.get(), pbuf, L2, s);
@@ -981,7 +981,7 @@ void kernel_grad_group(dcrf_model& m, const KgPlan& P, const float* b, const flo
             st.t[1] = SliceTerm{vtx, sw, need_fb ? fwd_of(i) + L : nullptr, d1, -1, nullptr, nullptr, nullptr, L2};  // K c
             launch_kg_x(b, lbl + (size_t)i * NL, t.norm.get(), N, L, st, t.ntype, x, s);
         }
-        launch_splat(P.ch1.get(), P.nch, P.ent.get(), xb, L, P.S1.get(), L, L, s);
+        launch_splat(P.ch1.get(), P.nch, P.ent.get(), xb, (size_t)T * N, L, P.S1.get(), L, L, s);
         launch_combine(P.cb1.get(), P.ncb, P.S1.get(), L, L, s);
         kg_blur(P, true, P.S1.get(), xbuf, L, s);
     }
@@ -1406,6 +1406,7 @@ BlurTable blur_table(const dcrf_model& m) {
 SliceTable slice_table(const dcrf_model& m, bool transpose, const float* kw, float* mout) {
     SliceTable st{};
     st.nterms = (int)m.terms.size();
+    st.rows = (size_t)m.V_total + 1;  // the slices read vertex rows (and the zero row)
     const size_t NL = (size_t)m.N() * m.L;
     for (int k = 0; k < st.nterms; k++) {
         const Term& t = *m.terms[k];
@@ -1440,6 +1441,11 @@ double splat_bytes(const dcrf_model& m) {
 }
 double meanfield_bytes(const dcrf_model& m) { return splat_bytes(m) + m.N() * (double)m.L * 4.0; }
 
+// Rows of the splat's input: the pixels, or the 8 x 8 block positions of entries ent_in.
+size_t in_rows(const dcrf_model& m, const int2* ent_in) {
+    return ent_in ? q_block_rows(m.geo.W[0], m.geo.H[0]) : (size_t)m.N();
+}
+
 // in: the [N] input rows with row stride ldi (floats).
 void run_filter(dcrf_model& m, const float* in, int ldi, bool transpose, hipStream_t s,
                 const int2* ent_in = nullptr) {
@@ -1450,7 +1456,8 @@ void run_filter(dcrf_model& m, const float* in, int ldi, bool transpose, hipStre
         if (m.tiled)
             launch_splat_tiled(m.tsplat, ent, in, m.vals[0].get(), m.ldv, L, m.lds_cap, s);  // ldi == L
         else
-            launch_splat(m.g_chunks.get(), m.C_total, ent, in, ldi, m.vals[0].get(), m.ldv, L, s);
+            launch_splat(m.g_chunks.get(), m.C_total, ent, in, in_rows(m, ent_in), ldi,
+                         m.vals[0].get(), m.ldv, L, s);
         t.done();
     }
     if (m.CB_total) {

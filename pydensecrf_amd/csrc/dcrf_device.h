@@ -31,8 +31,8 @@ constexpr int kXcds = 8;         // MI355X: 8 XCDs, each with its own L2
 // items: neighbouring vertices / pixels, whose rows the gathers share, then meet in
 // the same L2.  A bijection on [0, nb).
 __device__ __forceinline__ int xcd_block(int b, int nb) {
-    const int x = b % kXcds, i = b / kXcds;
-    const int q = nb / kXcds, r = nb % kXcds;
+    const int x = (unsigned)b % kXcds, i = (unsigned)b / kXcds;
+    const int q = (unsigned)nb / kXcds, r = (unsigned)nb % kXcds;
     return x * q + (x < r ? x : r) + i;
 }
 
@@ -121,17 +121,40 @@ __device__ __forceinline__ void store_piece(float* __restrict__ row, int k0, int
     *reinterpret_cast<Piece<R>*>(row + k0) = p;
 }
 
+// Pointer to the lane's piece of row `row` of rows of ld floats.  NARROW: the row index is
+// below 2^24 and the whole array below 4 GiB (narrow_rows on the host), so the offset is
+// one 24-bit multiply-add and the access takes a scalar base with a 32-bit lane offset.
+// The 64-bit form costs a 64-bit multiply and two 64-bit adds per gathered row.
+template <bool NARROW>
+__device__ __forceinline__ const float* row_piece(const float* __restrict__ base, int row, int ld, int k0) {
+    if (NARROW) {
+        const unsigned off = __umul24((unsigned)row, (unsigned)ld * 4u) + (unsigned)k0 * 4u;
+        return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + off);
+    }
+    return base + (size_t)row * ld + k0;
+}
+
+// Value x of lane `lane` of the wave (every lane of the wave calls).
+__device__ __forceinline__ float wave_read(float x, int lane) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(lane << 2, __float_as_int(x)));
+}
+__device__ __forceinline__ int wave_read(int x, int lane) { return __builtin_amdgcn_ds_bpermute(lane << 2, x); }
+
 template <bool WAVE, int R>
 struct LaneGroup {
     int L, S, g, l, k0, base, t, per;
+    int w;  // the thread's wave in its block (the same in every lane: a scalar)
     bool on;
     float* sh;  // block mode: block * R floats
 
     // per: groups per wave (WAVE) or per block
     __device__ __forceinline__ LaneGroup(int L_, int S_, int per_, float* sh_) : L(L_), S(S_), per(per_), sh(sh_) {
         t = threadIdx.x;
+        w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
         const int lane = WAVE ? (t & 63) : t;
-        g = lane / S;
+        // lane / S: (lane + 1/2) / S is at least 1 / 2048 away from an integer (S and lane
+        // stay below 1024), far more than the reciprocal's and the product's rounding
+        g = (int)(((float)lane + 0.5f) * __builtin_amdgcn_rcpf((float)S));
         l = lane - g * S;
         on = g < per;
         if (!on) {  // idle lanes shadow group 0 so that every shuffle index stays valid
@@ -139,11 +162,11 @@ struct LaneGroup {
             l = l < S ? l : 0;
         }
         k0 = l * R;
-        base = WAVE ? (t & ~63) + g * S : g * S;
+        base = g * S;  // the group's first lane (WAVE: in its wave, else in the block)
     }
     // Index of this group's item in block b of a grid.
     __device__ __forceinline__ int item_in(int b) const {
-        return WAVE ? (b * (kWaveBlock / 64) + (t >> 6)) * per + g : b * per + g;
+        return WAVE ? (b * (kWaveBlock / 64) + w) * per + g : b * per + g;
     }
     // Index of this group's item (blocks taken in XCD-contiguous order).
     __device__ __forceinline__ int item() const { return item_in(xcd_block(blockIdx.x, gridDim.x)); }
@@ -152,7 +175,7 @@ struct LaneGroup {
 
     // Value of lane s of this group (all lanes must call).
     __device__ __forceinline__ float lane_value(float x, int s) {
-        if (WAVE) return __shfl(x, (base + s) & 63);
+        if (WAVE) return wave_read(x, base + s);
         sh[t] = x;
         __syncthreads();
         const float v = sh[base + s];
@@ -170,7 +193,7 @@ struct LaneGroup {
             for (int k = 1; k < S; k <<= 1) {
                 int s = l + k;
                 if (s >= S) s -= S;
-                m = fmaxf(m, __shfl(m, (base + s) & 63));
+                m = fmaxf(m, wave_read(m, base + s));
             }
             return m;
         }
@@ -190,10 +213,10 @@ struct LaneGroup {
         if (WAVE) {
             // pairwise tree over the S lanes towards lane 0 of the group, then a broadcast
             for (int k = 1; k < S; k <<= 1) {
-                const float y = __shfl(a, (base + l + k) & 63);
+                const float y = wave_read(a, base + l + k);  // (lane numbers wrap at 64)
                 if ((l & (2 * k - 1)) == 0 && l + k < S) a = a + y;
             }
-            return __shfl(a, base & 63);
+            return wave_read(a, base);
         }
         sh[t] = a;
         __syncthreads();
@@ -290,10 +313,7 @@ __device__ __forceinline__ void slice_piece(const SliceTerm& T, int p, int k0, i
     for (int j = 0; j < kMaxD1; j++)
         if (j < d1) {
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                const float prod = w[j] * x[j][r];
-                m[r] = m[r] + prod;
-            }
+            for (int r = 0; r < R; r++) m[r] = fmaf(w[j], x[j][r], m[r]);
         }
 }
 
@@ -396,6 +416,22 @@ __device__ __forceinline__ void matrix_piece_rows(const float* __restrict__ w, i
         const float mv = mrow[b];
 #pragma unroll
         for (int r = 0; r < R; r++) c[r] = fmaf(w[(size_t)(k0 + r) * ldw + b], mv, c[r]);
+    }
+}
+
+// y[r] / s for the lane's values, s the same for all of them: one reciprocal (Newton's
+// step on the hardware's approximation), then per value the product and one residual
+// correction (Markstein), which gives the rounded quotient for the softmax's operands
+// (0 <= y <= 1 <= s <= DCRF_MAX_LABELS; NaNs pass through).  Three full divisions took a
+// tenth of the fused mean-field kernel's instructions.
+template <int R>
+__device__ __forceinline__ void divide_all(const float (&y)[R], float s, float (&q)[R]) {
+    float rc = __builtin_amdgcn_rcpf(s);
+    rc = fmaf(fmaf(-s, rc, 1.0f), rc, rc);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const float a = y[r] * rc;
+        q[r] = fmaf(fmaf(-s, a, y[r]), rc, a);
     }
 }
 

@@ -276,6 +276,7 @@ struct SliceTerm {
 struct SliceTable {
     int nterms;
     SliceTerm t[DCRF_MAX_TERMS];
+    size_t rows = ~(size_t)0;  // rows of the terms' value buffers (unknown: 64-bit offsets)
     int nstat = 0;  // terms with a statistic (gslot 0 .. nstat-1)
 };
 // Give each Matrix term an LDS copy of its L x L compatibility (cw_lds) while they fit
@@ -298,9 +299,10 @@ LaunchShape shape_for(int L);
 LaunchShape shape_for_r(int L, int R);  // the shape for R labels per lane
 
 // Splat: vals[out] = sum over a segment's entries i of w_i * in[p_i], in entry order;
-// ent[i] = (p_i, bits of w_i).  Global form: p_i is the pixel (row of `in`).
-void launch_splat(const Chunk* chunks, int n_chunks, const int2* ent, const float* in, int ldi, float* vals,
-                  int ldv, int L, hipStream_t s);
+// ent[i] = (p_i, bits of w_i).  Global form: p_i is the pixel (row of `in`, rows_in of them).
+void launch_splat(const Chunk* chunks, int n_chunks, const int2* ent, const float* in, size_t rows_in, int ldi,
+                  float* vals, int ldv, int L, hipStream_t s);
+bool narrow_rows(size_t rows, int ld);
 // Tiled form: one block per tile stages the tile's input rows, entries and segments in
 // LDS; p_i is then the index of the entry's pixel inside its tile (row-major in the
 // tile).  The entries of tile t are [tile_e[t], tile_e[t+1]), its segments

@@ -66,9 +66,19 @@ __global__ void k_fill(float* p, float v, size_t n) {
 //   serves 16 pairs instead of one load per lane and pair.  Input rows are gathered
 //   kBatch at a time.
 //   block mode (a group wider than a wave): the pairs are loaded by every lane.
+// The compiler must not sink a batch's loads into the masked additions that use them: it
+// had moved the first entry's LDS read and row load behind all the others of its batch,
+// two memory round trips per batch instead of one (loaded() keeps a value's load where
+// it is written).
 constexpr int kWin = 512;  // entry pairs per wave window
 
-template <bool WAVE, int R>
+template <int R>
+__device__ __forceinline__ void loaded(float (&x)[R]) {
+#pragma unroll
+    for (int r = 0; r < R; r++) asm volatile("" : "+v"(x[r]));
+}
+
+template <bool WAVE, int R, bool NARROW>
 __global__ void __launch_bounds__(1024) k_splat(const Chunk* __restrict__ chunks, int n,
                                                 const int2* __restrict__ ent, const float* __restrict__ in, int ldi,
                                                 float* __restrict__ vals, int ldv, int L, int S, int per) {
@@ -80,24 +90,28 @@ __global__ void __launch_bounds__(1024) k_splat(const Chunk* __restrict__ chunks
     for (int r = 0; r < R; r++) acc[r] = 0.0f;
     if (WAVE) {
         extern __shared__ int2 win_all[];
-        int2* win = win_all + (threadIdx.x >> 6) * (kWin + kBatch);
+        int2* win = win_all + G.w * (kWin + kBatch);
         const int lane = threadIdx.x & 63;
-        const int cw0 = c - G.g;  // the wave's first chunk
-        if (cw0 >= n) return;     // the whole wave is idle (no block barrier below)
+        // the wave's first chunk: the same in every lane (scalar bounds and loop)
+        const int cw0 = __builtin_amdgcn_readfirstlane(c - G.g);
+        if (cw0 >= n) return;  // the whole wave is idle (no block barrier below)
         const bool mine = G.on && c < n;
         const Chunk ch = chunks[mine ? c : cw0];
         const int r0 = chunks[cw0].beg, r1 = chunks[min(cw0 + per - 1, n - 1)].end;
-        for (int w0 = r0; w0 < r1; w0 += kWin) {  // wave-uniform
+        for (int w0 = r0; w0 < r1; w0 += kWin) {
             const int wn = min(kWin, r1 - w0);
-            // all loads first (clamped, unconditional), then the stores: the loads stay
-            // in flight together
-            int2 t[kWin / 64];
-#pragma unroll
-            for (int u = 0; u < kWin / 64; u++) t[u] = ent[w0 + min(lane + 64 * u, wn - 1)];
+            const int2* __restrict__ src = ent + w0;
             __builtin_amdgcn_wave_barrier();  // the previous window's reads come first
+            // four loads per lane and round (clamped, unconditional), then their stores:
+            // past wn they repeat the last pair, inside the window
+            for (int u0 = 0; u0 < wn; u0 += 256) {
+                long long t[4];
 #pragma unroll
-            for (int u = 0; u < kWin / 64; u++)
-                if (lane + 64 * u < wn) win[lane + 64 * u] = t[u];
+                for (int u = 0; u < 4; u++)
+                    t[u] = reinterpret_cast<const long long*>(src)[(unsigned)min(u0 + lane + 64 * u, wn - 1)];
+#pragma unroll
+                for (int u = 0; u < 4; u++) reinterpret_cast<long long*>(win)[u0 + lane + 64 * u] = t[u];
+            }
             if (lane < kBatch) win[wn + lane] = make_int2(0, 0);  // padding: pixel 0, weight 0
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -110,31 +124,30 @@ __global__ void __launch_bounds__(1024) k_splat(const Chunk* __restrict__ chunks
 #pragma unroll
                     for (int u = 0; u < kBatch; u++) e[u] = win[i + u];  // i + u < wn + kBatch
 #pragma unroll
-                    for (int u = 0; u < kBatch; u++) load_piece<R>(in + (size_t)e[u].x * ldi, k0, L, xx[u]);
+                    for (int u = 0; u < kBatch; u++) load_piece<R>(row_piece<NARROW>(in, e[u].x, ldi, k0), 0, L, xx[u]);
 #pragma unroll
-                    for (int u = 0; u < kBatch; u++)
+                    for (int u = 0; u < kBatch; u++) {
+                        loaded<R>(xx[u]);
                         if (i + u < b) {
                             const float wu = __int_as_float(e[u].y);
 #pragma unroll
-                            for (int r = 0; r < R; r++) {
-                                const float prod = wu * xx[u][r];
-                                acc[r] = acc[r] + prod;
-                            }
+                            for (int r = 0; r < R; r++) acc[r] = fmaf(wu, xx[u][r], acc[r]);
                         }
+                    }
                 }
             }
         }
         // A run of the wave's chunks with one vertex (the layout gives the later ones
         // out = -1): their sums are folded into the run's first group, right to left, in
         // a fixed order.  Lists without such runs skip this.
-        const int nv = __shfl(ch.v, (lane + S) & 63);
-        const int nout = __shfl(ch.out, (lane + S) & 63);
+        const int nv = wave_read(ch.v, lane + S);
+        const int nout = wave_read(ch.out, lane + S);
         const bool cont = mine && G.g + 1 < per && c + 1 < n && nout < 0 && nv == ch.v;
         if (__any(cont)) {
             for (int j = per - 2; j >= 0; j--) {  // wave-uniform
                 float y[R];
 #pragma unroll
-                for (int r = 0; r < R; r++) y[r] = __shfl(acc[r], (lane + S) & 63);
+                for (int r = 0; r < R; r++) y[r] = wave_read(acc[r], lane + S);
                 if (cont && G.g == j)
 #pragma unroll
                     for (int r = 0; r < R; r++) acc[r] = acc[r] + y[r];
@@ -151,17 +164,16 @@ __global__ void __launch_bounds__(1024) k_splat(const Chunk* __restrict__ chunks
 #pragma unroll
         for (int u = 0; u < kBatch; u++) e[u] = ent[min(i + u, ch.end - 1)];
 #pragma unroll
-        for (int u = 0; u < kBatch; u++) load_piece<R>(in + (size_t)e[u].x * ldi, k0, L, xx[u]);
+        for (int u = 0; u < kBatch; u++) load_piece<R>(row_piece<NARROW>(in, e[u].x, ldi, k0), 0, L, xx[u]);
 #pragma unroll
-        for (int u = 0; u < kBatch; u++)
+        for (int u = 0; u < kBatch; u++) {
+            loaded<R>(xx[u]);
             if (i + u < ch.end) {
                 const float wu = __int_as_float(e[u].y);
 #pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const float prod = wu * xx[u][r];
-                    acc[r] = acc[r] + prod;
-                }
+                for (int r = 0; r < R; r++) acc[r] = fmaf(wu, xx[u][r], acc[r]);
             }
+        }
     }
     store_piece<R>(vals + (size_t)ch.out * ldv, k0, L, acc);
 }
@@ -247,10 +259,7 @@ __global__ void __launch_bounds__(1024) k_splat_tiled(TiledSplat ts, const int2*
 #pragma unroll
             for (int u = 0; u < 4; u++)
 #pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const float prod = ww[u] * xx[u][r];
-                    acc[r] = acc[r] + prod;
-                }
+                for (int r = 0; r < R; r++) acc[r] = fmaf(ww[u], xx[u][r], acc[r]);
         }
         for (; i < e; i++) {
             float xx[R];
@@ -258,10 +267,7 @@ __global__ void __launch_bounds__(1024) k_splat_tiled(TiledSplat ts, const int2*
             const float ww = __int_as_float(x.y);
             load_piece<R>(tq + x.x * L, k0, L, xx);
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                const float prod = ww * xx[r];
-                acc[r] = acc[r] + prod;
-            }
+            for (int r = 0; r < R; r++) acc[r] = fmaf(ww, xx[r], acc[r]);
         }
         store_piece<R>(vals + (size_t)out * ldv, k0, L, acc);
     }
@@ -330,7 +336,7 @@ __global__ void __launch_bounds__(kWaveBlock) k_combine_waves(const Combine* __r
         if (rc.count > 0) store_piece<R>(vals + (size_t)rc.v * ldv, k0, L, acc);
         return;
     }
-    float* wrows = rows_lds + (size_t)(threadIdx.x >> 6) * per * L;
+    float* wrows = rows_lds + (size_t)G.w * per * L;
     if (G.on && G.g < head.pad) store_piece<R>(wrows + (size_t)G.g * L, k0, L, acc);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -378,8 +384,7 @@ __global__ void __launch_bounds__(1024) k_blur(const float* __restrict__ src, fl
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const float s2 = a[r] + b[r];
-        const float h = 0.5f * s2;
-        out[r] = o[r] + h;
+        out[r] = fmaf(0.5f, s2, o[r]);
     }
     store_piece<R>(dst + (size_t)v * ldv, k0, L, out);
 }
@@ -393,8 +398,7 @@ __global__ void __launch_bounds__(1024) k_blur(const float* __restrict__ src, fl
 // K launches of k_blur, with K-1 fewer launches and no intermediate rows written.
 __device__ __forceinline__ float blur_fold(float o, float a, float b) {
     const float s2 = a + b;
-    const float h = 0.5f * s2;
-    return o + h;
+    return fmaf(0.5f, s2, o);
 }
 
 // zr: the zero row (absent neighbours point to it; it holds zeros in every vertex
@@ -586,8 +590,7 @@ __global__ void __launch_bounds__(1024) k_meanfield(const float* __restrict__ U,
     const float s = G.all_sum(x);
     if (active) {
         float q[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) q[r] = x[r] / s;
+        divide_all<R>(x, s, q);
         store_piece<R>(Q + (size_t)p * L, k0, L, q);
         if (tmp1) store_piece<R>(tmp1 + (size_t)p * L, k0, L, e);
         if (tmp2) store_piece<R>(tmp2 + (size_t)p * L, k0, L, last);
@@ -611,10 +614,7 @@ __device__ __forceinline__ void term_message(const SliceTerm& T, int k, const in
     for (int j = jb; j < je; j++) {
         const float w = __int_as_float(e[j].y);
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            const float prod = w * x[j][r];
-            raw[r] = raw[r] + prod;
-        }
+        for (int r = 0; r < R; r++) raw[r] = fmaf(w, x[j][r], raw[r]);
     }
 #pragma unroll
     for (int r = 0; r < R; r++) m[r] = raw[r];
@@ -688,8 +688,7 @@ __device__ __forceinline__ void finish_pixel(LaneGroup<true, R>& G, const SliceT
     const float sum = G.all_sum(y);
     if (active) {
         float q[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) q[r] = y[r] / sum;
+        divide_all<R>(y, sum, q);
         store_piece<R>(qrow, G.k0, G.L, q);
 #pragma unroll
         for (int k = 0; k < NT; k++)
@@ -697,34 +696,44 @@ __device__ __forceinline__ void finish_pixel(LaneGroup<true, R>& G, const SliceT
     }
 }
 
-// One (vertex, weight bits) pair by a nontemporal 8-byte load (x in the low word).
-__device__ __forceinline__ int2 load_pair_nt(const int2* p) {
-    const long long v = __builtin_nontemporal_load(reinterpret_cast<const long long*>(p));
-    return make_int2((int)(unsigned)(v & 0xffffffffll), (int)(v >> 32));
-}
+// The pixels of a wave of the fused kernels: np >= 1 consecutive ones from p0 (a wave past
+// the last pixel repeats it; its results are not stored).  Both are the same in every
+// lane, so the wave's rows of the unary, Q and the slice pairs start at scalar addresses.
+struct WavePixels {
+    int p0, np;
+    template <int R>
+    __device__ __forceinline__ WavePixels(const LaneGroup<true, R>& G, int p, int N) {
+        p0 = __builtin_amdgcn_readfirstlane(min(p - G.g, N - 1));
+        np = min(G.per, N - p0);
+    }
+};
 
-// Stage the slice pairs of the wave's pixels (consecutive: one contiguous run of
-// per * DS pairs, 64 pairs per load instruction) into the wave's LDS slice wp; the
-// wave's groups then read their own.  `p` is the group's pixel.
+// LDS pairs of one wave's staged slice pairs: its per * ds pairs rounded up to whole rounds
+// of 128 (stage_wave_pairs stores whole rounds).
+__host__ __device__ inline int wave_pairs(int per, int ds) { return (per * ds + 127) & ~127; }
+
+// Stage the slice pairs of the wave's pixels (one contiguous run of np * DS pairs, 64 pairs
+// per load instruction) into the wave's LDS slice wp; the wave's groups then read their
+// own.  Past the run the last pair is repeated, so a group without a pixel reads valid
+// rows and needs no mask (a masked LDS read per entry, each waited for on its own, had
+// made nine round trips of one).
 template <int R, int DS>
-__device__ __forceinline__ void stage_wave_pairs(const LaneGroup<true, R>& G, int p, int N,
-                                                 const int2* __restrict__ slc, int2* wp) {
-    const int per = G.per;
-    const int pw0 = p - G.g;  // the wave's first pixel
-    const int np = max(0, min(per, N - pw0)) * DS;
+__device__ __forceinline__ void stage_wave_pairs(const WavePixels& W, int per, const int2* __restrict__ slc,
+                                                 int2* wp) {
+    const int np = W.np * DS;
     const int lane = threadIdx.x & 63;
     // two loads per lane per round (clamped, unconditional), then the stores.  The pairs
     // are read once per iteration: nontemporal loads keep them from displacing the Q rows
     // this kernel writes, which the next splat gathers (at 1024x768x21 the splat went from
     // 72.5 to 58.3 us; nontemporal loads of the splat's own entries or of the unary row
     // measured slower)
-    const size_t base = (size_t)pw0 * DS;
-    const int last = max(np - 1, 0);
-    for (int i0 = 0; i0 < np; i0 += 128) {
-        const int2 t0 = load_pair_nt(slc + base + min(i0 + lane, last));
-        const int2 t1 = load_pair_nt(slc + base + min(i0 + 64 + lane, last));
-        if (i0 + lane < np) wp[i0 + lane] = t0;
-        if (i0 + 64 + lane < np) wp[i0 + 64 + lane] = t1;
+    const long long* __restrict__ src = reinterpret_cast<const long long*>(slc + (size_t)W.p0 * DS);
+    long long* dst = reinterpret_cast<long long*>(wp);
+    for (int i0 = 0; i0 < per * DS; i0 += 128) {
+        const long long t0 = __builtin_nontemporal_load(src + (unsigned)min(i0 + lane, np - 1));
+        const long long t1 = __builtin_nontemporal_load(src + (unsigned)min(i0 + 64 + lane, np - 1));
+        dst[i0 + lane] = t0;
+        dst[i0 + 64 + lane] = t1;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -735,30 +744,30 @@ __device__ __forceinline__ void stage_wave_pairs(const LaneGroup<true, R>& G, in
 // entries per pixel: slc holds every pixel's (vertex, weight bits) pairs of both terms
 // side by side, so all D0 + D1 vertex rows are gathered after one dependent load.  Same
 // arithmetic, in the same order, as k_meanfield.
-template <int R, int D0, int D1, bool CWL>
-__global__ void __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(8)))  // <= 64 VGPRs
-k_meanfield_fused(const float* __restrict__ U, float* __restrict__ Q,
-                                                                int ldq, int N, int L, int S, int per,
-                                                                SliceTable st, const int2* __restrict__ slc,
-                                                                int cwf, int bw) {
+template <int R, int D0, int D1, bool CWL, bool NARROW>
+__global__ void __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(R <= 3 ? 8 : 7)))  // <= 64 (72) VGPRs
+k_meanfield_fused(const float* __restrict__ U, float* __restrict__ Q, int ldq, int N, int L, int S, int per,
+                  SliceTable st, const int2* __restrict__ slc, int cwf, int bw) {
     constexpr int DS = D0 + D1;
     LaneGroup<true, R> G(L, S, per, nullptr);
     const int p = G.item();
     const bool active = G.on && p < N;
     const int k0 = G.k0;
-    const int pc = active ? p : 0;  // idle lanes read pixel 0 (in bounds; results unused)
+    const WavePixels W(G, p, N);
+    const int gp = min(G.g, W.np - 1);  // groups without a pixel repeat the wave's last one
     extern __shared__ __align__(16) int2 pairs_all[];
-    int2* wp = pairs_all + (threadIdx.x >> 6) * (per * DS);
+    const int wpairs = wave_pairs(per, DS);
+    int2* wp = pairs_all + G.w * wpairs;
     // CWL: some Matrix term has an LDS copy of its weights (staging costs a barrier, so
     // it is compiled in only then)
-    float* shc = reinterpret_cast<float*>(pairs_all + (blockDim.x >> 6) * (per * DS));
+    float* shc = reinterpret_cast<float*>(pairs_all + (kWaveBlock / 64) * wpairs);
     // the unary row does not depend on the slice pairs: its load is in flight while they
     // are staged (not at four labels per lane, where the longer-lived row would spill)
     constexpr bool kEarlyU = R <= 3;
     float u[R];
     auto load_u = [&]() {
         if (U) {
-            load_piece<R>(U + (size_t)pc * L, k0, L, u);
+            load_piece<R>(U + (size_t)W.p0 * L + (unsigned)(gp * L + k0), 0, L, u);
         } else {
 #pragma unroll
             for (int r = 0; r < R; r++) u[r] = 0.0f;
@@ -766,30 +775,30 @@ k_meanfield_fused(const float* __restrict__ U, float* __restrict__ Q,
     };
     if (kEarlyU) load_u();
     if (CWL) stage_compat(st, L, shc);
-    stage_wave_pairs<R, DS>(G, p, N, slc, wp);
+    stage_wave_pairs<R, DS>(W, per, slc, wp);
     int2 e[DS];
 #pragma unroll
-    for (int j = 0; j < DS; j++) e[j] = active ? wp[G.g * DS + j] : make_int2(0, 0);
+    for (int j = 0; j < DS; j++) e[j] = wp[gp * DS + j];
     if (!kEarlyU) load_u();
     float x[DS][R];
 #pragma unroll
     for (int j = 0; j < DS; j++) {
         const SliceTerm& T = j < D0 ? st.t[0] : st.t[1];
-        load_piece<R>(T.vals + (size_t)e[j].x * T.ldv, k0, L, x[j]);
+        load_piece<R>(row_piece<NARROW>(T.vals, e[j].x, T.ldv, k0), 0, L, x[j]);
     }
     // CWL: the wave's message rows follow the compat region
-    float* msg = shc + cwf + (size_t)(threadIdx.x >> 6) * (D1 ? 2 : 1) * per * ((L + 3) & ~3);
+    float* msg = shc + cwf + (size_t)G.w * (D1 ? 2 : 1) * per * ((L + 3) & ~3);
     // bw > 0: Q is written in 8 x 8 pixel blocks of an image bw pixels wide (q_block_pos)
-    const int qpos = bw > 0 ? q_block_pos(pc, bw) : p;
-    finish_pixel<R, D0, D1, CWL>(G, st, e, x, u, active, Q + (size_t)qpos * ldq, shc, p, msg);
+    float* qrow = bw > 0 ? Q + (size_t)q_block_pos(W.p0 + gp, bw) * ldq : Q + (size_t)W.p0 * ldq + (unsigned)(gp * ldq);
+    finish_pixel<R, D0, D1, CWL>(G, st, e, x, u, active, qrow, shc, p, msg);
 }
 
 // The adjoint step of k_adjoint (adjoint.hip) over the same interleaved slice pairs:
 // g = sum_k C_k(w_k slice_k(filtered b)), b = sumAndNormalize(Q .* g, Q), dU += b, and
 // the terms' statistic rows (SliceTerm::gstat).  The pairs carry the transposed filter's
 // slice weights.  Same arithmetic, in the same order, as k_adjoint.
-template <int R, int D0, int D1, bool CWL>
-__global__ void __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(8)))
+template <int R, int D0, int D1, bool CWL, bool NARROW>
+__global__ void __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(R <= 3 ? 8 : 7)))
 k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __restrict__ dU, int N, int L, int S,
                 int per, SliceTable st, const int2* __restrict__ slc, int cwf) {
     constexpr int DS = D0 + D1;
@@ -797,29 +806,33 @@ k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __res
     const int p = G.item();
     const bool active = G.on && p < N;
     const int k0 = G.k0;
-    const int pc = active ? p : 0;
+    const WavePixels W(G, p, N);
+    const int gp = min(G.g, W.np - 1);
     extern __shared__ __align__(16) int2 pairs_all[];
-    int2* wp = pairs_all + (threadIdx.x >> 6) * (per * DS);
-    float* shc = reinterpret_cast<float*>(pairs_all + (blockDim.x >> 6) * (per * DS));
+    const int wpairs = wave_pairs(per, DS);
+    int2* wp = pairs_all + G.w * wpairs;
+    float* shc = reinterpret_cast<float*>(pairs_all + (kWaveBlock / 64) * wpairs);
+    const size_t wrow = (size_t)W.p0 * L;              // the wave's rows of Q, b and dU
+    const unsigned grow = (unsigned)(gp * L + k0);     // the lane's piece of them
     float q[R];
-    load_piece<R>(Q + (size_t)pc * L, k0, L, q);  // in flight while the pairs are staged
+    load_piece<R>(Q + wrow + grow, 0, L, q);  // in flight while the pairs are staged
     if (CWL) stage_compat(st, L, shc);
-    stage_wave_pairs<R, DS>(G, p, N, slc, wp);
+    stage_wave_pairs<R, DS>(W, per, slc, wp);
     int2 e[DS];
 #pragma unroll
-    for (int j = 0; j < DS; j++) e[j] = active ? wp[G.g * DS + j] : make_int2(0, 0);
+    for (int j = 0; j < DS; j++) e[j] = wp[gp * DS + j];
     float x[DS][R];
 #pragma unroll
     for (int j = 0; j < DS; j++) {
         const SliceTerm& T = j < D0 ? st.t[0] : st.t[1];
-        load_piece<R>(T.vals + (size_t)e[j].x * T.ldv, k0, L, x[j]);
+        load_piece<R>(row_piece<NARROW>(T.vals, e[j].x, T.ldv, k0), 0, L, x[j]);
     }
     constexpr int NT = D1 ? 2 : 1;
     float raw[NT][R], mk[NT][R], c[NT][R];  // (the adjoint stores no raw messages)
 #pragma unroll
     for (int k = 0; k < NT; k++) term_message<R, D0, D1>(st.t[k], k, e, x, raw[k], mk[k]);
     // statistic region after the message rows (present with a compat region)
-    float* sst = shc + cwf + (cwf ? (blockDim.x >> 6) * NT * per * ((L + 3) & ~3) : 0);
+    float* sst = shc + cwf + (cwf ? (kWaveBlock / 64) * NT * per * ((L + 3) & ~3) : 0);
 #pragma unroll
     for (int k = 0; k < NT; k++)
         if (st.t[k].gslot >= 0) {
@@ -828,7 +841,7 @@ k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __res
             for (int r = 0; r < R; r++) v[r] = active ? raw[k][r] * q[r] : 0.0f;
             stat_put<R>(sst, st.t[k].gslot, v);
         }
-    float* msg = shc + cwf + (size_t)(threadIdx.x >> 6) * NT * per * ((L + 3) & ~3);
+    float* msg = shc + cwf + (size_t)G.w * NT * per * ((L + 3) & ~3);
     compat_terms<R, NT, CWL>(G, st, mk, c, shc, msg);
     float gsum[R];
 #pragma unroll
@@ -841,11 +854,11 @@ k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __res
     sum_normalize<true, R>(q, gsum, bn, G);
     if (active) {
         float du[R];
-        load_piece<R>(dU + (size_t)p * L, k0, L, du);
+        load_piece<R>(dU + wrow + grow, 0, L, du);
 #pragma unroll
         for (int r = 0; r < R; r++) du[r] = du[r] + bn[r];
-        store_piece<R>(b + (size_t)p * L, k0, L, bn);
-        store_piece<R>(dU + (size_t)p * L, k0, L, du);
+        store_piece<R>(b + wrow + grow, 0, L, bn);
+        store_piece<R>(dU + wrow + grow, 0, L, du);
     }
     if (st.nstat) stat_finish<true, R, NT>(st, G, sst);  // uniform condition
 }
@@ -1140,13 +1153,23 @@ void launch_transpose(const float* in, float* out, int rows, int cols, hipStream
     DCRF_HIP_CHECK(hipGetLastError());
 }
 
-void launch_splat(const Chunk* chunks, int n_chunks, const int2* ent, const float* in, int ldi, float* vals,
-                  int ldv, int L, hipStream_t s) {
+// Rows whose offsets row_piece<true> can form: 24-bit row numbers and row sizes, 32-bit
+// byte offsets.
+bool narrow_rows(size_t rows, int ld) {
+    return rows <= ((size_t)1 << 24) && ld < (1 << 22) && rows * (size_t)ld * sizeof(float) <= 0xffffffffull;
+}
+
+void launch_splat(const Chunk* chunks, int n_chunks, const int2* ent, const float* in, size_t rows_in, int ldi,
+                  float* vals, int ldv, int L, hipStream_t s) {
     if (!n_chunks) return;
     const LaunchShape sh = shape_for(L);
     const size_t shm = sh.wave ? (size_t)(kWaveBlock / 64) * (kWin + kBatch) * sizeof(int2) : 0;
-    DCRF_DISPATCH(sh, k_splat, blocks_for(n_chunks, sh.items), shm, s, chunks, n_chunks, ent, in, ldi, vals, ldv, L,
-                  sh.S, sh.per);
+    if (narrow_rows(rows_in, ldi))
+        DCRF_DISPATCH_T(sh, k_splat, true, blocks_for(n_chunks, sh.items), shm, s, chunks, n_chunks, ent, in, ldi, vals,
+                        ldv, L, sh.S, sh.per);
+    else
+        DCRF_DISPATCH_T(sh, k_splat, false, blocks_for(n_chunks, sh.items), shm, s, chunks, n_chunks, ent, in, ldi,
+                        vals, ldv, L, sh.S, sh.per);
 }
 
 size_t tiled_splat_lds(int L, int side, int e_max, int s_max, size_t lds_cap) {
@@ -1258,13 +1281,19 @@ void launch_interleave_slice(const int* vtx, const float* sw, int N, int d1, int
 // and the adjoint's statistic region (stat_lds_floats)
 inline size_t fused_lds_bytes(const LaunchShape& sh, int ds, int nt, int L, int cwf, int nstat = 0) {
     const size_t waves = kWaveBlock / 64;
-    return waves * sh.per * ds * sizeof(int2) + (size_t)cwf * sizeof(float) +
+    return waves * wave_pairs(sh.per, ds) * sizeof(int2) + (size_t)cwf * sizeof(float) +
            (cwf ? waves * nt * sh.per * (size_t)((L + 3) & ~3) * sizeof(float) : 0) +
            stat_lds_floats(true, nstat, L, kWaveBlock, sh.R) * sizeof(float);
 }
 
+// One of a fused kernel's four forms: with or without the LDS copy of Matrix weights, with
+// 24-bit or 64-bit row offsets.
+#define DCRF_FUSED_FORM(kernel, R_, D0_, D1_)                                              \
+    (cwf ? (narrow ? kernel<R_, D0_, D1_, true, true> : kernel<R_, D0_, D1_, true, false>) \
+         : (narrow ? kernel<R_, D0_, D1_, false, true> : kernel<R_, D0_, D1_, false, false>))
+
 #define DCRF_FUSED(R_, D0_, D1_)                                                                          \
-    (cwf ? k_meanfield_fused<R_, D0_, D1_, true> : k_meanfield_fused<R_, D0_, D1_, false>)<<<                 \
+    DCRF_FUSED_FORM(k_meanfield_fused, R_, D0_, D1_)<<<                                                     \
         blocks_for(N, sh.items), kWaveBlock, fused_lds_bytes(sh, D0_ + D1_, D1_ ? 2 : 1, L, cwf), s>>>(       \
         U, Q, ldq, N, L, sh.S, sh.per, st, slc, cwf, bw)
 
@@ -1272,6 +1301,7 @@ template <int R>
 void launch_fused_r(const LaunchShape& sh, const float* U, float* Q, int ldq, int N, int L, const SliceTable& st,
                     const int2* slc, int cwf, int bw, hipStream_t s) {
     const int a = st.t[0].d1, b = st.nterms > 1 ? st.t[1].d1 : 0;
+    const bool narrow = narrow_rows(st.rows, st.t[0].ldv);
     if (a == 3 && b == 0) DCRF_FUSED(R, 3, 0);
     else if (a == 6 && b == 0) DCRF_FUSED(R, 6, 0);
     else if (a == 3 && b == 6) DCRF_FUSED(R, 3, 6);
@@ -1282,7 +1312,7 @@ void launch_fused_r(const LaunchShape& sh, const float* U, float* Q, int ldq, in
 #undef DCRF_FUSED
 
 #define DCRF_ADJ_FUSED(R_, D0_, D1_)                                                                      \
-    (cwf ? k_adjoint_fused<R_, D0_, D1_, true> : k_adjoint_fused<R_, D0_, D1_, false>)<<<                   \
+    DCRF_FUSED_FORM(k_adjoint_fused, R_, D0_, D1_)<<<                                                       \
         blocks_for(N, sh.items), kWaveBlock, fused_lds_bytes(sh, D0_ + D1_, D1_ ? 2 : 1, L, cwf, st.nstat),  \
         s>>>(Q, b, dU, N, L, sh.S, sh.per, st, slc, cwf)
 
@@ -1290,6 +1320,7 @@ template <int R>
 void launch_adj_fused_r(const LaunchShape& sh, const float* Q, float* b, float* dU, int N, int L,
                         const SliceTable& st, const int2* slc, int cwf, hipStream_t s) {
     const int a = st.t[0].d1, c = st.nterms > 1 ? st.t[1].d1 : 0;
+    const bool narrow = narrow_rows(st.rows, st.t[0].ldv);
     if (a == 3 && c == 0) DCRF_ADJ_FUSED(R, 3, 0);
     else if (a == 6 && c == 0) DCRF_ADJ_FUSED(R, 6, 0);
     else if (a == 3 && c == 6) DCRF_ADJ_FUSED(R, 3, 6);
@@ -1298,6 +1329,7 @@ void launch_adj_fused_r(const LaunchShape& sh, const float* Q, float* b, float* 
     DCRF_HIP_CHECK(hipGetLastError());
 }
 #undef DCRF_ADJ_FUSED
+#undef DCRF_FUSED_FORM
 
 #define DCRF_RUNS(R_, D0_, D1_)                                                                           \
     k_meanfield_runs<R_, D0_, D1_><<<rs.n_runs, kWaveBlock, lds, s>>>(U, Q, N, L, sh.S, sh.per, st, rs)
