@@ -31,7 +31,7 @@ inline unsigned blocks_for(size_t n, int t = kThreads) { return (unsigned)((n + 
 template <bool WAVE, int R>
 __global__ void __launch_bounds__(1024) k_sn_first(const float* __restrict__ Q, const float* __restrict__ dQ,
                                                    float* __restrict__ b, float* __restrict__ dU, int N, int L,
-                                                   int S, int per) {
+                                                   int Lv, int S, int per) {
     extern __shared__ float sh[];
     LaneGroup<WAVE, R> G(L, S, per, sh);
     const int p = G.item();
@@ -43,13 +43,13 @@ __global__ void __launch_bounds__(1024) k_sn_first(const float* __restrict__ Q, 
         gv[r] = 0.0f;
     }
     if (active) {
-        load_piece<R>(Q + (size_t)p * L, G.k0, L, q);
-        load_piece<R>(dQ + (size_t)p * L, G.k0, L, gv);
+        load_row(Q + (size_t)p * L, G, q);
+        load_row(dQ + (size_t)p * L, G, gv);
     }
     sum_normalize<WAVE, R>(q, gv, bn, G);
     if (active) {
-        store_piece<R>(b + (size_t)p * L, G.k0, L, bn);
-        store_piece<R>(dU + (size_t)p * L, G.k0, L, bn);
+        store_piece<R>(b + (size_t)p * Lv, G.k0, L, bn);
+        store_row(dU + (size_t)p * L, G, bn);
     }
 }
 
@@ -59,7 +59,7 @@ __global__ void __launch_bounds__(1024) k_sn_first(const float* __restrict__ Q, 
 // the compatibility gradient's statistic, with no message cache.
 template <bool WAVE, int R, bool CWL>
 __global__ void __launch_bounds__(1024) k_adjoint(const float* __restrict__ Q, float* __restrict__ b,
-                                                  float* __restrict__ dU, int N, int L, int S, int per,
+                                                  float* __restrict__ dU, int N, int L, int Lv, int S, int per,
                                                   SliceTable st, int cwf) {
     extern __shared__ float sh[];
     float* shc = sh + blockDim.x;
@@ -72,7 +72,7 @@ __global__ void __launch_bounds__(1024) k_adjoint(const float* __restrict__ Q, f
     float q[R];
 #pragma unroll
     for (int r = 0; r < R; r++) q[r] = 0.0f;
-    if (active) load_piece<R>(Q + (size_t)p * L, k0, L, q);
+    if (active) load_piece<R>(Q + (size_t)p * Lv, k0, L, q);
     float gsum[R];
 #pragma unroll
     for (int r = 0; r < R; r++) gsum[r] = 0.0f;
@@ -107,11 +107,11 @@ __global__ void __launch_bounds__(1024) k_adjoint(const float* __restrict__ Q, f
     sum_normalize<WAVE, R>(q, gsum, bn, G);
     if (active) {
         float du[R];
-        load_piece<R>(dU + (size_t)p * L, k0, L, du);
+        load_row(dU + (size_t)p * L, G, du);
 #pragma unroll
         for (int r = 0; r < R; r++) du[r] = du[r] + bn[r];
-        store_piece<R>(b + (size_t)p * L, k0, L, bn);
-        store_piece<R>(dU + (size_t)p * L, k0, L, du);
+        store_piece<R>(b + (size_t)p * Lv, k0, L, bn);
+        store_row(dU + (size_t)p * L, G, du);
     }
     if (st.nstat) stat_finish<WAVE, R>(st, G, sst);  // uniform condition
 }
@@ -126,8 +126,8 @@ __global__ void __launch_bounds__(1024) k_adjoint(const float* __restrict__ Q, f
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 constexpr int kMfmaBatch = 8;
 
-__global__ void __launch_bounds__(256) k_grad_mfma(const float* __restrict__ b, const float* __restrict__ M, int N,
-                                                   int L, int tiles1, int ppw, int ranges, size_t bstride,
+__global__ void __launch_bounds__(256) k_grad_mfma(const float* __restrict__ b, int ldb,
+                                                   const float* __restrict__ M, int N, int L, int tiles1, int ppw, int ranges, size_t bstride,
                                                    size_t mstride, int n_waves, float* __restrict__ partial) {
     const int w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     if (w >= n_waves) return;  // whole waves only; no barrier in this kernel
@@ -152,7 +152,7 @@ __global__ void __launch_bounds__(256) k_grad_mfma(const float* __restrict__ b, 
         for (int u = 0; u < kMfmaBatch; u++) {
             const int pp = p + 2 * u + k;
             const int pc = min(pp, p1 - 1);
-            av[u] = b[(size_t)pc * L + ac];
+            av[u] = b[(size_t)pc * ldb + ac];
             bv[u] = M[(size_t)pc * L + cc];
         }
 #pragma unroll
@@ -290,23 +290,24 @@ __global__ void k_set_compat(const float* __restrict__ raw, int ckind, int L, fl
 
 }  // namespace
 
-void launch_sn_first(const float* Q, const float* dQ, float* b, float* dU, int N, int L, hipStream_t s) {
-    const LaunchShape sh = shape_for(L);
-    DCRF_DISPATCH(sh, k_sn_first, blocks_for(N, sh.items), sizeof(float) * sh.block, s, Q, dQ, b, dU, N, L, sh.S,
+void launch_sn_first(const float* Q, const float* dQ, float* b, float* dU, int N, int L, int Lv, hipStream_t s) {
+    const LaunchShape sh = shape_for(Lv);
+    DCRF_DISPATCH(sh, k_sn_first, blocks_for(N, sh.items), sizeof(float) * sh.block, s, Q, dQ, b, dU, N, L, Lv, sh.S,
                   sh.per);
 }
 
-void launch_adjoint(const float* Q, float* b, float* dU, int N, int L, const SliceTable& st_in, hipStream_t s) {
+void launch_adjoint(const float* Q, float* b, float* dU, int N, int L, int Lv, const SliceTable& st_in, hipStream_t s) {
     SliceTable st = st_in;
     const int cwf = assign_compat_lds(st, L);
-    const LaunchShape sh = shape_for(L);
+    const LaunchShape sh = shape_for(Lv);
     const size_t lds =
         sizeof(float) * ((size_t)sh.block + cwf + stat_lds_floats(sh.wave, st.nstat, L, sh.block, sh.R));
-    DCRF_DISPATCH_CWL(sh, cwf, k_adjoint, blocks_for(N, sh.items), lds, s, Q, b, dU, N, L, sh.S, sh.per, st, cwf);
+    DCRF_DISPATCH_CWL(sh, cwf, k_adjoint, blocks_for(N, sh.items), lds, s, Q, b, dU, N, L, Lv, sh.S, sh.per, st,
+                      cwf);
 }
 
-int adjoint_blocks(int N, int L) {
-    const LaunchShape sh = shape_for(L);
+int adjoint_blocks(int N, int Lv) {
+    const LaunchShape sh = shape_for(Lv);
     return (int)blocks_for(N, sh.items);
 }
 
@@ -346,7 +347,7 @@ void launch_sum_rows(const float* part, long long rows, int cols, double* mid, d
     DCRF_HIP_CHECK(hipGetLastError());
 }
 
-void launch_grad_stat(const float* b, size_t bstride, const float* M, size_t mstride, int iters, int N, int L,
+void launch_grad_stat(const float* b, int ldb, size_t bstride, const float* M, size_t mstride, int iters, int N, int L,
                       float* partial, double* mid, double* acc, hipStream_t s) {
     if (iters < 1) return;
     int ppw;
@@ -356,7 +357,7 @@ void launch_grad_stat(const float* b, size_t bstride, const float* M, size_t mst
     const long long waves = (long long)iters * ranges * tiles1 * tiles1;
     if (waves > 0x7fffffffll / 64 || (long long)iters * ranges > 0x7fffffffll)
         throw Error{DCRF_ERR_VALUE, "gradient statistic too large"};
-    k_grad_mfma<<<(unsigned)((waves + 3) / 4), 256, 0, s>>>(b, M, N, L, tiles1, ppw, (int)ranges, bstride, mstride,
+    k_grad_mfma<<<(unsigned)((waves + 3) / 4), 256, 0, s>>>(b, ldb, M, N, L, tiles1, ppw, (int)ranges, bstride, mstride,
                                                             (int)waves, partial);
     DCRF_HIP_CHECK(hipGetLastError());
     launch_sum_rows(partial, (long long)iters * ranges, L * L, mid, acc, s);

@@ -306,7 +306,7 @@ struct dcrf_model {
     std::vector<std::unique_ptr<Term>> terms;
     DevBuf<float> Q, work, tmp1, tmp2, stage;
     DevBuf<float> Qp;  // inference iterate with the vertex-row stride (see run_inference)
-    int ldv = 0;       // row stride (floats) of the vertex rows: L rounded to a cache line
+    int ldv = 0;       // row stride (floats) of the vertex rows and Qp: padded_labels(L), or L
     float hash_load = 0.5f;
     int splat_chunk = 0;  // 0: default
     int tile_side = 0;  // 0: default_tile_side(L)
@@ -636,7 +636,7 @@ void compute_norm(dcrf_model& m, Term& t) {
     st.nterms = 1;
     st.t[0] = SliceTerm{gv.get(), sw.get(), bufs[d1 & 1], d1, -1, nullptr, nullptr, nullptr, 1};
     t.norm.reserve(N);
-    launch_slice_term(t.norm.get(), N, 1, st, 0, s);
+    launch_slice_term(t.norm.get(), N, 1, 1, st, 0, s);
     if (t.ntype == DCRF_NO_NORMALIZATION) {
         // mean_norm = N / sum(norm) per instance, in float (pairwise.cpp:46-53)
         std::vector<float> h(N);
@@ -953,7 +953,7 @@ void kernel_grad_group(dcrf_model& m, const KgPlan& P, const float* b, const flo
         SliceTable st{};
         st.nterms = 1;
         st.t[0] = SliceTerm{nullptr, nullptr, nullptr, 1, t.ckind, t.d_compat.get(), kw ? kw + k : nullptr, nullptr, L};
-        launch_kg_prepare(Qt, b, t.norm.get(), N, L, st, t.ntype, need_fa ? lbl + i * NL : nullptr,
+        launch_kg_prepare(Qt, b, m.ldv, t.norm.get(), N, L, st, t.ntype, need_fa ? lbl + i * NL : nullptr,
                           pk + (size_t)i * 2 * NL, s);
     }
     launch_splat(P.ch2.get(), P.nch, P.ent.get(), pk, (size_t)T * N, L2, P.S2.get(), L2, L2, s);
@@ -979,7 +979,7 @@ void kernel_grad_group(dcrf_model& m, const KgPlan& P, const float* b, const flo
             const int d1 = t.lat.d + 1;
             st.t[0] = SliceTerm{vtx, sw, need_fa ? rev_of(i) : nullptr, d1, -1, nullptr, nullptr, nullptr, L2};  // K^T a
             st.t[1] = SliceTerm{vtx, sw, need_fb ? fwd_of(i) + L : nullptr, d1, -1, nullptr, nullptr, nullptr, L2};  // K c
-            launch_kg_x(b, lbl + (size_t)i * NL, t.norm.get(), N, L, st, t.ntype, x, s);
+            launch_kg_x(b, m.ldv, lbl + (size_t)i * NL, t.norm.get(), N, L, st, t.ntype, x, s);
         }
         launch_splat(P.ch1.get(), P.nch, P.ent.get(), xb, (size_t)T * N, L, P.S1.get(), L, L, s);
         launch_combine(P.cb1.get(), P.ncb, P.S1.get(), L, L, s);
@@ -1138,7 +1138,6 @@ void ensure_layout(dcrf_model& m) {
     // Segments and entries, tile by tile, the terms in layout order inside a tile: tile
     // t's entries of term k (sorted positions tile_ptr[t] ..) move to ebase[k][t] + j.
     const int NT = m.tiles.n_tiles();
-    const LaunchShape csh = shape_for(L);
     // the LDS-tiled splat (small tiles only) if the largest tile's entries and segments fit
     int e_max = 0, s_max = 0;
     for (int t = 0; t < NT; t++) {
@@ -1164,6 +1163,9 @@ void ensure_layout(dcrf_model& m) {
     // empty segments of vertices that only padding lanes touch go to waves of their own
     // at the end.  An instance of a batch then gets the bits of the same image alone.
     // Block-mode shapes and the tiled splat keep one row per segment.
+    // (the LDS-tiled splat stages unpadded rows)
+    m.ldv = m.tiled ? L : padded_labels(L);
+    const LaunchShape csh = shape_for(m.ldv);
     const bool runs = csh.wave && !m.tiled;
     const int per = csh.per;
     std::vector<Chunk>& gch = m.gch_scratch;  // (capacity kept between layout builds)
@@ -1295,9 +1297,6 @@ void ensure_layout(dcrf_model& m) {
     upload(m.g_comb2, gcb2, s);
     m.tsplat = TiledSplat{m.g_chunks.get(), m.g_tile_seg.get(), m.g_tile_e.get(), NT, tg, e_max, s_max};
 
-    // vertex rows packed (stride L): rows padded to start cache lines (32 floats at
-    // L = 21, for Q between iterations too) measured 8 % slower per step at 1024x768x21
-    m.ldv = L;
     m.vals[0].reserve((size_t)m.rows0 * m.ldv);
     m.vals[1].reserve((size_t)(V + 1) * m.ldv);
     launch_fill(m.vals[0].get(), 0.f, (size_t)m.rows0 * m.ldv, s);
@@ -1368,11 +1367,10 @@ void ensure_layout(dcrf_model& m) {
             // rectangles of 2 waves' pixels per row x 16 rows (18 x 16 at 21 labels)
             // rectangles two waves of pixels wide, at most run_rows high and at most
             // 24 KiB of slice pairs
-            const LaunchShape shp = shape_for(L);
-            const int TW = 2 * shp.per;
+            const int TW = 2 * shape_for(L).per;
             const int TH = std::max(1, std::min(m.run_rows, (24 * 1024) / (TW * ds * 8)));
             build_run_slice(m.geo, m.geod, m.g_slc.get(), ds, par, TW, TH, m.rslice, s);
-            m.rows_lds = (m.rslice.u_max * L + 1) & ~1;
+            m.rows_lds = (m.rslice.u_max * m.ldv + 1) & ~1;
             SliceTable probe = slice_table(m, false);
             const int cwf = assign_compat_lds(probe, L);
             const size_t lds = meanfield_runs_lds(L, ds, m.rslice.P, m.rows_lds, cwf);
@@ -1446,27 +1444,25 @@ size_t in_rows(const dcrf_model& m, const int2* ent_in) {
     return ent_in ? q_block_rows(m.geo.W[0], m.geo.H[0]) : (size_t)m.N();
 }
 
-// in: the [N] input rows with row stride ldi (floats).
-void run_filter(dcrf_model& m, const float* in, int ldi, bool transpose, hipStream_t s,
-                const int2* ent_in = nullptr) {
-    const int L = m.L;
+// in: the [N] input rows with row stride m.ldv (floats).
+void run_filter(dcrf_model& m, const float* in, bool transpose, hipStream_t s, const int2* ent_in = nullptr) {
+    const int L = m.L, Lv = m.ldv;  // the filter works on whole rows, padding labels included
     const int2* ent = ent_in ? ent_in : ((transpose && !m.all_symmetric) ? m.g_entT.get() : m.g_entF.get());
     {
         Timed t(m, s, KC_SPLAT, splat_bytes(m));
         if (m.tiled)
-            launch_splat_tiled(m.tsplat, ent, in, m.vals[0].get(), m.ldv, L, m.lds_cap, s);  // ldi == L
+            launch_splat_tiled(m.tsplat, ent, in, m.vals[0].get(), m.ldv, L, m.lds_cap, s);  // ldv == L
         else
-            launch_splat(m.g_chunks.get(), m.C_total, ent, in, in_rows(m, ent_in), ldi,
-                         m.vals[0].get(), m.ldv, L, s);
+            launch_splat(m.g_chunks.get(), m.C_total, ent, in, in_rows(m, ent_in), Lv, m.vals[0].get(), Lv, Lv, s);
         t.done();
     }
     if (m.CB_total) {
         Timed t(m, s, KC_COMBINE, 0.0);
         if (m.comb_waves)
-            launch_combine_waves(m.g_comb.get(), m.CB_total, m.vals[0].get(), m.ldv, L, s);
+            launch_combine_waves(m.g_comb.get(), m.CB_total, m.vals[0].get(), Lv, Lv, s);
         else
-            launch_combine(m.g_comb.get(), m.CB_total, m.vals[0].get(), m.ldv, L, s);
-        if (m.CB2_total) launch_combine(m.g_comb2.get(), m.CB2_total, m.vals[0].get(), m.ldv, L, s);
+            launch_combine(m.g_comb.get(), m.CB_total, m.vals[0].get(), Lv, Lv, s);
+        if (m.CB2_total) launch_combine(m.g_comb2.get(), m.CB2_total, m.vals[0].get(), Lv, Lv, s);
         t.done();
     }
     if (m.pairs) {
@@ -1490,7 +1486,7 @@ void run_filter(dcrf_model& m, const float* in, int ldi, bool transpose, hipStre
             }
             Timed t(m, s, KC_BLUR, bytes);
             const int pr = m.blur_r > 0 && (m.blur_small_v <= 0 || m.prefixP[p] < m.blur_small_v) ? m.blur_r : 0;
-            launch_blur_pass(m.vals[p & 1].get(), m.vals[(p + 1) & 1].get(), 0, m.prefixP[p], m.ldv, L, pt, s, pr);
+            launch_blur_pass(m.vals[p & 1].get(), m.vals[(p + 1) & 1].get(), 0, m.prefixP[p], Lv, Lv, pt, s, pr);
             t.done();
         }
         return;
@@ -1498,7 +1494,7 @@ void run_filter(dcrf_model& m, const float* in, int ldi, bool transpose, hipStre
     const BlurTable bt = blur_table(m);
     for (int step = 0; step <= m.max_d; step++) {
         Timed t(m, s, KC_BLUR, (double)m.prefixV[step] * (2.0 * L * 4 + 8));
-        launch_blur(m.vals[step & 1].get(), m.vals[(step + 1) & 1].get(), 0, m.prefixV[step], m.ldv, L, bt, step,
+        launch_blur(m.vals[step & 1].get(), m.vals[(step + 1) & 1].get(), 0, m.prefixV[step], Lv, Lv, bt, step,
                     transpose ? 1 : 0, s);
         t.done();
     }
@@ -1510,50 +1506,59 @@ void prepare(dcrf_model& m) {
     ensure_layout(m);
     const size_t n = (size_t)m.N() * m.L;
     m.Q.reserve(n);
-    if (m.fused && m.ldv != m.L) m.Qp.reserve((size_t)m.N() * m.ldv);  // before any graph capture
-    if (m.qblocks && !m.qblocks_ready && m.fused && !m.runs && !m.tiled && m.ldv == m.L && m.geo.is2d &&
+    if (m.ldv != m.L) m.Qp.reserve((size_t)m.N() * m.ldv);  // before any graph capture
+    if (m.qblocks && !m.qblocks_ready && m.fused && !m.runs && !m.tiled && m.geo.is2d &&
         m.geo.n_inst == 1) {
         m.g_entB.reserve(m.E_total);
         launch_entry_block(m.g_entF.get(), (size_t)m.E_total, m.geo.W[0], m.g_entB.get(), m.stream);
-        m.Qb.reserve(q_block_rows(m.geo.W[0], m.geo.H[0]) * m.L);
+        m.Qb.reserve(q_block_rows(m.geo.W[0], m.geo.H[0]) * m.ldv);
         DCRF_HIP_CHECK(hipStreamSynchronize(m.stream));
         m.qblocks_ready = true;
     }
 }
 
-// With the fused kernel (and the global splat), the iterations between the first and
-// the last keep Q in m.Qp with the vertex-row stride: every row the splat gathers then
-// starts a cache line.  The first splat reads the caller's Q, the last update writes it.
-void run_inference(dcrf_model& m, int n_iter, const float* U, float* Q, hipStream_t s, bool allow_pad = true) {
-    const int L = m.L, N = m.N();
-    launch_softmax_neg(U, Q, N, L, s);
+// Splat input rows from rows in the caller's layout ([N][L]): themselves, or m.Qp with the
+// padding labels added.
+const float* splat_rows(dcrf_model& m, const float* Q, hipStream_t s) {
+    if (m.ldv == m.L) return Q;
+    launch_pad_rows(Q, m.Qp.get(), m.N(), m.L, m.ldv, s);
+    return m.Qp.get();
+}
+
+// Q between the iterations has rows of ldv floats: where those are padded it stays in m.Qp
+// and only the last update writes the caller's Q.
+void run_inference(dcrf_model& m, int n_iter, const float* U, float* Q, hipStream_t s) {
+    const int L = m.L, N = m.N(), Lv = m.ldv;
+    float* Qi = Lv != L && n_iter > 0 ? m.Qp.get() : Q;
+    launch_softmax_neg(U, Qi, Qi == Q ? L : Lv, N, L, Lv, s);
     const SliceTable st = slice_table(m, false, m.kw_set ? m.kw.get() : nullptr);
-    const bool pad = allow_pad && m.fused && !m.runs && !m.tiled && n_iter > 1 && m.ldv != L && m.Qp.get();
-    // Q in 8 x 8 blocks between iterations: the first splat reads the caller's Q, the
+    // Q in 8 x 8 blocks between iterations: the first splat reads Q_0 in pixel order, the
     // later ones m.Qb through the block-position entries; the last update writes Q
-    const bool blk = !pad && m.qblocks_ready && n_iter > 1 && m.fused && !m.runs && !m.tiled;
+    const bool blk = m.qblocks_ready && n_iter > 1 && m.fused && !m.runs && !m.tiled;
     for (int it = 0; it < n_iter; it++) {
+        const bool last = it + 1 == n_iter;
         if (blk) {
-            run_filter(m, it > 0 ? m.Qb.get() : Q, L, false, s, it > 0 ? m.g_entB.get() : nullptr);
+            run_filter(m, it > 0 ? m.Qb.get() : Qi, false, s, it > 0 ? m.g_entB.get() : nullptr);
             Timed t(m, s, KC_MEANFIELD, meanfield_bytes(m));
-            const bool last = it + 1 == n_iter;
-            launch_meanfield_fused(U, last ? Q : m.Qb.get(), L, N, L, st, m.g_slc.get(), s, last ? 0 : m.geo.W[0]);
+            launch_meanfield_fused(U, last ? Q : m.Qb.get(), last ? L : Lv, N, L, Lv, st, m.g_slc.get(), s,
+                                   last ? 0 : m.geo.W[0]);
             t.done();
             continue;
         }
-        const bool in_p = pad && it > 0, out_p = pad && it + 1 < n_iter;
-        run_filter(m, in_p ? m.Qp.get() : Q, in_p ? m.ldv : L, false, s);
+        run_filter(m, Qi, false, s);
+        float* Qo = last ? Q : Qi;
+        const int ldo = last ? L : Lv;
         Timed t(m, s, KC_MEANFIELD, meanfield_bytes(m));
         if (m.runs)
-            launch_meanfield_runs(U, Q, m.N(), m.L, st,
+            launch_meanfield_runs(U, Qo, ldo, N, L, Lv, st,
                                   RunSliceDev{m.rslice.P, m.rslice.n_runs, m.rows_lds, m.rslice.base.get(),
                                               m.rslice.rows.get(), m.rslice.pix_base.get(), m.rslice.rpix.get(),
                                               m.rslice.loc.get(), m.vals[0].get(), m.vals[1].get()},
                                   s);
         else if (m.fused)
-            launch_meanfield_fused(U, out_p ? m.Qp.get() : Q, out_p ? m.ldv : L, N, L, st, m.g_slc.get(), s);
+            launch_meanfield_fused(U, Qo, ldo, N, L, Lv, st, m.g_slc.get(), s);
         else
-            launch_meanfield(U, Q, m.N(), m.L, st, nullptr, nullptr, s);
+            launch_meanfield(U, Qo, ldo, N, L, Lv, st, nullptr, nullptr, s);
         t.done();
     }
 }
@@ -1568,7 +1573,8 @@ int matrix_terms(const dcrf_model& m) {
 void forward_train(dcrf_model& m, int n_iter, const float* U, const float* compat_raw, const float* kw,
                    hipStream_t s) {
     const int N = m.N(), L = m.L, T = (int)m.terms.size();
-    const size_t NL = (size_t)N * L;
+    const int Lv = m.ldv;
+    const size_t NL = (size_t)N * L, NLv = (size_t)N * Lv;  // Q_t (t < n): rows of ldv floats; Q_n: of L
     if (compat_raw) {
         size_t off = 0;
         for (auto& t : m.terms) {
@@ -1576,24 +1582,25 @@ void forward_train(dcrf_model& m, int n_iter, const float* U, const float* compa
             off += compat_raw_len(t->ckind, L);
         }
     }
-    m.qcache.reserve((size_t)(n_iter + 1) * NL);
+    m.qcache.reserve((size_t)n_iter * NLv + NL);
     // raw messages of the Matrix terms only (their statistic is a full L x L product
     // taken after the adjoint loop); the others' statistic comes from the adjoint kernels
     const int nm = matrix_terms(m);
     m.mcache.reserve(std::max<size_t>((size_t)n_iter * nm * NL, 1));
-    launch_softmax_neg(U, m.qcache.get(), N, L, s);
+    launch_softmax_neg(U, m.qcache.get(), n_iter ? Lv : L, N, L, Lv, s);
     for (int it = 0; it < n_iter; it++) {
-        const float* Qt = m.qcache.get() + (size_t)it * NL;
-        float* Qn = m.qcache.get() + (size_t)(it + 1) * NL;
-        run_filter(m, Qt, L, false, s);
+        const float* Qt = m.qcache.get() + (size_t)it * NLv;
+        float* Qn = m.qcache.get() + (size_t)(it + 1) * NLv;
+        const int ldn = it + 1 < n_iter ? Lv : L;
+        run_filter(m, Qt, false, s);
         SliceTable st = slice_table(m, false, kw);
         for (int k = 0, j = 0; k < T; k++)
             if (m.terms[k]->ckind == DCRF_COMPAT_MATRIX)
                 st.t[k].mout = m.mcache.get() + ((size_t)it * nm + j++) * NL;
         if (m.fused)  // same arithmetic as k_meanfield, gathers of all entries up front
-            launch_meanfield_fused(U, Qn, L, N, L, st, m.g_slc.get(), s);
+            launch_meanfield_fused(U, Qn, ldn, N, L, Lv, st, m.g_slc.get(), s);
         else
-            launch_meanfield(U, Qn, N, L, st, nullptr, nullptr, s);
+            launch_meanfield(U, Qn, ldn, N, L, Lv, st, nullptr, nullptr, s);
     }
     m.train_n = n_iter;
     m.train_kw = kw;
@@ -1626,16 +1633,16 @@ const int2* adjoint_pairs(dcrf_model& m, hipStream_t s) {
 void backward(dcrf_model& m, const float* dQ, float* dU, float* dcompat, float* dkw, hipStream_t s,
               bool kernel = false) {
     if (m.train_n < 0) throw Error{DCRF_ERR_STATE, "backward needs a preceding training forward"};
-    const int N = m.N(), L = m.L, T = (int)m.terms.size(), n = m.train_n;
-    const size_t NL = (size_t)N * L;
+    const int N = m.N(), L = m.L, Lv = m.ldv, T = (int)m.terms.size(), n = m.train_n;
+    const size_t NL = (size_t)N * L, NLv = (size_t)N * Lv;
     // b_t, the adjoint entering reverse iteration t - 1, in slot t (t = n .. 0).  The
     // Matrix terms' statistic reads every b_t after the loop, so with such a term every
     // slot stays; otherwise two slots alternate.
     const int nm = matrix_terms(m);
-    m.bbuf.reserve((size_t)(nm ? n + 1 : std::min(n + 1, 2)) * NL);
-    auto bslot = [&](int t) { return m.bbuf.get() + (size_t)(nm ? t : (t & 1)) * NL; };
+    m.bbuf.reserve((size_t)(nm ? n + 1 : std::min(n + 1, 2)) * NLv);
+    auto bslot = [&](int t) { return m.bbuf.get() + (size_t)(nm ? t : (t & 1)) * NLv; };
     const float* Qc = m.qcache.get();
-    launch_sn_first(Qc + (size_t)n * NL, dQ, bslot(n), dU, N, L, s);
+    launch_sn_first(Qc + (size_t)n * NLv, dQ, bslot(n), dU, N, L, Lv, s);
     std::vector<size_t> goff(T + 1, 0);
     for (int k = 0; k < T; k++) goff[k + 1] = goff[k] + stat_len(m.terms[k]->ckind, L);
     m.gacc.reserve(std::max<size_t>(goff[T], 1));
@@ -1643,7 +1650,7 @@ void backward(dcrf_model& m, const float* dQ, float* dU, float* dcompat, float* 
     // the other terms' statistic rows: term j (in term order among them), iteration it
     // at partial + (j * n + it) * nblk * L, one row of L sums per adjoint block
     const int nd = T - nm;
-    const size_t nblk = (size_t)adjoint_blocks(N, L);
+    const size_t nblk = (size_t)adjoint_blocks(N, Lv);
     size_t pf = std::max<size_t>((size_t)nd * n * nblk * L, 1);
     if (nm) pf = std::max(pf, grad_partial_floats(N, L, n));
     m.partial.reserve(pf);
@@ -1678,9 +1685,9 @@ void backward(dcrf_model& m, const float* dQ, float* dU, float* dcompat, float* 
             // DenseCRF::gradient takes the kernel gradient with b before its update
             // (densecrf.cpp:280-284)
             for (const auto& P : m.kgplans)
-                kernel_grad_group(m, *P, b, Qc + (size_t)it * NL, m.train_kw, koff, pstride, s);
+                kernel_grad_group(m, *P, b, Qc + (size_t)it * NLv, m.train_kw, koff, pstride, s);
         }
-        run_filter(m, b, L, true, s);
+        run_filter(m, b, true, s);
         SliceTable st = slice_table(m, true, m.train_kw);
         for (int k = 0, j = 0; k < T; k++)
             if (m.terms[k]->ckind != DCRF_COMPAT_MATRIX) {
@@ -1689,9 +1696,9 @@ void backward(dcrf_model& m, const float* dQ, float* dU, float* dcompat, float* 
                 st.nstat = j;
             }
         if (m.fused)
-            launch_adjoint_fused(Qc + (size_t)it * NL, bslot(it), dU, N, L, st, adjoint_pairs(m, s), s);
+            launch_adjoint_fused(Qc + (size_t)it * NLv, bslot(it), dU, N, L, Lv, st, adjoint_pairs(m, s), s);
         else
-            launch_adjoint(Qc + (size_t)it * NL, bslot(it), dU, N, L, st, s);
+            launch_adjoint(Qc + (size_t)it * NLv, bslot(it), dU, N, L, Lv, st, s);
     }
     if (kernel)  // the one-pass kernel gradient's partial rows hold all iterations
         for (int k = 0; k < T; k++)
@@ -1710,7 +1717,7 @@ void backward(dcrf_model& m, const float* dQ, float* dU, float* dcompat, float* 
         }
     for (int k = 0, j = 0; k < T; k++)
         if (m.terms[k]->ckind == DCRF_COMPAT_MATRIX) {
-            launch_grad_stat(bslot(1), NL, m.mcache.get() + (size_t)j * NL, (size_t)nm * NL, n, N, L,
+            launch_grad_stat(bslot(1), Lv, NLv, m.mcache.get() + (size_t)j * NL, (size_t)nm * NL, n, N, L,
                              m.partial.get(), m.rmid.get(), m.gacc.get() + goff[k], s);
             j++;
         }
@@ -1775,7 +1782,10 @@ double objective_value(int kind, const std::vector<double>& OP, int L) {
 // device array per GPU instead of the model's buffers.  Host code must not use the
 // array's name as an address: the address comes from hipGetSymbolAddress, once per
 // device, and is kept in scratch_dev.
-constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;
+// The limit counts rows of L floats; the array holds them padded (at most 8 floats for 5
+// labels) and the second buffer's alignment.
+constexpr size_t kNoAllocRowBytes = (size_t)64 << 20;
+constexpr size_t kNoAllocScratchBytes = kNoAllocRowBytes / 5 * 8 + 4096;
 constexpr int kMaxDevices = 64;
 static __device__ __align__(256) float scratch[kNoAllocScratchBytes / sizeof(float)];
 float* scratch_dev[kMaxDevices] = {};
@@ -2164,10 +2174,11 @@ int dcrf_inference_device_noalloc(dcrf_model* m, int n_iter, const float* U_dev,
         const size_t n0 = (size_t)m->rows0 * m->ldv, n1 = (size_t)(m->V_total + 1) * m->ldv;
         const size_t off1 = (n0 + 63) / 64 * 64;  // second buffer 256-byte aligned
         const size_t need = off1 + n1;
-        if (need > kNoAllocScratchBytes / sizeof(float))
-            throw Error{DCRF_ERR_VALUE, "the model needs " + std::to_string(need * sizeof(float)) +
+        const size_t unpadded = ((size_t)m->rows0 + m->V_total + 1) * m->L * sizeof(float);
+        if (unpadded > kNoAllocRowBytes || need > kNoAllocScratchBytes / sizeof(float))
+            throw Error{DCRF_ERR_VALUE, "the model needs " + std::to_string(unpadded) +
                                             " bytes of vertex rows; the allocation-free inference holds at most " +
-                                            std::to_string(kNoAllocScratchBytes) + " (use dcrf_inference_device)"};
+                                            std::to_string(kNoAllocRowBytes) + " (use dcrf_inference_device)"};
         float* base = scratch_for_current_device();
         hipStream_t s = (hipStream_t)stream;
         // the rows start at zero, as the layout leaves the model's own buffers (the
@@ -2175,7 +2186,7 @@ int dcrf_inference_device_noalloc(dcrf_model* m, int n_iter, const float* U_dev,
         launch_fill(base, 0.f, need, s);
         BorrowedRows rows(*m, base, n0, base + off1, n1);
         const float* U = U_dev ? U_dev : (m->has_unary ? m->unary.get() : nullptr);
-        run_inference(*m, n_iter, U, Q_dev, s, false);
+        run_inference(*m, n_iter, U, Q_dev, s);
     });
 }
 
@@ -2190,7 +2201,7 @@ int dcrf_start_inference(dcrf_model* m, float* Q) {
         ensure_device(*m);
         ensure_unary(*m);
         m->Q.reserve(n);
-        launch_softmax_neg(m->unary.get(), m->Q.get(), m->N(), m->L, m->stream);
+        launch_softmax_neg(m->unary.get(), m->Q.get(), m->L, m->N(), m->L, padded_labels(m->L), m->stream);
         copy_to_host(Q, m->Q.get(), sizeof(float) * n, m->stream);
     });
 }
@@ -2205,8 +2216,8 @@ int dcrf_step_inference(dcrf_model* m, float* Q, float* tmp1, float* tmp2) {
         hipStream_t s = m->stream;
         copy_to_device(m->Q.get(), Q, sizeof(float) * n, s);
         if (m->terms.empty()) launch_fill(m->tmp2.get(), 0.f, n, s);
-        run_filter(*m, m->Q.get(), m->L, false, s);
-        launch_meanfield(m->has_unary ? m->unary.get() : nullptr, m->Q.get(), m->N(), m->L,
+        run_filter(*m, splat_rows(*m, m->Q.get(), s), false, s);
+        launch_meanfield(m->has_unary ? m->unary.get() : nullptr, m->Q.get(), m->L, m->N(), m->L, m->ldv,
                          slice_table(*m, false, m->kw_set ? m->kw.get() : nullptr), m->tmp1.get(), m->terms.empty() ? nullptr : m->tmp2.get(), s);
         copy_to_host(Q, m->Q.get(), sizeof(float) * n, s);
         if (tmp1) copy_to_host(tmp1, m->tmp1.get(), sizeof(float) * n, s);
@@ -2223,12 +2234,11 @@ int dcrf_kl_divergence(dcrf_model* m, const float* Q, double* kl) {
         m->work.reserve(n);
         hipStream_t s = m->stream;
         copy_to_device(m->work.get(), Q, sizeof(float) * n, s);
-        run_filter(*m, m->work.get(), m->L, false, s);
-        const LaunchShape sh = shape_for(m->L);
-        const int nb = (m->N() + sh.items - 1) / sh.items;
+        run_filter(*m, splat_rows(*m, m->work.get(), s), false, s);
+        const int nb = kl_blocks(m->N(), m->ldv);
         DevBuf<double> part;
         part.reserve(nb);
-        launch_kl(m->work.get(), m->has_unary ? m->unary.get() : nullptr, m->N(), m->L,
+        launch_kl(m->work.get(), m->has_unary ? m->unary.get() : nullptr, m->N(), m->L, m->ldv,
                   slice_table(*m, false, m->kw_set ? m->kw.get() : nullptr), part.get(), s);
         std::vector<double> h(nb);
         DCRF_HIP_CHECK(hipMemcpyAsync(h.data(), part.get(), sizeof(double) * nb, hipMemcpyDeviceToHost, s));
@@ -2250,8 +2260,8 @@ int dcrf_apply_pairwise(dcrf_model* m, int term, const float* Q, float* out, int
         m->tmp1.reserve(n);
         hipStream_t s = m->stream;
         copy_to_device(m->work.get(), Q, sizeof(float) * n, s);
-        run_filter(*m, m->work.get(), m->L, transpose != 0, s);
-        launch_slice_term(m->tmp1.get(), m->N(), m->L,
+        run_filter(*m, splat_rows(*m, m->work.get(), s), transpose != 0, s);
+        launch_slice_term(m->tmp1.get(), m->N(), m->L, m->ldv,
                           slice_table(*m, transpose != 0, m->kw_set ? m->kw.get() : nullptr), term, s);
         copy_to_host(out, m->tmp1.get(), sizeof(float) * n, s);
         if (m->timing) collect_timing(*m);
@@ -2318,10 +2328,10 @@ int dcrf_pairwise_energy(dcrf_model* m, const int16_t* labels, int term, float* 
         m->tmp1.reserve(n);
         hipStream_t s = m->stream;
         copy_to_device(m->work.get(), Q.data(), sizeof(float) * n, s);
-        run_filter(*m, m->work.get(), L, false, s);
+        run_filter(*m, splat_rows(*m, m->work.get(), s), false, s);
         const SliceTable st = slice_table(*m, false, m->kw_set ? m->kw.get() : nullptr);
         for (int k = term < 0 ? 0 : term; k < (term < 0 ? T : term + 1); k++) {
-            launch_slice_term(m->tmp1.get(), N, L, st, k, s);
+            launch_slice_term(m->tmp1.get(), N, L, m->ldv, st, k, s);
             copy_to_host(x.data(), m->tmp1.get(), sizeof(float) * n, s);
             for (int i = 0; i < N; i++) {
                 const float e = labels[i] >= 0 && labels[i] < L ? -0.5f * x[(size_t)i * L + labels[i]] : 0.0f;
@@ -2521,7 +2531,7 @@ int dcrf_gradient_objective(dcrf_model* m, int n_iter, int objective_kind, const
         }
         const int npart = objective_partials(objective_kind, N, L);
         m->obj_partial.reserve(npart);
-        launch_objective(objective_kind, m->qcache.get() + (size_t)n_iter * NL, m->gt_dev.get(), N, L, param,
+        launch_objective(objective_kind, m->qcache.get() + (size_t)n_iter * N * m->ldv, m->gt_dev.get(), N, L, param,
                          hw.empty() ? nullptr : m->obj_w.get(), m->work.get(), m->obj_partial.get(), s);
         std::vector<double> OP(npart);
         DCRF_HIP_CHECK(hipMemcpyAsync(OP.data(), m->obj_partial.get(), sizeof(double) * npart,
@@ -2613,7 +2623,7 @@ int dcrf_forward_device(dcrf_model* m, int n_iter, const float* U_dev, const flo
         forward_train(*m, n_iter, U, compat_dev, kw, s);
         if (Q_dev) {
             const size_t NL = (size_t)m->N() * m->L;
-            DCRF_HIP_CHECK(hipMemcpyAsync(Q_dev, m->qcache.get() + (size_t)n_iter * NL, sizeof(float) * NL,
+            DCRF_HIP_CHECK(hipMemcpyAsync(Q_dev, m->qcache.get() + (size_t)n_iter * m->N() * m->ldv, sizeof(float) * NL,
                                           hipMemcpyDeviceToDevice, s));
         }
     });

@@ -1,11 +1,14 @@
 // Device helpers shared by the lattice-filter, mean-field and adjoint kernels.
 //
-// Lane groups.  A group of S = L / R lanes owns one item (a splat chunk, a vertex, a
-// pixel); lane l owns the R consecutive labels [l*R, l*R + R) of the item's row, so a
-// row of L floats is read and written as S contiguous R-float pieces (dwordx R
-// accesses).  R is the largest of 4, 3, 2 dividing L, else 1 (choose_labels_per_lane):
-// no lane holds a partial piece, so no access is conditional; per-item work (addresses,
-// reductions, exp) is shared by R labels.
+// Lane groups.  A group of S lanes owns one item (a splat chunk, a vertex, a pixel);
+// lane l owns the R consecutive labels [l*R, l*R + R) of the item's row, so a row is
+// read and written as S contiguous R-float pieces (dwordx R accesses); per-item work
+// (addresses, reductions, exp) is shared by R labels.
+//   The rows that are gathered (vertex rows, Q between iterations, the adjoint's b) have
+//   padded_labels(L) floats: R is the largest of 4, 3, 2 dividing that, no piece is
+//   partial and no access conditional.  The padding labels hold zeros.
+//   Rows of the caller's layout ([N][L]: unary, final Q, gradients) may end inside the
+//   last lane's piece (LaneGroup::tail): load_row and store_row handle that lane.
 //   WAVE = true  (S <= 64): 64 / S groups per 64-wide wave, the block is 4 waves.  A
 //                 group never spans waves; group-wide max / sum / peer reads are
 //                 ds_bpermute shuffles with no block barrier.
@@ -144,11 +147,13 @@ template <bool WAVE, int R>
 struct LaneGroup {
     int L, S, g, l, k0, base, t, per;
     int w;  // the thread's wave in its block (the same in every lane: a scalar)
+    bool tail;  // R does not divide L (uniform): the last lane holds padding labels
     bool on;
     float* sh;  // block mode: block * R floats
 
     // per: groups per wave (WAVE) or per block
     __device__ __forceinline__ LaneGroup(int L_, int S_, int per_, float* sh_) : L(L_), S(S_), per(per_), sh(sh_) {
+        tail = L % R != 0;
         t = threadIdx.x;
         w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
         const int lane = WAVE ? (t & 63) : t;
@@ -171,7 +176,13 @@ struct LaneGroup {
     // Index of this group's item (blocks taken in XCD-contiguous order).
     __device__ __forceinline__ int item() const { return item_in(xcd_block(blockIdx.x, gridDim.x)); }
     __device__ static __forceinline__ int items_per_block(int per) { return WAVE ? (kWaveBlock / 64) * per : per; }
-    __device__ __forceinline__ bool has(int) const { return true; }  // R divides L: every slot is a label
+    __device__ __forceinline__ bool has(int r) const { return !tail || k0 + r < L; }  // slot r is a label
+    // Padding slots of x set to v.
+    __device__ __forceinline__ void pad(float (&x)[R], float v) const {
+        if (tail)
+#pragma unroll
+            for (int r = 1; r < R; r++) x[r] = k0 + r < L ? x[r] : v;
+    }
 
     // Value of lane s of this group (all lanes must call).
     __device__ __forceinline__ float lane_value(float x, int s) {
@@ -183,11 +194,11 @@ struct LaneGroup {
         return v;
     }
 
+    // (all_max and all_sum take the padding slots as well: -infinity and 0 there)
     __device__ __forceinline__ float all_max(const float (&x)[R]) {
         float m = x[0];
 #pragma unroll
-        for (int r = 1; r < R; r++)
-            if (has(r)) m = fmaxf(m, x[r]);
+        for (int r = 1; r < R; r++) m = fmaxf(m, x[r]);
         if (WAVE) {
             // ring doubling over the S lanes; max is idempotent, so overlap is harmless
             for (int k = 1; k < S; k <<= 1) {
@@ -208,8 +219,7 @@ struct LaneGroup {
     __device__ __forceinline__ float all_sum(const float (&x)[R]) {
         float a = x[0];
 #pragma unroll
-        for (int r = 1; r < R; r++)
-            if (has(r)) a = a + x[r];
+        for (int r = 1; r < R; r++) a = a + x[r];
         if (WAVE) {
             // pairwise tree over the S lanes towards lane 0 of the group, then a broadcast
             for (int k = 1; k < S; k <<= 1) {
@@ -226,6 +236,56 @@ struct LaneGroup {
         return v;
     }
 };
+
+// The lane's labels of a row of L floats (row: its first float); 0 in padding slots.  A
+// partial last piece is read from the row's end instead, R floats that the row has, and
+// shifted into place: no access leaves the row.
+template <bool WAVE, int R>
+__device__ __forceinline__ void load_row(const float* __restrict__ row, const LaneGroup<WAVE, R>& G, float (&x)[R]) {
+    if (R < 4 || !G.tail) {
+        load_piece<R>(row, G.k0, G.L, x);
+        return;
+    }
+    const int sh = max(G.k0 + R - G.L, 0);  // > 0 in the last lane only
+    load_piece<R>(row, G.k0 - sh, G.L, x);
+#pragma unroll
+    for (int b = 1; b < R; b <<= 1)
+        if (sh & b) {
+#pragma unroll
+            for (int r = 0; r + b < R; r++) x[r] = x[r + b];
+        }
+    G.pad(x, 0.0f);
+}
+
+// Store the lane's labels to a row of L floats (padding slots are not stored).
+template <bool WAVE, int R>
+__device__ __forceinline__ void store_row(float* __restrict__ row, const LaneGroup<WAVE, R>& G, const float (&x)[R]) {
+    if (R < 4 || !G.tail || G.k0 + R <= G.L) {
+        store_piece<R>(row, G.k0, G.L, x);
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r + 1 < R; r++)
+        if (G.k0 + r < G.L) row[G.k0 + r] = x[r];
+}
+
+// The same for rows of ld floats, which hold the padding labels where ld > L.
+template <bool WAVE, int R>
+__device__ __forceinline__ void load_row(const float* __restrict__ row, int ld, const LaneGroup<WAVE, R>& G,
+                                         float (&x)[R]) {
+    if (ld > G.L)
+        load_piece<R>(row, G.k0, G.L, x);
+    else
+        load_row(row, G, x);
+}
+template <bool WAVE, int R>
+__device__ __forceinline__ void store_row(float* __restrict__ row, int ld, const LaneGroup<WAVE, R>& G,
+                                          const float (&x)[R]) {
+    if (ld > G.L)
+        store_piece<R>(row, G.k0, G.L, x);
+    else
+        store_row(row, G, x);
+}
 
 // The adjoint kernels' per-block compatibility statistic (SliceTerm::gstat): the sum of
 // each label's products over the block's groups, in a fixed order.  stat_put leaves the
@@ -347,8 +407,12 @@ template <bool WAVE, int R>
 __device__ __forceinline__ void matrix_piece(const float* __restrict__ cw, int ldw, const float (&m)[R],
                                              float (&c)[R], LaneGroup<WAVE, R>& G) {
     const int L = G.L;
+    const float* wr[R];  // the lane's weight rows (a padding slot repeats the last one)
 #pragma unroll
-    for (int r = 0; r < R; r++) c[r] = 0.0f;
+    for (int r = 0; r < R; r++) {
+        c[r] = 0.0f;
+        wr[r] = cw + (size_t)min(G.k0 + r, L - 1) * ldw;
+    }
     for (int s = 0; s < G.S; s++) {
 #pragma unroll
         for (int rr = 0; rr < R; rr++) {
@@ -356,11 +420,11 @@ __device__ __forceinline__ void matrix_piece(const float* __restrict__ cw, int l
             const int b = s * R + rr;
             if (b < L) {
 #pragma unroll
-                for (int r = 0; r < R; r++)
-                    if (G.has(r)) c[r] = fmaf(cw[(size_t)(G.k0 + r) * ldw + b], mb, c[r]);
+                for (int r = 0; r < R; r++) c[r] = fmaf(wr[r][b], mb, c[r]);
             }
         }
     }
+    G.pad(c, 0.0f);
 }
 
 // Compatibility transform of the lane's message values (labelcompatibility.cpp:46-48,
@@ -377,8 +441,10 @@ __device__ __forceinline__ void compat_piece(const SliceTerm& T, const float (&m
         return;
     }
     if (T.ckind == DCRF_COMPAT_DIAGONAL) {
+        float w[R];
+        load_row(T.cw, G, w);
 #pragma unroll
-        for (int r = 0; r < R; r++) c[r] = G.has(r) ? T.cw[G.k0 + r] * m[r] : 0.0f;
+        for (int r = 0; r < R; r++) c[r] = w[r] * m[r];
         return;
     }
     // two copies of the loop, one per weight source, so that each pointer keeps its
@@ -395,16 +461,22 @@ __device__ __forceinline__ void compat_piece(const SliceTerm& T, const float (&m
 // order, so the results are bit-identical to matrix_piece's.
 template <int R>
 __device__ __forceinline__ void matrix_piece_rows(const float* __restrict__ w, int ldw,
-                                                  const float* __restrict__ mrow, int L, int k0, float (&c)[R]) {
+                                                  const float* __restrict__ mrow, const LaneGroup<true, R>& G,
+                                                  float (&c)[R]) {
+    const int L = G.L;
+    int wo[R];
 #pragma unroll
-    for (int r = 0; r < R; r++) c[r] = 0.0f;
+    for (int r = 0; r < R; r++) {
+        c[r] = 0.0f;
+        wo[r] = min(G.k0 + r, L - 1) * ldw;
+    }
     int b = 0;
 #pragma unroll 1
     for (; b + 4 <= L; b += 4) {
         const float4 mv = *reinterpret_cast<const float4*>(mrow + b);
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            const float4 wv = *reinterpret_cast<const float4*>(w + (size_t)(k0 + r) * ldw + b);
+            const float4 wv = *reinterpret_cast<const float4*>(w + wo[r] + b);
             c[r] = fmaf(wv.x, mv.x, c[r]);
             c[r] = fmaf(wv.y, mv.y, c[r]);
             c[r] = fmaf(wv.z, mv.z, c[r]);
@@ -415,8 +487,9 @@ __device__ __forceinline__ void matrix_piece_rows(const float* __restrict__ w, i
     for (; b < L; b++) {
         const float mv = mrow[b];
 #pragma unroll
-        for (int r = 0; r < R; r++) c[r] = fmaf(w[(size_t)(k0 + r) * ldw + b], mv, c[r]);
+        for (int r = 0; r < R; r++) c[r] = fmaf(w[wo[r] + b], mv, c[r]);
     }
+    G.pad(c, 0.0f);
 }
 
 // y[r] / s for the lane's values, s the same for all of them: one reciprocal (Newton's

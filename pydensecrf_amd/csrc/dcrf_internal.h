@@ -1,7 +1,9 @@
 // Internal declarations shared by the HIP translation units of libdcrf_hip.so.
 //
 // Device layout of a model (N variables over all instances, L labels):
-//   Q, unary                [N][L] float, label fastest (the reference's Eigen storage)
+//   Q, unary                [N][L] float, label fastest (the reference's Eigen storage);
+//                           Q between iterations and the vertex rows have rows of
+//                           padded_labels(L) floats (dcrf_model::ldv)
 // Per pairwise term k with feature dimension d (term-local vertex ids 0..V_k-1):
 //   vtx, bary, rank         [N][d+1]   lattice vertex / barycentric weight / rank per
 //                                      (pixel, remainder)   (Permutohedral offset_ ...)
@@ -295,6 +297,10 @@ struct LaunchShape {
     int S;      // lanes per item, ceil(L / R)
 };
 int choose_labels_per_lane(int L);
+// Floats of a gathered row (vertex rows, Q between iterations) of L labels: L where three or
+// four labels per lane divide it (or all fit one lane), else L rounded up to 4.
+int padded_labels(int L);
+// The shape for rows of L floats, every lane's piece whole.
 LaunchShape shape_for(int L);
 LaunchShape shape_for_r(int L, int R);  // the shape for R labels per lane
 
@@ -336,7 +342,8 @@ void launch_pass_table(const int2* nbr, int V, int vbase, int zero_row, int K, c
                        hipStream_t s);
 // Mean-field update: E = -U - sum_k compat_k(slice_k); Q = softmax(E).  U may be null.
 // tmp1/tmp2 optional outputs (energy, last term's message).
-void launch_meanfield(const float* U, float* Q, int N, int L, const SliceTable& st, float* tmp1,
+// Lv: floats of the vertex rows (padded_labels(L), or L); Q has rows of ldq floats, L or Lv.
+void launch_meanfield(const float* U, float* Q, int ldq, int N, int L, int Lv, const SliceTable& st, float* tmp1,
                       float* tmp2, hipStream_t s);
 // The same update for models of one term with d+1 in {3, 6} or two terms with
 // (d+1) = (3, 6) / (6, 3) (fused_meanfield_ok): slc[p] holds the (vertex, weight bits)
@@ -366,11 +373,11 @@ struct RunSlice {
 void build_run_slice(const Geometry& g, const GeometryDev& gd, const int2* slc, int ds, unsigned par_mask, int TW,
                      int TH, RunSlice& rs, hipStream_t s);
 size_t meanfield_runs_lds(int L, int ds, int P, int rows_lds, int cwf);
-void launch_meanfield_runs(const float* U, float* Q, int N, int L, const SliceTable& st, const RunSliceDev& rs,
-                           hipStream_t s);
+void launch_meanfield_runs(const float* U, float* Q, int ldq, int N, int L, int Lv, const SliceTable& st,
+                           const RunSliceDev& rs, hipStream_t s);
 // bw > 0: Q is written in 8 x 8 pixel blocks of an image bw pixels wide (q_block_pos,
 // rows of ldq floats), for the splat over block-position entries (launch_entry_block).
-void launch_meanfield_fused(const float* U, float* Q, int ldq, int N, int L, const SliceTable& st,
+void launch_meanfield_fused(const float* U, float* Q, int ldq, int N, int L, int Lv, const SliceTable& st,
                             const int2* slc, hipStream_t s, int bw = 0);
 void launch_entry_block(const int2* ent, size_t E, int W, int2* out, hipStream_t s);
 // rows of a Q held in 8 x 8 pixel blocks for an image of W x H pixels
@@ -378,12 +385,15 @@ inline size_t q_block_rows(int W, int H) { return (size_t)((W + 7) / 8) * ((H + 
 void launch_interleave_slice(const int* vtx, const float* sw, int N, int d1, int ds, int off, int2* slc,
                              hipStream_t s);
 // out = compat_k(slice_k) for term index `which` of st.
-void launch_slice_term(float* out, int N, int L, const SliceTable& st, int which, hipStream_t s);
-// Q0 = softmax(-U).
-void launch_softmax_neg(const float* U, float* Q, int N, int L, hipStream_t s);
-// KL divergence partial sums (one double per block).
-int launch_kl(const float* Q, const float* U, int N, int L, const SliceTable& st, double* partials,
-              hipStream_t s);
+void launch_slice_term(float* out, int N, int L, int Lv, const SliceTable& st, int which, hipStream_t s);
+// Q0 = softmax(-U), rows of ldq floats.
+void launch_softmax_neg(const float* U, float* Q, int ldq, int N, int L, int Lv, hipStream_t s);
+// out [N][Lv] = in [N][L] with zeros in the padding labels.
+void launch_pad_rows(const float* in, float* out, int N, int L, int Lv, hipStream_t s);
+// KL divergence partial sums (one double per block, kl_blocks of them).
+int kl_blocks(int N, int Lv);
+void launch_kl(const float* Q, const float* U, int N, int L, int Lv, const SliceTable& st, double* partials,
+               hipStream_t s);
 // norm = f(K*1) per the normalisation type, from the sliced values (L = 1).
 void launch_norm_finish(float* norm, int N, int ntype, hipStream_t s);
 void launch_fill(float* p, float v, size_t n, hipStream_t s);
@@ -392,23 +402,24 @@ void launch_transpose(const float* in, float* out, int rows, int cols, hipStream
 // out[p] = the first label of the largest Q[p][l] (DenseCRF::currentMap), Q row stride ldq.
 void launch_argmax(const float* Q, int ldq, int N, int L, int16_t* out, hipStream_t s);
 // ---------------------------------------------------------------- adjoint kernels
-// b = sumAndNormalize(Q .* dQ, Q); dU = b.
-void launch_sn_first(const float* Q, const float* dQ, float* b, float* dU, int N, int L, hipStream_t s);
+// b = sumAndNormalize(Q .* dQ, Q); dU = b.  Q, dQ, dU [N][L]; b rows of Lv floats.
+void launch_sn_first(const float* Q, const float* dQ, float* b, float* dU, int N, int L, int Lv, hipStream_t s);
 // b <- sumAndNormalize(Q .* sum_k w_k C_k^T slice^T_k, Q) (b is written, not read); dU += b.
 // Terms with st.t[k].gstat also get their statistic rows (see SliceTerm).
-void launch_adjoint(const float* Q, float* b, float* dU, int N, int L, const SliceTable& st, hipStream_t s);
+// Q and b have rows of Lv floats, dU of L.
+void launch_adjoint(const float* Q, float* b, float* dU, int N, int L, int Lv, const SliceTable& st, hipStream_t s);
 // The same over interleaved slice pairs (those of launch_meanfield_fused, with the
 // transposed filter's slice weights); models that fused_meanfield_ok accepts.
-void launch_adjoint_fused(const float* Q, float* b, float* dU, int N, int L, const SliceTable& st, const int2* slc,
-                          hipStream_t s);
+void launch_adjoint_fused(const float* Q, float* b, float* dU, int N, int L, int Lv, const SliceTable& st,
+                          const int2* slc, hipStream_t s);
 // Blocks of one adjoint launch over N pixels (the rows of its statistic output).
-int adjoint_blocks(int N, int L);
-// acc += sum_{t < iters} sum_p b_t[p] M_t[p]^T (L x L), with b_t = b + t * bstride and
-// M_t = M + t * mstride, on the matrix cores; one launch and one reduction for all
+int adjoint_blocks(int N, int Lv);
+// acc += sum_{t < iters} sum_p b_t[p] M_t[p]^T (L x L), with b_t = b + t * bstride (rows of
+// ldb floats) and M_t = M + t * mstride (rows of L), on the matrix cores; one launch and one reduction for all
 // iterations.  partial holds grad_partial_floats(N, L, iters) floats, mid
 // rows_mid_doubles(L * L) doubles.
 size_t grad_partial_floats(int N, int L, int iters);
-void launch_grad_stat(const float* b, size_t bstride, const float* M, size_t mstride, int iters, int N, int L,
+void launch_grad_stat(const float* b, int ldb, size_t bstride, const float* M, size_t mstride, int iters, int N, int L,
                       float* partial, double* mid, double* acc, hipStream_t s);
 // acc[j] += sum_{r < rows} part[r * cols + j] for j < cols, in double, in a fixed order
 // (two kernels; mid holds rows_mid_doubles(cols) doubles).
@@ -423,11 +434,12 @@ void launch_set_compat(const float* raw, int ckind, int L, float* cw, hipStream_
 // lbl (optional) = C (w Q_t) of the term in st.t[0] (its compatibility and weight), and
 // P [N][2L] = [a | c], a = b (times n for SYMMETRIC / AFTER), c = lbl (times n for
 // SYMMETRIC / BEFORE).
-void launch_kg_prepare(const float* Qt, const float* b, const float* norm, int N, int L, const SliceTable& st,
+// Qt and b have rows of ldq floats.
+void launch_kg_prepare(const float* Qt, const float* b, int ldq, const float* norm, int N, int L, const SliceTable& st,
                        int ntype, float* lbl, float* P, hipStream_t s);
 // The normaliser-derivative input x of featureGradient for ntype, with fa sliced by
 // st.t[0] and fb by st.t[1] (a term with null vals: not needed).
-void launch_kg_x(const float* b, const float* lbl, const float* norm, int N, int L, const SliceTable& st, int ntype,
+void launch_kg_x(const float* b, int ldb, const float* lbl, const float* norm, int N, int L, const SliceTable& st, int ntype,
                  float* x, hipStream_t s);
 // Whether launch_kg_grad has a kernel for L labels and feature dimension d.
 bool kg_grad_fused(int L, int d);

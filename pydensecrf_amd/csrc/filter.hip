@@ -35,6 +35,17 @@ int choose_labels_per_lane(int L) {
     return 1;
 }
 
+// Rows of L floats that neither 4 nor 3 divides took one or two labels per lane: at 19
+// labels 19 lanes and 3 rows per wave instruction, each with its own addresses and
+// weights.  Padded to 20, five lanes of four labels and 12 rows: 1021x511x19, 10
+// iterations, 1745 -> 1006 us.  Three labels per lane stay: 21 labels padded to 24 (6
+// lanes for 7, aligned 16-byte pieces, but 14 % more bytes in every gathered row) measured
+// 1514 against 1464 us at 1024x768, 10 iterations.
+int padded_labels(int L) {
+    const int R = choose_labels_per_lane(L);
+    return L >= 5 && R < 3 ? (L + 3) & ~3 : L;
+}
+
 LaunchShape shape_for(int L) { return shape_for_r(L, choose_labels_per_lane(L)); }
 
 LaunchShape shape_for_r(int L, int R) {
@@ -537,9 +548,9 @@ __global__ void k_pass_table(const int2* __restrict__ nbr, int V, int vbase, int
 // Mean-field update of one pixel: E = -U - sum_k C_k(w_k slice_k), Q = softmax(-E)
 // (densecrf.cpp:122-129, with the per-term weight w_k = 1 unless set).
 template <bool WAVE, int R, bool CWL>
-__global__ void __launch_bounds__(1024) k_meanfield(const float* __restrict__ U, float* __restrict__ Q, int N,
-                                                    int L, int S, int per, SliceTable st, float* __restrict__ tmp1,
-                                                    float* __restrict__ tmp2) {
+__global__ void __launch_bounds__(1024) k_meanfield(const float* __restrict__ U, float* __restrict__ Q, int ldq,
+                                                    int N, int L, int S, int per, SliceTable st,
+                                                    float* __restrict__ tmp1, float* __restrict__ tmp2) {
     extern __shared__ float sh[];
     float* shc = sh + blockDim.x;  // compat region after the group scratch
     if (CWL) stage_compat(st, L, shc);
@@ -554,7 +565,7 @@ __global__ void __launch_bounds__(1024) k_meanfield(const float* __restrict__ U,
         last[r] = 0.0f;
     }
     if (active && U) {
-        load_piece<R>(U + (size_t)p * L, k0, L, e);
+        load_row(U + (size_t)p * L, G, e);
 #pragma unroll
         for (int r = 0; r < R; r++) e[r] = -e[r];
     }
@@ -565,7 +576,7 @@ __global__ void __launch_bounds__(1024) k_meanfield(const float* __restrict__ U,
             float m[R], c[R];
             if (active) {
                 slice_piece<R>(T, p, k0, L, m);
-                if (T.mout) store_piece<R>(T.mout + (size_t)p * L, k0, L, m);
+                if (T.mout) store_row(T.mout + (size_t)p * L, G, m);
             } else {
 #pragma unroll
                 for (int r = 0; r < R; r++) m[r] = 0.0f;
@@ -583,6 +594,7 @@ __global__ void __launch_bounds__(1024) k_meanfield(const float* __restrict__ U,
             }
         }
     }
+    G.pad(e, -INFINITY);
     const float mx = G.all_max(e);
     float x[R];
 #pragma unroll
@@ -591,9 +603,9 @@ __global__ void __launch_bounds__(1024) k_meanfield(const float* __restrict__ U,
     if (active) {
         float q[R];
         divide_all<R>(x, s, q);
-        store_piece<R>(Q + (size_t)p * L, k0, L, q);
-        if (tmp1) store_piece<R>(tmp1 + (size_t)p * L, k0, L, e);
-        if (tmp2) store_piece<R>(tmp2 + (size_t)p * L, k0, L, last);
+        store_row(Q + (size_t)p * ldq, ldq, G, q);
+        if (tmp1) store_row(tmp1 + (size_t)p * L, G, e);
+        if (tmp2) store_row(tmp2 + (size_t)p * L, G, last);
     }
 }
 
@@ -656,7 +668,7 @@ __device__ __forceinline__ void compat_terms(LaneGroup<true, R>& G, const SliceT
     for (int k = 0; k < NT; k++) {
         const SliceTerm& T = st.t[k];
         if (ROWS && T.ckind == DCRF_COMPAT_MATRIX && T.cw_lds >= 0)
-            matrix_piece_rows<R>(shc + T.cw_lds, T.ldw, msg + ((size_t)k * G.per + G.g) * ldm, G.L, G.k0, c[k]);
+            matrix_piece_rows<R>(shc + T.cw_lds, T.ldw, msg + ((size_t)k * G.per + G.g) * ldm, G, c[k]);
         else
             compat_piece<true, R>(T, mk[k], c[k], G, shc);
     }
@@ -668,7 +680,7 @@ __device__ __forceinline__ void compat_terms(LaneGroup<true, R>& G, const SliceT
 template <int R, int D0, int D1, bool ROWS>
 __device__ __forceinline__ void finish_pixel(LaneGroup<true, R>& G, const SliceTable& st, const int2 (&e)[D0 + D1],
                                              const float (&x)[D0 + D1][R], const float (&u)[R], bool active,
-                                             float* __restrict__ qrow, const float* shc, int p, float* msg) {
+                                             float* __restrict__ qrow, int ldq, const float* shc, int p, float* msg) {
     constexpr int NT = D1 ? 2 : 1;
     float raw[NT][R], mk[NT][R], c[NT][R];
 #pragma unroll
@@ -681,6 +693,7 @@ __device__ __forceinline__ void finish_pixel(LaneGroup<true, R>& G, const SliceT
     for (int k = 0; k < NT; k++)
 #pragma unroll
         for (int r = 0; r < R; r++) en[r] = en[r] - c[k][r];
+    G.pad(en, -INFINITY);
     const float mx = G.all_max(en);
     float y[R];
 #pragma unroll
@@ -689,10 +702,10 @@ __device__ __forceinline__ void finish_pixel(LaneGroup<true, R>& G, const SliceT
     if (active) {
         float q[R];
         divide_all<R>(y, sum, q);
-        store_piece<R>(qrow, G.k0, G.L, q);
+        store_row(qrow, ldq, G, q);
 #pragma unroll
         for (int k = 0; k < NT; k++)
-            if (st.t[k].mout) store_piece<R>(st.t[k].mout + (size_t)p * G.L, G.k0, G.L, raw[k]);
+            if (st.t[k].mout) store_row(st.t[k].mout + (size_t)p * G.L, G, raw[k]);
     }
 }
 
@@ -767,7 +780,7 @@ k_meanfield_fused(const float* __restrict__ U, float* __restrict__ Q, int ldq, i
     float u[R];
     auto load_u = [&]() {
         if (U) {
-            load_piece<R>(U + (size_t)W.p0 * L + (unsigned)(gp * L + k0), 0, L, u);
+            load_row(U + (size_t)W.p0 * L + (unsigned)(gp * L), G, u);
         } else {
 #pragma unroll
             for (int r = 0; r < R; r++) u[r] = 0.0f;
@@ -790,7 +803,7 @@ k_meanfield_fused(const float* __restrict__ U, float* __restrict__ Q, int ldq, i
     float* msg = shc + cwf + (size_t)G.w * (D1 ? 2 : 1) * per * ((L + 3) & ~3);
     // bw > 0: Q is written in 8 x 8 pixel blocks of an image bw pixels wide (q_block_pos)
     float* qrow = bw > 0 ? Q + (size_t)q_block_pos(W.p0 + gp, bw) * ldq : Q + (size_t)W.p0 * ldq + (unsigned)(gp * ldq);
-    finish_pixel<R, D0, D1, CWL>(G, st, e, x, u, active, qrow, shc, p, msg);
+    finish_pixel<R, D0, D1, CWL>(G, st, e, x, u, active, qrow, ldq, shc, p, msg);
 }
 
 // The adjoint step of k_adjoint (adjoint.hip) over the same interleaved slice pairs:
@@ -799,8 +812,8 @@ k_meanfield_fused(const float* __restrict__ U, float* __restrict__ Q, int ldq, i
 // slice weights.  Same arithmetic, in the same order, as k_adjoint.
 template <int R, int D0, int D1, bool CWL, bool NARROW>
 __global__ void __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(R <= 3 ? 8 : 7)))
-k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __restrict__ dU, int N, int L, int S,
-                int per, SliceTable st, const int2* __restrict__ slc, int cwf) {
+k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __restrict__ dU, int N, int L, int Lv,
+                int S, int per, SliceTable st, const int2* __restrict__ slc, int cwf) {
     constexpr int DS = D0 + D1;
     LaneGroup<true, R> G(L, S, per, nullptr);
     const int p = G.item();
@@ -812,8 +825,8 @@ k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __res
     const int wpairs = wave_pairs(per, DS);
     int2* wp = pairs_all + G.w * wpairs;
     float* shc = reinterpret_cast<float*>(pairs_all + (kWaveBlock / 64) * wpairs);
-    const size_t wrow = (size_t)W.p0 * L;              // the wave's rows of Q, b and dU
-    const unsigned grow = (unsigned)(gp * L + k0);     // the lane's piece of them
+    const size_t wrow = (size_t)W.p0 * Lv;           // the wave's rows of Q and b
+    const unsigned grow = (unsigned)(gp * Lv + k0);  // the lane's piece of them
     float q[R];
     load_piece<R>(Q + wrow + grow, 0, L, q);  // in flight while the pairs are staged
     if (CWL) stage_compat(st, L, shc);
@@ -854,11 +867,12 @@ k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __res
     sum_normalize<true, R>(q, gsum, bn, G);
     if (active) {
         float du[R];
-        load_piece<R>(dU + wrow + grow, 0, L, du);
+        float* urow = dU + (size_t)W.p0 * L + (unsigned)(gp * L);
+        load_row(urow, G, du);
 #pragma unroll
         for (int r = 0; r < R; r++) du[r] = du[r] + bn[r];
         store_piece<R>(b + wrow + grow, 0, L, bn);
-        store_piece<R>(dU + wrow + grow, 0, L, du);
+        store_row(urow, G, du);
     }
     if (st.nstat) stat_finish<true, R, NT>(st, G, sst);  // uniform condition
 }
@@ -870,8 +884,8 @@ k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __res
 // list, in run-major pixel order).
 template <int R, int D0, int D1>
 __global__ void __launch_bounds__(kWaveBlock) k_meanfield_runs(const float* __restrict__ U, float* __restrict__ Q,
-                                                               int N, int L, int S, int per, SliceTable st,
-                                                               RunSliceDev rs) {
+                                                               int ldq, int N, int L, int Lv, int S, int per,
+                                                               SliceTable st, RunSliceDev rs) {
     (void)N;  // the runs cover the pixels exactly (rs.pix_base)
     constexpr int DS = D0 + D1;
     extern __shared__ float lds[];
@@ -899,7 +913,7 @@ __global__ void __launch_bounds__(kWaveBlock) k_meanfield_runs(const float* __re
 #pragma unroll
         for (int b = 0; b < 4; b++) {
             const int q = q0 + b * items + gi;
-            if (G.on && q < nu) store_piece<R>(tq + (size_t)q * L, k0, L, xs[b]);
+            if (G.on && q < nu) store_piece<R>(tq + (size_t)q * Lv, k0, L, xs[b]);
         }
     }
     {
@@ -922,7 +936,7 @@ __global__ void __launch_bounds__(kWaveBlock) k_meanfield_runs(const float* __re
     float un[R];
     int pn = pixel(0);
     if (U) {
-        load_piece<R>(U + (size_t)pn * L, k0, L, un);
+        load_row(U + (size_t)pn * L, G, un);
     } else {
 #pragma unroll
         for (int r = 0; r < R; r++) un[r] = 0.0f;
@@ -935,15 +949,15 @@ __global__ void __launch_bounds__(kWaveBlock) k_meanfield_runs(const float* __re
         for (int r = 0; r < R; r++) u[r] = un[r];
         if (b0 + items < np) {
             pn = pixel(b0 + items);
-            if (U) load_piece<R>(U + (size_t)pn * L, k0, L, un);
+            if (U) load_row(U + (size_t)pn * L, G, un);
         }
         int2 e[DS];
 #pragma unroll
         for (int j = 0; j < DS; j++) e[j] = active ? tp[(b0 + gi) * DS + j] : make_int2(0, 0);
         float x[DS][R];
 #pragma unroll
-        for (int j = 0; j < DS; j++) load_piece<R>(tq + (size_t)e[j].x * L, k0, L, x[j]);
-        finish_pixel<R, D0, D1, false>(G, st, e, x, u, active, Q + (size_t)p * L, shc, p, nullptr);
+        for (int j = 0; j < DS; j++) load_piece<R>(tq + (size_t)e[j].x * Lv, k0, L, x[j]);
+        finish_pixel<R, D0, D1, false>(G, st, e, x, u, active, Q + (size_t)p * ldq, ldq, shc, p, nullptr);
     }
 }
 
@@ -988,7 +1002,7 @@ __global__ void __launch_bounds__(1024) k_slice_term(float* __restrict__ out, in
 #pragma unroll
         for (int r = 0; r < R; r++) c[r] = m[r];
     }
-    if (active) store_piece<R>(out + (size_t)p * L, G.k0, L, c);
+    if (active) store_row(out + (size_t)p * L, G, c);
 }
 
 // KL divergence terms per pixel, reduced per block in double in a fixed order
@@ -1012,8 +1026,8 @@ __global__ void __launch_bounds__(1024) k_kl(const float* __restrict__ Q, const 
     }
     double acc = 0.0;
     if (active) {
-        load_piece<R>(Q + (size_t)p * L, k0, L, q);
-        if (U) load_piece<R>(U + (size_t)p * L, k0, L, u);
+        load_row(Q + (size_t)p * L, G, q);
+        if (U) load_row(U + (size_t)p * L, G, u);
 #pragma unroll
         for (int r = 0; r < R; r++)
             if (G.has(r)) {
@@ -1116,6 +1130,15 @@ __global__ void k_argmax(const float* __restrict__ Q, int ldq, int N, int L, int
     out[p] = (int16_t)arg;
 }
 
+// out [N][Lv] = in [N][L], zeros in the padding labels.
+__global__ void k_pad_rows(const float* __restrict__ in, float* __restrict__ out, size_t n, int L, int Lv) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const size_t p = i / Lv;
+    const int l = (int)(i - p * Lv);
+    out[i] = l < L ? in[p * L + l] : 0.0f;
+}
+
 // out[c][r] = in[r][c] for an rows x cols row-major input, 32x32 tiles through LDS.
 __global__ void k_transpose(const float* __restrict__ in, float* __restrict__ out, int rows, int cols) {
     __shared__ float tile[32][33];
@@ -1143,6 +1166,13 @@ void launch_fill(float* p, float v, size_t n, hipStream_t s) {
 void launch_argmax(const float* Q, int ldq, int N, int L, int16_t* out, hipStream_t s) {
     if (N <= 0) return;
     k_argmax<<<blocks_for(N), kThreads, 0, s>>>(Q, ldq, N, L, out);
+    DCRF_HIP_CHECK(hipGetLastError());
+}
+
+void launch_pad_rows(const float* in, float* out, int N, int L, int Lv, hipStream_t s) {
+    const size_t n = (size_t)N * Lv;
+    if (!n) return;
+    k_pad_rows<<<blocks_for(n), kThreads, 0, s>>>(in, out, n, L, Lv);
     DCRF_HIP_CHECK(hipGetLastError());
 }
 
@@ -1263,7 +1293,7 @@ void launch_pass_table(const int2* nbr, int V, int vbase, int zero_row, int K, c
 }
 
 bool fused_meanfield_ok(int L, int nterms, int d1_0, int d1_1) {
-    if (!shape_for(L).wave) return false;
+    if (!shape_for(padded_labels(L)).wave) return false;
     if (nterms == 1) return d1_0 == 3 || d1_0 == 6;
     if (nterms == 2) return (d1_0 == 3 && d1_1 == 6) || (d1_0 == 6 && d1_1 == 3);
     return false;
@@ -1314,10 +1344,10 @@ void launch_fused_r(const LaunchShape& sh, const float* U, float* Q, int ldq, in
 #define DCRF_ADJ_FUSED(R_, D0_, D1_)                                                                      \
     DCRF_FUSED_FORM(k_adjoint_fused, R_, D0_, D1_)<<<                                                       \
         blocks_for(N, sh.items), kWaveBlock, fused_lds_bytes(sh, D0_ + D1_, D1_ ? 2 : 1, L, cwf, st.nstat),  \
-        s>>>(Q, b, dU, N, L, sh.S, sh.per, st, slc, cwf)
+        s>>>(Q, b, dU, N, L, Lv, sh.S, sh.per, st, slc, cwf)
 
 template <int R>
-void launch_adj_fused_r(const LaunchShape& sh, const float* Q, float* b, float* dU, int N, int L,
+void launch_adj_fused_r(const LaunchShape& sh, const float* Q, float* b, float* dU, int N, int L, int Lv,
                         const SliceTable& st, const int2* slc, int cwf, hipStream_t s) {
     const int a = st.t[0].d1, c = st.nterms > 1 ? st.t[1].d1 : 0;
     const bool narrow = narrow_rows(st.rows, st.t[0].ldv);
@@ -1332,11 +1362,11 @@ void launch_adj_fused_r(const LaunchShape& sh, const float* Q, float* b, float* 
 #undef DCRF_FUSED_FORM
 
 #define DCRF_RUNS(R_, D0_, D1_)                                                                           \
-    k_meanfield_runs<R_, D0_, D1_><<<rs.n_runs, kWaveBlock, lds, s>>>(U, Q, N, L, sh.S, sh.per, st, rs)
+    k_meanfield_runs<R_, D0_, D1_><<<rs.n_runs, kWaveBlock, lds, s>>>(U, Q, ldq, N, L, Lv, sh.S, sh.per, st, rs)
 
 template <int R>
-void launch_runs_r(const LaunchShape& sh, const float* U, float* Q, int N, int L, const SliceTable& st,
-                   const RunSliceDev& rs, size_t lds, hipStream_t s) {
+void launch_runs_r(const LaunchShape& sh, const float* U, float* Q, int ldq, int N, int L, int Lv,
+                   const SliceTable& st, const RunSliceDev& rs, size_t lds, hipStream_t s) {
     const int a = st.t[0].d1, b = st.nterms > 1 ? st.t[1].d1 : 0;
     if (a == 3 && b == 0) DCRF_RUNS(R, 3, 0);
     else if (a == 6 && b == 0) DCRF_RUNS(R, 6, 0);
@@ -1352,11 +1382,11 @@ size_t meanfield_runs_lds(int L, int ds, int P, int rows_lds, int cwf) {
     return (size_t)rows_lds * sizeof(float) + (size_t)P * ds * sizeof(int2) + (size_t)cwf * sizeof(float);
 }
 
-void launch_meanfield_runs(const float* U, float* Q, int N, int L, const SliceTable& st_in, const RunSliceDev& rs,
-                           hipStream_t s) {
+void launch_meanfield_runs(const float* U, float* Q, int ldq, int N, int L, int Lv, const SliceTable& st_in,
+                           const RunSliceDev& rs, hipStream_t s) {
     SliceTable st = st_in;
     const int cwf = assign_compat_lds(st, L);
-    const LaunchShape sh = shape_for(L);
+    const LaunchShape sh = shape_for(Lv);
     if (!fused_meanfield_ok(L, st.nterms, st.t[0].d1, st.nterms > 1 ? st.t[1].d1 : 0))
         throw Error{DCRF_ERR_VALUE, "no run mean-field kernel for these terms"};
     const int ds = st.t[0].d1 + (st.nterms > 1 ? st.t[1].d1 : 0);
@@ -1377,18 +1407,18 @@ void launch_meanfield_runs(const float* U, float* Q, int N, int L, const SliceTa
         return reinterpret_cast<const void*>(&k_meanfield_runs<R_, 6, 3>);
     };
     switch (sh.R) {
-        case 1: grant(fn_for(std::integral_constant<int, 1>{}), 1); launch_runs_r<1>(sh, U, Q, N, L, st, rs, lds, s); break;
-        case 2: grant(fn_for(std::integral_constant<int, 2>{}), 2); launch_runs_r<2>(sh, U, Q, N, L, st, rs, lds, s); break;
-        case 3: grant(fn_for(std::integral_constant<int, 3>{}), 3); launch_runs_r<3>(sh, U, Q, N, L, st, rs, lds, s); break;
-        default: grant(fn_for(std::integral_constant<int, 4>{}), 4); launch_runs_r<4>(sh, U, Q, N, L, st, rs, lds, s); break;
+        case 1: grant(fn_for(std::integral_constant<int, 1>{}), 1); launch_runs_r<1>(sh, U, Q, ldq, N, L, Lv, st, rs, lds, s); break;
+        case 2: grant(fn_for(std::integral_constant<int, 2>{}), 2); launch_runs_r<2>(sh, U, Q, ldq, N, L, Lv, st, rs, lds, s); break;
+        case 3: grant(fn_for(std::integral_constant<int, 3>{}), 3); launch_runs_r<3>(sh, U, Q, ldq, N, L, Lv, st, rs, lds, s); break;
+        default: grant(fn_for(std::integral_constant<int, 4>{}), 4); launch_runs_r<4>(sh, U, Q, ldq, N, L, Lv, st, rs, lds, s); break;
     }
 }
 
-void launch_meanfield_fused(const float* U, float* Q, int ldq, int N, int L, const SliceTable& st_in,
+void launch_meanfield_fused(const float* U, float* Q, int ldq, int N, int L, int Lv, const SliceTable& st_in,
                             const int2* slc, hipStream_t s, int bw) {
     SliceTable st = st_in;
     const int cwf = assign_compat_lds(st, L, true);  // 16-byte rows for matrix_piece_rows
-    const LaunchShape sh = shape_for(L);
+    const LaunchShape sh = shape_for(Lv);
     if (!fused_meanfield_ok(L, st.nterms, st.t[0].d1, st.nterms > 1 ? st.t[1].d1 : 0))
         throw Error{DCRF_ERR_VALUE, "no fused mean-field kernel for these terms"};
     switch (sh.R) {
@@ -1416,18 +1446,18 @@ void launch_entry_block(const int2* ent, size_t E, int W, int2* out, hipStream_t
     DCRF_HIP_CHECK(hipGetLastError());
 }
 
-void launch_adjoint_fused(const float* Q, float* b, float* dU, int N, int L, const SliceTable& st_in,
+void launch_adjoint_fused(const float* Q, float* b, float* dU, int N, int L, int Lv, const SliceTable& st_in,
                           const int2* slc, hipStream_t s) {
     SliceTable st = st_in;
     const int cwf = assign_compat_lds(st, L, true);  // 16-byte rows for matrix_piece_rows
-    const LaunchShape sh = shape_for(L);
+    const LaunchShape sh = shape_for(Lv);
     if (!fused_meanfield_ok(L, st.nterms, st.t[0].d1, st.nterms > 1 ? st.t[1].d1 : 0))
         throw Error{DCRF_ERR_VALUE, "no fused adjoint kernel for these terms"};
     switch (sh.R) {
-        case 1: launch_adj_fused_r<1>(sh, Q, b, dU, N, L, st, slc, cwf, s); break;
-        case 2: launch_adj_fused_r<2>(sh, Q, b, dU, N, L, st, slc, cwf, s); break;
-        case 3: launch_adj_fused_r<3>(sh, Q, b, dU, N, L, st, slc, cwf, s); break;
-        default: launch_adj_fused_r<4>(sh, Q, b, dU, N, L, st, slc, cwf, s); break;
+        case 1: launch_adj_fused_r<1>(sh, Q, b, dU, N, L, Lv, st, slc, cwf, s); break;
+        case 2: launch_adj_fused_r<2>(sh, Q, b, dU, N, L, Lv, st, slc, cwf, s); break;
+        case 3: launch_adj_fused_r<3>(sh, Q, b, dU, N, L, Lv, st, slc, cwf, s); break;
+        default: launch_adj_fused_r<4>(sh, Q, b, dU, N, L, Lv, st, slc, cwf, s); break;
     }
 }
 
@@ -1446,38 +1476,38 @@ int assign_compat_lds(SliceTable& st, int L, bool pad) {
     return total;
 }
 
-void launch_meanfield(const float* U, float* Q, int N, int L, const SliceTable& st_in, float* tmp1, float* tmp2,
-                      hipStream_t s) {
+void launch_meanfield(const float* U, float* Q, int ldq, int N, int L, int Lv, const SliceTable& st_in, float* tmp1,
+                      float* tmp2, hipStream_t s) {
     SliceTable st = st_in;
     const int cwf = assign_compat_lds(st, L);
-    const LaunchShape sh = shape_for(L);
-    DCRF_DISPATCH_CWL(sh, cwf, k_meanfield, blocks_for(N, sh.items), sizeof(float) * (sh.block + cwf), s, U, Q, N,
-                      L, sh.S, sh.per, st, tmp1, tmp2);
+    const LaunchShape sh = shape_for(Lv);
+    DCRF_DISPATCH_CWL(sh, cwf, k_meanfield, blocks_for(N, sh.items), sizeof(float) * (sh.block + cwf), s, U, Q, ldq,
+                      N, L, sh.S, sh.per, st, tmp1, tmp2);
 }
 
-void launch_softmax_neg(const float* U, float* Q, int N, int L, hipStream_t s) {
+void launch_softmax_neg(const float* U, float* Q, int ldq, int N, int L, int Lv, hipStream_t s) {
     SliceTable st{};
     st.nterms = 0;
-    launch_meanfield(U, Q, N, L, st, nullptr, nullptr, s);
+    launch_meanfield(U, Q, ldq, N, L, Lv, st, nullptr, nullptr, s);
 }
 
-void launch_slice_term(float* out, int N, int L, const SliceTable& st_in, int which, hipStream_t s) {
+void launch_slice_term(float* out, int N, int L, int Lv, const SliceTable& st_in, int which, hipStream_t s) {
     SliceTable st = st_in;
     const int cwf = assign_compat_lds(st, L);
-    const LaunchShape sh = shape_for(L);
+    const LaunchShape sh = shape_for(Lv);
     DCRF_DISPATCH_CWL(sh, cwf, k_slice_term, blocks_for(N, sh.items), sizeof(float) * (sh.block + cwf), s, out, N,
                       L, sh.S, sh.per, st, which);
 }
 
-int launch_kl(const float* Q, const float* U, int N, int L, const SliceTable& st_in, double* partials,
-              hipStream_t s) {
+int kl_blocks(int N, int Lv) { return (int)blocks_for(N, shape_for(Lv).items); }
+
+void launch_kl(const float* Q, const float* U, int N, int L, int Lv, const SliceTable& st_in, double* partials,
+               hipStream_t s) {
     SliceTable st = st_in;
     const int cwf = assign_compat_lds(st, L);
-    const LaunchShape sh = shape_for(L);
-    const int nb = (int)blocks_for(N, sh.items);
-    DCRF_DISPATCH_CWL(sh, cwf, k_kl, nb, sizeof(float) * (sh.block + cwf), s, Q, U, N, L, sh.S, sh.per, st,
+    const LaunchShape sh = shape_for(Lv);
+    DCRF_DISPATCH_CWL(sh, cwf, k_kl, kl_blocks(N, Lv), sizeof(float) * (sh.block + cwf), s, Q, U, N, L, sh.S, sh.per, st,
                       partials);
-    return nb;
 }
 
 void launch_norm_finish(float* norm, int N, int ntype, hipStream_t s) {

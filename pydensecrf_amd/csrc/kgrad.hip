@@ -45,7 +45,7 @@ inline unsigned blocks_for(size_t n, int t = kThreads) { return (unsigned)((n + 
 // (the normaliser input x reads it).
 template <bool WAVE, int R, bool CWL>
 __global__ void __launch_bounds__(1024) k_kg_prepare(const float* __restrict__ Qt, const float* __restrict__ b,
-                                                     const float* __restrict__ norm, int N, int L, int S, int per,
+                                                     int ldq, const float* __restrict__ norm, int N, int L, int S, int per,
                                                      SliceTable st, int ntype, float* __restrict__ lbl,
                                                      float* __restrict__ P) {
     extern __shared__ float sh[];
@@ -58,8 +58,8 @@ __global__ void __launch_bounds__(1024) k_kg_prepare(const float* __restrict__ Q
     float m[R], bv[R], c[R];
     float n = 0.0f;
     if (active) {
-        load_piece<R>(Qt + (size_t)p * L, G.k0, L, m);
-        load_piece<R>(b + (size_t)p * L, G.k0, L, bv);
+        load_piece<R>(Qt + (size_t)p * ldq, G.k0, L, m);
+        load_piece<R>(b + (size_t)p * ldq, G.k0, L, bv);
         n = norm[p];
     } else {
 #pragma unroll
@@ -94,7 +94,8 @@ __global__ void __launch_bounds__(1024) k_kg_prepare(const float* __restrict__ Q
 //   AFTER      x = (b fb) n^2                     (:98-105)
 //   BEFORE     x = (fa lbl) n^2                   (:106-113)
 template <bool WAVE, int R>
-__global__ void __launch_bounds__(1024) k_kg_x(const float* __restrict__ b, const float* __restrict__ lbl,
+__global__ void __launch_bounds__(1024) k_kg_x(const float* __restrict__ b, int ldb,
+                                               const float* __restrict__ lbl,
                                                const float* __restrict__ norm, int N, int L, int S, int per,
                                                SliceTable st, int ntype, float* __restrict__ x) {
     LaneGroup<WAVE, R> G(L, S, per, nullptr);  // no group-wide operation here
@@ -104,7 +105,7 @@ __global__ void __launch_bounds__(1024) k_kg_x(const float* __restrict__ b, cons
     const bool sym = ntype == DCRF_NORMALIZE_SYMMETRIC, after = ntype == DCRF_NORMALIZE_AFTER;
     if (st.t[0].vals) slice_piece<R>(st.t[0], p, G.k0, L, fa);
     if (st.t[1].vals) slice_piece<R>(st.t[1], p, G.k0, L, fb);
-    if (sym || after) load_piece<R>(b + (size_t)p * L, G.k0, L, bv);
+    if (sym || after) load_piece<R>(b + (size_t)p * ldb, G.k0, L, bv);
     if (!after) load_piece<R>(lbl + (size_t)p * L, G.k0, L, lv);
     const float n = norm[p];
     const float n2 = n * n;
@@ -522,21 +523,21 @@ static GradScale grad_scale(int d) {
     return gs;
 }
 
-void launch_kg_prepare(const float* Qt, const float* b, const float* norm, int N, int L, const SliceTable& st_in,
+void launch_kg_prepare(const float* Qt, const float* b, int ldq, const float* norm, int N, int L, const SliceTable& st_in,
                        int ntype, float* lbl, float* P, hipStream_t s) {
     if (!N) return;
     SliceTable st = st_in;
     const int cwf = assign_compat_lds(st, L);
     const LaunchShape sh = shape_for(L);
     DCRF_DISPATCH_CWL(sh, cwf, k_kg_prepare, blocks_for(N, sh.items), sizeof(float) * (sh.block + cwf), s, Qt, b,
-                      norm, N, L, sh.S, sh.per, st, ntype, lbl, P);
+                      ldq, norm, N, L, sh.S, sh.per, st, ntype, lbl, P);
 }
 
-void launch_kg_x(const float* b, const float* lbl, const float* norm, int N, int L, const SliceTable& st, int ntype,
+void launch_kg_x(const float* b, int ldb, const float* lbl, const float* norm, int N, int L, const SliceTable& st, int ntype,
                  float* x, hipStream_t s) {
     if (!N) return;
     const LaunchShape sh = shape_for(L);
-    DCRF_DISPATCH(sh, k_kg_x, blocks_for(N, sh.items), 0, s, b, lbl, norm, N, L, sh.S, sh.per, st, ntype, x);
+    DCRF_DISPATCH(sh, k_kg_x, blocks_for(N, sh.items), 0, s, b, ldb, lbl, norm, N, L, sh.S, sh.per, st, ntype, x);
 }
 
 bool kg_grad_fused(int L, int d) { return d >= 1 && d <= 6 && shape_for(L).wave; }
