@@ -1167,7 +1167,7 @@ void ensure_layout(dcrf_model& m) {
     m.ldv = m.tiled ? L : padded_labels(L);
     const LaunchShape csh = shape_for(m.ldv);
     const bool runs = csh.wave && !m.tiled;
-    const int per = csh.per;
+    const int per = splat_shape(m.ldv).per;  // segments per wave of the splat
     std::vector<Chunk>& gch = m.gch_scratch;  // (capacity kept between layout builds)
     gch.clear();
     std::vector<int>& nruns = m.runs_scratch;

@@ -300,6 +300,13 @@ int choose_labels_per_lane(int L);
 // Floats of a gathered row (vertex rows, Q between iterations) of L labels: L where three or
 // four labels per lane divide it (or all fit one lane), else L rounded up to 4.
 int padded_labels(int L);
+// The splat's: K lanes share each lane position of a segment's row (kSplitLanes for rows of
+// one or two lanes, else 1), per segments per wave.
+constexpr int kSplitLanes = 4;
+struct SplatShape {
+    int K, per;
+};
+SplatShape splat_shape(int L);
 // The shape for rows of L floats, every lane's piece whole.
 LaunchShape shape_for(int L);
 LaunchShape shape_for_r(int L, int R);  // the shape for R labels per lane

@@ -46,6 +46,17 @@ int padded_labels(int L) {
     return L >= 5 && R < 3 ? (L + 3) & ~3 : L;
 }
 
+// Rows of one or two lanes (up to 8 labels) take the quad form of the splat
+// (k_splat_split).  10 iterations, k_splat -> quads: 1920x1080x2 1421 -> 1127 us,
+// 200x150x3 390 -> 230 us, training on 1.5 M voxels with 4 labels 2892 -> 2366 us; eight
+// lanes per segment: the same within 2 %.  From three lanes on (9 labels: 21 segments a
+// wave) one window holds nearly all of a wave's entries.
+SplatShape splat_shape(int L) {
+    const LaunchShape sh = shape_for(L);
+    if (!sh.wave || sh.S > 2) return SplatShape{1, sh.per};
+    return SplatShape{kSplitLanes, 64 / (sh.S * kSplitLanes)};
+}
+
 LaunchShape shape_for(int L) { return shape_for_r(L, choose_labels_per_lane(L)); }
 
 LaunchShape shape_for_r(int L, int R) {
@@ -189,14 +200,94 @@ __global__ void __launch_bounds__(1024) k_splat(const Chunk* __restrict__ chunks
     store_piece<R>(vals + (size_t)ch.out * ldv, k0, L, acc);
 }
 
+// Splat for rows of few lanes (S <= 2 lanes of R labels, up to 8 labels).  With one lane
+// per row piece and segment (k_splat) the wave's lanes are on up to 64 different segments:
+// each LDS window of entries covers a third of them while the others wait, and every
+// lane's row is a cache line of its own.  Here the K = kSplitLanes = 4 lanes of a quad
+// share a segment: lane kk loads every K-th entry, straight from memory (32 consecutive
+// bytes per segment and load; kSplitBatch entries per lane, so a segment of 32 in one
+// round), and its row.  Neighbouring entries of a segment are mostly neighbouring pixels:
+// their rows share lines.  Every lane of the quad then adds all the products in entry
+// order, reading them from the other lanes as DPP operands: the rounding of a sequential
+// sum, which a tree of the four shares would lose.  Same segments and in-wave runs as
+// k_splat, in groups of S quads.
+constexpr int kSplitBatch = 8;
+
+template <int J>
+__device__ __forceinline__ float quad_value(float x) {  // x of lane J of the quad
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), J * 0x55, 0xf, 0xf, true));
+}
+
+template <int R, bool NARROW>
+__global__ void __launch_bounds__(kWaveBlock) k_splat_split(const Chunk* __restrict__ chunks, int n,
+                                                            const int2* __restrict__ ent, const float* __restrict__ in,
+                                                            int ldi, float* __restrict__ vals, int ldv, int S,
+                                                            int per) {
+    constexpr int K = kSplitLanes;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int gs = S * K;                  // lanes of a group: 4 or 8
+    const int g = S == 1 ? lane >> 2 : lane >> 3;
+    const int kk = lane & 3, k0 = S == 1 ? 0 : ((lane >> 2) & 1) * R;
+    const int cw0 = (xcd_block(blockIdx.x, gridDim.x) * (kWaveBlock / 64) + w) * per;
+    if (cw0 >= n) return;  // the whole wave is idle (no block barrier below)
+    const int c = cw0 + g;
+    const bool mine = c < n;
+    const Chunk ch = chunks[mine ? c : cw0];
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = 0.0f;
+    for (int i0 = ch.beg; i0 < ch.end; i0 += kSplitBatch * K) {  // the same in all lanes of a group
+        int2 e[kSplitBatch];
+        float x[kSplitBatch][R];
+#pragma unroll
+        for (int u = 0; u < kSplitBatch; u++) e[u] = ent[min(i0 + kk + u * K, ch.end - 1)];
+#pragma unroll
+        for (int u = 0; u < kSplitBatch; u++) load_piece<R>(row_piece<NARROW>(in, e[u].x, ldi, k0), 0, 0, x[u]);
+#pragma unroll
+        for (int u = 0; u < kSplitBatch; u++) {
+            loaded<R>(x[u]);
+            const bool on = i0 + kk + u * K < ch.end;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const float prod = __int_as_float(e[u].y) * x[u][r];
+                x[u][r] = on ? prod : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kSplitBatch; u++)
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                acc[r] = acc[r] + quad_value<0>(x[u][r]);
+                acc[r] = acc[r] + quad_value<1>(x[u][r]);
+                acc[r] = acc[r] + quad_value<2>(x[u][r]);
+                acc[r] = acc[r] + quad_value<3>(x[u][r]);
+            }
+    }
+    const int nv = wave_read(ch.v, lane + gs);
+    const int nout = wave_read(ch.out, lane + gs);
+    const bool cont = mine && g + 1 < per && c + 1 < n && nout < 0 && nv == ch.v;
+    if (__any(cont)) {
+        for (int j = per - 2; j >= 0; j--) {  // wave-uniform
+            float y[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) y[r] = wave_read(acc[r], lane + gs);
+            if (cont && g == j)
+#pragma unroll
+                for (int r = 0; r < R; r++) acc[r] = acc[r] + y[r];
+        }
+    }
+    if (mine && kk == 0 && ch.out >= 0) store_piece<R>(vals + (size_t)ch.out * ldv, k0, 0, acc);
+}
+
 // Tiled splat: block = one tile.  Stage 1 copies the tile's input rows, its entries
 // (pixel index in the tile, weight) and its segments (beg, end, out) into LDS, every
 // thread keeping kStage loads in flight; stage 2 gives the segments to the lane groups
-// of the block, which sum them from LDS in entry order (the same order, hence the same
-// bits, as k_splat).
+// of the block, which sum them from LDS in the order of k_splat or k_splat_split (hence
+// the same bits).
 constexpr int kStage = 32;
 
-template <int R>
+// FMA: k_splat's additions, else k_splat_split's.
+template <int R, bool FMA>
 __global__ void __launch_bounds__(1024) k_splat_tiled(TiledSplat ts, const int2* __restrict__ ent,
                                                             const float* __restrict__ in, float* __restrict__ vals,
                                                             int ldv, int L, int S, int per, int q_max) {
@@ -255,6 +346,17 @@ __global__ void __launch_bounds__(1024) k_splat_tiled(TiledSplat ts, const int2*
         float acc[R];
 #pragma unroll
         for (int r = 0; r < R; r++) acc[r] = 0.0f;
+        auto add = [&](float ww, const float (&x)[R]) {
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if (FMA) {
+                    acc[r] = fmaf(ww, x[r], acc[r]);
+                } else {
+                    const float prod = ww * x[r];
+                    acc[r] = acc[r] + prod;
+                }
+            }
+        };
         int i = b;
         for (; i + 4 <= e; i += 4) {
             int pp[4];
@@ -268,17 +370,13 @@ __global__ void __launch_bounds__(1024) k_splat_tiled(TiledSplat ts, const int2*
 #pragma unroll
             for (int u = 0; u < 4; u++) load_piece<R>(tq + pp[u] * L, k0, L, xx[u]);
 #pragma unroll
-            for (int u = 0; u < 4; u++)
-#pragma unroll
-                for (int r = 0; r < R; r++) acc[r] = fmaf(ww[u], xx[u][r], acc[r]);
+            for (int u = 0; u < 4; u++) add(ww[u], xx[u]);
         }
         for (; i < e; i++) {
             float xx[R];
             const int2 x = te[i];
-            const float ww = __int_as_float(x.y);
             load_piece<R>(tq + x.x * L, k0, L, xx);
-#pragma unroll
-            for (int r = 0; r < R; r++) acc[r] = fmaf(ww, xx[r], acc[r]);
+            add(__int_as_float(x.y), xx);
         }
         store_piece<R>(vals + (size_t)out * ldv, k0, L, acc);
     }
@@ -1193,6 +1291,23 @@ void launch_splat(const Chunk* chunks, int n_chunks, const int2* ent, const floa
                   float* vals, int ldv, int L, hipStream_t s) {
     if (!n_chunks) return;
     const LaunchShape sh = shape_for(L);
+    const SplatShape sp = splat_shape(L);
+    if (sp.K > 1) {
+        const bool narrow = narrow_rows(rows_in, ldi);
+        const unsigned grid = blocks_for(n_chunks, (kWaveBlock / 64) * sp.per);
+#define DCRF_SPLIT(R_)                                                                              \
+    case R_:                                                                                        \
+        (narrow ? k_splat_split<R_, true> : k_splat_split<R_, false>)<<<grid, kWaveBlock, 0, s>>>(    \
+            chunks, n_chunks, ent, in, ldi, vals, ldv, sh.S, sp.per);                                 \
+        break;
+        switch (sh.R) {
+            DCRF_SPLIT(1) DCRF_SPLIT(2) DCRF_SPLIT(3) DCRF_SPLIT(4)
+            default: throw Error{DCRF_ERR_STATE, "no split splat kernel for this shape"};
+        }
+#undef DCRF_SPLIT
+        DCRF_HIP_CHECK(hipGetLastError());
+        return;
+    }
     const size_t shm = sh.wave ? (size_t)(kWaveBlock / 64) * (kWin + kBatch) * sizeof(int2) : 0;
     if (narrow_rows(rows_in, ldi))
         DCRF_DISPATCH_T(sh, k_splat, true, blocks_for(n_chunks, sh.items), shm, s, chunks, n_chunks, ent, in, ldi, vals,
@@ -1223,25 +1338,25 @@ void launch_splat_tiled(const TiledSplat& ts, const int2* ent, const float* in, 
     const int q_max = (ts.geom.side * ts.geom.side * L + 1) & ~1;  // the entry pairs start 8-byte aligned
     const int block = tiled_splat_block(lds, lds_cap);
     // dynamic LDS beyond the default launch limit must be granted per kernel
-    static size_t granted[5] = {};
+    static size_t granted[10] = {};
     auto grant = [&](const void* fn, int r) {
         if (lds > granted[r]) {
             DCRF_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
             granted[r] = lds;
         }
     };
-    switch (sh.R) {
-        case 1: grant(reinterpret_cast<const void*>(&k_splat_tiled<1>), 1); break;
-        case 2: grant(reinterpret_cast<const void*>(&k_splat_tiled<2>), 2); break;
-        case 3: grant(reinterpret_cast<const void*>(&k_splat_tiled<3>), 3); break;
-        default: grant(reinterpret_cast<const void*>(&k_splat_tiled<4>), 4); break;
+    const bool fma = splat_shape(L).K == 1;
+#define DCRF_TILED(R_, F_)                                                                                   \
+    case R_ * 2 + F_:                                                                                        \
+        grant(reinterpret_cast<const void*>(&k_splat_tiled<R_, F_>), R_ * 2 + F_);                            \
+        k_splat_tiled<R_, F_><<<ts.n_tiles, block, lds, s>>>(ts, ent, in, vals, ldv, L, sh.S, sh.per, q_max); \
+        break;
+    switch (sh.R * 2 + (fma ? 1 : 0)) {
+        DCRF_TILED(1, 0) DCRF_TILED(2, 0) DCRF_TILED(3, 0) DCRF_TILED(4, 0)
+        DCRF_TILED(1, 1) DCRF_TILED(2, 1) DCRF_TILED(3, 1) DCRF_TILED(4, 1)
+        default: throw Error{DCRF_ERR_STATE, "no tiled splat kernel for this shape"};
     }
-    switch (sh.R) {
-        case 1: k_splat_tiled<1><<<ts.n_tiles, block, lds, s>>>(ts, ent, in, vals, ldv, L, sh.S, sh.per, q_max); break;
-        case 2: k_splat_tiled<2><<<ts.n_tiles, block, lds, s>>>(ts, ent, in, vals, ldv, L, sh.S, sh.per, q_max); break;
-        case 3: k_splat_tiled<3><<<ts.n_tiles, block, lds, s>>>(ts, ent, in, vals, ldv, L, sh.S, sh.per, q_max); break;
-        default: k_splat_tiled<4><<<ts.n_tiles, block, lds, s>>>(ts, ent, in, vals, ldv, L, sh.S, sh.per, q_max); break;
-    }
+#undef DCRF_TILED
     DCRF_HIP_CHECK(hipGetLastError());
 }
 
