@@ -353,7 +353,7 @@ void launch_pass_table(const int2* nbr, int V, int vbase, int zero_row, int K, c
 void launch_meanfield(const float* U, float* Q, int ldq, int N, int L, int Lv, const SliceTable& st, float* tmp1,
                       float* tmp2, hipStream_t s);
 // The same update for models of one term with d+1 in {3, 6} or two terms with
-// (d+1) = (3, 6) / (6, 3) (fused_meanfield_ok): slc[p] holds the (vertex, weight bits)
+// (d+1) = (3, 6), (4, 5) in either order (fused_meanfield_ok): slc[p] holds the (vertex, weight bits)
 // pairs of every term of pixel p, term 0 first (launch_interleave_slice builds it).
 bool fused_meanfield_ok(int L, int nterms, int d1_0, int d1_1);
 // Run form of the fused update: pixels grouped into runs (TW x TH rectangles of 2-D
