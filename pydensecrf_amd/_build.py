@@ -24,8 +24,8 @@ INCLUDE = os.path.join(ROOT, "include")
 ORACLE = os.path.join(ROOT, "oracle")
 REFERENCE = "/root/reference"
 
-HIP_SOURCES = ["pool.hip", "lattice.hip", "filter.hip", "adjoint.hip", "kgrad.hip", "unary.hip", "objective.hip",
-               "capi.hip"]
+HIP_SOURCES = ["pool.hip", "lattice.hip", "filter.hip", "meanfield.hip", "adjoint.hip", "adjoint_fused.hip", "kgrad.hip",
+               "unary.hip", "objective.hip", "capi.hip"]
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     # keep the compiler from forming packed-FP32 instructions
@@ -37,7 +37,7 @@ CY_MODULES = ["eigen", "densecrf"]
 # and per-vertex filter, adjoint and kernel-gradient kernels keep every array in
 # registers or LDS.  The compiler's resource-usage remarks are read at every build and
 # the build fails on a kernel with ScratchSize > 0.
-NO_SCRATCH_SOURCES = ["filter.hip", "adjoint.hip", "kgrad.hip"]
+NO_SCRATCH_SOURCES = ["filter.hip", "meanfield.hip", "adjoint.hip", "adjoint_fused.hip", "kgrad.hip"]
 
 
 def _hipcc():

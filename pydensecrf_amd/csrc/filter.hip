@@ -707,360 +707,6 @@ __global__ void __launch_bounds__(1024) k_meanfield(const float* __restrict__ U,
     }
 }
 
-// Term k's message in a fused pixel update: the weighted sum of its gathered rows (entry
-// order, as slice_piece) into raw, and raw times the term weight into m.  The caller
-// stores raw to the term's `mout` (as k_meanfield does) only after its last read of
-// the terms' weights: once a kernel may have stored to global memory, the compiler
-// reads those weights through the vector memory path and waits for every load in
-// flight (the row gathers among them).
-template <int R, int D0, int D1>
-__device__ __forceinline__ void term_message(const SliceTerm& T, int k, const int2 (&e)[D0 + D1],
-                                             const float (&x)[D0 + D1][R], float (&raw)[R], float (&m)[R]) {
-    constexpr int DS = D0 + D1;
-    const int jb = k ? D0 : 0, je = k ? DS : D0;
-#pragma unroll
-    for (int r = 0; r < R; r++) raw[r] = 0.0f;
-#pragma unroll
-    for (int j = jb; j < je; j++) {
-        const float w = __int_as_float(e[j].y);
-#pragma unroll
-        for (int r = 0; r < R; r++) raw[r] = fmaf(w, x[j][r], raw[r]);
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) m[r] = raw[r];
-    if (T.kw) {
-        const float kw = T.kw[0];
-#pragma unroll
-        for (int r = 0; r < R; r++) m[r] = m[r] * kw;
-    }
-}
-
-// The compatibility transforms c[k] of the pixel's NT term messages.  ROWS: the Matrix
-// terms whose weights have an LDS copy (16-byte aligned rows) first write the group's
-// message vector into the wave's message region `msg` (NT rows of (L + 3) & ~3 floats
-// per group), then read it back whole with matrix_piece_rows: no cross-lane shuffles.
-// The other terms go through compat_piece.  Same results either way.
-template <int R, int NT, bool ROWS>
-__device__ __forceinline__ void compat_terms(LaneGroup<true, R>& G, const SliceTable& st, const float (&mk)[NT][R],
-                                             float (&c)[NT][R], const float* shc, float* msg) {
-    const int ldm = (G.L + 3) & ~3;
-    if (ROWS) {
-        bool any = false;
-#pragma unroll
-        for (int k = 0; k < NT; k++)
-            if (st.t[k].ckind == DCRF_COMPAT_MATRIX && st.t[k].cw_lds >= 0) {
-                any = true;
-                if (G.on) {  // idle lanes shadow group 0: they must not write its row
-                    float* row = msg + ((size_t)k * G.per + G.g) * ldm + G.k0;
-#pragma unroll
-                    for (int r = 0; r < R; r++) row[r] = mk[k][r];
-                }
-            }
-        if (any) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < NT; k++) {
-        const SliceTerm& T = st.t[k];
-        if (ROWS && T.ckind == DCRF_COMPAT_MATRIX && T.cw_lds >= 0)
-            matrix_piece_rows<R>(shc + T.cw_lds, T.ldw, msg + ((size_t)k * G.per + G.g) * ldm, G, c[k]);
-        else
-            compat_piece<true, R>(T, mk[k], c[k], G, shc);
-    }
-}
-
-// The per-pixel tail of the fused mean-field kernels: the terms' compatibility
-// messages subtracted from -U, then the softmax over the lane group, stored when
-// `active`.
-template <int R, int D0, int D1, bool ROWS>
-__device__ __forceinline__ void finish_pixel(LaneGroup<true, R>& G, const SliceTable& st, const int2 (&e)[D0 + D1],
-                                             const float (&x)[D0 + D1][R], const float (&u)[R], bool active,
-                                             float* __restrict__ qrow, int ldq, const float* shc, int p, float* msg) {
-    constexpr int NT = D1 ? 2 : 1;
-    float raw[NT][R], mk[NT][R], c[NT][R];
-#pragma unroll
-    for (int k = 0; k < NT; k++) term_message<R, D0, D1>(st.t[k], k, e, x, raw[k], mk[k]);
-    compat_terms<R, NT, ROWS>(G, st, mk, c, shc, msg);
-    float en[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) en[r] = -u[r];
-#pragma unroll
-    for (int k = 0; k < NT; k++)
-#pragma unroll
-        for (int r = 0; r < R; r++) en[r] = en[r] - c[k][r];
-    G.pad(en, -INFINITY);
-    const float mx = G.all_max(en);
-    float y[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) y[r] = expf(en[r] - mx);
-    const float sum = G.all_sum(y);
-    if (active) {
-        float q[R];
-        divide_all<R>(y, sum, q);
-        store_row(qrow, ldq, G, q);
-#pragma unroll
-        for (int k = 0; k < NT; k++)
-            if (st.t[k].mout) store_row(st.t[k].mout + (size_t)p * G.L, G, raw[k]);
-    }
-}
-
-// The pixels of a wave of the fused kernels: np >= 1 consecutive ones from p0 (a wave past
-// the last pixel repeats it; its results are not stored).  Both are the same in every
-// lane, so the wave's rows of the unary, Q and the slice pairs start at scalar addresses.
-struct WavePixels {
-    int p0, np;
-    template <int R>
-    __device__ __forceinline__ WavePixels(const LaneGroup<true, R>& G, int p, int N) {
-        p0 = __builtin_amdgcn_readfirstlane(min(p - G.g, N - 1));
-        np = min(G.per, N - p0);
-    }
-};
-
-// LDS pairs of one wave's staged slice pairs: its per * ds pairs rounded up to whole rounds
-// of 128 (stage_wave_pairs stores whole rounds).
-__host__ __device__ inline int wave_pairs(int per, int ds) { return (per * ds + 127) & ~127; }
-
-// Stage the slice pairs of the wave's pixels (one contiguous run of np * DS pairs, 64 pairs
-// per load instruction) into the wave's LDS slice wp; the wave's groups then read their
-// own.  Past the run the last pair is repeated, so a group without a pixel reads valid
-// rows and needs no mask (a masked LDS read per entry, each waited for on its own, had
-// made nine round trips of one).
-template <int R, int DS>
-__device__ __forceinline__ void stage_wave_pairs(const WavePixels& W, int per, const int2* __restrict__ slc,
-                                                 int2* wp) {
-    const int np = W.np * DS;
-    const int lane = threadIdx.x & 63;
-    // two loads per lane per round (clamped, unconditional), then the stores.  The pairs
-    // are read once per iteration: nontemporal loads keep them from displacing the Q rows
-    // this kernel writes, which the next splat gathers (at 1024x768x21 the splat went from
-    // 72.5 to 58.3 us; nontemporal loads of the splat's own entries or of the unary row
-    // measured slower)
-    const long long* __restrict__ src = reinterpret_cast<const long long*>(slc + (size_t)W.p0 * DS);
-    long long* dst = reinterpret_cast<long long*>(wp);
-    for (int i0 = 0; i0 < per * DS; i0 += 128) {
-        const long long t0 = __builtin_nontemporal_load(src + (unsigned)min(i0 + lane, np - 1));
-        const long long t1 = __builtin_nontemporal_load(src + (unsigned)min(i0 + 64 + lane, np - 1));
-        dst[i0 + lane] = t0;
-        dst[i0 + 64 + lane] = t1;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Mean-field update for models of one or two terms with d+1 = D0 (and D1) lattice
-// (3, 6: images; 4 and 5: volumes with intensity, where the generic kernels took 45 us
-// (mean-field) and 62 us (adjoint) per launch on 1.5 M voxels with 4 labels)
-// entries per pixel: slc holds every pixel's (vertex, weight bits) pairs of both terms
-// side by side, so all D0 + D1 vertex rows are gathered after one dependent load.  Same
-// arithmetic, in the same order, as k_meanfield.
-template <int R, int D0, int D1, bool CWL, bool NARROW>
-__global__ void __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(R <= 3 ? 8 : 7)))  // <= 64 (72) VGPRs
-k_meanfield_fused(const float* __restrict__ U, float* __restrict__ Q, int ldq, int N, int L, int S, int per,
-                  SliceTable st, const int2* __restrict__ slc, int cwf, int bw) {
-    constexpr int DS = D0 + D1;
-    LaneGroup<true, R> G(L, S, per, nullptr);
-    const int p = G.item();
-    const bool active = G.on && p < N;
-    const int k0 = G.k0;
-    const WavePixels W(G, p, N);
-    const int gp = min(G.g, W.np - 1);  // groups without a pixel repeat the wave's last one
-    extern __shared__ __align__(16) int2 pairs_all[];
-    const int wpairs = wave_pairs(per, DS);
-    int2* wp = pairs_all + G.w * wpairs;
-    // CWL: some Matrix term has an LDS copy of its weights (staging costs a barrier, so
-    // it is compiled in only then)
-    float* shc = reinterpret_cast<float*>(pairs_all + (kWaveBlock / 64) * wpairs);
-    // the unary row does not depend on the slice pairs: its load is in flight while they
-    // are staged (not at four labels per lane, where the longer-lived row would spill)
-    constexpr bool kEarlyU = R <= 3;
-    float u[R];
-    auto load_u = [&]() {
-        if (U) {
-            load_row(U + (size_t)W.p0 * L + (unsigned)(gp * L), G, u);
-        } else {
-#pragma unroll
-            for (int r = 0; r < R; r++) u[r] = 0.0f;
-        }
-    };
-    if (kEarlyU) load_u();
-    if (CWL) stage_compat(st, L, shc);
-    stage_wave_pairs<R, DS>(W, per, slc, wp);
-    int2 e[DS];
-#pragma unroll
-    for (int j = 0; j < DS; j++) e[j] = wp[gp * DS + j];
-    if (!kEarlyU) load_u();
-    float x[DS][R];
-#pragma unroll
-    for (int j = 0; j < DS; j++) {
-        const SliceTerm& T = j < D0 ? st.t[0] : st.t[1];
-        load_piece<R>(row_piece<NARROW>(T.vals, e[j].x, T.ldv, k0), 0, L, x[j]);
-    }
-    // CWL: the wave's message rows follow the compat region
-    float* msg = shc + cwf + (size_t)G.w * (D1 ? 2 : 1) * per * ((L + 3) & ~3);
-    // bw > 0: Q is written in 8 x 8 pixel blocks of an image bw pixels wide (q_block_pos)
-    float* qrow = bw > 0 ? Q + (size_t)q_block_pos(W.p0 + gp, bw) * ldq : Q + (size_t)W.p0 * ldq + (unsigned)(gp * ldq);
-    finish_pixel<R, D0, D1, CWL>(G, st, e, x, u, active, qrow, ldq, shc, p, msg);
-}
-
-// The adjoint step of k_adjoint (adjoint.hip) over the same interleaved slice pairs:
-// g = sum_k C_k(w_k slice_k(filtered b)), b = sumAndNormalize(Q .* g, Q), dU += b, and
-// the terms' statistic rows (SliceTerm::gstat).  The pairs carry the transposed filter's
-// slice weights.  Same arithmetic, in the same order, as k_adjoint.
-template <int R, int D0, int D1, bool CWL, bool NARROW>
-__global__ void __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(R <= 3 ? 8 : 7)))
-k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __restrict__ dU, int N, int L, int Lv,
-                int S, int per, SliceTable st, const int2* __restrict__ slc, int cwf) {
-    constexpr int DS = D0 + D1;
-    LaneGroup<true, R> G(L, S, per, nullptr);
-    const int p = G.item();
-    const bool active = G.on && p < N;
-    const int k0 = G.k0;
-    const WavePixels W(G, p, N);
-    const int gp = min(G.g, W.np - 1);
-    extern __shared__ __align__(16) int2 pairs_all[];
-    const int wpairs = wave_pairs(per, DS);
-    int2* wp = pairs_all + G.w * wpairs;
-    float* shc = reinterpret_cast<float*>(pairs_all + (kWaveBlock / 64) * wpairs);
-    const size_t wrow = (size_t)W.p0 * Lv;           // the wave's rows of Q and b
-    const unsigned grow = (unsigned)(gp * Lv + k0);  // the lane's piece of them
-    float q[R];
-    load_piece<R>(Q + wrow + grow, 0, L, q);  // in flight while the pairs are staged
-    if (CWL) stage_compat(st, L, shc);
-    stage_wave_pairs<R, DS>(W, per, slc, wp);
-    int2 e[DS];
-#pragma unroll
-    for (int j = 0; j < DS; j++) e[j] = wp[gp * DS + j];
-    float x[DS][R];
-#pragma unroll
-    for (int j = 0; j < DS; j++) {
-        const SliceTerm& T = j < D0 ? st.t[0] : st.t[1];
-        load_piece<R>(row_piece<NARROW>(T.vals, e[j].x, T.ldv, k0), 0, L, x[j]);
-    }
-    constexpr int NT = D1 ? 2 : 1;
-    float raw[NT][R], mk[NT][R], c[NT][R];  // (the adjoint stores no raw messages)
-#pragma unroll
-    for (int k = 0; k < NT; k++) term_message<R, D0, D1>(st.t[k], k, e, x, raw[k], mk[k]);
-    // statistic region after the message rows (present with a compat region)
-    float* sst = shc + cwf + (cwf ? (kWaveBlock / 64) * NT * per * ((L + 3) & ~3) : 0);
-#pragma unroll
-    for (int k = 0; k < NT; k++)
-        if (st.t[k].gslot >= 0) {
-            float v[R];
-#pragma unroll
-            for (int r = 0; r < R; r++) v[r] = active ? raw[k][r] * q[r] : 0.0f;
-            stat_put<R>(sst, st.t[k].gslot, v);
-        }
-    float* msg = shc + cwf + (size_t)G.w * NT * per * ((L + 3) & ~3);
-    compat_terms<R, NT, CWL>(G, st, mk, c, shc, msg);
-    float gsum[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) gsum[r] = 0.0f;
-#pragma unroll
-    for (int k = 0; k < NT; k++)
-#pragma unroll
-        for (int r = 0; r < R; r++) gsum[r] = gsum[r] + c[k][r];
-    float bn[R];
-    sum_normalize<true, R>(q, gsum, bn, G);
-    if (active) {
-        float du[R];
-        float* urow = dU + (size_t)W.p0 * L + (unsigned)(gp * L);
-        load_row(urow, G, du);
-#pragma unroll
-        for (int r = 0; r < R; r++) du[r] = du[r] + bn[r];
-        store_piece<R>(b + wrow + grow, 0, L, bn);
-        store_row(urow, G, du);
-    }
-    if (st.nstat) stat_finish<true, R, NT>(st, G, sst);  // uniform condition
-}
-
-// The same update over pixel runs (2-D rectangles whose rows hold whole waves of
-// pixels), one workgroup per run: the run's distinct vertex rows (a few hundred, against
-// P*(D0+D1) gathers) are staged in LDS once, then every pixel's slice reads them from
-// there (rs.loc holds the pairs with the vertex replaced by its index in the run's
-// list, in run-major pixel order).
-template <int R, int D0, int D1>
-__global__ void __launch_bounds__(kWaveBlock) k_meanfield_runs(const float* __restrict__ U, float* __restrict__ Q,
-                                                               int ldq, int N, int L, int Lv, int S, int per,
-                                                               SliceTable st, RunSliceDev rs) {
-    (void)N;  // the runs cover the pixels exactly (rs.pix_base)
-    constexpr int DS = D0 + D1;
-    extern __shared__ float lds[];
-    float* tq = lds;  // rs.rows_lds floats: the run's rows
-    int2* tp = reinterpret_cast<int2*>(lds + rs.rows_lds);  // rs.P * DS pairs: the run's slice pairs
-    float* shc = reinterpret_cast<float*>(tp + (size_t)rs.P * DS);
-    stage_compat(st, L, shc);
-    LaneGroup<true, R> G(L, S, per, nullptr);
-    const int k0 = G.k0;
-    const int run = xcd_block(blockIdx.x, gridDim.x);
-    const int k0r = rs.pix_base[run], np = rs.pix_base[run + 1] - k0r;  // run-major positions
-    const int u0 = rs.base[run], nu = rs.base[run + 1] - u0;
-    const int items = (blockDim.x >> 6) * per;
-    const int gi = (threadIdx.x >> 6) * per + G.g;
-    // stage the rows (group gi takes rows gi, gi + items, ...) and the pairs (all threads,
-    // consecutive words): loads first, then stores
-    for (int q0 = 0; q0 < nu; q0 += 4 * items) {
-        float xs[4][R];
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const int q = min(q0 + b * items + gi, nu - 1);
-            const int tag = rs.rows[u0 + q];
-            load_piece<R>(((tag & 1) ? rs.v1 : rs.v0) + (size_t)(tag >> 1) * st.t[0].ldv, k0, L, xs[b]);
-        }
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const int q = q0 + b * items + gi;
-            if (G.on && q < nu) store_piece<R>(tq + (size_t)q * Lv, k0, L, xs[b]);
-        }
-    }
-    {
-        const int npairs = np * DS;
-        const int2* src = rs.loc + (size_t)k0r * DS;
-        for (int i0 = 0; i0 < npairs; i0 += 4 * (int)blockDim.x) {
-            int2 t[4];
-#pragma unroll
-            for (int b = 0; b < 4; b++) t[b] = src[min(i0 + b * (int)blockDim.x + (int)threadIdx.x, npairs - 1)];
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const int i = i0 + b * (int)blockDim.x + (int)threadIdx.x;
-                if (i < npairs) tp[i] = t[b];
-            }
-        }
-    }
-    __syncthreads();
-    // pixel passes: each pass's unary rows are loaded one pass ahead
-    auto pixel = [&](int b0) { return rs.rpix[b0 + gi < np && G.on ? k0r + b0 + gi : k0r]; };
-    float un[R];
-    int pn = pixel(0);
-    if (U) {
-        load_row(U + (size_t)pn * L, G, un);
-    } else {
-#pragma unroll
-        for (int r = 0; r < R; r++) un[r] = 0.0f;
-    }
-    for (int b0 = 0; b0 < np; b0 += items) {
-        const bool active = G.on && b0 + gi < np;
-        const int p = pn;
-        float u[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) u[r] = un[r];
-        if (b0 + items < np) {
-            pn = pixel(b0 + items);
-            if (U) load_row(U + (size_t)pn * L, G, un);
-        }
-        int2 e[DS];
-#pragma unroll
-        for (int j = 0; j < DS; j++) e[j] = active ? tp[(b0 + gi) * DS + j] : make_int2(0, 0);
-        float x[DS][R];
-#pragma unroll
-        for (int j = 0; j < DS; j++) load_piece<R>(tq + (size_t)e[j].x * Lv, k0, L, x[j]);
-        finish_pixel<R, D0, D1, false>(G, st, e, x, u, active, Q + (size_t)p * ldq, ldq, shc, p, nullptr);
-    }
-}
-
 // slc[p][off + j] = (vtx[p][j], bits of sw[p][j]) for j < d1; rows of ds pairs.
 __global__ void k_interleave_slice(const int* __restrict__ vtx, const float* __restrict__ sw, int N, int d1, int ds,
                                    int off, int2* __restrict__ slc) {
@@ -1425,137 +1071,6 @@ void launch_interleave_slice(const int* vtx, const float* sw, int N, int d1, int
     DCRF_HIP_CHECK(hipGetLastError());
 }
 
-// dynamic LDS of the fused kernels: the wave's slice pairs, the compat region (cwf
-// floats), with a compat region the message rows (NT per group, (L + 3) & ~3 floats),
-// and the adjoint's statistic region (stat_lds_floats)
-inline size_t fused_lds_bytes(const LaunchShape& sh, int ds, int nt, int L, int cwf, int nstat = 0) {
-    const size_t waves = kWaveBlock / 64;
-    return waves * wave_pairs(sh.per, ds) * sizeof(int2) + (size_t)cwf * sizeof(float) +
-           (cwf ? waves * nt * sh.per * (size_t)((L + 3) & ~3) * sizeof(float) : 0) +
-           stat_lds_floats(true, nstat, L, kWaveBlock, sh.R) * sizeof(float);
-}
-
-// One of a fused kernel's four forms: with or without the LDS copy of Matrix weights, with
-// 24-bit or 64-bit row offsets.
-#define DCRF_FUSED_FORM(kernel, R_, D0_, D1_)                                              \
-    (cwf ? (narrow ? kernel<R_, D0_, D1_, true, true> : kernel<R_, D0_, D1_, true, false>) \
-         : (narrow ? kernel<R_, D0_, D1_, false, true> : kernel<R_, D0_, D1_, false, false>))
-
-#define DCRF_FUSED(R_, D0_, D1_)                                                                          \
-    DCRF_FUSED_FORM(k_meanfield_fused, R_, D0_, D1_)<<<                                                     \
-        blocks_for(N, sh.items), kWaveBlock, fused_lds_bytes(sh, D0_ + D1_, D1_ ? 2 : 1, L, cwf), s>>>(       \
-        U, Q, ldq, N, L, sh.S, sh.per, st, slc, cwf, bw)
-
-template <int R>
-void launch_fused_r(const LaunchShape& sh, const float* U, float* Q, int ldq, int N, int L, const SliceTable& st,
-                    const int2* slc, int cwf, int bw, hipStream_t s) {
-    const int a = st.t[0].d1, b = st.nterms > 1 ? st.t[1].d1 : 0;
-    const bool narrow = narrow_rows(st.rows, st.t[0].ldv);
-    if (a == 3 && b == 0) DCRF_FUSED(R, 3, 0);
-    else if (a == 6 && b == 0) DCRF_FUSED(R, 6, 0);
-    else if (a == 3 && b == 6) DCRF_FUSED(R, 3, 6);
-    else if (a == 6 && b == 3) DCRF_FUSED(R, 6, 3);
-    else if (a == 4 && b == 5) DCRF_FUSED(R, 4, 5);
-    else if (a == 5 && b == 4) DCRF_FUSED(R, 5, 4);
-    else throw Error{DCRF_ERR_VALUE, "no fused mean-field kernel for these terms"};
-    DCRF_HIP_CHECK(hipGetLastError());
-}
-#undef DCRF_FUSED
-
-#define DCRF_ADJ_FUSED(R_, D0_, D1_)                                                                      \
-    DCRF_FUSED_FORM(k_adjoint_fused, R_, D0_, D1_)<<<                                                       \
-        blocks_for(N, sh.items), kWaveBlock, fused_lds_bytes(sh, D0_ + D1_, D1_ ? 2 : 1, L, cwf, st.nstat),  \
-        s>>>(Q, b, dU, N, L, Lv, sh.S, sh.per, st, slc, cwf)
-
-template <int R>
-void launch_adj_fused_r(const LaunchShape& sh, const float* Q, float* b, float* dU, int N, int L, int Lv,
-                        const SliceTable& st, const int2* slc, int cwf, hipStream_t s) {
-    const int a = st.t[0].d1, c = st.nterms > 1 ? st.t[1].d1 : 0;
-    const bool narrow = narrow_rows(st.rows, st.t[0].ldv);
-    if (a == 3 && c == 0) DCRF_ADJ_FUSED(R, 3, 0);
-    else if (a == 6 && c == 0) DCRF_ADJ_FUSED(R, 6, 0);
-    else if (a == 3 && c == 6) DCRF_ADJ_FUSED(R, 3, 6);
-    else if (a == 6 && c == 3) DCRF_ADJ_FUSED(R, 6, 3);
-    else if (a == 4 && c == 5) DCRF_ADJ_FUSED(R, 4, 5);
-    else if (a == 5 && c == 4) DCRF_ADJ_FUSED(R, 5, 4);
-    else throw Error{DCRF_ERR_VALUE, "no fused adjoint kernel for these terms"};
-    DCRF_HIP_CHECK(hipGetLastError());
-}
-#undef DCRF_ADJ_FUSED
-#undef DCRF_FUSED_FORM
-
-#define DCRF_RUNS(R_, D0_, D1_)                                                                           \
-    k_meanfield_runs<R_, D0_, D1_><<<rs.n_runs, kWaveBlock, lds, s>>>(U, Q, ldq, N, L, Lv, sh.S, sh.per, st, rs)
-
-template <int R>
-void launch_runs_r(const LaunchShape& sh, const float* U, float* Q, int ldq, int N, int L, int Lv,
-                   const SliceTable& st, const RunSliceDev& rs, size_t lds, hipStream_t s) {
-    const int a = st.t[0].d1, b = st.nterms > 1 ? st.t[1].d1 : 0;
-    if (a == 3 && b == 0) DCRF_RUNS(R, 3, 0);
-    else if (a == 6 && b == 0) DCRF_RUNS(R, 6, 0);
-    else if (a == 3 && b == 6) DCRF_RUNS(R, 3, 6);
-    else if (a == 6 && b == 3) DCRF_RUNS(R, 6, 3);
-    else if (a == 4 && b == 5) DCRF_RUNS(R, 4, 5);
-    else if (a == 5 && b == 4) DCRF_RUNS(R, 5, 4);
-    else throw Error{DCRF_ERR_VALUE, "no run mean-field kernel for these terms"};
-    DCRF_HIP_CHECK(hipGetLastError());
-}
-#undef DCRF_RUNS
-
-size_t meanfield_runs_lds(int L, int ds, int P, int rows_lds, int cwf) {
-    (void)L;
-    return (size_t)rows_lds * sizeof(float) + (size_t)P * ds * sizeof(int2) + (size_t)cwf * sizeof(float);
-}
-
-void launch_meanfield_runs(const float* U, float* Q, int ldq, int N, int L, int Lv, const SliceTable& st_in,
-                           const RunSliceDev& rs, hipStream_t s) {
-    SliceTable st = st_in;
-    const int cwf = assign_compat_lds(st, L);
-    const LaunchShape sh = shape_for(Lv);
-    if (!fused_meanfield_ok(L, st.nterms, st.t[0].d1, st.nterms > 1 ? st.t[1].d1 : 0))
-        throw Error{DCRF_ERR_VALUE, "no run mean-field kernel for these terms"};
-    const int ds = st.t[0].d1 + (st.nterms > 1 ? st.t[1].d1 : 0);
-    const size_t lds = meanfield_runs_lds(L, ds, rs.P, rs.rows_lds, cwf);
-    static size_t granted[5] = {};
-    auto grant = [&](const void* fn, int r) {
-        if (lds > granted[r]) {
-            DCRF_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            granted[r] = lds;
-        }
-    };
-    const int a = st.t[0].d1, b = st.nterms > 1 ? st.t[1].d1 : 0;
-    auto fn_for = [&](auto rtag) -> const void* {
-        constexpr int R_ = decltype(rtag)::value;
-        if (a == 3 && b == 0) return reinterpret_cast<const void*>(&k_meanfield_runs<R_, 3, 0>);
-        if (a == 6 && b == 0) return reinterpret_cast<const void*>(&k_meanfield_runs<R_, 6, 0>);
-        if (a == 3 && b == 6) return reinterpret_cast<const void*>(&k_meanfield_runs<R_, 3, 6>);
-        if (a == 4 && b == 5) return reinterpret_cast<const void*>(&k_meanfield_runs<R_, 4, 5>);
-        if (a == 5 && b == 4) return reinterpret_cast<const void*>(&k_meanfield_runs<R_, 5, 4>);
-        return reinterpret_cast<const void*>(&k_meanfield_runs<R_, 6, 3>);
-    };
-    switch (sh.R) {
-        case 1: grant(fn_for(std::integral_constant<int, 1>{}), 1); launch_runs_r<1>(sh, U, Q, ldq, N, L, Lv, st, rs, lds, s); break;
-        case 2: grant(fn_for(std::integral_constant<int, 2>{}), 2); launch_runs_r<2>(sh, U, Q, ldq, N, L, Lv, st, rs, lds, s); break;
-        case 3: grant(fn_for(std::integral_constant<int, 3>{}), 3); launch_runs_r<3>(sh, U, Q, ldq, N, L, Lv, st, rs, lds, s); break;
-        default: grant(fn_for(std::integral_constant<int, 4>{}), 4); launch_runs_r<4>(sh, U, Q, ldq, N, L, Lv, st, rs, lds, s); break;
-    }
-}
-
-void launch_meanfield_fused(const float* U, float* Q, int ldq, int N, int L, int Lv, const SliceTable& st_in,
-                            const int2* slc, hipStream_t s, int bw) {
-    SliceTable st = st_in;
-    const int cwf = assign_compat_lds(st, L, true);  // 16-byte rows for matrix_piece_rows
-    const LaunchShape sh = shape_for(Lv);
-    if (!fused_meanfield_ok(L, st.nterms, st.t[0].d1, st.nterms > 1 ? st.t[1].d1 : 0))
-        throw Error{DCRF_ERR_VALUE, "no fused mean-field kernel for these terms"};
-    switch (sh.R) {
-        case 1: launch_fused_r<1>(sh, U, Q, ldq, N, L, st, slc, cwf, bw, s); break;
-        case 2: launch_fused_r<2>(sh, U, Q, ldq, N, L, st, slc, cwf, bw, s); break;
-        case 3: launch_fused_r<3>(sh, U, Q, ldq, N, L, st, slc, cwf, bw, s); break;
-        default: launch_fused_r<4>(sh, U, Q, ldq, N, L, st, slc, cwf, bw, s); break;
-    }
-}
-
 namespace {
 // Entry (pixel, weight) -> (its 8 x 8 block position, weight) for an image W pixels wide.
 __global__ void k_entry_block(const int2* __restrict__ ent, size_t E, int W, int2* __restrict__ out) {
@@ -1571,21 +1086,6 @@ void launch_entry_block(const int2* ent, size_t E, int W, int2* out, hipStream_t
     if (!E) return;
     k_entry_block<<<blocks_for(E), kThreads, 0, s>>>(ent, E, W, out);
     DCRF_HIP_CHECK(hipGetLastError());
-}
-
-void launch_adjoint_fused(const float* Q, float* b, float* dU, int N, int L, int Lv, const SliceTable& st_in,
-                          const int2* slc, hipStream_t s) {
-    SliceTable st = st_in;
-    const int cwf = assign_compat_lds(st, L, true);  // 16-byte rows for matrix_piece_rows
-    const LaunchShape sh = shape_for(Lv);
-    if (!fused_meanfield_ok(L, st.nterms, st.t[0].d1, st.nterms > 1 ? st.t[1].d1 : 0))
-        throw Error{DCRF_ERR_VALUE, "no fused adjoint kernel for these terms"};
-    switch (sh.R) {
-        case 1: launch_adj_fused_r<1>(sh, Q, b, dU, N, L, Lv, st, slc, cwf, s); break;
-        case 2: launch_adj_fused_r<2>(sh, Q, b, dU, N, L, Lv, st, slc, cwf, s); break;
-        case 3: launch_adj_fused_r<3>(sh, Q, b, dU, N, L, Lv, st, slc, cwf, s); break;
-        default: launch_adj_fused_r<4>(sh, Q, b, dU, N, L, Lv, st, slc, cwf, s); break;
-    }
 }
 
 int assign_compat_lds(SliceTable& st, int L, bool pad) {
