@@ -37,7 +37,6 @@ void set_error(int code, const std::string& msg) {
 namespace {
 
 constexpr int kDefaultChunk = 32;
-constexpr int kCombineSplit = 16;  // longest serial chain of partial rows in one combine
 
 struct TermLayout {
     DevBuf<int2> nbr;    // [(d+1)][V] global rows
@@ -315,17 +314,11 @@ struct dcrf_model {
 
     // global filter layout
     bool layout_valid = false;
-    int V_total = 0, rows0 = 0, E_total = 0, C_total = 0, CB_total = 0, CB2_total = 0, max_d = 0;
+    int V_total = 0, rows0 = 0, E_total = 0, max_d = 0;
     std::vector<int> order, vbase;
     std::vector<int> prefixV;
     DevBuf<float> vals[2];
-    DevBuf<Chunk> g_chunks;
-    DevBuf<Combine> g_comb, g_comb2;  // combine pieces, then the second level of split vertices
-    // host scratch of the layout's in-wave runs, kept between layout builds (a kernel-
-    // parameter change rebuilds the layout; fresh vectors cost their page faults each time)
-    std::vector<Chunk> gch_scratch;
-    std::vector<int> runs_scratch, first_scratch;
-    bool comb_waves = false;          // g_comb is a one-launch list (launch_combine_waves)
+    SegLists seg;                      // splat segments and recombination items
     DevBuf<int> g_tile_seg, g_tile_e;  // first segment / entry of each tile
     bool tiled = false;                // splat through LDS tiles (else the global form)
     size_t lds_cap = 0;                // LDS bytes one workgroup may allocate
@@ -566,96 +559,6 @@ TileGeom tile_geom(const dcrf_model& m) {
                     m.geo.n_inst, m.geo.is2d ? 1 : 0, m.tiles.side};
 }
 
-// Most entries and segments of one tile, from first-of-tile tables.
-int max_run(const std::vector<int>& first) {
-    int mx = 0;
-    for (size_t t = 0; t + 1 < first.size(); t++) mx = std::max(mx, first[t + 1] - first[t]);
-    return mx;
-}
-
-// The splat's wave mode loads a wave's entries as one range: consecutive segments must
-// adjoin (segment c+1 begins where segment c ends), which the tile-major layout gives.
-void require_adjoining(const std::vector<Chunk>& ch) {
-    for (size_t c = 1; c < ch.size(); c++)
-        if (ch[c].beg != ch[c - 1].end) throw Error{DCRF_ERR_STATE, "splat layout: segments do not adjoin"};
-}
-
-// norm = K*1 for one term (pairwise.cpp:44), then the normalisation of :46-61.
-void compute_norm(dcrf_model& m, Term& t) {
-    TermLattice& lat = t.lat;
-    const int N = m.N(), d1 = lat.d + 1, V = lat.V, E = N * d1;
-    hipStream_t s = m.stream;
-    DevBuf<int> tseg, te;
-    DevBuf<int2> ent;
-    DevBuf<float> sw, vals0, vals1, ones;
-    DevBuf<Chunk> ch;
-    DevBuf<Combine> cb;
-    DevBuf<int2> nbr;
-    ent.reserve(E);
-    sw.reserve(E);
-    // one term: entry positions are the sorted positions; rows V+1.. hold the partials
-    std::vector<Chunk> hch = lat.chunks;
-    for (auto& c : hch) c.out = c.out >= 0 ? c.out : V + 1 + (-c.out - 1);
-    require_adjoining(hch);
-    std::vector<Combine> hcb = lat.combines;
-    for (auto& c : hcb) c.first += V + 1;
-    upload(ch, hch, s);
-    upload(cb, hcb, s);
-    upload(tseg, lat.chunk_tile_ptr, s);
-    upload(te, lat.tile_ptr, s);
-    const TileGeom tg = tile_geom(m);
-    const TiledSplat ts{ch.get(), tseg.get(), te.get(), lat.n_tiles, tg, max_run(lat.tile_ptr),
-                        max_run(lat.chunk_tile_ptr)};
-    const bool tiled = tiled_splat_lds(1, tg.side, ts.e_max, ts.s_max, m.lds_cap) > 0;
-    launch_entry_gather(lat.csr_e.get(), E, d1, lat.bary.get(), nullptr, 0, nullptr, nullptr, 0, tiled ? &tg : nullptr,
-                        ent.get(), s);
-    const int rows = V + 1 + lat.n_partials;
-    vals0.reserve(rows);
-    vals1.reserve(V + 1);
-    launch_fill(vals0.get(), 0.f, rows, s);
-    launch_fill(vals1.get(), 0.f, V + 1, s);
-    nbr.reserve((size_t)d1 * V);
-    launch_remap_nbr(lat.nbr.get(), nbr.get(), d1 * V, 0, V, s);
-    ones.reserve(N);
-    launch_fill(ones.get(), 1.f, N, s);
-    if (tiled)
-        launch_splat_tiled(ts, ent.get(), ones.get(), vals0.get(), 1, 1, m.lds_cap, s);
-    else
-        launch_splat(ch.get(), (int)hch.size(), ent.get(), ones.get(), N, 1, vals0.get(), 1, 1, s);
-    launch_combine(cb.get(), (int)hcb.size(), vals0.get(), 1, 1, s);
-    BlurTable bt{};
-    bt.nterms = 1;
-    bt.t[0] = BlurTerm{0, V, lat.d, nbr.get()};
-    float* bufs[2] = {vals0.get(), vals1.get()};
-    for (int step = 0; step <= lat.d; step++)
-        launch_blur(bufs[step & 1], bufs[(step + 1) & 1], 0, V, 1, 1, bt, step, 0, s);
-    DevBuf<int> gv;
-    gv.reserve(E);
-    launch_slice_weights(lat.vtx.get(), lat.bary.get(), nullptr, 0, slice_alpha(lat.d), N, d1, 0, gv.get(), sw.get(), s);
-    SliceTable st{};
-    st.nterms = 1;
-    st.t[0] = SliceTerm{gv.get(), sw.get(), bufs[d1 & 1], d1, -1, nullptr, nullptr, nullptr, 1};
-    t.norm.reserve(N);
-    launch_slice_term(t.norm.get(), N, 1, 1, st, 0, s);
-    if (t.ntype == DCRF_NO_NORMALIZATION) {
-        // mean_norm = N / sum(norm) per instance, in float (pairwise.cpp:46-53)
-        std::vector<float> h(N);
-        DCRF_HIP_CHECK(hipMemcpyAsync(h.data(), t.norm.get(), sizeof(float) * N, hipMemcpyDeviceToHost, s));
-        DCRF_HIP_CHECK(hipStreamSynchronize(s));
-        for (int i = 0; i < m.geo.n_inst; i++) {
-            const int b = m.geo.pix_base[i], e = m.geo.pix_base[i + 1];
-            float mean = 0.f;
-            for (int p = b; p < e; p++) mean += h[p];
-            mean = (float)(e - b) / mean;
-            for (int p = b; p < e; p++) h[p] = mean;
-        }
-        DCRF_HIP_CHECK(hipMemcpyAsync(t.norm.get(), h.data(), sizeof(float) * N, hipMemcpyHostToDevice, s));
-    } else {
-        launch_norm_finish(t.norm.get(), N, t.ntype, s);
-    }
-    DCRF_HIP_CHECK(hipStreamSynchronize(s));
-}
-
 // Multi-step blur schedule: a lattice runs its d+1 steps in ceil((d+1)/K) passes of at
 // most K steps, spread as evenly as possible (longer passes first); the number of passes
 // falls with d, so in the global filter pass p covers a prefix of the vertex space.
@@ -705,6 +608,26 @@ void build_pass_tables(const int2* nbr, int V, int d, int vbase, int zero_row, s
     }
 }
 
+// The counting of the segment lists for rows of Lr floats (padding included): in-wave runs
+// where a segment's lanes fit a wave (and runs is set), recombination in one launch.
+void plan_segments(const RunSet& rs, int Lr, bool runs, SegPlan& P, hipStream_t s) {
+    const LaunchShape sh = shape_for(Lr);
+    count_segments(rs, sh.wave && runs ? splat_shape(Lr).per : 0, sh.wave ? sh.per : 0, P, s);
+}
+
+// Splat of rows of Lr floats (stride Lr) over a list, and its recombination.
+void splat_lists(const SegLists& l, const int2* ent, const float* in, size_t rows_in, int Lr, float* vals,
+                 hipStream_t s) {
+    launch_splat(l.ch.get(), l.nch, ent, in, rows_in, Lr, vals, Lr, Lr, s);
+}
+void combine_lists(const SegLists& l, int Lr, float* vals, hipStream_t s) {
+    if (l.waves)
+        launch_combine_waves(l.cb.get(), l.ncb, vals, Lr, Lr, s);
+    else
+        launch_combine(l.cb.get(), l.ncb, vals, Lr, Lr, s);
+    launch_combine(l.cb2.get(), l.ncb2, vals, Lr, Lr, s);
+}
+
 // ---------------------------------------------------------------- kernel-parameter gradient
 // The blur passes of one layout (x: the x chains, else the forward and reverse chains
 // of the paired inputs) from the splat rows src through the ping-pong pair buf: pass p
@@ -749,7 +672,7 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
     std::vector<KgPart> old = std::move(P.parts);
     P.parts.clear();
     P.passes = 0;
-    int row = 0, xrow = 0, parts_total = 0;
+    int row = 0, xrow = 0;
     size_t E = 0;
     for (size_t i = 0; i < terms.size(); i++) {
         const int k = terms[i];
@@ -765,41 +688,36 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
         part.X = xrow;
         row += 2 * lat.V;
         xrow += lat.V;
-        parts_total += lat.n_partials;
         E += (size_t)N * (lat.d + 1);
         P.passes = std::max(P.passes, part.passes);
         P.parts.push_back(std::move(part));
     }
     P.Z2 = row;
     P.Z1 = xrow;
-    // merged segments: entries of the i-th term from e0, its partial rows from p0 after
-    // the zero row
-    std::vector<Chunk> ch2;
-    std::vector<Combine> cb2;
-    P.ent.reserve(E);
-    size_t e0 = 0;
-    int p0 = 0;
-    for (size_t i = 0; i < P.parts.size(); i++) {
-        const KgPart& part = P.parts[i];
-        const TermLattice& lat = m.terms[part.term]->lat;
-        const int d1 = lat.d + 1;
-        launch_entry_gather(lat.csr_e.get(), N * d1, d1, lat.bary.get(), nullptr, 0, nullptr, nullptr, 0, nullptr,
-                            P.ent.get() + e0, s, (int)i * N);
-        for (const Chunk& c : lat.chunks)
-            ch2.push_back(Chunk{part.F + c.v, c.beg + (int)e0, c.end + (int)e0,
-                                c.out >= 0 ? part.F + c.out : P.Z2 + 1 + p0 + (-c.out - 1)});
-        for (const Combine& c : lat.combines)
-            cb2.push_back(Combine{part.F + c.v, P.Z2 + 1 + p0 + c.first, c.count, c.pad});
-        e0 += (size_t)N * d1;
-        p0 += lat.n_partials;
+    // merged segment lists in the x layout's rows (the terms' vertices one after another):
+    // one for x (L floats a row), one for [a | c] and one for the all-ones input (one
+    // float), whose rows are then moved to the paired layout
+    RunSet rs;
+    {
+        std::vector<const TermLattice*> lats;
+        std::vector<int> xbase;
+        for (const KgPart& part : P.parts) {
+            lats.push_back(&m.terms[part.term]->lat);
+            xbase.push_back(part.X);
+        }
+        build_run_set(lats, xbase, m.tiles.n_tiles(), m.chunk(), rs, s);
     }
-    require_adjoining(ch2);
-    if (!ch2.empty() && (ch2.front().beg != 0 || (size_t)ch2.back().end != E))
-        throw Error{DCRF_ERR_STATE, "kernel gradient: segments do not cover the entries"};
-    upload(P.ch2, ch2, s);
-    upload(P.cb2, cb2, s);
-    P.nch = (int)ch2.size();
-    P.ncb = (int)cb2.size();
+    SegPlan s1, s2, so;
+    plan_segments(rs, (int)L, true, s1, s);
+    plan_segments(rs, (int)(2 * L), true, s2, s);
+    plan_segments(rs, 1, true, so, s);
+    P.ent.reserve(E);
+    for (size_t i = 0; i < P.parts.size(); i++) {
+        const TermLattice& lat = m.terms[P.parts[i].term]->lat;
+        const int d1 = lat.d + 1;
+        launch_entry_gather(lat.csr_e.get(), N * d1, d1, lat.bary.get(), nullptr, 0, lat.tile_ptr.get(),
+                            rs.gebase.get(), rs.NT, rs.T, (int)i, nullptr, P.ent.get(), s, (int)i * N);
+    }
     KgRowMap rm{};
     rm.n = (int)P.parts.size();
     rm.Z2 = P.Z2;
@@ -808,9 +726,15 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
         rm.F[i] = P.parts[i].F;
         rm.X[i] = P.parts[i].X;
     }
-    P.ch1.reserve(P.nch);
-    P.cb1.reserve(P.ncb);
-    launch_kg_relayout(P.ch2.get(), P.nch, P.cb2.get(), P.ncb, rm, P.ch1.get(), P.cb1.get(), s);
+    DCRF_HIP_CHECK(hipStreamSynchronize(s));  // the counts
+    emit_segments(rs, s1, P.Z1 + 1, P.l1, s);
+    for (auto q : {std::make_pair(&s2, &P.l2), std::make_pair(&so, &P.lo)}) {
+        SegLists& l = *q.second;
+        emit_segments(rs, *q.first, P.Z1 + 1, l, s);
+        launch_kg_relayout(l.ch.get(), l.nch, l.cb.get(), l.ncb, rm, s);
+        launch_kg_relayout(nullptr, 0, l.cb2.get(), l.ncb2, rm, s);
+        l.rows += P.Z2 - P.Z1;
+    }
     // pass tables: pass p of term i expands the axes of its p-th pass; the forward chain
     // reads rows from F, the reverse chain from F in its first pass (the splat rows) and
     // from R after, the x chain from X
@@ -871,22 +795,21 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
         b.reserve(n);
         launch_fill(b.get(), 0.f, n, s);
     };
-    const size_t rows2 = (size_t)P.Z2 + 1 + parts_total;
-    zeroed(P.S2, rows2 * 2 * L);
+    zeroed(P.S2, (size_t)P.l2.rows * 2 * L);
     zeroed(P.X2[0], (size_t)(P.Z2 + 1) * 2 * L);
     zeroed(P.X2[1], (size_t)(P.Z2 + 1) * 2 * L);
-    zeroed(P.S1, ((size_t)P.Z1 + 1 + parts_total) * L);
+    zeroed(P.S1, (size_t)P.l1.rows * L);
     zeroed(P.B1, (size_t)(P.Z1 + 1) * L);
     // the all-ones input of every term (stacked, one value per pixel) through the plan's
     // splat and both chains; the reverse rows are the terms' K^T 1
-    zeroed(P.ones[0], rows2);
+    zeroed(P.ones[0], (size_t)P.lo.rows);
     zeroed(P.ones[1], (size_t)P.Z2 + 1);
     zeroed(P.ones[2], (size_t)P.Z2 + 1);
     DevBuf<float> in1;
     in1.reserve((size_t)P.parts.size() * N);
     launch_fill(in1.get(), 1.f, (size_t)P.parts.size() * N, s);
-    launch_splat(P.ch2.get(), P.nch, P.ent.get(), in1.get(), P.parts.size() * (size_t)N, 1, P.ones[0].get(), 1, 1, s);
-    launch_combine(P.cb2.get(), P.ncb, P.ones[0].get(), 1, 1, s);
+    splat_lists(P.lo, P.ent.get(), in1.get(), P.parts.size() * (size_t)N, 1, P.ones[0].get(), s);
+    combine_lists(P.lo, 1, P.ones[0].get(), s);
     float* const obuf[2] = {P.ones[1].get(), P.ones[2].get()};
     kg_blur(P, false, P.ones[0].get(), obuf, 1, s);
     for (KgPart& part : P.parts) part.ones_rev = obuf[(part.passes - 1) & 1] + part.R;
@@ -906,7 +829,8 @@ void ensure_kg_plans(dcrf_model& m) {
     for (int k = 0; k < (int)m.terms.size(); k++) {
         const Term& t = *m.terms[k];
         if (!t.num_kparams()) continue;
-        const long long ek = N * (t.lat.d + 1), rk = 2LL * t.lat.V + t.lat.n_partials;
+        // (at most one partial row per entry, and per 16 of those a second-level row)
+        const long long ek = N * (t.lat.d + 1), rk = 2LL * t.lat.V + ek / std::max(1, m.chunk()) + t.lat.n_runs;
         if (!g.empty() && ((int)g.size() == DCRF_MAX_TERMS / 2 || e + ek > lim || rows + rk + 1 > lim ||
                            (long long)(g.size() + 1) * N > lim)) {
             groups.push_back(g);
@@ -956,8 +880,8 @@ void kernel_grad_group(dcrf_model& m, const KgPlan& P, const float* b, const flo
         launch_kg_prepare(Qt, b, m.ldv, t.norm.get(), N, L, st, t.ntype, need_fa ? lbl + i * NL : nullptr,
                           pk + (size_t)i * 2 * NL, s);
     }
-    launch_splat(P.ch2.get(), P.nch, P.ent.get(), pk, (size_t)T * N, L2, P.S2.get(), L2, L2, s);
-    launch_combine(P.cb2.get(), P.ncb, P.S2.get(), L2, L2, s);
+    splat_lists(P.l2, P.ent.get(), pk, (size_t)T * N, L2, P.S2.get(), s);
+    combine_lists(P.l2, L2, P.S2.get(), s);
     float* const pbuf[2] = {P.X2[0].get(), P.X2[1].get()};
     kg_blur(P, false, P.S2.get(), pbuf, L2, s);
     float* const xbuf[2] = {P.B1.get(), P.S1.get()};  // pass 0 reads the splat rows S1
@@ -981,8 +905,8 @@ void kernel_grad_group(dcrf_model& m, const KgPlan& P, const float* b, const flo
             st.t[1] = SliceTerm{vtx, sw, need_fb ? fwd_of(i) + L : nullptr, d1, -1, nullptr, nullptr, nullptr, L2};  // K c
             launch_kg_x(b, m.ldv, lbl + (size_t)i * NL, t.norm.get(), N, L, st, t.ntype, x, s);
         }
-        launch_splat(P.ch1.get(), P.nch, P.ent.get(), xb, (size_t)T * N, L, P.S1.get(), L, L, s);
-        launch_combine(P.cb1.get(), P.ncb, P.S1.get(), L, L, s);
+        splat_lists(P.l1, P.ent.get(), xb, (size_t)T * N, L, P.S1.get(), s);
+        combine_lists(P.l1, L, P.S1.get(), s);
         kg_blur(P, true, P.S1.get(), xbuf, L, s);
     }
     for (int i = 0; i < T; i++) {
@@ -1066,8 +990,7 @@ void add_term(dcrf_model& m, int d, int ckind, const float* compat, int ktype, i
     if (t->lat.overflow)
         throw Error{DCRF_ERR_OVERFLOW,
                     "a lattice coordinate exceeds the int16 range of the lattice keys; scale the features down"};
-    build_chunks(t->lat, m.chunk());
-    compute_norm(m, *t);
+    // (the normaliser is computed with the layout)
     // DenseKernel keeps f_ and starts from unit scales / the identity (pairwise.cpp:116-122)
     t->feat0 = std::move(feat);
     t->kparams.assign(ktype == DCRF_FULL_KERNEL ? (size_t)d * d : (size_t)d, 0.0f);
@@ -1094,6 +1017,113 @@ int blur_launches(const dcrf_model& m) {
     return P;
 }
 
+BlurTable blur_table(const dcrf_model& m);
+
+// All blur passes over rows of Lv floats, between the buffers v0 (the splat rows) and v1:
+// afterwards term k's rows are in the one of result_parity(m, k).
+void blur_rows(dcrf_model& m, float* v0, float* v1, int Lv, bool transpose, hipStream_t s) {
+    float* const v[2] = {v0, v1};
+    const int L = m.L;
+    if (m.pairs) {
+        // up to three blur steps per pass; terms in layout order, pass p covers the
+        // terms with more than p passes (a prefix of the vertex space)
+        for (int p = 0; p < m.n_passes; p++) {
+            PassTable pt{};
+            pt.nterms = (int)m.order.size();
+            pt.zero_row = m.V_total;  // zero in both vertex buffers
+            double bytes = 0.0;
+            for (int i = 0; i < pt.nterms; i++) {
+                const int k = m.order[i];
+                const TermLattice& lat = m.terms[k]->lat;
+                const TermLayout& lay = *m.tl[k];
+                const bool on = (int)lay.pass_steps.size() > p;
+                const int steps = on ? lay.pass_steps[p] : 1;
+                pt.t[i] = PassTerm{m.vbase[k], lat.V,
+                                   on ? (transpose ? lay.passT.get() : lay.passF.get()) + lay.pass_off[p] : nullptr,
+                                   steps};
+                if (on) bytes += (double)lat.V * steps * (2.0 * L * 4 + 8);
+            }
+            Timed t(m, s, KC_BLUR, bytes);
+            const int pr = m.blur_r > 0 && (m.blur_small_v <= 0 || m.prefixP[p] < m.blur_small_v) ? m.blur_r : 0;
+            launch_blur_pass(v[p & 1], v[(p + 1) & 1], 0, m.prefixP[p], Lv, Lv, pt, s, pr);
+            t.done();
+        }
+        return;
+    }
+    const BlurTable bt = blur_table(m);
+    for (int step = 0; step <= m.max_d; step++) {
+        Timed t(m, s, KC_BLUR, (double)m.prefixV[step] * (2.0 * L * 4 + 8));
+        launch_blur(v[step & 1], v[(step + 1) & 1], 0, m.prefixV[step], Lv, Lv, bt, step,
+                    transpose ? 1 : 0, s);
+        t.done();
+    }
+}
+
+// The normalisers of all terms: norm = K 1 (pairwise.cpp:44), then the normalisation of
+// :46-61.  One filter of the all-ones input over every term's lattice, one float a row,
+// through the layout's run set and pass tables (so: the counts `so` for rows of one float).
+void compute_norms(dcrf_model& m, const RunSet& rs, const SegPlan& so, hipStream_t s) {
+    const int N = m.N(), T = (int)m.order.size(), V = m.V_total;
+    struct Untimed {  // these launches are no part of the timed classes
+        dcrf_model& m;
+        bool was;
+        explicit Untimed(dcrf_model& m_) : m(m_), was(m_.timing) { m.timing = false; }
+        ~Untimed() { m.timing = was; }
+    } untimed(m);
+    SegLists l;
+    emit_segments(rs, so, V + 1, l, s);
+    for (int i = 0; i < T; i++) {
+        const TermLattice& lat = m.terms[m.order[i]]->lat;
+        const int d1 = lat.d + 1;
+        launch_entry_gather(lat.csr_e.get(), N * d1, d1, lat.bary.get(), nullptr, 0, lat.tile_ptr.get(),
+                            rs.gebase.get(), rs.NT, T, i, nullptr, m.g_entF.get(), s);
+    }
+    DevBuf<float> ones, v0, v1;
+    ones.reserve(N);
+    v0.reserve(l.rows);
+    v1.reserve((size_t)V + 1);
+    launch_fill(ones.get(), 1.f, N, s);
+    launch_fill(v0.get(), 0.f, l.rows, s);
+    launch_fill(v1.get(), 0.f, (size_t)V + 1, s);
+    splat_lists(l, m.g_entF.get(), ones.get(), N, 1, v0.get(), s);
+    combine_lists(l, 1, v0.get(), s);
+    blur_rows(m, v0.get(), v1.get(), 1, false, s);
+    DevBuf<int> gv;
+    DevBuf<float> sw;
+    for (int k : m.order) {
+        Term& t = *m.terms[k];
+        const TermLattice& lat = t.lat;
+        const int d1 = lat.d + 1;
+        gv.reserve((size_t)N * d1);
+        sw.reserve((size_t)N * d1);
+        launch_slice_weights(lat.vtx.get(), lat.bary.get(), nullptr, 0, slice_alpha(lat.d), N, d1, m.vbase[k], gv.get(),
+                             sw.get(), s);
+        SliceTable st{};
+        st.nterms = 1;
+        st.t[0] = SliceTerm{gv.get(), sw.get(), result_parity(m, k) ? v1.get() : v0.get(), d1, -1, nullptr, nullptr,
+                            nullptr, 1};
+        t.norm.reserve(N);
+        launch_slice_term(t.norm.get(), N, 1, 1, st, 0, s);
+        if (t.ntype != DCRF_NO_NORMALIZATION) {
+            launch_norm_finish(t.norm.get(), N, t.ntype, s);
+            continue;
+        }
+        // mean_norm = N / sum(norm) per instance, in float (pairwise.cpp:46-53)
+        std::vector<float> h(N);
+        DCRF_HIP_CHECK(hipMemcpyAsync(h.data(), t.norm.get(), sizeof(float) * N, hipMemcpyDeviceToHost, s));
+        DCRF_HIP_CHECK(hipStreamSynchronize(s));
+        for (int i = 0; i < m.geo.n_inst; i++) {
+            const int b = m.geo.pix_base[i], e = m.geo.pix_base[i + 1];
+            float mean = 0.f;
+            for (int p = b; p < e; p++) mean += h[p];
+            mean = (float)(e - b) / mean;
+            for (int p = b; p < e; p++) h[p] = mean;
+        }
+        DCRF_HIP_CHECK(hipMemcpyAsync(t.norm.get(), h.data(), sizeof(float) * N, hipMemcpyHostToDevice, s));
+        DCRF_HIP_CHECK(hipStreamSynchronize(s));
+    }
+}
+
 void ensure_layout(dcrf_model& m) {
     if (m.layout_valid) return;
     m.drop_graph();
@@ -1101,8 +1131,6 @@ void ensure_layout(dcrf_model& m) {
     hipStream_t s = m.stream;
     const int T = (int)m.terms.size();
     const int N = m.N(), L = m.L;
-    for (auto& t : m.terms)
-        if (t->lat.chunk_len != m.chunk()) build_chunks(t->lat, m.chunk());
     // terms in layout order: more blur passes first (then higher d), so that the terms
     // of pass p are a prefix of the vertex space
     const std::vector<int> step_limit = pass_step_limits(m);
@@ -1115,8 +1143,7 @@ void ensure_layout(dcrf_model& m) {
         return m.terms[a]->lat.d > m.terms[b]->lat.d;
     });
     m.vbase.assign(T, 0);
-    std::vector<int> pbase(T, 0);
-    int V = 0, P = 0, E = 0;
+    int V = 0, E = 0;
     m.max_d = -1;
     m.all_symmetric = true;
     for (int k : m.order) {
@@ -1128,216 +1155,121 @@ void ensure_layout(dcrf_model& m) {
         if (m.terms[k]->ntype != DCRF_NORMALIZE_SYMMETRIC && m.terms[k]->ntype != DCRF_NO_NORMALIZATION)
             m.all_symmetric = false;
     }
-    for (int k : m.order) {
-        pbase[k] = V + 1 + P;
-        P += m.terms[k]->lat.n_partials;
-    }
     m.V_total = V;
-    m.rows0 = V + 1 + P;
     m.E_total = E;
-    // Segments and entries, tile by tile, the terms in layout order inside a tile: tile
-    // t's entries of term k (sorted positions tile_ptr[t] ..) move to ebase[k][t] + j.
+    // Segments and entries, tile by tile, the terms in layout order inside a tile
+    // (segments.hip).  In-wave runs: a vertex's segments that sit side by side in one wave
+    // are added inside the wave (k_splat folds each such run into its first lane group),
+    // which at 1024x768x21 cuts the partial rows from 188 k to 72 k and the vertices with
+    // more than 16 of them from 2,581 to 52.  The runs are part of the summation order, so
+    // every (tile, term) group starts a wave: an instance of a batch then gets the bits of
+    // the same image alone.  Vertices with more than 16 partial rows are recombined by a
+    // whole wave (their rows in pieces summed side by side), in block-mode shapes in two
+    // levels.  Block-mode shapes and the tiled splat have no in-wave runs.
     const int NT = m.tiles.n_tiles();
-    // the LDS-tiled splat (small tiles only) if the largest tile's entries and segments fit
-    int e_max = 0, s_max = 0;
-    for (int t = 0; t < NT; t++) {
-        int et = 0, st = 0;
+    RunSet rs;
+    {
+        std::vector<const TermLattice*> lats;
+        std::vector<int> vb;
         for (int k : m.order) {
-            const TermLattice& lat = m.terms[k]->lat;
-            et += lat.tile_ptr[t + 1] - lat.tile_ptr[t];
-            st += lat.chunk_tile_ptr[t + 1] - lat.chunk_tile_ptr[t];
+            lats.push_back(&m.terms[k]->lat);
+            vb.push_back(m.vbase[k]);
         }
-        e_max = std::max(e_max, et);
-        s_max = std::max(s_max, st);
+        build_run_set(lats, vb, NT, m.chunk(), rs, s);
     }
+    // the LDS-tiled splat (a tile side set by the caller) if the largest tile's entries and
+    // segments fit
     const TileGeom tg = tile_geom(m);
-    m.tiled = tiled_splat_lds(L, tg.side, e_max, s_max, m.lds_cap) > 0;
-    // In-wave runs (wave-mode shapes, global splat): a vertex's segments that sit side by
-    // side in one wave are added inside the wave (k_splat folds each such run into its
-    // first lane group); the later segments of a run get out = -1 and write nothing, and
-    // the vertex gets one partial row per run, or its final row when it has one run.  At
-    // 1024x768x21 this cuts the partial rows from 188 k to 72 k and the vertices with more
-    // than 16 of them from 2,581 to 52.  The runs are part of the summation order, so
-    // they must not depend on where a segment sits in the whole list: every (tile, term)
-    // group starts a wave (empty fillers, v = out = -1, pad the group before), and the
-    // empty segments of vertices that only padding lanes touch go to waves of their own
-    // at the end.  An instance of a batch then gets the bits of the same image alone.
-    // Block-mode shapes and the tiled splat keep one row per segment.
+    int e_max = 0, s_max = 0;
+    m.tiled = false;
+    SegPlan sp, so;
+    if (m.tile_side && T) {
+        count_segments(rs, 0, 0, sp, s);
+        std::vector<int> gs(rs.G + 1), ge(rs.G + 1), ts(NT + 1), te(NT + 1);
+        copy_to_host(gs.data(), sp.gseg.get(), sizeof(int) * gs.size(), s);
+        copy_to_host(ge.data(), rs.gebase.get(), sizeof(int) * ge.size(), s);
+        for (int t = 0; t <= NT; t++) {
+            ts[t] = gs[(size_t)t * T];
+            te[t] = ge[(size_t)t * T];
+        }
+        for (int t = 0; t < NT; t++) {
+            e_max = std::max(e_max, te[t + 1] - te[t]);
+            s_max = std::max(s_max, ts[t + 1] - ts[t]);
+        }
+        s_max += sp.host[0].empty;  // the empty segments go with the last tile
+        m.tiled = tiled_splat_lds(L, tg.side, e_max, s_max, m.lds_cap) > 0;
+        if (m.tiled) {
+            ts[NT] += sp.host[0].empty;
+            upload(m.g_tile_seg, ts, s);
+            upload(m.g_tile_e, te, s);
+            DCRF_HIP_CHECK(hipStreamSynchronize(s));  // (the lists above are on this frame)
+        }
+    }
     // (the LDS-tiled splat stages unpadded rows)
     m.ldv = m.tiled ? L : padded_labels(L);
-    const LaunchShape csh = shape_for(m.ldv);
-    const bool runs = csh.wave && !m.tiled;
-    const int per = splat_shape(m.ldv).per;  // segments per wave of the splat
-    std::vector<Chunk>& gch = m.gch_scratch;  // (capacity kept between layout builds)
-    gch.clear();
-    std::vector<int>& nruns = m.runs_scratch;
-    std::vector<int>& pfirst = m.first_scratch;
-    if (runs) {
-        nruns.assign(V + 1, 0);
-        pfirst.assign(V + 1, -1);
+    if (T) {
+        plan_segments(rs, m.ldv, !m.tiled, sp, s);
+        plan_segments(rs, 1, true, so, s);
     }
-    int slot = 0, prev = -1;  // position inside the current wave, the vertex before it
-    auto put = [&](const Chunk& x) {  // marks run heads (out = 1) and continuations (out = -1)
-        const bool h = x.v >= 0 && (slot == 0 || prev != x.v);
-        gch.push_back(Chunk{x.v, x.beg, x.end, h ? 1 : -1});
-        if (h) nruns[x.v]++;
-        prev = x.v;
-        if (++slot == per) slot = 0;
-    };
-    std::vector<Combine> gcb;
-    std::vector<int> gts(NT + 1), gte(NT + 1);
-    std::vector<std::vector<int>> ebase(T, std::vector<int>(NT));
-    std::vector<int> empty_segs;  // vertices of the empty segments (padding lanes only)
-    int e = 0;
-    for (int t = 0; t < NT; t++) {
-        gts[t] = (int)gch.size();
-        gte[t] = e;
-        for (int k : m.order) {
-            const TermLattice& lat = m.terms[k]->lat;
-            const int eb = e - lat.tile_ptr[t];
-            ebase[k][t] = eb;
-            for (int c = lat.chunk_tile_ptr[t]; c < lat.chunk_tile_ptr[t + 1]; c++) {
-                Chunk x = lat.chunks[c];
-                x.v += m.vbase[k];
-                x.beg += eb;
-                x.end += eb;
-                if (runs) {
-                    if (x.beg == x.end)
-                        empty_segs.push_back(x.v);
-                    else
-                        put(x);
-                    continue;
-                }
-                x.out = x.out >= 0 ? x.out + m.vbase[k] : pbase[k] + (-x.out - 1);
-                gch.push_back(x);
-            }
-            e += lat.tile_ptr[t + 1] - lat.tile_ptr[t];
-            if (runs)
-                while (slot) put(Chunk{-1, e, e, 0});
-        }
-    }
-    if (e != E) throw Error{DCRF_ERR_STATE, "splat layout: entry count mismatch"};
-    if (runs) {
-        for (int v : empty_segs) put(Chunk{v, e, e, 0});
-        while (slot) put(Chunk{-1, e, e, 0});
-    }
-    gts[NT] = (int)gch.size();
-    gte[NT] = e;
-    require_adjoining(gch);
-    upload(m.g_tile_seg, gts, s);
-    upload(m.g_tile_e, gte, s);
-    std::vector<Combine> combs;  // (vertex, first partial row, rows) of every split vertex
-    if (runs) {  // outputs: partial rows contiguous per vertex, in the order of its first run
-        int prow = V + 1;
-        for (Chunk& x : gch) {
-            if (x.out < 0) continue;  // a filler or a run's continuation
-            const int v = x.v;
-            if (nruns[v] == 1) {
-                x.out = v;
-                continue;
-            }
-            if (pfirst[v] < 0) {
-                pfirst[v] = prow;
-                combs.push_back(Combine{v, prow, nruns[v], 0});
-                prow += nruns[v];
-            }
-            x.out = pfirst[v]++;  // pfirst[v] walks the vertex's partial rows
-        }
-        m.rows0 = prow;
-    } else {
-        for (int k : m.order)
-            for (Combine c : m.terms[k]->lat.combines) {
-                c.v += m.vbase[k];
-                c.first += pbase[k];
-                combs.push_back(c);
-            }
-    }
-    // Vertices split into more than kCombineSplit partial rows must not leave one lane
-    // group a long serial chain (before the in-wave runs, the heaviest bilateral vertices
-    // at 1024x768 had ~245 partial rows).  Wave-mode shapes recombine in one launch
-    // (launch_combine_waves): such a vertex fills a whole wave, its rows cut into up to
-    // `per` pieces summed side by side and then added in piece order.  Block-mode shapes
-    // recombine in two levels: pieces of about kCombineSplit rows into second-level rows
-    // (appended after the partial rows), then those into the vertex row (a second launch).
-    std::vector<Combine> gcb2, heavy;
-    m.comb_waves = csh.wave;
-    for (const Combine& c : combs) {
-        if (c.count <= kCombineSplit) {
-            gcb.push_back(c);
-            continue;
-        }
-        if (m.comb_waves) {
-            const int pieces = std::min(csh.per, (c.count + kCombineSplit - 1) / kCombineSplit);
-            for (int j = 0, off = 0; j < csh.per; j++) {
-                const int n = j < pieces ? (c.count - off) / (pieces - j) : 0;
-                heavy.push_back(Combine{c.v, c.first + off, n, pieces});
-                off += n;
-            }
-            continue;
-        }
-        const int pieces = (c.count + kCombineSplit - 1) / kCombineSplit;
-        const int row2 = m.rows0;
-        m.rows0 += pieces;
-        for (int j = 0, off = 0; j < pieces; j++) {
-            const int n = (c.count - off) / (pieces - j);
-            gcb.push_back(Combine{row2 + j, c.first + off, n, 0});
-            off += n;
-        }
-        gcb2.push_back(Combine{c.v, row2, pieces, 0});
-    }
-    if (!heavy.empty()) {  // light items padded to whole waves, then one wave per heavy vertex
-        while (gcb.size() % csh.per) gcb.push_back(Combine{0, 0, 0, 0});
-        gcb.insert(gcb.end(), heavy.begin(), heavy.end());
-    }
-    m.C_total = (int)gch.size();
-    m.CB_total = (int)gcb.size();
-    m.CB2_total = (int)gcb2.size();
-    upload(m.g_chunks, gch, s);
-    upload(m.g_comb, gcb, s);
-    upload(m.g_comb2, gcb2, s);
-    m.tsplat = TiledSplat{m.g_chunks.get(), m.g_tile_seg.get(), m.g_tile_e.get(), NT, tg, e_max, s_max};
-
-    m.vals[0].reserve((size_t)m.rows0 * m.ldv);
-    m.vals[1].reserve((size_t)(V + 1) * m.ldv);
-    launch_fill(m.vals[0].get(), 0.f, (size_t)m.rows0 * m.ldv, s);
-    launch_fill(m.vals[1].get(), 0.f, (size_t)(V + 1) * m.ldv, s);
-    m.g_entF.reserve(E);
-    if (!m.all_symmetric) m.g_entT.reserve(E);
     m.tl.clear();
     m.tl.resize(T);
-    std::vector<DevBuf<int>> staging(2 * T);  // live until the synchronisation below
-    for (int i = 0; i < T; i++) {
-        const int k = m.order[i];
-        Term& t = *m.terms[k];
-        const TermLattice& lat = t.lat;
-        const int d1 = lat.d + 1, Ek = N * d1;
-        DevBuf<int>& tptr = staging[2 * i];
-        DevBuf<int>& eb = staging[2 * i + 1];
-        upload(tptr, lat.tile_ptr, s);
-        upload(eb, ebase[k], s);
-        const TileGeom* local = m.tiled ? &tg : nullptr;
-        launch_entry_gather(lat.csr_e.get(), Ek, d1, lat.bary.get(), t.norm.get(), pre_norm(t.ntype, false),
-                            tptr.get(), eb.get(), NT, local, m.g_entF.get(), s);
-        if (!m.all_symmetric)
-            launch_entry_gather(lat.csr_e.get(), Ek, d1, lat.bary.get(), t.norm.get(), pre_norm(t.ntype, true),
-                                tptr.get(), eb.get(), NT, local, m.g_entT.get(), s);
+    for (int k : m.order) {  // what the normalisers need
+        const TermLattice& lat = m.terms[k]->lat;
+        const int d1 = lat.d + 1;
         auto lay = std::make_unique<TermLayout>();
         lay->nbr.reserve((size_t)d1 * lat.V);
         launch_remap_nbr(lat.nbr.get(), lay->nbr.get(), d1 * lat.V, m.vbase[k], V, s);
         if (m.pairs)  // forward passes walk axes 0..d, the transpose's d..0 (permutohedral.cpp:556)
             build_pass_tables(lay->nbr.get(), lat.V, lat.d, m.vbase[k], V, lay->pass_steps, lay->pass_off,
                               lay->passF, lay->passT, s, step_limit[k]);
-        lay->vtx.reserve(Ek);
-        lay->swF.reserve(Ek);
+        m.tl[k] = std::move(lay);
+    }
+    m.n_passes = m.pairs ? blur_launches(m) : 0;
+    m.prefixP.assign(m.n_passes, 0);
+    for (int p = 0; p < m.n_passes; p++)
+        for (int k = 0; k < T; k++)
+            if ((int)m.tl[k]->pass_steps.size() > p) m.prefixP[p] += m.terms[k]->lat.V;
+    m.prefixV.assign(std::max(m.max_d + 1, 0), 0);
+    for (int st = 0; st <= m.max_d; st++)
+        for (int k = 0; k < T; k++)
+            if (m.terms[k]->lat.d >= st) m.prefixV[st] += m.terms[k]->lat.V;
+    m.g_entF.reserve(E);
+    if (!m.all_symmetric) m.g_entT.reserve(E);
+    DCRF_HIP_CHECK(hipStreamSynchronize(s));  // the counts
+    m.rows0 = V + 1;
+    if (T) {
+        emit_segments(rs, sp, V + 1, m.seg, s);
+        m.rows0 = m.seg.rows;
+        compute_norms(m, rs, so, s);
+    }
+    m.tsplat = TiledSplat{m.seg.ch.get(), m.g_tile_seg.get(), m.g_tile_e.get(), NT, tg, e_max, s_max};
+
+    m.vals[0].reserve((size_t)m.rows0 * m.ldv);
+    m.vals[1].reserve((size_t)(V + 1) * m.ldv);
+    launch_fill(m.vals[0].get(), 0.f, (size_t)m.rows0 * m.ldv, s);
+    launch_fill(m.vals[1].get(), 0.f, (size_t)(V + 1) * m.ldv, s);
+    for (int i = 0; i < T; i++) {
+        const int k = m.order[i];
+        Term& t = *m.terms[k];
+        const TermLattice& lat = t.lat;
+        TermLayout& lay = *m.tl[k];
+        const int d1 = lat.d + 1, Ek = N * d1;
+        const TileGeom* local = m.tiled ? &tg : nullptr;
+        launch_entry_gather(lat.csr_e.get(), Ek, d1, lat.bary.get(), t.norm.get(), pre_norm(t.ntype, false),
+                            lat.tile_ptr.get(), rs.gebase.get(), NT, T, i, local, m.g_entF.get(), s);
+        if (!m.all_symmetric)
+            launch_entry_gather(lat.csr_e.get(), Ek, d1, lat.bary.get(), t.norm.get(), pre_norm(t.ntype, true),
+                                lat.tile_ptr.get(), rs.gebase.get(), NT, T, i, local, m.g_entT.get(), s);
+        lay.vtx.reserve(Ek);
+        lay.swF.reserve(Ek);
         const float alpha = slice_alpha(lat.d);
         launch_slice_weights(lat.vtx.get(), lat.bary.get(), t.norm.get(), post_norm(t.ntype, false), alpha, N, d1,
-                             m.vbase[k], lay->vtx.get(), lay->swF.get(), s);
+                             m.vbase[k], lay.vtx.get(), lay.swF.get(), s);
         if (!m.all_symmetric) {
-            lay->swT.reserve(Ek);
+            lay.swT.reserve(Ek);
             launch_slice_weights(lat.vtx.get(), lat.bary.get(), t.norm.get(), post_norm(t.ntype, true), alpha, N, d1,
-                                 m.vbase[k], lay->vtx.get(), lay->swT.get(), s);
+                                 m.vbase[k], lay.vtx.get(), lay.swT.get(), s);
         }
-        m.tl[k] = std::move(lay);
     }
     // interleaved slice pairs for the fused mean-field kernel
     m.runs = false;
@@ -1377,15 +1309,6 @@ void ensure_layout(dcrf_model& m) {
             m.runs = m.mf_mode == 3 && lds <= 64 * 1024 && lds <= m.lds_cap;
         }
     }
-    m.prefixV.assign(std::max(m.max_d + 1, 0), 0);
-    for (int st = 0; st <= m.max_d; st++)
-        for (int k = 0; k < T; k++)
-            if (m.terms[k]->lat.d >= st) m.prefixV[st] += m.terms[k]->lat.V;
-    m.n_passes = m.pairs ? blur_launches(m) : 0;
-    m.prefixP.assign(m.n_passes, 0);
-    for (int p = 0; p < m.n_passes; p++)
-        for (int k = 0; k < T; k++)
-            if ((int)m.tl[k]->pass_steps.size() > p) m.prefixP[p] += m.terms[k]->lat.V;
     DCRF_HIP_CHECK(hipStreamSynchronize(s));
     m.layout_valid = true;
 }
@@ -1453,51 +1376,15 @@ void run_filter(dcrf_model& m, const float* in, bool transpose, hipStream_t s, c
         if (m.tiled)
             launch_splat_tiled(m.tsplat, ent, in, m.vals[0].get(), m.ldv, L, m.lds_cap, s);  // ldv == L
         else
-            launch_splat(m.g_chunks.get(), m.C_total, ent, in, in_rows(m, ent_in), Lv, m.vals[0].get(), Lv, Lv, s);
+            splat_lists(m.seg, ent, in, in_rows(m, ent_in), Lv, m.vals[0].get(), s);
         t.done();
     }
-    if (m.CB_total) {
+    if (m.seg.ncb) {
         Timed t(m, s, KC_COMBINE, 0.0);
-        if (m.comb_waves)
-            launch_combine_waves(m.g_comb.get(), m.CB_total, m.vals[0].get(), Lv, Lv, s);
-        else
-            launch_combine(m.g_comb.get(), m.CB_total, m.vals[0].get(), Lv, Lv, s);
-        if (m.CB2_total) launch_combine(m.g_comb2.get(), m.CB2_total, m.vals[0].get(), Lv, Lv, s);
+        combine_lists(m.seg, Lv, m.vals[0].get(), s);
         t.done();
     }
-    if (m.pairs) {
-        // up to three blur steps per pass; terms in layout order, pass p covers the
-        // terms with more than p passes (a prefix of the vertex space)
-        for (int p = 0; p < m.n_passes; p++) {
-            PassTable pt{};
-            pt.nterms = (int)m.order.size();
-            pt.zero_row = m.V_total;  // zero in both vertex buffers
-            double bytes = 0.0;
-            for (int i = 0; i < pt.nterms; i++) {
-                const int k = m.order[i];
-                const TermLattice& lat = m.terms[k]->lat;
-                const TermLayout& lay = *m.tl[k];
-                const bool on = (int)lay.pass_steps.size() > p;
-                const int steps = on ? lay.pass_steps[p] : 1;
-                pt.t[i] = PassTerm{m.vbase[k], lat.V,
-                                   on ? (transpose ? lay.passT.get() : lay.passF.get()) + lay.pass_off[p] : nullptr,
-                                   steps};
-                if (on) bytes += (double)lat.V * steps * (2.0 * L * 4 + 8);
-            }
-            Timed t(m, s, KC_BLUR, bytes);
-            const int pr = m.blur_r > 0 && (m.blur_small_v <= 0 || m.prefixP[p] < m.blur_small_v) ? m.blur_r : 0;
-            launch_blur_pass(m.vals[p & 1].get(), m.vals[(p + 1) & 1].get(), 0, m.prefixP[p], Lv, Lv, pt, s, pr);
-            t.done();
-        }
-        return;
-    }
-    const BlurTable bt = blur_table(m);
-    for (int step = 0; step <= m.max_d; step++) {
-        Timed t(m, s, KC_BLUR, (double)m.prefixV[step] * (2.0 * L * 4 + 8));
-        launch_blur(m.vals[step & 1].get(), m.vals[(step + 1) & 1].get(), 0, m.prefixV[step], Lv, Lv, bt, step,
-                    transpose ? 1 : 0, s);
-        t.done();
-    }
+    blur_rows(m, m.vals[0].get(), m.vals[1].get(), Lv, transpose, s);
 }
 
 void prepare(dcrf_model& m) {
@@ -2449,7 +2336,7 @@ int dcrf_set_kernel_params(dcrf_model* m, const float* params) {
         for (int i = 0; i < np; i++) require(std::isfinite(params[i]), "kernel parameters must be finite");
         ensure_device(*m);
         hipStream_t s = m->stream;
-        // new lattices and normalisers of every scaled term first, then commit them all
+        // new lattices of every scaled term first, then commit them all
         struct Rebuilt {
             Term* t;
             Term tmp;
@@ -2476,13 +2363,10 @@ int dcrf_set_kernel_params(dcrf_model* m, const float* params) {
             if (r->tmp.lat.overflow)
                 throw Error{DCRF_ERR_OVERFLOW, "a scaled lattice coordinate exceeds the int16 range of the lattice "
                                                "keys; scale the kernel parameters down"};
-            build_chunks(r->tmp.lat, m->chunk());
-            compute_norm(*m, r->tmp);
             done.push_back(std::move(r));
         }
         for (auto& r : done) {
             r->t->lat = std::move(r->tmp.lat);
-            r->t->norm = std::move(r->tmp.norm);
             r->t->kparams = std::move(r->kp);
         }
         if (!done.empty()) {
@@ -2670,12 +2554,14 @@ int dcrf_term_instance_vertices(const dcrf_model* m, int term, int inst, int* V)
     });
 }
 
-int dcrf_get_lattice(const dcrf_model* m, int term, int inst, int* offset, int* rank, float* bary, int* nbr,
+int dcrf_get_lattice(const dcrf_model* cm, int term, int inst, int* offset, int* rank, float* bary, int* nbr,
                      int16_t* keys, float* norm) {
     return guard([&] {
+        dcrf_model* m = const_cast<dcrf_model*>(cm);  // the normalisers come with the (cached) layout
         require(m != nullptr, "null model");
         require(term >= 0 && term < (int)m->terms.size(), "pairwise term index out of range");
         require(inst >= 0 && inst < m->geo.n_inst, "instance index out of range");
+        if (norm) ensure_layout(*m);
         const Term& t = *m->terms[term];
         const TermLattice& lat = t.lat;
         const int d1 = lat.d + 1;
@@ -2828,7 +2714,7 @@ int dcrf_splat_layout(dcrf_model* m, int* tiled, int* tile_side, int* n_tiles, i
         *tiled = m->tiled ? 1 : 0;
         *tile_side = m->tiles.side;
         *n_tiles = m->tiles.n_tiles();
-        *segments = m->C_total;
+        *segments = m->seg.nch;
         *partials = m->rows0 - m->V_total - 1;
         *meanfield = m->runs ? 2 : (m->fused ? 1 : 0);
     });

@@ -111,18 +111,47 @@ struct TermLattice {
     DevBuf<int> nbr;     // [(d+1)][V][2]
     DevBuf<int16_t> keys;  // [V][d]
     DevBuf<int> csr_e;     // [N*(d+1)] entry index p*(d+1)+r, sorted by (tile of p, vertex, p)
-    int n_tiles = 0;
-    std::vector<int> run_beg;   // runs of equal (tile, vertex) in csr_e order (size n_runs + 1)
-    std::vector<int> run_v, run_t;
-    std::vector<int> tile_ptr;  // first csr_e position of each tile (size n_tiles + 1)
-    // splat segments, term-local, listed tile by tile: out >= 0 vertex row, < 0 partial
-    // row -(r+1); chunk_tile_ptr[t] = first segment of tile t
-    std::vector<Chunk> chunks;
-    std::vector<int> chunk_tile_ptr;
-    std::vector<Combine> combines;  // vertices with more than one segment
-    int n_partials = 0;
-    int chunk_len = 0;
+    int n_tiles = 0, n_entries = 0;
+    int n_runs = 0;                      // runs of equal (tile, vertex) in csr_e order:
+    DevBuf<int> run_beg, run_v, run_t;   // first position (n_runs + 1 of them), vertex, tile
+    DevBuf<int> tile_run, tile_ptr;      // first run / csr_e position of each tile (n_tiles + 1)
 };
+
+// ---------------------------------------------------------------- splat segment lists
+// The runs of several terms merged tile by tile, terms in the given order inside a tile
+// (group g = tile * T + term); see segments.hip.
+struct RunSet {
+    int T = 0, NT = 0, G = 0, R = 0, V = 0, E = 0, C = 0;
+    DevBuf<int> mbase, gebase;   // [G + 1] first merged run / entry of each group
+    DevBuf<int> rv, rb, rl, rg;  // [R] vertex, first entry, entries, group
+    DevBuf<int> S;               // [R + 1] segments before each run
+    DevBuf<int> sv, si;          // [R] the runs sorted by vertex: vertex, merged index
+};
+struct SegCounts {
+    int partial, light, heavy, empty, pieces;
+};
+// The list sizes for per segments a splat wave (0: no in-wave runs) and perc lane groups a
+// recombination wave (0: two levels).
+struct SegPlan {
+    int per = 0, perc = 0;
+    DevBuf<int> gseg, H, vcount, vfirst;
+    DevBuf<SegCounts> vs;
+    SegCounts host[2] = {};  // totals; [1].partial: the groups' segments
+};
+struct SegLists {
+    DevBuf<Chunk> ch;
+    DevBuf<Combine> cb, cb2;
+    int nch = 0, ncb = 0, ncb2 = 0;
+    int rows = 0;        // rows up to the last partial (or second-level) row
+    bool waves = false;  // cb is a one-launch list (launch_combine_waves)
+};
+// vbase[i]: the first vertex of term i, the terms' vertices one after another.
+void build_run_set(const std::vector<const TermLattice*>& lats, const std::vector<int>& vbase, int n_tiles, int C,
+                   RunSet& rs, hipStream_t s);
+// Queues the counting; P.host is valid after the stream has been synchronised.
+void count_segments(const RunSet& rs, int per, int perc, SegPlan& P, hipStream_t s);
+// The lists, partial rows from row0 (after P's counts have arrived).
+void emit_segments(const RunSet& rs, const SegPlan& P, int row0, SegLists& L, hipStream_t s);
 
 // The lattice filters of the kernel-parameter gradient (the lattice_.compute and
 // Permutohedral::gradient calls of DenseKernel::featureGradient, pairwise.cpp:88-114,
@@ -147,10 +176,9 @@ struct KgPart {
 struct KgPlan {
     std::vector<KgPart> parts;
     int gen = -1;  // the model's lattice generation the plan was built for
-    int Z2 = 0, Z1 = 0, passes = 0, nch = 0, ncb = 0;
-    DevBuf<int2> ent;          // (stacked input row, barycentric weight bits) in segment order
-    DevBuf<Chunk> ch2, ch1;    // segments with output rows of the [a | c] and x layouts
-    DevBuf<Combine> cb2, cb1;  // vertices with several segments, in the two layouts
+    int Z2 = 0, Z1 = 0, passes = 0;
+    DevBuf<int2> ent;    // (stacked input row, barycentric weight bits) in segment order
+    SegLists l2, l1, lo;  // segment lists of the [a | c] and x layouts, and of the ones (paired rows)
     std::vector<int> vp2, vp1;  // per pass: one past the last row it writes
     DevBuf<int> tab;            // the pass tables of all chains
     std::vector<std::vector<int>> tab_off;  // per pass: forward, reverse, x table of each part
@@ -217,9 +245,6 @@ struct TileGeom {
 // (pad points zero).  Fills lat.{vtx,bary,rank,nbr,keys,csr_ptr,csr_e,V,inst_vbase}.
 void build_lattice(const Geometry& g, const GeometryDev& gd, const TileMap& tm, const float* feat, int d,
                    TermLattice& lat, float hash_load, hipStream_t s);
-// Splat segments (host): the runs of equal (tile, vertex) cut into pieces of at most
-// `chunk` entries, listed tile by tile.
-void build_chunks(TermLattice& lat, int chunk);
 // Feature generators into padded point-major layout [npad][d].
 void features_from_dxN(const Geometry& g, const GeometryDev& gd, const float* feat_dxN, int d,
                        float* out, hipStream_t s);
@@ -479,9 +504,8 @@ struct KgRowMap {
     int n, Z2, Z1;
     int F[DCRF_MAX_TERMS / 2], X[DCRF_MAX_TERMS / 2];
 };
-// ch1 / cb1 = ch / cb with their rows in the x layout.
-void launch_kg_relayout(const Chunk* ch, int nch, const Combine* cb, int ncb, const KgRowMap& m, Chunk* ch1,
-                        Combine* cb1, hipStream_t s);
+// The lists' rows from the x layout to the paired layout, in place.
+void launch_kg_relayout(Chunk* ch, int nch, Combine* cb, int ncb, const KgRowMap& m, hipStream_t s);
 // out[i] = (float)acc[i].
 void launch_kparam_store(const double* acc, int n, float* out, hipStream_t s);
 // Scaled features diag(P) f or P f (P column-major) over the padded table.
@@ -512,13 +536,13 @@ void launch_gram(const float* A, int LA, const float* B, int LB, int N, float* p
 
 // Global layout remaps.
 void launch_remap_nbr(const int* src, int2* dst, int n, int vbase, int zero_row, hipStream_t s);
-// Entry arrays of one term: sorted entry j (csr_e[j] = p*(d+1)+r) goes to position
-// base[t] + j, t the tile of j (tile_ptr: first j of each tile; base null: position j);
-// ent = (the pixel p, or its index inside its tile when `local` is given, plus pix_off;
+// Entry arrays of one term, the i-th of T merged ones: sorted entry j (csr_e[j] =
+// p*(d+1)+r) of tile t (tile_ptr: first j of each tile) goes to position gebase[t*T + i] +
+// j - tile_ptr[t]; ent = (the pixel p, or its index inside its tile when `local` is given, plus pix_off;
 // bits of the barycentric weight, times norm[p] when use_norm).
 void launch_entry_gather(const int* csr_e, int E, int d1, const float* bary, const float* norm, int use_norm,
-                         const int* tile_ptr, const int* base, int n_tiles, const TileGeom* local, int2* ent_out,
-                         hipStream_t s, int pix_off = 0);
+                         const int* tile_ptr, const int* gebase, int n_tiles, int T, int i, const TileGeom* local,
+                         int2* ent_out, hipStream_t s, int pix_off = 0);
 void launch_slice_weights(const int* vtx, const float* bary, const float* norm, int use_norm,
                           float alpha, int N, int d1, int vbase, int* gvtx, float* sw,
                           hipStream_t s);

@@ -351,10 +351,11 @@ __global__ void k_iota(int* p, int n) {
     if (i < n) p[i] = i;
 }
 
-// Sort key of a real entry: (tile of its pixel << vbits) | vertex.
+// Sort key of a real entry: (tile of its pixel << vbits) | vertex, in 32 bits where they
+// suffice (half the bytes of every pass of the sort).
+template <typename K>
 __global__ void k_entry_keys(const int* __restrict__ vtx, int Er, int d1, const int* pix_base, const int* Wd,
-                             const int* tile_base, int n_inst, int is2d, int side, int vbits,
-                             unsigned long long* __restrict__ key) {
+                             const int* tile_base, int n_inst, int is2d, int side, int vbits, K* __restrict__ key) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= Er) return;
     const int p = e / d1;
@@ -368,23 +369,43 @@ __global__ void k_entry_keys(const int* __restrict__ vtx, int Er, int d1, const 
     } else {
         tile = tile_base[i] + local / (side * side);
     }
-    key[e] = ((unsigned long long)(unsigned)tile << vbits) | (unsigned)vtx[e];
+    key[e] = ((K)(unsigned)tile << vbits) | (K)(unsigned)vtx[e];
 }
 
 // Starts of the runs of equal keys in a sorted array.
-__global__ void k_run_flags(const unsigned long long* __restrict__ key, int n, int* __restrict__ flag) {
+template <typename K>
+__global__ void k_run_flags(const K* __restrict__ key, int n, int* __restrict__ flag) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     flag[i] = (i == 0 || key[i] != key[i - 1]) ? 1 : 0;
 }
 
-__global__ void k_run_compact(const unsigned long long* __restrict__ key, const int* __restrict__ flag,
-                              const int* __restrict__ rid, int n, int* __restrict__ beg,
-                              unsigned long long* __restrict__ rkey) {
+// The runs: first position, vertex and tile of each, and the first run and position of
+// every tile (every tile has pixels, hence runs).
+template <typename K>
+__global__ void k_run_compact(const K* __restrict__ key, const int* __restrict__ flag, const int* __restrict__ rid,
+                              int n, int vbits, int n_tiles, int* __restrict__ beg, int* __restrict__ rv,
+                              int* __restrict__ rt, int* __restrict__ tile_run, int* __restrict__ tile_ptr) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !flag[i]) return;
-    beg[rid[i]] = i;
-    rkey[rid[i]] = key[i];
+    if (i >= n) return;
+    const int r = rid[i];
+    const K k = key[i];
+    const int t = (int)(k >> vbits);
+    if (flag[i]) {
+        beg[r] = i;
+        rv[r] = (int)(k & (((K)1 << vbits) - 1));
+        rt[r] = t;
+        if (i == 0 || (int)(key[i - 1] >> vbits) != t) {
+            tile_run[t] = r;
+            tile_ptr[t] = i;
+        }
+    }
+    if (i == n - 1) {
+        const int runs = r + flag[i];
+        beg[runs] = n;
+        tile_run[n_tiles] = runs;
+        tile_ptr[n_tiles] = n;
+    }
 }
 
 __global__ void k_gather_int(const int* __restrict__ src, const int* __restrict__ idx, int n,
@@ -398,6 +419,55 @@ uint32_t next_pow2(uint64_t x) {
     while (p < x) p <<= 1;
     if (p > (1ull << 31)) throw Error{DCRF_ERR_VALUE, "lattice hash table would exceed 2^31 slots"};
     return (uint32_t)p;
+}
+
+// Entries sorted by (tile of the pixel, vertex), stably (pixel order within a key), and the
+// runs of equal (tile, vertex): the splat segments are cut from the runs (segments.hip).
+template <typename K>
+void sort_entries(const Geometry& g, const GeometryDev& gd, const TileMap& tm, TermLattice& lat, int vbits, int tbits,
+                  hipStream_t s) {
+    const int Er = lat.n_entries, D1 = lat.d + 1;
+    DevBuf<int> iota, flag, rid;
+    DevBuf<K> key, sorted_key;
+    iota.reserve(Er);
+    key.reserve(Er);
+    sorted_key.reserve(Er);
+    k_iota<<<blocks_for(Er), kThreads, 0, s>>>(iota.get(), Er);
+    DCRF_HIP_CHECK(hipGetLastError());
+    k_entry_keys<K><<<blocks_for(Er), kThreads, 0, s>>>(lat.vtx.get(), Er, D1, gd.pix_base.get(), gd.W.get(),
+                                                        tm.base_dev.get(), g.n_inst, g.is2d ? 1 : 0, tm.side, vbits,
+                                                        key.get());
+    DCRF_HIP_CHECK(hipGetLastError());
+    size_t tb = 0;
+    DCRF_HIP_CHECK(rocprim::radix_sort_pairs(nullptr, tb, key.get(), sorted_key.get(), iota.get(), lat.csr_e.get(),
+                                             (size_t)Er, 0, vbits + tbits, s));
+    DevBuf<char> tmp;
+    tmp.reserve(tb);
+    DCRF_HIP_CHECK(rocprim::radix_sort_pairs(tmp.get(), tb, key.get(), sorted_key.get(), iota.get(), lat.csr_e.get(),
+                                             (size_t)Er, 0, vbits + tbits, s));
+    flag.reserve(Er);
+    rid.reserve(Er);
+    k_run_flags<K><<<blocks_for(Er), kThreads, 0, s>>>(sorted_key.get(), Er, flag.get());
+    DCRF_HIP_CHECK(hipGetLastError());
+    size_t sb = 0;
+    DCRF_HIP_CHECK(rocprim::exclusive_scan(nullptr, sb, flag.get(), rid.get(), 0, (size_t)Er, rocprim::plus<int>(), s));
+    DevBuf<char> stmp;
+    stmp.reserve(sb);
+    DCRF_HIP_CHECK(rocprim::exclusive_scan(stmp.get(), sb, flag.get(), rid.get(), 0, (size_t)Er, rocprim::plus<int>(), s));
+    int tail[2];
+    DCRF_HIP_CHECK(hipMemcpyAsync(&tail[0], rid.get() + (Er - 1), sizeof(int), hipMemcpyDeviceToHost, s));
+    DCRF_HIP_CHECK(hipMemcpyAsync(&tail[1], flag.get() + (Er - 1), sizeof(int), hipMemcpyDeviceToHost, s));
+    DCRF_HIP_CHECK(hipStreamSynchronize(s));
+    lat.n_runs = tail[0] + tail[1];
+    lat.run_beg.reserve(lat.n_runs + 1);
+    lat.run_v.reserve(lat.n_runs);
+    lat.run_t.reserve(lat.n_runs);
+    lat.tile_run.reserve(lat.n_tiles + 1);
+    lat.tile_ptr.reserve(lat.n_tiles + 1);
+    k_run_compact<K><<<blocks_for(Er), kThreads, 0, s>>>(sorted_key.get(), flag.get(), rid.get(), Er, vbits,
+                                                         lat.n_tiles, lat.run_beg.get(), lat.run_v.get(),
+                                                         lat.run_t.get(), lat.tile_run.get(), lat.tile_ptr.get());
+    DCRF_HIP_CHECK(hipGetLastError());
 }
 
 template <int D>
@@ -495,74 +565,18 @@ void build_lattice_d(const Geometry& g, const GeometryDev& gd, const TileMap& tm
         DCRF_HIP_CHECK(hipStreamSynchronize(s));
     }
 
-    // Entries sorted by (tile of the pixel, vertex), stably (pixel order within a key),
-    // and the runs of equal (tile, vertex): the splat segments are cut from the runs.
     lat.csr_e.reserve((size_t)Er);
     lat.n_tiles = tm.n_tiles();
-    {
-        int vbits = 1;
-        while ((1ll << vbits) <= (long long)V) vbits++;
-        int tbits = 1;
-        while ((1ll << tbits) <= (long long)lat.n_tiles) tbits++;
-        if (vbits + tbits > 63) throw Error{DCRF_ERR_VALUE, "too many lattice vertices and tiles"};
-        DevBuf<int> iota, flag2, rid;
-        DevBuf<unsigned long long> key, sorted_key;
-        iota.reserve(Er);
-        key.reserve(Er);
-        sorted_key.reserve(Er);
-        k_iota<<<blocks_for(Er), kThreads, 0, s>>>(iota.get(), Er);
-        DCRF_HIP_CHECK(hipGetLastError());
-        k_entry_keys<<<blocks_for(Er), kThreads, 0, s>>>(lat.vtx.get(), Er, D1, gd.pix_base.get(), gd.W.get(),
-                                                         tm.base_dev.get(), g.n_inst, g.is2d ? 1 : 0, tm.side,
-                                                         vbits, key.get());
-        DCRF_HIP_CHECK(hipGetLastError());
-        size_t tmp_bytes = 0;
-        DCRF_HIP_CHECK(rocprim::radix_sort_pairs(nullptr, tmp_bytes, key.get(), sorted_key.get(), iota.get(),
-                                                 lat.csr_e.get(), (size_t)Er, 0, vbits + tbits, s));
-        DevBuf<char> tmp;
-        tmp.reserve(tmp_bytes);
-        DCRF_HIP_CHECK(rocprim::radix_sort_pairs(tmp.get(), tmp_bytes, key.get(), sorted_key.get(), iota.get(),
-                                                 lat.csr_e.get(), (size_t)Er, 0, vbits + tbits, s));
-        flag2.reserve(Er);
-        rid.reserve(Er);
-        k_run_flags<<<blocks_for(Er), kThreads, 0, s>>>(sorted_key.get(), Er, flag2.get());
-        DCRF_HIP_CHECK(hipGetLastError());
-        size_t scan_bytes = 0;
-        DCRF_HIP_CHECK(rocprim::exclusive_scan(nullptr, scan_bytes, flag2.get(), rid.get(), 0, (size_t)Er,
-                                               rocprim::plus<int>(), s));
-        DevBuf<char> stmp;
-        stmp.reserve(scan_bytes);
-        DCRF_HIP_CHECK(rocprim::exclusive_scan(stmp.get(), scan_bytes, flag2.get(), rid.get(), 0, (size_t)Er,
-                                               rocprim::plus<int>(), s));
-        int tail[2];
-        DCRF_HIP_CHECK(hipMemcpyAsync(&tail[0], rid.get() + (Er - 1), sizeof(int), hipMemcpyDeviceToHost, s));
-        DCRF_HIP_CHECK(hipMemcpyAsync(&tail[1], flag2.get() + (Er - 1), sizeof(int), hipMemcpyDeviceToHost, s));
-        DCRF_HIP_CHECK(hipStreamSynchronize(s));
-        const int n_runs = tail[0] + tail[1];
-        DevBuf<int> rbeg;
-        DevBuf<unsigned long long> rkey;
-        rbeg.reserve(n_runs);
-        rkey.reserve(n_runs);
-        k_run_compact<<<blocks_for(Er), kThreads, 0, s>>>(sorted_key.get(), flag2.get(), rid.get(), Er, rbeg.get(),
-                                                          rkey.get());
-        DCRF_HIP_CHECK(hipGetLastError());
-        lat.run_beg.resize(n_runs + 1);
-        std::vector<unsigned long long> hk(n_runs);
-        copy_to_host(lat.run_beg.data(), rbeg.get(), sizeof(int) * n_runs, s);
-        copy_to_host(hk.data(), rkey.get(), sizeof(unsigned long long) * n_runs, s);
-        lat.run_beg[n_runs] = Er;
-        lat.run_v.resize(n_runs);
-        lat.run_t.resize(n_runs);
-        const unsigned long long vmask = (1ull << vbits) - 1;
-        for (int r = 0; r < n_runs; r++) {
-            lat.run_v[r] = (int)(hk[r] & vmask);
-            lat.run_t[r] = (int)(hk[r] >> vbits);
-        }
-        // first sorted entry of every tile
-        lat.tile_ptr.assign(lat.n_tiles + 1, Er);
-        for (int r = n_runs - 1; r >= 0; r--) lat.tile_ptr[lat.run_t[r]] = lat.run_beg[r];
-        for (int t = lat.n_tiles - 1; t >= 0; t--) lat.tile_ptr[t] = std::min(lat.tile_ptr[t], lat.tile_ptr[t + 1]);
-    }
+    lat.n_entries = Er;
+    int vbits = 1;
+    while ((1ll << vbits) <= (long long)V) vbits++;
+    int tbits = 1;
+    while ((1ll << tbits) <= (long long)lat.n_tiles) tbits++;
+    if (vbits + tbits > 63) throw Error{DCRF_ERR_VALUE, "too many lattice vertices and tiles"};
+    if (vbits + tbits <= 32)
+        sort_entries<unsigned>(g, gd, tm, lat, vbits, tbits, s);
+    else
+        sort_entries<unsigned long long>(g, gd, tm, lat, vbits, tbits, s);
 }
 
 // Run of pixel p: a TW x TH rectangle of its 2-D instance (row-major over the image), or
@@ -699,7 +713,7 @@ void build_run_slice(const Geometry& g, const GeometryDev& gd, const int2* slc, 
     tmp.reserve(tb);
     DCRF_HIP_CHECK(rocprim::radix_sort_pairs(tmp.get(), tb, key.get(), skey.get(), iota.get(), perm.get(), (size_t)n, 0,
                                              32 + rbits, s));
-    k_run_flags<<<blocks_for(n), kThreads, 0, s>>>(skey.get(), n, flag.get());
+    k_run_flags<unsigned long long><<<blocks_for(n), kThreads, 0, s>>>(skey.get(), n, flag.get());
     DCRF_HIP_CHECK(hipGetLastError());
     size_t sb = 0;
     DCRF_HIP_CHECK(rocprim::exclusive_scan(nullptr, sb, flag.get(), uid.get(), 0, (size_t)n, rocprim::plus<int>(), s));
@@ -760,55 +774,6 @@ void build_lattice(const Geometry& g, const GeometryDev& gd, const TileMap& tm, 
             throw Error{DCRF_ERR_VALUE, "feature dimension must be between 1 and " +
                                             std::to_string(DCRF_MAX_DIM)};
     }
-}
-
-void build_chunks(TermLattice& lat, int chunk) {
-    const int V = lat.V, n_runs = (int)lat.run_v.size(), T = lat.n_tiles;
-    std::vector<Chunk>& ch = lat.chunks;
-    ch.clear();
-    ch.reserve(n_runs + n_runs / 4 + 16);
-    std::vector<int> seg_tile;
-    seg_tile.reserve(ch.capacity());
-    // vertices without real contributors (created by padding lanes only) still need
-    // their row zeroed every iteration: an empty segment each, listed with tile 0
-    std::vector<char> seen(V, 0);
-    for (int r = 0; r < n_runs; r++) seen[lat.run_v[r]] = 1;
-    for (int v = 0; v < V; v++)
-        if (!seen[v]) {
-            ch.push_back(Chunk{v, 0, 0, v});
-            seg_tile.push_back(0);
-        }
-    std::vector<int> cnt(V, 0);
-    const size_t first_real = ch.size();
-    for (int r = 0; r < n_runs; r++) {
-        const int b = lat.run_beg[r], e = lat.run_beg[r + 1], v = lat.run_v[r];
-        for (int i = b; i < e; i += chunk) {
-            ch.push_back(Chunk{v, i, std::min(e, i + chunk), 0});
-            seg_tile.push_back(lat.run_t[r]);
-            cnt[v]++;
-        }
-    }
-    // vertices with one segment write their row directly; the others get partial rows,
-    // contiguous per vertex in segment (= tile) order, recombined by the combine pass
-    std::vector<int> pfirst(V, -1);
-    lat.combines.clear();
-    int prow = 0;
-    for (int v = 0; v < V; v++)
-        if (cnt[v] > 1) {
-            pfirst[v] = prow;
-            lat.combines.push_back(Combine{v, prow, cnt[v], 0});
-            prow += cnt[v];
-        }
-    std::vector<int> used(V, 0);
-    for (size_t c = first_real; c < ch.size(); c++) {
-        const int v = ch[c].v;
-        ch[c].out = pfirst[v] < 0 ? v : -(pfirst[v] + used[v]++) - 1;
-    }
-    lat.chunk_tile_ptr.assign(T + 1, (int)ch.size());
-    for (int c = (int)ch.size() - 1; c >= 0; c--) lat.chunk_tile_ptr[seg_tile[c]] = c;
-    for (int t = T - 1; t >= 0; t--) lat.chunk_tile_ptr[t] = std::min(lat.chunk_tile_ptr[t], lat.chunk_tile_ptr[t + 1]);
-    lat.n_partials = prow;
-    lat.chunk_len = chunk;
 }
 
 void features_from_dxN(const Geometry& g, const GeometryDev& gd, const float* feat_dxN, int d, float* out,
