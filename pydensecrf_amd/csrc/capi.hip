@@ -361,8 +361,8 @@ struct dcrf_model {
     DevBuf<float> obj_w;
     DevBuf<double> obj_partial;
     // kernel-parameter gradient: the filter plans (built on first use for the lattices of
-    // generation lat_gen, which every lattice change advances), 4 [N][L] work slabs per
-    // term of a plan (lbl, [a | c], x), 2 [N][d] feature gradients (one-thread-per-point
+    // generation lat_gen, which every lattice change advances), 3 [N][L] work slabs per
+    // term of a plan ([a | c], x), 2 [N][d] feature gradients (one-thread-per-point
     // form), per-block partials and the accumulated gradient of all terms
     std::vector<std::unique_ptr<KgPlan>> kgplans;
     int lat_gen = 0;
@@ -851,7 +851,7 @@ void ensure_kg_plans(dcrf_model& m) {
 
 // acc_k += kernelGradient(b, Q_t) for every term k of plan P (pairwise.cpp:202-207,
 // 152-163, 88-114): fg = -G(x, 1) + G(a, c) with a, c and x per the normalisation type.
-// Per term one pass forms lbl = C (w Q_t) and the inputs a and c; the [a | c] of all the
+// One pass forms the terms' inputs a and c from C (w Q_t) and b; the [a | c] of all the
 // plan's terms are splatted together and blurred in both orders: the forward rows give
 // K a (G(a, c), direction 0) and K c, the reverse rows K^T a and K^T c (G(a, c),
 // direction 1).  x (from the slices K^T a and K c in one pass per term) needs one more
@@ -864,22 +864,21 @@ void kernel_grad_group(dcrf_model& m, const KgPlan& P, const float* b, const flo
     const int N = m.N(), L = m.L, L2 = 2 * L;
     const size_t NL = (size_t)N * L;
     const int T = (int)P.parts.size();
-    float* lbl = m.kgbuf.get();                // [T][N][L]
-    float* pk = lbl + (size_t)T * NL;          // [T][N][2L]
-    float* xb = pk + (size_t)2 * T * NL;       // [T][N][L]
+    float* pk = m.kgbuf.get();            // [T][N][2L]
+    float* xb = pk + (size_t)2 * T * NL;  // [T][N][L]
     bool any_x = false;
+    SliceTable pst{};
+    KgInputs in{};
+    pst.nterms = T;
     for (int i = 0; i < T; i++) {
         const int k = P.parts[i].term;
         const Term& t = *m.terms[k];
-        const bool has_x = t.ntype != DCRF_NO_NORMALIZATION;
-        const bool need_fa = has_x && t.ntype != DCRF_NORMALIZE_AFTER;  // x reads fa and lbl
-        any_x = any_x || has_x;
-        SliceTable st{};
-        st.nterms = 1;
-        st.t[0] = SliceTerm{nullptr, nullptr, nullptr, 1, t.ckind, t.d_compat.get(), kw ? kw + k : nullptr, nullptr, L};
-        launch_kg_prepare(Qt, b, m.ldv, t.norm.get(), N, L, st, t.ntype, need_fa ? lbl + i * NL : nullptr,
-                          pk + (size_t)i * 2 * NL, s);
+        any_x = any_x || t.ntype != DCRF_NO_NORMALIZATION;
+        pst.t[i] = SliceTerm{nullptr, nullptr, nullptr, 1, t.ckind, t.d_compat.get(), kw ? kw + k : nullptr, nullptr, L};
+        in.norm[i] = t.norm.get();
+        in.ntype[i] = t.ntype;
     }
+    launch_kg_prepare(Qt, b, m.ldv, in, N, L, pst, pk, s);
     splat_lists(P.l2, P.ent.get(), pk, (size_t)T * N, L2, P.S2.get(), s);
     combine_lists(P.l2, L2, P.S2.get(), s);
     float* const pbuf[2] = {P.X2[0].get(), P.X2[1].get()};
@@ -903,7 +902,7 @@ void kernel_grad_group(dcrf_model& m, const KgPlan& P, const float* b, const flo
             const int d1 = t.lat.d + 1;
             st.t[0] = SliceTerm{vtx, sw, need_fa ? rev_of(i) : nullptr, d1, -1, nullptr, nullptr, nullptr, L2};  // K^T a
             st.t[1] = SliceTerm{vtx, sw, need_fb ? fwd_of(i) + L : nullptr, d1, -1, nullptr, nullptr, nullptr, L2};  // K c
-            launch_kg_x(b, m.ldv, lbl + (size_t)i * NL, t.norm.get(), N, L, st, t.ntype, x, s);
+            launch_kg_x(pk + (size_t)i * 2 * NL, t.norm.get(), N, L, st, t.ntype, x, s);
         }
         splat_lists(P.l1, P.ent.get(), xb, (size_t)T * N, L, P.S1.get(), s);
         combine_lists(P.l1, L, P.S1.get(), s);
@@ -1555,7 +1554,7 @@ void backward(dcrf_model& m, const float* dQ, float* dU, float* dcompat, float* 
         }
         size_t tmax = 1;
         for (const auto& P : m.kgplans) tmax = std::max(tmax, P->parts.size());
-        m.kgbuf.reserve(4 * tmax * NL);
+        m.kgbuf.reserve(3 * tmax * NL);
         if (dslow) m.kgdf.reserve((size_t)2 * N * dslow);
         pstride = kparam_partial_doubles(dmax);
         m.kpartial.reserve(pstride * T);

@@ -463,16 +463,19 @@ void launch_compat_finish(const double* G, int ckind, int L, const float* cw, co
 void launch_set_compat(const float* raw, int ckind, int L, float* cw, hipStream_t s);
 
 // ---------------------------------------------------------------- kernel-parameter gradient
-// lbl (optional) = C (w Q_t) of the term in st.t[0] (its compatibility and weight), and
-// P [N][2L] = [a | c], a = b (times n for SYMMETRIC / AFTER), c = lbl (times n for
-// SYMMETRIC / BEFORE).
-// Qt and b have rows of ldq floats.
-void launch_kg_prepare(const float* Qt, const float* b, int ldq, const float* norm, int N, int L, const SliceTable& st,
-                       int ntype, float* lbl, float* P, hipStream_t s);
-// The normaliser-derivative input x of featureGradient for ntype, with fa sliced by
-// st.t[0] and fb by st.t[1] (a term with null vals: not needed).
-void launch_kg_x(const float* b, int ldb, const float* lbl, const float* norm, int N, int L, const SliceTable& st, int ntype,
-                 float* x, hipStream_t s);
+// Per term k of st (its compatibility and weight) with normaliser norm[k] (n) of type
+// ntype[k]: the rows [a | c] of 2L floats at P + k N 2L, a = b (times n for SYMMETRIC /
+// AFTER), c = C (w Q_t) (times n for SYMMETRIC / BEFORE).  Qt and b have rows of ldq floats.
+struct KgInputs {
+    const float* norm[DCRF_MAX_TERMS / 2];
+    int ntype[DCRF_MAX_TERMS / 2];
+};
+void launch_kg_prepare(const float* Qt, const float* b, int ldq, const KgInputs& in, int N, int L, const SliceTable& st,
+                       float* P, hipStream_t s);
+// The normaliser-derivative input x of featureGradient for ntype from the term's rows
+// P, with fa sliced by st.t[0] and fb by st.t[1] (the same entries; null vals: not needed).
+void launch_kg_x(const float* P, const float* norm, int N, int L, const SliceTable& st, int ntype, float* x,
+                 hipStream_t s);
 // Whether launch_kg_grad has a kernel for L labels and feature dimension d.
 bool kg_grad_fused(int L, int d);
 // The parameter gradient of fg = -G(x, 1) + G(a, c) (xr null: fg = G(a, c)) against

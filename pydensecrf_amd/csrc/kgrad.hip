@@ -36,96 +36,172 @@ namespace {
 constexpr int kThreads = 256;
 inline unsigned blocks_for(size_t n, int t = kThreads) { return (unsigned)((n + t - 1) / t); }
 
-// lbl = C (w Q_t), the term's compatibility applied to its weighted Q_t
-// (PairwisePotential::kernelGradient, pairwise.cpp:202-207; st.t[0] carries the
-// compatibility and the weight), and the two filter inputs of featureGradient
-// (pairwise.cpp:88-114) side by side, P[p] = [a | c] (2L floats): a = b n (SYMMETRIC,
-// AFTER) or b, c = lbl n (SYMMETRIC, BEFORE) or lbl.  One splat and the two blur orders
-// of P give K a, K^T a, K c, K^T c.  lbl is stored only where the caller gives a buffer
-// (the normaliser input x reads it).
+// The two filter inputs of featureGradient (pairwise.cpp:88-114) of every term of a plan,
+// from one read of Q_t and b: per term lbl = C (w Q_t), the compatibility applied to the
+// weighted Q_t (PairwisePotential::kernelGradient, pairwise.cpp:202-207; st.t[k] carries
+// the compatibility and the weight), and the row P[k N + p] = [a | c] (2L floats), a = b n
+// (SYMMETRIC, AFTER) or b, c = lbl n (SYMMETRIC, BEFORE) or lbl.  One splat and the two
+// blur orders of P give K a, K^T a, K c, K^T c.  Matrix weights with an LDS copy read the
+// pixel's messages as rows there in wave mode (msg; matrix_piece_rows).
+// Bound: memory, 2 rows read and 2 written per term and point.  One launch per term, with
+// lbl stored beside P and the messages passed by shuffles, took 2 x 29 us at 512x512x21
+// with two Matrix terms; this form 44 us.
 template <bool WAVE, int R, bool CWL>
 __global__ void __launch_bounds__(1024) k_kg_prepare(const float* __restrict__ Qt, const float* __restrict__ b,
-                                                     int ldq, const float* __restrict__ norm, int N, int L, int S, int per,
-                                                     SliceTable st, int ntype, float* __restrict__ lbl,
-                                                     float* __restrict__ P) {
-    extern __shared__ float sh[];
+                                                     int ldq, KgInputs in, int N, int L, int S, int per,
+                                                     SliceTable st, int cwf, float* __restrict__ P) {
+    extern __shared__ __align__(16) float sh[];
     float* shc = sh + blockDim.x;
     if (CWL) stage_compat(st, L, shc);
     LaneGroup<WAVE, R> G(L, S, per, sh);
     const int p = G.item();
     const bool active = G.on && p < N;
-    const SliceTerm& T = st.t[0];
-    float m[R], bv[R], c[R];
-    float n = 0.0f;
+    float m[R], bv[R];
     if (active) {
         load_piece<R>(Qt + (size_t)p * ldq, G.k0, L, m);
         load_piece<R>(b + (size_t)p * ldq, G.k0, L, bv);
-        n = norm[p];
     } else {
 #pragma unroll
         for (int r = 0; r < R; r++) m[r] = bv[r] = 0.0f;
     }
-    if (T.kw) {
-        const float kw = T.kw[0];
+    const int ldm = (L + 3) & ~3;
+    float* msg = shc + cwf + (size_t)G.w * per * ldm;  // WAVE and CWL: the wave's message rows
+    for (int k = 0; k < st.nterms; k++) {
+        const SliceTerm& T = st.t[k];
+        float mk[R], c[R];
+        const float kw = T.kw ? T.kw[0] : 1.0f;
 #pragma unroll
-        for (int r = 0; r < R; r++) m[r] = m[r] * kw;
-    }
-    compat_piece<WAVE, R>(T, m, c, G, shc);  // every lane: Matrix reads its group
-    if (!active) return;
-    if (lbl) store_piece<R>(lbl + (size_t)p * L, G.k0, L, c);
-    const bool na = ntype == DCRF_NORMALIZE_SYMMETRIC || ntype == DCRF_NORMALIZE_AFTER;
-    const bool nc = ntype == DCRF_NORMALIZE_SYMMETRIC || ntype == DCRF_NORMALIZE_BEFORE;
-    float av[R], cv[R];
+        for (int r = 0; r < R; r++) mk[r] = T.kw ? m[r] * kw : m[r];
+        if constexpr (WAVE && CWL) {
+            if (T.ckind == DCRF_COMPAT_MATRIX && T.cw_lds >= 0) {
+                // (between fences: the last term's reads, these rows, their reads)
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                if (G.on) {
+                    float* row = msg + (size_t)G.g * ldm + G.k0;
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        av[r] = na ? bv[r] * n : bv[r];
-        cv[r] = nc ? c[r] * n : c[r];
+                    for (int r = 0; r < R; r++) row[r] = mk[r];
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                matrix_piece_rows<R>(shc + T.cw_lds, T.ldw, msg + (size_t)G.g * ldm, G, c);
+            } else {
+                compat_piece<WAVE, R>(T, mk, c, G, shc);
+            }
+        } else {
+            compat_piece<WAVE, R>(T, mk, c, G, shc);  // every lane: Matrix reads its group
+        }
+        if (!active) continue;
+        const int nt = in.ntype[k];
+        const float n = in.norm[k][p];
+        const bool na = nt == DCRF_NORMALIZE_SYMMETRIC || nt == DCRF_NORMALIZE_AFTER;
+        const bool nc = nt == DCRF_NORMALIZE_SYMMETRIC || nt == DCRF_NORMALIZE_BEFORE;
+        float av[R], cv[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            av[r] = na ? bv[r] * n : bv[r];
+            cv[r] = nc ? c[r] * n : c[r];
+        }
+        float* row = P + ((size_t)k * N + p) * 2 * L;
+        store_piece<R>(row, G.k0, L, av);
+        store_piece<R>(row + L, G.k0, L, cv);
     }
-    float* row = P + (size_t)p * 2 * L;
-    store_piece<R>(row, G.k0, L, av);
-    store_piece<R>(row + L, G.k0, L, cv);
 }
 
-// The first argument x of featureGradient's norm-derivative term, with fa = K^T a
-// (st.t[0]: the reverse-blurred rows of P) and fb = K c (st.t[1]: the forward-blurred
+// The first argument x of featureGradient's norm-derivative term from fa = K^T a, fb = K c
+// and the point's row [a | c] of P, whose halves carry one factor n of the reference's
+// forms already:
+//   SYMMETRIC  x = (0.5 (b fb + fa lbl)) n^3 = (0.5 (a fb + fa c)) n^2   (pairwise.cpp:90-97)
+//   AFTER      x = (b fb) n^2 = (a fb) n                                 (:98-105)
+//   BEFORE     x = (fa lbl) n^2 = (fa c) n                               (:106-113)
+template <int R>
+__device__ __forceinline__ void kg_x_value(const float* __restrict__ prow, int k0, int L, float n, int ntype,
+                                           const float (&fa)[R], const float (&fb)[R], float (&v)[R]) {
+    float a[R] = {}, c[R] = {};
+    if (ntype != DCRF_NORMALIZE_BEFORE) load_piece<R>(prow, k0, L, a);
+    if (ntype != DCRF_NORMALIZE_AFTER) load_piece<R>(prow + L, k0, L, c);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (ntype == DCRF_NORMALIZE_SYMMETRIC)
+            v[r] = 0.5f * fmaf(a[r], fb[r], fa[r] * c[r]) * (n * n);
+        else if (ntype == DCRF_NORMALIZE_AFTER)
+            v[r] = a[r] * fb[r] * n;
+        else
+            v[r] = fa[r] * c[r] * n;
+    }
+}
+
+// x with fa (st.t[0]: the reverse-blurred rows of P) and fb (st.t[1]: the forward-blurred
 // rows, from label L on) sliced in the same pass; a slice whose rows are null is not
-// needed by the normalisation type:
-//   SYMMETRIC  x = (0.5 (b fb + fa lbl)) n^3      (pairwise.cpp:90-97)
-//   AFTER      x = (b fb) n^2                     (:98-105)
-//   BEFORE     x = (fa lbl) n^2                   (:106-113)
+// needed by the normalisation type.  For the shapes that k_kg_x_rows does not cover.
 template <bool WAVE, int R>
-__global__ void __launch_bounds__(1024) k_kg_x(const float* __restrict__ b, int ldb,
-                                               const float* __restrict__ lbl,
-                                               const float* __restrict__ norm, int N, int L, int S, int per,
-                                               SliceTable st, int ntype, float* __restrict__ x) {
+__global__ void __launch_bounds__(1024) k_kg_x(const float* __restrict__ P, const float* __restrict__ norm, int N,
+                                               int L, int S, int per, SliceTable st, int ntype,
+                                               float* __restrict__ x) {
     LaneGroup<WAVE, R> G(L, S, per, nullptr);  // no group-wide operation here
     const int p = G.item();
     if (!G.on || p >= N) return;
-    float fa[R] = {}, fb[R] = {}, bv[R] = {}, lv[R] = {}, v[R];
-    const bool sym = ntype == DCRF_NORMALIZE_SYMMETRIC, after = ntype == DCRF_NORMALIZE_AFTER;
+    float fa[R] = {}, fb[R] = {}, v[R];
     if (st.t[0].vals) slice_piece<R>(st.t[0], p, G.k0, L, fa);
     if (st.t[1].vals) slice_piece<R>(st.t[1], p, G.k0, L, fb);
-    if (sym || after) load_piece<R>(b + (size_t)p * ldb, G.k0, L, bv);
-    if (!after) load_piece<R>(lbl + (size_t)p * L, G.k0, L, lv);
-    const float n = norm[p];
-    const float n2 = n * n;
+    kg_x_value<R>(P + (size_t)p * 2 * L, G.k0, L, norm[p], ntype, fa, fb, v);
+    store_piece<R>(x + (size_t)p * L, G.k0, L, v);
+}
+
+// n consecutive words from src into the wave's LDS words dst, repeating the last of the m
+// >= 1 that exist: the points' entries are read once per wave, not once per lane of every
+// group (12 broadcast loads of the 64 lanes at d = 5).
+template <typename T>
+__device__ __forceinline__ void stage_words(const T* __restrict__ src, int n, int m, T* dst) {
+    for (int i = threadIdx.x & 63; i < n; i += 64) dst[i] = src[min(i, m - 1)];
+}
+__device__ __forceinline__ void stage_done() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The same for lane groups inside a wave and d = D: both slices use the lattice's entries
+// once, all 2 (D + 1) rows are in flight together.
+// Bound: the row gathers.  512x512x21: the form above took 38 us a term (mean of d = 2 and
+// 5), this one 19 (d = 2) and 27 us (d = 5).
+template <int R, int D>
+__global__ void __launch_bounds__(kWaveBlock) k_kg_x_rows(const float* __restrict__ P, const int* __restrict__ vtx,
+                                                          const float* __restrict__ sw, const float* __restrict__ ra,
+                                                          const float* __restrict__ rb, const float* __restrict__ norm,
+                                                          int N, int L, int S, int per, int ntype,
+                                                          float* __restrict__ x) {
+    constexpr int D1 = D + 1, W = kWaveBlock / 64;
+    __shared__ int sv[W][64 * D1];
+    __shared__ float ss[W][64 * D1];
+    LaneGroup<true, R> G(L, S, per, nullptr);
+    const int p0 = __builtin_amdgcn_readfirstlane(G.item() - G.g);
+    const int np = min(per, N - p0);
+    if (np <= 0) return;  // the whole wave
+    stage_words(vtx + (size_t)p0 * D1, per * D1, np * D1, sv[G.w]);
+    stage_words(sw + (size_t)p0 * D1, per * D1, np * D1, ss[G.w]);
+    stage_done();
+    const int gp = min(G.g, np - 1), p = p0 + gp, L2 = 2 * L;
+    float ua[D1][R], ub[D1][R];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        if (sym) {
-            const float p1 = bv[r] * fb[r], p2 = fa[r] * lv[r];
-            const float sum = p1 + p2;
-            const float h = 0.5f * sum;
-            const float n3 = n2 * n;
-            v[r] = h * n3;
-        } else if (after) {
-            const float q = bv[r] * fb[r];
-            v[r] = q * n2;
-        } else {
-            const float q = fa[r] * lv[r];
-            v[r] = q * n2;
+    for (int q = 0; q < D1; q++) {
+        const size_t o = (size_t)sv[G.w][gp * D1 + q] * L2 + G.k0;
+        if (ra) load_piece<R>(ra + o, 0, L, ua[q]);
+        if (rb) load_piece<R>(rb + o, 0, L, ub[q]);
+    }
+    float fa[R] = {}, fb[R] = {}, v[R];
+#pragma unroll
+    for (int q = 0; q < D1; q++) {
+        const float w = ss[G.w][gp * D1 + q];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if (ra) fa[r] = fmaf(w, ua[q][r], fa[r]);
+            if (rb) fb[r] = fmaf(w, ub[q][r], fb[r]);
         }
     }
-    store_piece<R>(x + (size_t)p * L, G.k0, L, v);
+    kg_x_value<R>(P + (size_t)p * L2, G.k0, L, norm[p], ntype, fa, fb, v);
+    if (G.on && G.g < np) store_piece<R>(x + (size_t)p * L, G.k0, L, v);
 }
 
 struct GradScale {
@@ -200,66 +276,6 @@ __global__ void __launch_bounds__(kThreads) k_slice_grad(const float* __restrict
     }
 }
 
-// The lane's pieces of the point's d+1 vertex rows for one direction of the slicing
-// gradient: au[q][r] = vals[v[q]][k0 + r] (row stride ldv), or with per_vertex the one
-// value per vertex for every label.
-template <int R, int D>
-__device__ __forceinline__ void grad_rows(const float* __restrict__ vals, int ldv, bool per_vertex,
-                                          const int (&v)[D + 1], int k0, int L, float (&au)[D + 1][R]) {
-#pragma unroll
-    for (int q = 0; q < D + 1; q++) {
-        if (!per_vertex) {
-            load_piece<R>(vals + (size_t)v[q] * ldv, k0, L, au[q]);
-        } else {
-            const float x = vals[v[q]];
-#pragma unroll
-            for (int r = 0; r < R; r++) au[q][r] = x;
-        }
-    }
-}
-
-// The lane's share of one direction of the slicing gradient (the loop body of
-// k_slice_grad) for its R consecutive labels, from the rows grad_rows loaded: the rotated
-// differences of alpha * au are formed by select, elevated and paired with cv; grad[j]
-// sums the lane's labels in order.  The lane group adds the shares afterwards.
-template <int R, int D>
-__device__ __forceinline__ void grad_share(const float (&au_in)[D + 1][R], const int (&r0)[D + 1],
-                                           const float (&cv)[R], const GradScale& gs, float* grad) {
-    constexpr int D1 = D + 1;
-    float au[D1][R];
-#pragma unroll
-    for (int q = 0; q < D1; q++)
-#pragma unroll
-        for (int r = 0; r < R; r++) au[q][r] = gs.alpha * au_in[q][r];
-#pragma unroll
-    for (int j = 0; j < D; j++) grad[j] = 0.0f;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        float ra[D1];
-#pragma unroll
-        for (int j = 0; j < D1; j++) {
-            const int a = r0[j], b = a + 1 > D ? 0 : a + 1;
-            float x0 = au[0][r], x1 = au[0][r];
-#pragma unroll
-            for (int q = 1; q < D1; q++) {
-                x0 = a == q ? au[q][r] : x0;
-                x1 = b == q ? au[q][r] : x1;
-            }
-            ra[j] = x0 - x1;
-        }
-        float sm = ra[0];
-#pragma unroll
-        for (int j = 1; j <= D; j++) {
-            const float jr = (float)j * ra[j];
-            const float diff = sm - jr;
-            const float e = gs.sf[j - 1] * diff;
-            const float prod = cv[r] * e;
-            grad[j - 1] = grad[j - 1] + prod;
-            sm = sm + ra[j];
-        }
-    }
-}
-
 // The operands of k_kg_grad.
 struct KgGrad {
     const float* fwd;   // forward-blurred rows of P (stride 2L): K a in labels 0..L-1
@@ -275,119 +291,171 @@ struct KgGrad {
     int full;  // FULL_KERNEL: d*d parameters, else d
 };
 
+// t[q - 1] += sign * (sum over the lane's labels of c (u_q - u_0)), q = 1..D, u_q the
+// lane's piece of the point's vertex row q (rows of ld floats from vals).
+template <int R, int D>
+__device__ __forceinline__ void grad_dots(const float* __restrict__ vals, int ld, const int* v, int k0, int L,
+                                          const float (&c)[R], float (&t)[D]) {
+    float u0[R], u[D][R];
+    load_piece<R>(vals + (size_t)v[0] * ld + k0, 0, L, u0);
+#pragma unroll
+    for (int q = 1; q <= D; q++) load_piece<R>(vals + (size_t)v[q] * ld + k0, 0, L, u[q - 1]);
+#pragma unroll
+    for (int q = 0; q < D; q++)
+#pragma unroll
+        for (int r = 0; r < R; r++) t[q] = fmaf(c[r], u[q][r] - u0[r], t[q]);
+}
+
 // The whole per-point part of one term's kernel gradient in one pass, S lanes per point
 // and R labels per lane (S <= 64: lane groups inside one wave), d <= 6:
 //   g = G(a, c) = dir 0 (K a rows, paired with c) + dir 1 (K^T c rows, paired with a),
 //   r = G(x, 1) = dir 0 (K x rows, paired with ones) + dir 1 (K^T 1, paired with x),
-//   fg = -r + g (g alone without a normaliser term: x and its rows are not read),
-// each direction summed over the group's lanes (a pairwise tree towards the group's
-// first lane) before the two are added; the 4d lane shares go through one tree together.
+//   fg = -r + g (g alone without a normaliser term: x and its rows are not read).
+// A direction's share is linear in the products T_q = sum_k c_k u_q[k] of the paired row
+// with the point's vertex rows, and only differences of the T_q enter it: each lane
+// accumulates T_q - T_0 of all four directions over its labels (D values), the group adds
+// them (a pairwise tree towards its first lane), and the rotation by rank and the
+// elevation (k_slice_grad's, on alpha T) follow once per point, one lane each, for up to
+// 64 points of the wave's rounds together.  (Rotated and elevated per label, as
+// k_slice_grad does, the selections were most of the instructions: 90 us at 512x512x21
+// with d = 5 and 36 us with d = 2; this form 45 and 25 us, bound by the 3 (d + 1) row
+// gathers.)
 // The parameter products (pairwise.cpp:157-161), DIAG f[q(p)][j] fg[j], FULL fg[r]
-// f[q(p)][c] at c*d + r (column-major, like the reference), are added in double by one
-// lane per parameter.  Per round the group leaders leave fg and the point's feature row
-// in LDS, and lane q of the wave adds its product for the wave's points in point order,
-// over the block's `rounds` consecutive blocks' worth of points.  At the end the waves'
-// sums are added in wave order, and the block adds them to partial[blockIdx.x][q]: one
-// row per block sums all reverse iterations, in iteration order.  The label order of
-// each direction's sum differs from the reference's sequential one (float tolerance).
+// f[q(p)][c] at c*d + r (column-major, like the reference), are added in double in a fixed
+// order: DIAG by each point's lane over the batches, then a tree over the lanes; FULL by
+// lane q of the wave for parameter q, over the batch's points in order.  At the end the
+// waves' sums are added in wave order, and the block adds them to partial[blockIdx.x][q]:
+// one row per block sums all reverse iterations, in iteration order.
 template <int R, int D>
 __global__ void __launch_bounds__(kWaveBlock) k_kg_grad(const int* __restrict__ vtx, const int* __restrict__ rank,
                                                         KgGrad a, int N, int L, int S, int per, int rounds,
                                                         GradScale gs, double* __restrict__ partial) {
     constexpr int D1 = D + 1, W = kWaveBlock / 64;
-    __shared__ float fgl[W][64][D];  // per wave: fg of each group's point
-    __shared__ float ffl[W][64][D];  // and the point's feature row
+    __shared__ int sv[W][64 * D1];   // per wave: the round's vertices
+    __shared__ float tl[W][64][D];   // T_q - T_0 of the batch's points, then FULL: fg
+    __shared__ float ffl[W][64][D];  // FULL: the points' feature rows
     __shared__ double wsum[W][D * D];
     const int np = a.full ? D * D : D;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     LaneGroup<true, R> G(L, S, per, nullptr);
     const int L2 = 2 * L;
-    const bool nx = a.xr != nullptr;
     // lane q < np: parameter q = (row, col) of the products fg[row] * f[col]
-    const int prow = a.full ? lane % D : lane, pcol = a.full ? lane / D : lane;
-    double acc = 0.0;
+    const int prow = lane % D, pcol = min(lane / D, D - 1);
+    double acc[D];  // FULL: acc[0]
+#pragma unroll
+    for (int j = 0; j < D; j++) acc[j] = 0.0;
     const int b0 = xcd_block(blockIdx.x, gridDim.x) * rounds;
-    for (int i = 0; i < rounds; i++) {  // uniform over the block: every lane takes part in every shuffle
-        const int p = G.item_in(b0 + i);
-        const bool active = G.on && p < N;
-        const int pp = active ? p : 0;
-        const bool lead = active && G.l == 0;
-        int v[D1], r0[D1];
+    const int batch = 64 / per;  // rounds whose points one lane each holds
+    const int pstep = W * per;   // from a round's points of the wave to the next round's
+    const int li = lane / per, lg = lane - li * per;
+    for (int i0 = 0; i0 < rounds; i0 += batch) {
+        const int nb = min(batch, rounds - i0);
+        const int pb = __builtin_amdgcn_readfirstlane(G.item_in(b0 + i0) - G.g);
+        for (int i = 0; i < nb; i++) {
+            const int p0 = pb + i * pstep, n = min(per, N - p0);
+            if (n <= 0) break;  // the wave's further rounds lie behind the last point too
+            stage_words(vtx + (size_t)p0 * D1, per * D1, n * D1, sv[w]);
+            stage_done();
+            const int gp = min(G.g, n - 1);
+            const size_t p = p0 + gp;
+            int v[D1];
 #pragma unroll
-        for (int q = 0; q < D1; q++) {
-            v[q] = vtx[(size_t)pp * D1 + q];
-            r0[q] = D - rank[(size_t)pp * D1 + q];
-        }
-        // the leader's feature row of the point, for the products below
-        float fv[D];
-        {
-            int fq = 0;
-            if (lead) {
-                const int inst = a.n_inst > 1 ? last_le(a.pix_base, a.n_inst, p) : 0;
-                fq = a.pad_base[inst] + (p - a.pix_base[inst]);
+            for (int q = 0; q < D1; q++) v[q] = sv[w][gp * D1 + q];
+            float t[D], cv[R];
+#pragma unroll
+            for (int q = 0; q < D; q++) t[q] = 0.0f;
+            if (a.xr) {
+                float u[R];
+                load_piece<R>(a.x + p * L, G.k0, L, cv);
+                float o[D1], xs = cv[0];
+#pragma unroll
+                for (int q = 0; q < D1; q++) o[q] = a.ones[v[q]];
+#pragma unroll
+                for (int r = 1; r < R; r++) xs = xs + cv[r];
+#pragma unroll
+                for (int r = 0; r < R; r++) u[r] = 1.0f;
+                grad_dots<R, D>(a.xr, L, v, G.k0, L, u, t);
+#pragma unroll
+                for (int q = 0; q < D; q++) t[q] = -fmaf(xs, o[q + 1] - o[0], t[q]);
             }
+            load_piece<R>(a.P + p * L2 + L, G.k0, L, cv);
+            grad_dots<R, D>(a.fwd, L2, v, G.k0, L, cv, t);
+            load_piece<R>(a.P + p * L2, G.k0, L, cv);
+            grad_dots<R, D>(a.rev + L, L2, v, G.k0, L, cv, t);
+            for (int k = 1; k < S; k <<= 1) {
+                float y[D];
 #pragma unroll
-            for (int j = 0; j < D; j++) fv[j] = lead ? a.f[(size_t)fq * D + j] : 0.0f;
-        }
-        // shares [dir 0 of G(a, c) | dir 1 | dir 0 of G(x, 1) | dir 1], d each; a
-        // direction's rows are loaded where its share is formed
-        float sh[4 * D];
-        {
-            float u[D1][R], cv[R];
-            load_piece<R>(a.P + (size_t)pp * L2 + L, G.k0, L, cv);
-            grad_rows<R, D>(a.fwd, L2, false, v, G.k0, L, u);
-            grad_share<R, D>(u, r0, cv, gs, sh);
-            load_piece<R>(a.P + (size_t)pp * L2, G.k0, L, cv);
-            grad_rows<R, D>(a.rev + L, L2, false, v, G.k0, L, u);
-            grad_share<R, D>(u, r0, cv, gs, sh + D);
-            if (nx) {
+                for (int j = 0; j < D; j++) y[j] = wave_read(t[j], G.base + G.l + k);  // (wraps at 64)
+                if ((G.l & (2 * k - 1)) == 0 && G.l + k < S) {
 #pragma unroll
-                for (int r = 0; r < R; r++) cv[r] = 1.0f;
-                grad_rows<R, D>(a.xr, L, false, v, G.k0, L, u);
-                grad_share<R, D>(u, r0, cv, gs, sh + 2 * D);
-                load_piece<R>(a.x + (size_t)pp * L, G.k0, L, cv);
-                grad_rows<R, D>(a.ones, 1, true, v, G.k0, L, u);
-                grad_share<R, D>(u, r0, cv, gs, sh + 3 * D);
-            } else {
-#pragma unroll
-                for (int j = 2 * D; j < 4 * D; j++) sh[j] = 0.0f;
+                    for (int j = 0; j < D; j++) t[j] = t[j] + y[j];
+                }
             }
-        }
-        // the group's sums in its first lane (the tree of LaneGroup::all_sum)
-        for (int k = 1; k < S; k <<= 1) {
-            float y[4 * D];
+            if (G.on && G.l == 0) {
 #pragma unroll
-            for (int j = 0; j < 4 * D; j++) y[j] = __shfl(sh[j], (G.base + G.l + k) & 63);
-            if ((G.l & (2 * k - 1)) == 0 && G.l + k < S) {
-#pragma unroll
-                for (int j = 0; j < 4 * D; j++) sh[j] = sh[j] + y[j];
+                for (int j = 0; j < D; j++) tl[w][i * per + G.g][j] = t[j];
             }
         }
-        if (lead) {
+        stage_done();
+        const int p = pb + li * pstep + lg;
+        const bool real = li < nb && p < N;  // a prefix of the wave's lanes
+        float fg[D], fv[D];
+#pragma unroll
+        for (int j = 0; j < D; j++) fg[j] = fv[j] = 0.0f;
+        if (real) {
+            const int inst = a.n_inst > 1 ? last_le(a.pix_base, a.n_inst, p) : 0;
+            const int fq = a.pad_base[inst] + (p - a.pix_base[inst]);
+            float T[D1];
+            T[0] = 0.0f;
 #pragma unroll
             for (int j = 0; j < D; j++) {
-                const float g = sh[j] + sh[D + j];
-                const float r = sh[2 * D + j] + sh[3 * D + j];
-                fgl[w][G.g][j] = nx ? -r + g : g;
-                ffl[w][G.g][j] = fv[j];
+                fv[j] = a.f[(size_t)fq * D + j];
+                T[j + 1] = gs.alpha * tl[w][lane][j];
             }
-        }
-        __syncthreads();
-        if (lane < np) {
-            const int ng = min(per, N - (G.item_in(b0 + i) - G.g));  // the wave's points in this round
-            for (int gi = 0; gi < ng; gi++) {
-                float fgv = fgl[w][gi][0], fcv = ffl[w][gi][0];
+            float ra[D1];
 #pragma unroll
-                for (int j = 1; j < D; j++) {
-                    fgv = prow == j ? fgl[w][gi][j] : fgv;
-                    fcv = pcol == j ? ffl[w][gi][j] : fcv;
+            for (int j = 0; j < D1; j++) {
+                const int r0 = D - rank[(size_t)p * D1 + j], r1 = r0 + 1 > D ? 0 : r0 + 1;
+                float x0 = T[0], x1 = T[0];
+#pragma unroll
+                for (int q = 1; q < D1; q++) {
+                    x0 = r0 == q ? T[q] : x0;
+                    x1 = r1 == q ? T[q] : x1;
                 }
-                acc += (double)fgv * (double)fcv;
+                ra[j] = x0 - x1;
+            }
+            float sm = ra[0];
+#pragma unroll
+            for (int j = 1; j <= D; j++) {
+                fg[j - 1] = gs.sf[j - 1] * (sm - (float)j * ra[j]);
+                sm = sm + ra[j];
             }
         }
-        __syncthreads();
+        if (!a.full) {
+#pragma unroll
+            for (int j = 0; j < D; j++) acc[j] += (double)fg[j] * (double)fv[j];
+        } else {
+            stage_done();  // every lane has read its T
+#pragma unroll
+            for (int j = 0; j < D; j++) {
+                tl[w][lane][j] = fg[j];
+                ffl[w][lane][j] = fv[j];
+            }
+            stage_done();
+            const int n = __popcll(__ballot(real));
+            for (int g = 0; g < n; g++) acc[0] += (double)tl[w][g][prow] * (double)ffl[w][g][pcol];
+        }
+        stage_done();  // (the next batch writes tl)
     }
-    if (lane < np) wsum[w][lane] = acc;
+    if (!a.full) {
+#pragma unroll
+        for (int j = 0; j < D; j++) {
+            for (int k = 32; k > 0; k >>= 1) acc[j] += __shfl_down(acc[j], k);
+            if (lane == 0) wsum[w][j] = acc[j];
+        }
+    } else if (lane < np) {
+        wsum[w][lane] = acc[0];
+    }
     __syncthreads();
     for (int q = threadIdx.x; q < np; q += blockDim.x) {
         double s = 0.0;
@@ -523,21 +591,42 @@ static GradScale grad_scale(int d) {
     return gs;
 }
 
-void launch_kg_prepare(const float* Qt, const float* b, int ldq, const float* norm, int N, int L, const SliceTable& st_in,
-                       int ntype, float* lbl, float* P, hipStream_t s) {
+void launch_kg_prepare(const float* Qt, const float* b, int ldq, const KgInputs& in, int N, int L,
+                       const SliceTable& st_in, float* P, hipStream_t s) {
     if (!N) return;
     SliceTable st = st_in;
-    const int cwf = assign_compat_lds(st, L);
     const LaunchShape sh = shape_for(L);
-    DCRF_DISPATCH_CWL(sh, cwf, k_kg_prepare, blocks_for(N, sh.items), sizeof(float) * (sh.block + cwf), s, Qt, b,
-                      ldq, norm, N, L, sh.S, sh.per, st, ntype, lbl, P);
+    const int cwf = assign_compat_lds(st, L, sh.wave);  // 16-byte rows for matrix_piece_rows
+    const size_t msg = sh.wave && cwf ? (size_t)(kWaveBlock / 64) * sh.per * ((L + 3) & ~3) : 0;
+    DCRF_DISPATCH_CWL(sh, cwf, k_kg_prepare, blocks_for(N, sh.items), sizeof(float) * (sh.block + cwf + msg), s, Qt, b,
+                      ldq, in, N, L, sh.S, sh.per, st, cwf, P);
 }
 
-void launch_kg_x(const float* b, int ldb, const float* lbl, const float* norm, int N, int L, const SliceTable& st, int ntype,
-                 float* x, hipStream_t s) {
+void launch_kg_x(const float* P, const float* norm, int N, int L, const SliceTable& st, int ntype, float* x,
+                 hipStream_t s) {
     if (!N) return;
     const LaunchShape sh = shape_for(L);
-    DCRF_DISPATCH(sh, k_kg_x, blocks_for(N, sh.items), 0, s, b, ldb, lbl, norm, N, L, sh.S, sh.per, st, ntype, x);
+    const int d = st.t[0].d1 - 1;
+#define DCRF_KGX(RR, DD)                                                                                         \
+    case RR * 8 + DD:                                                                                            \
+        k_kg_x_rows<RR, DD><<<blocks_for(N, sh.items), kWaveBlock, 0, s>>>(P, st.t[0].vtx, st.t[0].sw,           \
+                                                                           st.t[0].vals, st.t[1].vals, norm, N, \
+                                                                           L, sh.S, sh.per, ntype, x);          \
+        break;
+    if (kg_grad_fused(L, d)) {
+        switch (sh.R * 8 + d) {
+            DCRF_KGX(1, 1) DCRF_KGX(1, 2) DCRF_KGX(1, 3) DCRF_KGX(1, 4) DCRF_KGX(1, 5) DCRF_KGX(1, 6)
+            DCRF_KGX(2, 1) DCRF_KGX(2, 2) DCRF_KGX(2, 3) DCRF_KGX(2, 4) DCRF_KGX(2, 5) DCRF_KGX(2, 6)
+            DCRF_KGX(3, 1) DCRF_KGX(3, 2) DCRF_KGX(3, 3) DCRF_KGX(3, 4) DCRF_KGX(3, 5) DCRF_KGX(3, 6)
+            DCRF_KGX(4, 1) DCRF_KGX(4, 2) DCRF_KGX(4, 3) DCRF_KGX(4, 4) DCRF_KGX(4, 5) DCRF_KGX(4, 6)
+            default:
+                throw Error{DCRF_ERR_STATE, "kernel gradient: no lane-group kernel for this shape"};
+        }
+        DCRF_HIP_CHECK(hipGetLastError());
+        return;
+    }
+#undef DCRF_KGX
+    DCRF_DISPATCH(sh, k_kg_x, blocks_for(N, sh.items), 0, s, P, norm, N, L, sh.S, sh.per, st, ntype, x);
 }
 
 bool kg_grad_fused(int L, int d) { return d >= 1 && d <= 6 && shape_for(L).wave; }

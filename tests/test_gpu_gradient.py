@@ -411,6 +411,33 @@ def test_kernel_gradient_multi_round(nt):
     assert err <= KG_TOL_L21, (err, kg, kgo)
 
 
+@pytest.mark.parametrize("L,W,H", [(2, 1024, 513), (64, 203, 199), (21, 61, 1)])
+def test_kernel_gradient_batches(L, W, H):
+    """k_kg_grad holds the points of up to 64 / per rounds of a wave before it elevates
+    them: per = 64 points a round in several batches of one (L = 2: R = 2, one lane a
+    point; 2053 blocks of 256 points, 2 rounds), per = 4 (L = 64), and one round with a
+    last wave that has fewer points than lane groups.  FULL kernels against the oracle
+    (which adds their products in double); the DIAG gradient is the diagonal of the FULL
+    one, up to the order of the additions in double and the rounding of the result."""
+    img, U, gt = image_case(W, H, L, seed=51)
+
+    def build(m, ktype):
+        m.set_unary(U)
+        m.add_gaussian(3.0, 3.0, 3.0, ktype=ktype)
+        m.add_bilateral(40.0, 40.0, 13.0, 13.0, 13.0, img, 10.0, ktype=ktype)
+        return m
+
+    full = build(capi.Model.create_2d(W, H, L), capi.FULL_KERNEL).gradient(2, gt, kernel=True)[4]
+    diag = build(capi.Model.create_2d(W, H, L), capi.DIAG_KERNEL).gradient(2, gt, kernel=True)[4]
+    want = build(po.OracleCRF(W=W, H=H, L=L), capi.FULL_KERNEL).gradient(2, gt, kernel=True)[3]
+    assert full.shape == want.shape == (4 + 25,)
+    err = np.abs(full - want).max() / np.abs(want).max()
+    print("kernel gradient %dx%dx%d: max error / max entry %.3g" % (W, H, L, err))
+    assert err <= KG_TOL_L21, (err, full, want)
+    of = np.concatenate([full[:4].reshape(2, 2).diagonal(), full[4:].reshape(5, 5).diagonal()])
+    assert np.abs(diag - of).max() <= 1e-6 * np.abs(of).max()
+
+
 @pytest.mark.parametrize("case", ["mixed_normalisation", "five_terms", "high_dim"])
 def test_kernel_gradient_term_mixes(case):
     """The kernel-parameter gradient's shared filter plans: an unnormalised term beside
