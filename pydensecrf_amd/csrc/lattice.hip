@@ -244,15 +244,33 @@ __global__ void __launch_bounds__(kThreads) k_embed(const float* __restrict__ fe
     if (ovf) overflow[threadIdx.x & 63] = 1;
 }
 
+// slot[e] = the table slot of entry e's key; a key's slot keeps its smallest entry.
+// Consecutive points often share a vertex: of a wave's entries, one that has the key of
+// the previous point's entry of the same remainder takes that entry's slot, and only the
+// first of such a chain, its smallest, goes to the table.
+// Bound: latency of the table's and the keys' random reads, and atomics of many entries on
+// one new slot.  1024x768, every entry for itself: 242 us (d = 5), 121 us (d = 2); with
+// chains 210 and 45 us.
 template <int D>
 __global__ void __launch_bounds__(kThreads) k_hash_insert(const Key<D>* __restrict__ keys, int E,
                                                           int* table, uint32_t mask,
                                                           int* __restrict__ slot) {
+    constexpr int D1 = D + 1;
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= E) return;
-    const Key<D> k = keys[e];
+    const int lane = threadIdx.x & 63;
+    const Key<D> k = keys[min(e, E - 1)];
+    bool same = lane >= D1;
+#pragma unroll
+    for (int i = 0; i < Key<D>::W; i++) {
+        const uint64_t w = __shfl(k.w[i], (lane - D1) & 63);
+        same = same && w == k.w[i];
+    }
+    int lead = same ? lane - D1 : lane;
+#pragma unroll
+    for (int n = 1; n <= 63 / D1; n *= 2) lead = __shfl(lead, lead);
     uint32_t h = key_hash<D>(k) & mask;
-    for (;;) {
+    bool look = e < E && lead == lane;
+    while (look) {
         // a workgroup-scope read may return a stale value from the CU's cache, which is
         // safe: a slot only goes from empty to entries of one key, whose value then only
         // falls, so a stale non-empty value names the right key and is >= the current one
@@ -260,23 +278,21 @@ __global__ void __launch_bounds__(kThreads) k_hash_insert(const Key<D>* __restri
         // which reads the slot at device scope
         int cur = __hip_atomic_load(&table[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (cur == kEmpty) {
-            const int old = atomicCAS(&table[h], kEmpty, e);
-            if (old == kEmpty) {
-                slot[e] = (int)h;
-                return;
-            }
-            cur = old;
+            cur = atomicCAS(&table[h], kEmpty, e);
+            if (cur == kEmpty) break;
         }
         if (key_eq<D>(keys[cur], k)) {
             // the slot keeps the smallest entry of its key (first occurrence); the value
             // only falls, so an entry above the one just read cannot lower it: most
             // entries of a popular vertex skip the atomic
             if (e < cur) atomicMin(&table[h], e);
-            slot[e] = (int)h;
-            return;
+            look = false;
+        } else {
+            h = (h + 1) & mask;
         }
-        h = (h + 1) & mask;
     }
+    h = __shfl(h, lead);
+    if (e < E) slot[e] = (int)h;
 }
 
 template <int D>
