@@ -49,7 +49,7 @@ __global__ void __launch_bounds__(1024) k_sn_first(const float* __restrict__ Q, 
     sum_normalize<WAVE, R>(q, gv, bn, G);
     if (active) {
         store_piece<R>(b + (size_t)p * Lv, G.k0, L, bn);
-        store_row(dU + (size_t)p * L, G, bn);
+        if (dU) store_row(dU + (size_t)p * L, G, bn);
     }
 }
 
@@ -59,7 +59,7 @@ __global__ void __launch_bounds__(1024) k_sn_first(const float* __restrict__ Q, 
 // the compatibility gradient's statistic, with no message cache.
 template <bool WAVE, int R, bool CWL>
 __global__ void __launch_bounds__(1024) k_adjoint(const float* __restrict__ Q, float* __restrict__ b,
-                                                  float* __restrict__ dU, int N, int L, int Lv, int S, int per,
+                                                  float* __restrict__ dU, UnarySum us, int N, int L, int Lv, int S, int per,
                                                   SliceTable st, int cwf) {
     extern __shared__ float sh[];
     float* shc = sh + blockDim.x;
@@ -106,12 +106,8 @@ __global__ void __launch_bounds__(1024) k_adjoint(const float* __restrict__ Q, f
     float bn[R];
     sum_normalize<WAVE, R>(q, gsum, bn, G);
     if (active) {
-        float du[R];
-        load_row(dU + (size_t)p * L, G, du);
-#pragma unroll
-        for (int r = 0; r < R; r++) du[r] = du[r] + bn[r];
         store_piece<R>(b + (size_t)p * Lv, k0, L, bn);
-        store_row(dU + (size_t)p * L, G, du);
+        add_unary(us, (size_t)p * Lv + k0, dU + (size_t)p * L, G, bn);
     }
     if (st.nstat) stat_finish<WAVE, R>(st, G, sst);  // uniform condition
 }
@@ -296,13 +292,14 @@ void launch_sn_first(const float* Q, const float* dQ, float* b, float* dU, int N
                   sh.per);
 }
 
-void launch_adjoint(const float* Q, float* b, float* dU, int N, int L, int Lv, const SliceTable& st_in, hipStream_t s) {
+void launch_adjoint(const float* Q, float* b, float* dU, const UnarySum& us, int N, int L, int Lv,
+                    const SliceTable& st_in, hipStream_t s) {
     SliceTable st = st_in;
     const int cwf = assign_compat_lds(st, L);
     const LaunchShape sh = shape_for(Lv);
     const size_t lds =
         sizeof(float) * ((size_t)sh.block + cwf + stat_lds_floats(sh.wave, st.nstat, L, sh.block, sh.R));
-    DCRF_DISPATCH_CWL(sh, cwf, k_adjoint, blocks_for(N, sh.items), lds, s, Q, b, dU, N, L, Lv, sh.S, sh.per, st,
+    DCRF_DISPATCH_CWL(sh, cwf, k_adjoint, blocks_for(N, sh.items), lds, s, Q, b, dU, us, N, L, Lv, sh.S, sh.per, st,
                       cwf);
 }
 

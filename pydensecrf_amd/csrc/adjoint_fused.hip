@@ -9,12 +9,12 @@ namespace {
 inline unsigned blocks_for(size_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
 // The adjoint step of k_adjoint (adjoint.hip) over the same interleaved slice pairs:
-// g = sum_k C_k(w_k slice_k(filtered b)), b = sumAndNormalize(Q .* g, Q), dU += b, and
+// g = sum_k C_k(w_k slice_k(filtered b)), b = sumAndNormalize(Q .* g, Q), dU (UnarySum) and
 // the terms' statistic rows (SliceTerm::gstat).  The pairs carry the transposed filter's
 // slice weights.  Same arithmetic, in the same order, as k_adjoint.
 template <int R, int D0, int D1, bool CWL, bool NARROW>
 __global__ void __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(R <= 3 ? 8 : 7)))
-k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __restrict__ dU, int N, int L, int Lv,
+k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __restrict__ dU, UnarySum us, int N, int L, int Lv,
                 int S, int per, SliceTable st, const int2* __restrict__ slc, int cwf) {
     constexpr int DS = D0 + D1;
     LaneGroup<true, R> G(L, S, per, nullptr);
@@ -68,13 +68,8 @@ k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __res
     float bn[R];
     sum_normalize<true, R>(q, gsum, bn, G);
     if (active) {
-        float du[R];
-        float* urow = dU + (size_t)W.p0 * L + (unsigned)(gp * L);
-        load_row(urow, G, du);
-#pragma unroll
-        for (int r = 0; r < R; r++) du[r] = du[r] + bn[r];
         store_piece<R>(b + wrow + grow, 0, L, bn);
-        store_row(urow, G, du);
+        add_unary(us, wrow + grow, dU + (size_t)W.p0 * L + (unsigned)(gp * L), G, bn);
     }
     if (st.nstat) stat_finish<true, R, NT>(st, G, sst);  // uniform condition
 }
@@ -84,10 +79,10 @@ k_adjoint_fused(const float* __restrict__ Q, float* __restrict__ b, float* __res
 #define DCRF_ADJ_FUSED(R_, D0_, D1_)                                                                      \
     DCRF_FUSED_FORM(k_adjoint_fused, R_, D0_, D1_)<<<                                                       \
         blocks_for(N, sh.items), kWaveBlock, fused_lds_bytes(sh, D0_ + D1_, D1_ ? 2 : 1, L, cwf, st.nstat),  \
-        s>>>(Q, b, dU, N, L, Lv, sh.S, sh.per, st, slc, cwf)
+        s>>>(Q, b, dU, us, N, L, Lv, sh.S, sh.per, st, slc, cwf)
 
 template <int R>
-void launch_adj_fused_r(const LaunchShape& sh, const float* Q, float* b, float* dU, int N, int L, int Lv,
+void launch_adj_fused_r(const LaunchShape& sh, const float* Q, float* b, float* dU, const UnarySum& us, int N, int L, int Lv,
                         const SliceTable& st, const int2* slc, int cwf, hipStream_t s) {
     const int a = st.t[0].d1, c = st.nterms > 1 ? st.t[1].d1 : 0;
     const bool narrow = narrow_rows(st.rows, st.t[0].ldv);
@@ -101,7 +96,7 @@ void launch_adj_fused_r(const LaunchShape& sh, const float* Q, float* b, float* 
     DCRF_HIP_CHECK(hipGetLastError());
 }
 #undef DCRF_ADJ_FUSED
-void launch_adjoint_fused(const float* Q, float* b, float* dU, int N, int L, int Lv, const SliceTable& st_in,
+void launch_adjoint_fused(const float* Q, float* b, float* dU, const UnarySum& us, int N, int L, int Lv, const SliceTable& st_in,
                           const int2* slc, hipStream_t s) {
     SliceTable st = st_in;
     const int cwf = assign_compat_lds(st, L, true);  // 16-byte rows for matrix_piece_rows
@@ -109,10 +104,10 @@ void launch_adjoint_fused(const float* Q, float* b, float* dU, int N, int L, int
     if (!fused_meanfield_ok(L, st.nterms, st.t[0].d1, st.nterms > 1 ? st.t[1].d1 : 0))
         throw Error{DCRF_ERR_VALUE, "no fused adjoint kernel for these terms"};
     switch (sh.R) {
-        case 1: launch_adj_fused_r<1>(sh, Q, b, dU, N, L, Lv, st, slc, cwf, s); break;
-        case 2: launch_adj_fused_r<2>(sh, Q, b, dU, N, L, Lv, st, slc, cwf, s); break;
-        case 3: launch_adj_fused_r<3>(sh, Q, b, dU, N, L, Lv, st, slc, cwf, s); break;
-        default: launch_adj_fused_r<4>(sh, Q, b, dU, N, L, Lv, st, slc, cwf, s); break;
+        case 1: launch_adj_fused_r<1>(sh, Q, b, dU, us, N, L, Lv, st, slc, cwf, s); break;
+        case 2: launch_adj_fused_r<2>(sh, Q, b, dU, us, N, L, Lv, st, slc, cwf, s); break;
+        case 3: launch_adj_fused_r<3>(sh, Q, b, dU, us, N, L, Lv, st, slc, cwf, s); break;
+        default: launch_adj_fused_r<4>(sh, Q, b, dU, us, N, L, Lv, st, slc, cwf, s); break;
     }
 }
 

@@ -1523,12 +1523,14 @@ void backward(dcrf_model& m, const float* dQ, float* dU, float* dcompat, float* 
     const size_t NL = (size_t)N * L, NLv = (size_t)N * Lv;
     // b_t, the adjoint entering reverse iteration t - 1, in slot t (t = n .. 0).  The
     // Matrix terms' statistic reads every b_t after the loop, so with such a term every
-    // slot stays; otherwise two slots alternate.
+    // slot stays; otherwise a ring of the slots that dU still needs and the step's own.
     const int nm = matrix_terms(m);
-    m.bbuf.reserve((size_t)(nm ? n + 1 : std::min(n + 1, 2)) * NLv);
-    auto bslot = [&](int t) { return m.bbuf.get() + (size_t)(nm ? t : (t & 1)) * NLv; };
+    const int ring = nm ? n + 1 : std::min(n + 1, UnarySum::kPending + 1);
+    m.bbuf.reserve((size_t)ring * NLv);
+    auto bslot = [&](int t) { return m.bbuf.get() + (size_t)(t % ring) * NLv; };
     const float* Qc = m.qcache.get();
-    launch_sn_first(Qc + (size_t)n * NLv, dQ, bslot(n), dU, N, L, Lv, s);
+    launch_sn_first(Qc + (size_t)n * NLv, dQ, bslot(n), n ? nullptr : dU, N, L, Lv, s);
+    int first_pending = n;  // slots first_pending .. it + 1 are not in dU yet
     std::vector<size_t> goff(T + 1, 0);
     for (int k = 0; k < T; k++) goff[k + 1] = goff[k] + stat_len(m.terms[k]->ckind, L);
     m.gacc.reserve(std::max<size_t>(goff[T], 1));
@@ -1581,10 +1583,17 @@ void backward(dcrf_model& m, const float* dQ, float* dU, float* dcompat, float* 
                 st.t[k].gslot = j++;
                 st.nstat = j;
             }
+        UnarySum us{};
+        us.n = first_pending - it;
+        if (us.n == UnarySum::kPending || it == 0) {
+            us.mode = first_pending == n ? UnarySum::START : UnarySum::ADD;
+            for (int i = 0; i < us.n; i++) us.prev[i] = bslot(first_pending - i);
+            first_pending = it - 1;
+        }
         if (m.fused)
-            launch_adjoint_fused(Qc + (size_t)it * NLv, bslot(it), dU, N, L, Lv, st, adjoint_pairs(m, s), s);
+            launch_adjoint_fused(Qc + (size_t)it * NLv, bslot(it), dU, us, N, L, Lv, st, adjoint_pairs(m, s), s);
         else
-            launch_adjoint(Qc + (size_t)it * NLv, bslot(it), dU, N, L, Lv, st, s);
+            launch_adjoint(Qc + (size_t)it * NLv, bslot(it), dU, us, N, L, Lv, st, s);
     }
     if (kernel)  // the one-pass kernel gradient's partial rows hold all iterations
         for (int k = 0; k < T; k++)

@@ -524,6 +524,29 @@ __device__ __forceinline__ void sum_normalize(const float (&q)[R], const float (
     }
 }
 
+// The point's share of dU for an adjoint step (UnarySum): its pieces of the pending
+// slots' rows (boff: the piece's offset in a slot) and bn, added to the row urow in the
+// order the steps wrote them, so the sums are those of one addition per step.
+template <bool WAVE, int R>
+__device__ __forceinline__ void add_unary(const UnarySum& us, size_t boff, float* __restrict__ urow,
+                                          const LaneGroup<WAVE, R>& G, const float (&bn)[R]) {
+    if (us.mode == UnarySum::NONE) return;
+    float du[R] = {}, y[UnarySum::kPending][R];
+    if (us.mode == UnarySum::ADD) load_row(urow, G, du);
+#pragma unroll
+    for (int i = 0; i < UnarySum::kPending; i++)
+        if (i < us.n) load_piece<R>(us.prev[i] + boff, 0, G.L, y[i]);
+#pragma unroll
+    for (int i = 0; i < UnarySum::kPending; i++)
+        if (i < us.n) {
+#pragma unroll
+            for (int r = 0; r < R; r++) du[r] = i || us.mode == UnarySum::ADD ? du[r] + y[i][r] : y[i][r];
+        }
+#pragma unroll
+    for (int r = 0; r < R; r++) du[r] = du[r] + bn[r];
+    store_row(urow, G, du);
+}
+
 }  // namespace dcrf
 
 // Launch a lane-group kernel template <WAVE, R> (DCRF_DISPATCH) or <WAVE, R, C>

@@ -434,16 +434,30 @@ void launch_transpose(const float* in, float* out, int rows, int cols, hipStream
 // out[p] = the first label of the largest Q[p][l] (DenseCRF::currentMap), Q row stride ldq.
 void launch_argmax(const float* Q, int ldq, int N, int L, int16_t* out, hipStream_t s);
 // ---------------------------------------------------------------- adjoint kernels
-// b = sumAndNormalize(Q .* dQ, Q); dU = b.  Q, dQ, dU [N][L]; b rows of Lv floats.
+// What an adjoint step adds to dU = sum_t b_t.  The steps write their b_t to slots that
+// keep them for a while, and one step in kPending + 1 adds the pending slots' (prev[0 ..
+// n), oldest first) and its own b_t: the others leave dU alone.  START: dU = the sum (the
+// first such step; n >= 1), ADD: dU += it.
+// (One addition per step read and wrote dU, 132 MB at 1024x768x21, each time, in a kernel
+// that memory bounds: 84 us a launch, now @ADJ@ on average.)
+struct UnarySum {
+    static constexpr int kPending = 3;
+    enum Mode { NONE, START, ADD };
+    const float* prev[kPending];
+    int n, mode;
+};
+// b = sumAndNormalize(Q .* dQ, Q), and dU = b unless dU is null.  Q, dQ, dU [N][L]; b rows
+// of Lv floats.
 void launch_sn_first(const float* Q, const float* dQ, float* b, float* dU, int N, int L, int Lv, hipStream_t s);
-// b <- sumAndNormalize(Q .* sum_k w_k C_k^T slice^T_k, Q) (b is written, not read); dU += b.
+// b <- sumAndNormalize(Q .* sum_k w_k C_k^T slice^T_k, Q) (b is written, not read); dU as us says.
 // Terms with st.t[k].gstat also get their statistic rows (see SliceTerm).
 // Q and b have rows of Lv floats, dU of L.
-void launch_adjoint(const float* Q, float* b, float* dU, int N, int L, int Lv, const SliceTable& st, hipStream_t s);
+void launch_adjoint(const float* Q, float* b, float* dU, const UnarySum& us, int N, int L, int Lv,
+                    const SliceTable& st, hipStream_t s);
 // The same over interleaved slice pairs (those of launch_meanfield_fused, with the
 // transposed filter's slice weights); models that fused_meanfield_ok accepts.
-void launch_adjoint_fused(const float* Q, float* b, float* dU, int N, int L, int Lv, const SliceTable& st,
-                          const int2* slc, hipStream_t s);
+void launch_adjoint_fused(const float* Q, float* b, float* dU, const UnarySum& us, int N, int L, int Lv,
+                          const SliceTable& st, const int2* slc, hipStream_t s);
 // Blocks of one adjoint launch over N pixels (the rows of its statistic output).
 int adjoint_blocks(int N, int Lv);
 // acc += sum_{t < iters} sum_p b_t[p] M_t[p]^T (L x L), with b_t = b + t * bstride (rows of

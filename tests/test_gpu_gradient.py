@@ -411,6 +411,27 @@ def test_kernel_gradient_multi_round(nt):
     assert err <= KG_TOL_L21, (err, kg, kgo)
 
 
+@pytest.mark.parametrize("n", [0, 1, 2, 3, 4, 5, 7, 8, 9])
+@pytest.mark.parametrize("terms,L", [(2, 19), (3, 21)])
+def test_unary_gradient_pending_slots(n, terms, L):
+    """dL/dU is added up from up to four adjoint slots at a time: every count of reverse
+    iterations around the multiples of four, through the fused kernel (two terms; 19
+    labels in slots of 20) and the general one (three terms), against the oracle."""
+    W, H = 37, 23
+    img, U, gt = image_case(W, H, L, seed=61)
+    g = capi.Model.create_2d(W, H, L)
+    o = po.OracleCRF(W=W, H=H, L=L)
+    for m in (g, o):
+        m.set_unary(U)
+        m.add_gaussian(3.0, 3.0, 3.0)
+        m.add_bilateral(40.0, 40.0, 13.0, 13.0, 13.0, img, 5.0)
+        if terms == 3:
+            m.add_gaussian(6.0, 5.0, 1.0)
+    ug = g.gradient(n, gt)[1]
+    ugo = o.gradient(n, gt)[1]
+    assert _rel_close(ug, ugo, 1e-4)
+
+
 @pytest.mark.parametrize("L,W,H", [(2, 1024, 513), (64, 203, 199), (21, 61, 1)])
 def test_kernel_gradient_batches(L, W, H):
     """k_kg_grad holds the points of up to 64 / per rounds of a wave before it elevates
