@@ -11,11 +11,13 @@
 #include <sys/mman.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
 #include <limits>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <new>
@@ -91,10 +93,10 @@ int copy_threads(size_t n) {
 // Chunk t of n bytes split T ways, 4 KiB aligned: [off(t), off(t + 1)).
 inline size_t chunk_off(size_t n, int T, int t) { return t >= T ? n : (n / T * t) & ~(size_t)4095; }
 
-// Chunks of one staged window of n bytes moved by T threads: about 2 MiB each, at least
-// one and at most 8 per thread (thread t takes chunks t, t + T, ...).  The host copy
-// left after the window's last DMA (downloads), or made before its first (uploads), is
-// then one small chunk rather than a thread's whole share.
+// Chunks of one staged window of n bytes uploaded by T threads: about 2 MiB each, at
+// least one and at most 8 per thread (thread t takes chunks t, t + T, ...).  The host copy
+// made before the window's first DMA is then one small chunk rather than a thread's whole
+// share.
 inline int window_chunks(size_t n, int T) { return (int)std::clamp<size_t>(n >> 21, (size_t)T, (size_t)8 * T); }
 
 // work(t) for t < T: t = 0 on this thread, the others on threads of their own where the
@@ -145,6 +147,106 @@ char* stage_reserve(HostStage& H, size_t n) {
         H.cap = n;
     }
     return H.p;
+}
+
+// Page-locked buffers that hold a unary between dcrf_set_unary and its upload.  At most
+// kPinnedMax bytes exist at a time, in use or kept for the next model (until
+// dcrf_release_cached_memory); a request beyond that, or one that the runtime refuses,
+// gets none and the caller uses pageable memory.  Nothing is allocated before the process
+// has used a device: setting a unary alone does not initialise one.
+constexpr size_t kPinnedMax = (size_t)512 << 20;
+constexpr size_t kPinnedMin = (size_t)1 << 20;  // smaller unaries: pageable, the copies cost less than the events
+std::atomic<bool> g_device_used{false};
+
+struct PinnedPool {
+    std::mutex mu;
+    std::multimap<size_t, void*> free;
+    size_t total = 0;  // bytes allocated: in use and free
+};
+PinnedPool& pinned_pool() {
+    static PinnedPool* p = new PinnedPool;  // never destroyed: no runtime call at process exit
+    return *p;
+}
+
+// Frees the buffers not in use; returns their bytes.  The caller holds the lock.
+size_t release_pinned(PinnedPool& P) {
+    size_t b = 0;
+    for (auto& f : P.free) {
+        (void)hipHostFree(f.second);
+        b += f.first;
+    }
+    P.free.clear();
+    P.total -= b;
+    return b;
+}
+size_t release_pinned() {
+    PinnedPool& P = pinned_pool();
+    std::lock_guard<std::mutex> lk(P.mu);
+    return release_pinned(P);
+}
+
+// A buffer taken from the pool.
+struct PinnedBuf {
+    char* p = nullptr;
+    size_t cap = 0;
+    PinnedBuf() = default;
+    PinnedBuf(const PinnedBuf&) = delete;
+    PinnedBuf& operator=(const PinnedBuf&) = delete;
+    ~PinnedBuf() { give(); }
+    void give() {
+        if (!p) return;
+        PinnedPool& P = pinned_pool();
+        std::lock_guard<std::mutex> lk(P.mu);
+        P.free.emplace(cap, p);
+        p = nullptr;
+        cap = 0;
+    }
+    // At least n bytes in p, or false.
+    bool take(size_t n) {
+        if (p && cap >= n && cap <= 4 * n) return true;
+        give();
+        if (!g_device_used || n < kPinnedMin || n > kPinnedMax) return false;
+        PinnedPool& P = pinned_pool();
+        std::lock_guard<std::mutex> lk(P.mu);
+        auto it = P.free.lower_bound(n);
+        if (it == P.free.end() || it->first > 4 * n) {
+            const size_t size = (n + ((size_t)2 << 20) - 1) & ~(((size_t)2 << 20) - 1);
+            if (P.total + size > kPinnedMax) release_pinned(P);
+            if (P.total + size > kPinnedMax) return false;
+            // (a stream capture that another part of the program has open is not touched)
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            void* q = nullptr;
+            const hipError_t e = hipHostMalloc(&q, size, hipHostMallocPortable);
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            if (e != hipSuccess) {
+                (void)hipGetLastError();  // clear the failure
+                return false;
+            }
+            P.total += size;
+            it = P.free.emplace(size, q);
+        }
+        p = static_cast<char*>(it->second);
+        cap = it->first;
+        P.free.erase(it);
+        return true;
+    }
+};
+
+// The stream of the current device that uploads unaries beside the models' own work.
+hipStream_t upload_stream() {
+    static std::mutex* mu = new std::mutex;
+    static std::map<int, hipStream_t>* streams = new std::map<int, hipStream_t>;
+    int dev = 0;
+    DCRF_HIP_CHECK(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(*mu);
+    auto it = streams->find(dev);
+    if (it == streams->end()) {
+        hipStream_t s = nullptr;
+        DCRF_HIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+        it = streams->emplace(dev, s).first;
+    }
+    return it->second;
 }
 
 // Events of one staged copy, destroyed on every exit.
@@ -202,23 +304,37 @@ void copy_to_device(void* dst, const void* src, size_t n, hipStream_t s) {
 }
 
 // One window (n <= the staging area's size) of copy_to_host: every chunk's DMA is
-// queued at once, in order, and each chunk is copied out as soon as its event fires.
+// queued at once, in order; while the device works the threads touch the pages the copy
+// will fill (their contents kept), then each chunk is copied out by all of them as soon
+// as its event fires.  Chunks of 8 MiB, or a quarter of less: each costs a launch and an
+// event, and the host copy left after the last one is a thread's share of it.  (In chunks
+// of 2 MiB, one thread each and the pages not touched before, 66 MB into fresh memory
+// took 2.2 ms behind 1.5 ms of iterations; now 1.55.)
 void copy_to_host_window(char* stage, void* dst, const void* src, size_t n, hipStream_t s) {
-    const int T = copy_threads(n), C = window_chunks(n, T);
+    const int T = copy_threads(n), C = (int)std::max<size_t>({n >> 23, std::min<size_t>(n >> 21, 4), 1});
     ChunkEvents E(C);
     for (int c = 0; c < C; c++) {  // all chunks queued before any thread starts
         const size_t a = chunk_off(n, C, c), b = chunk_off(n, C, c + 1);
         DCRF_HIP_CHECK(hipMemcpyAsync(stage + a, (const char*)src + a, b - a, hipMemcpyDeviceToHost, s));
         DCRF_HIP_CHECK(hipEventRecord(E.ev[c], s));
     }
-    std::vector<hipError_t> err(C, hipSuccess);
+    std::vector<hipError_t> err(T, hipSuccess);
     run_parallel(T, [&](int t) {  // each chunk leaves the staging area as soon as it arrived
-        for (int c = t; c < C; c += T) {
-            err[c] = hipEventSynchronize(E.ev[c]);
-            if (err[c] != hipSuccess) return;
-            const size_t a = chunk_off(n, C, c), b = chunk_off(n, C, c + 1);
-            std::memcpy((char*)dst + a, stage + a, b - a);
-        }
+        for (int pass = 0; pass < 2; pass++)
+            for (int c = 0; c < C; c++) {
+                const size_t a = chunk_off(n, C, c), m = chunk_off(n, C, c + 1) - a;
+                const size_t x = a + chunk_off(m, T, t), y = a + chunk_off(m, T, t + 1);
+                if (pass == 0) {  // while the device works: the pages the copy will fill
+                    for (size_t o = x; o < y; o += 4096) {
+                        volatile char* q = (volatile char*)dst + o;
+                        *q = *q;
+                    }
+                    continue;
+                }
+                err[t] = hipEventSynchronize(E.ev[c]);
+                if (err[t] != hipSuccess) return;
+                std::memcpy((char*)dst + x, stage + x, y - x);
+            }
     });
     for (hipError_t e : err) DCRF_HIP_CHECK(e);
 }
@@ -292,7 +408,12 @@ struct dcrf_model {
     int L = 0;
     bool dev_ready = false;
     hipStream_t stream = nullptr;
-    HostFloats unary_host;  // (L, N) row-major as given
+    HostFloats unary_host;  // (L, N) row-major as given, unless unary_pin holds it
+    // a single instance's unary on its way to the device: set, and (unary_ev) being copied
+    // to `stage` by the device's upload stream
+    PinnedBuf unary_pin;
+    hipEvent_t unary_ev = nullptr;
+    bool unary_uploading = false;
     std::vector<char> unary_unset;  // per instance: its columns of unary_host hold no data yet
     bool has_unary = false, unary_dirty = false;
     DevBuf<float> unary;  // [N][L]
@@ -389,6 +510,8 @@ struct dcrf_model {
         }
         for (auto e : free_events) (void)hipEventDestroy(e);
         drop_graph();
+        if (unary_uploading) (void)hipEventSynchronize(unary_ev);
+        if (unary_ev) (void)hipEventDestroy(unary_ev);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -502,6 +625,30 @@ void ensure_device(dcrf_model& m) {
     std::vector<int> W = g.is2d ? g.W : std::vector<int>(g.n_inst, 1);
     DCRF_HIP_CHECK(hipMemcpy(m.geod.W.get(), W.data(), sizeof(int) * g.n_inst, hipMemcpyHostToDevice));
     m.dev_ready = true;
+    g_device_used = true;
+}
+
+// Waits for the unary's copy in flight, if any; the page-locked buffer is free after.
+void finish_unary_upload(dcrf_model& m) {
+    if (!m.unary_uploading) return;
+    DCRF_HIP_CHECK(hipEventSynchronize(m.unary_ev));
+    m.unary_uploading = false;
+}
+
+// Starts the copy of a unary that waits in page-locked memory, so that it runs beside the
+// lattice builds (one copy of 66 MB takes 1.2 ms, the two builds at 1024x768 about as
+// long).
+void start_unary_upload(dcrf_model& m) {
+    if (!m.unary_pin.p || m.unary_uploading) return;
+    const size_t n = (size_t)m.N() * m.L;
+    m.stage.reserve(n);
+    if (!m.unary_ev) DCRF_HIP_CHECK(hipEventCreateWithFlags(&m.unary_ev, hipEventDisableTiming));
+    hipStream_t s = upload_stream();
+    DCRF_HIP_CHECK(hipMemcpyAsync(m.stage.get(), m.unary_pin.p, sizeof(float) * n, hipMemcpyHostToDevice, s));
+    const hipError_t e = hipEventRecord(m.unary_ev, s);
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);
+    DCRF_HIP_CHECK(e);
+    m.unary_uploading = true;
 }
 
 // dst = src on the device (large lists through the staging area; then the copy is
@@ -526,6 +673,17 @@ void ensure_unary(dcrf_model& m) {
         upload(m.lL_dev, m.lL, m.stream);
         launch_logistic_unary(m.lfFN.get(), m.lL_dev.get(), m.N(), m.lF, m.L, m.unary.get(), m.stream);
         DCRF_HIP_CHECK(hipStreamSynchronize(m.stream));
+        m.unary_dirty = false;
+        return;
+    }
+    if (m.unary_pin.p) {
+        m.unary.reserve(n);
+        start_unary_upload(m);
+        DCRF_HIP_CHECK(hipStreamWaitEvent(m.stream, m.unary_ev, 0));
+        launch_transpose(m.stage.get(), m.unary.get(), m.L, m.N(), m.stream);
+        DCRF_HIP_CHECK(hipStreamSynchronize(m.stream));
+        m.unary_uploading = false;
+        m.unary_pin.give();
         m.unary_dirty = false;
         return;
     }
@@ -974,6 +1132,10 @@ void add_term(dcrf_model& m, int d, int ckind, const float* compat, int ktype, i
                 const float s = compat[a * L + b] + compat[b * L + a];
                 t->compat[(size_t)a * L + b] = 0.5f * s;
             }
+    }
+    try {
+        start_unary_upload(m);
+    } catch (const Error&) {  // no memory for it yet: the first inference uploads
     }
     t->d_compat.reserve(t->compat.size());
     DCRF_HIP_CHECK(hipMemcpy(t->d_compat.get(), t->compat.data(), sizeof(float) * t->compat.size(),
@@ -1764,7 +1926,7 @@ const char* dcrf_last_error(void) { return g_last_error.c_str(); }
 
 int dcrf_release_cached_memory(size_t* bytes) {
     return guard([&] {
-        const size_t b = pool_release_all() + release_host_stage();
+        const size_t b = pool_release_all() + release_host_stage() + release_pinned();
         if (bytes) *bytes = b;
     });
 }
@@ -1821,8 +1983,16 @@ int dcrf_set_unary(dcrf_model* m, const float* U) {
     return guard([&] {
         require(m && U, "null argument");
         const size_t n = (size_t)m->N() * m->L;
-        m->unary_host.resize(n);
-        host_copy(m->unary_host.data(), U, sizeof(float) * n);
+        finish_unary_upload(*m);
+        // one instance: page-locked memory, from which the upload is one asynchronous copy
+        // (several instances may be set one by one later, beside this call's values)
+        if (m->geo.n_inst == 1 && m->unary_pin.take(sizeof(float) * n)) {
+            host_copy(m->unary_pin.p, U, sizeof(float) * n);
+        } else {
+            m->unary_pin.give();
+            m->unary_host.resize(n);
+            host_copy(m->unary_host.data(), U, sizeof(float) * n);
+        }
         m->unary_unset.clear();
         m->has_unary = true;
         m->unary_dirty = true;
@@ -1845,6 +2015,8 @@ int dcrf_set_logistic_unary(dcrf_model* m, const float* Lmat, int F, const float
         DCRF_HIP_CHECK(hipMemcpyAsync(m->lfFN.get(), feat, sizeof(float) * N * F, hipMemcpyHostToDevice, s));
         launch_transpose(m->lfFN.get(), m->lf.get(), F, N, s);
         DCRF_HIP_CHECK(hipStreamSynchronize(s));
+        finish_unary_upload(*m);
+        m->unary_pin.give();
         m->lF = F;
         m->logistic = true;
         m->has_unary = true;
@@ -1893,6 +2065,8 @@ int dcrf_set_unary_instance(dcrf_model* m, int i, const float* U) {
         require(!m->logistic, "the model has a logistic unary: set a full unary with dcrf_set_unary first");
         require(i >= 0 && i < m->geo.n_inst, "instance index out of range");
         const int N = m->N(), L = m->L, b = m->geo.pix_base[i], Ni = m->geo.N[i];
+        finish_unary_upload(*m);
+        m->unary_pin.give();  // (held by single-instance models: this call sets all of it)
         if (m->unary_host.size() != (size_t)N * L) {  // instances not set are zero at the upload
             m->unary_host.resize((size_t)N * L);
             m->unary_unset.assign(m->geo.n_inst, 1);
