@@ -16,6 +16,7 @@
 //   6. CSR          -> stable radix sort of entries by vertex: each vertex's contributors
 //                      in ascending pixel order, for the atomic-free splat
 #include "dcrf_internal.h"
+#include "dcrf_device.h"
 
 #include <cstring>
 
@@ -249,14 +250,15 @@ __global__ void __launch_bounds__(kThreads) k_embed(const float* __restrict__ fe
 // the previous point's entry of the same remainder takes that entry's slot, and only the
 // first of such a chain, its smallest, goes to the table.
 // Bound: latency of the table's and the keys' random reads, and atomics of many entries on
-// one new slot.  1024x768, every entry for itself: 242 us (d = 5), 121 us (d = 2); with
-// chains 210 and 45 us.
+// one new slot.  The slots and keys that one image region needs fit an XCD's L2, so each
+// XCD takes one range of entries.  1024x768, every entry for itself: 242 us (d = 5),
+// 121 us (d = 2); with chains 210 and 45 us, by ranges as well 84 and 49 us.
 template <int D>
 __global__ void __launch_bounds__(kThreads) k_hash_insert(const Key<D>* __restrict__ keys, int E,
                                                           int* table, uint32_t mask,
                                                           int* __restrict__ slot) {
     constexpr int D1 = D + 1;
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    const int e = xcd_block(blockIdx.x, gridDim.x) * kThreads + (int)threadIdx.x;
     const int lane = threadIdx.x & 63;
     const Key<D> k = keys[min(e, E - 1)];
     bool same = lane >= D1;
