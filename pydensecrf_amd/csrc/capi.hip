@@ -11,6 +11,7 @@
 #include <sys/mman.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cmath>
 #include <cstdlib>
@@ -482,8 +483,8 @@ struct dcrf_model {
     DevBuf<float> obj_w;
     DevBuf<double> obj_partial;
     // kernel-parameter gradient: the filter plans (built on first use for the lattices of
-    // generation lat_gen, which every lattice change advances), 3 [N][L] work slabs per
-    // term of a plan ([a | c], x), 2 [N][d] feature gradients (one-thread-per-point
+    // generation lat_gen, which every lattice change advances), 4 [N][L] work slabs per
+    // term of a plan ([a | c], x, lbl), 2 [N][d] feature gradients (one-thread-per-point
     // form), per-block partials and the accumulated gradient of all terms
     std::vector<std::unique_ptr<KgPlan>> kgplans;
     int lat_gen = 0;
@@ -745,8 +746,8 @@ std::vector<int> pass_step_limits(const dcrf_model& m) {
 // Pass tables of one lattice (forward axes 0..d, reverse d..0) over its neighbour rows
 // nbr [(d+1)][V] (global rows from vbase, zero row zero_row), passes of at most K steps.
 void build_pass_tables(const int2* nbr, int V, int d, int vbase, int zero_row, std::vector<int>& steps,
-                       std::vector<int>& off, DevBuf<int>& fwd, DevBuf<int>& rev, hipStream_t s,
-                       int K = kMaxPassSteps) {
+                       std::vector<int>& off, DevBuf<int>& fwd, DevBuf<int>& rev, int K,
+                       std::vector<PassTableJob>& jobs) {
     steps = pass_schedule(d + 1, K);
     off.assign(1, 0);
     for (int q : steps) off.push_back(off.back() + V * (q == 1 ? 3 : q == 2 ? 9 : 27));
@@ -755,13 +756,14 @@ void build_pass_tables(const int2* nbr, int V, int d, int vbase, int zero_row, s
     int first = 0;
     for (size_t p = 0; p < steps.size(); p++) {
         const int q = steps[p];
-        int fa[3], ta[3];
+        PassTableJob f{nbr, fwd.get() + off[p], V, vbase, zero_row, q, {}};
+        PassTableJob r{nbr, rev.get() + off[p], V, vbase, zero_row, q, {}};
         for (int j = 0; j < q; j++) {
-            fa[j] = first + j;
-            ta[j] = d - first - j;
+            f.axes[j] = first + j;
+            r.axes[j] = d - first - j;
         }
-        launch_pass_table(nbr, V, vbase, zero_row, q, fa, fwd.get() + off[p], s);
-        launch_pass_table(nbr, V, vbase, zero_row, q, ta, rev.get() + off[p], s);
+        jobs.push_back(f);
+        jobs.push_back(r);
         first += q;
     }
 }
@@ -770,8 +772,16 @@ void build_pass_tables(const int2* nbr, int V, int d, int vbase, int zero_row, s
 // where a segment's lanes fit a wave (and runs is set), recombination in one launch.
 void plan_segments(const RunSet& rs, int Lr, bool runs, SegPlan& P, hipStream_t s) {
     const LaunchShape sh = shape_for(Lr);
-    count_segments(rs, sh.wave && runs ? splat_shape(Lr).per : 0, sh.wave ? sh.per : 0, P, s);
+    count_segments(rs, sh.wave && runs ? splat_shape(Lr).per : 0, sh.wave ? sh.per : 0, false, P, s);
 }
+
+// The same for the filters of the normalisers and of the kernel-parameter gradient: every
+// vertex's segments in one sequence, whatever the row length and the other terms.  The
+// parameter gradient amplifies the last bits of its vertex rows and of the normalisers a
+// hundred times (two orders of summation differ by 1e-5 of the result at 512x512x21), so
+// these sums keep one order; it costs 11 us a recombination there against in-wave runs
+// and whole waves for the long ones.
+void plan_sequential(const RunSet& rs, SegPlan& P, hipStream_t s) { count_segments(rs, 0, 0, true, P, s); }
 
 // Splat of rows of Lr floats (stride Lr) over a list, and its recombination.
 void splat_lists(const SegLists& l, const int2* ent, const float* in, size_t rows_in, int Lr, float* vals,
@@ -853,8 +863,8 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
     P.Z2 = row;
     P.Z1 = xrow;
     // merged segment lists in the x layout's rows (the terms' vertices one after another):
-    // one for x (L floats a row), one for [a | c] and one for the all-ones input (one
-    // float), whose rows are then moved to the paired layout
+    // one for x, one for [a | c] and the all-ones input, whose rows are then moved to the
+    // paired layout
     RunSet rs;
     {
         std::vector<const TermLattice*> lats;
@@ -865,10 +875,8 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
         }
         build_run_set(lats, xbase, m.tiles.n_tiles(), m.chunk(), rs, s);
     }
-    SegPlan s1, s2, so;
-    plan_segments(rs, (int)L, true, s1, s);
-    plan_segments(rs, (int)(2 * L), true, s2, s);
-    plan_segments(rs, 1, true, so, s);
+    SegPlan sp;
+    plan_sequential(rs, sp, s);
     P.ent.reserve(E);
     for (size_t i = 0; i < P.parts.size(); i++) {
         const TermLattice& lat = m.terms[P.parts[i].term]->lat;
@@ -885,14 +893,10 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
         rm.X[i] = P.parts[i].X;
     }
     DCRF_HIP_CHECK(hipStreamSynchronize(s));  // the counts
-    emit_segments(rs, s1, P.Z1 + 1, P.l1, s);
-    for (auto q : {std::make_pair(&s2, &P.l2), std::make_pair(&so, &P.lo)}) {
-        SegLists& l = *q.second;
-        emit_segments(rs, *q.first, P.Z1 + 1, l, s);
-        launch_kg_relayout(l.ch.get(), l.nch, l.cb.get(), l.ncb, rm, s);
-        launch_kg_relayout(nullptr, 0, l.cb2.get(), l.ncb2, rm, s);
-        l.rows += P.Z2 - P.Z1;
-    }
+    emit_segments(rs, sp, P.Z1 + 1, P.l1, s);
+    emit_segments(rs, sp, P.Z1 + 1, P.l2, s);
+    launch_kg_relayout(P.l2.ch.get(), P.l2.nch, P.l2.cb.get(), P.l2.ncb, rm, s);
+    P.l2.rows += P.Z2 - P.Z1;
     // pass tables: pass p of term i expands the axes of its p-th pass; the forward chain
     // reads rows from F, the reverse chain from F in its first pass (the splat rows) and
     // from R after, the x chain from X
@@ -904,11 +908,13 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
     P.vp2.assign(P.passes, 0);
     P.vp1.assign(P.passes, 0);
     size_t toff = 0;
+    std::vector<PassTableJob> jobs;
+    std::vector<std::array<DevBuf<int2>, 3>> nbrs(P.parts.size());  // until the tables are built
     for (size_t i = 0; i < P.parts.size(); i++) {
         KgPart& part = P.parts[i];
         const TermLattice& lat = m.terms[part.term]->lat;
         const int V = lat.V, d = lat.d, d1 = d + 1;
-        DevBuf<int2> nF, nR, nX;  // the neighbour rows in each chain's numbering
+        DevBuf<int2>&nF = nbrs[i][0], &nR = nbrs[i][1], &nX = nbrs[i][2];  // the neighbour rows in each chain's numbering
         nF.reserve((size_t)d1 * V);
         nR.reserve((size_t)d1 * V);
         nX.reserve((size_t)d1 * V);
@@ -926,16 +932,21 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
             const size_t n = (size_t)V * (q == 1 ? 3 : 9);
             std::vector<int>& off = P.tab_off[p];
             off[3 * i] = (int)toff;
-            launch_pass_table(nF.get(), V, part.F, P.Z2, q, fa, P.tab.get() + toff, s);
+            auto table = [&](const int2* nbr, int base, int zero_row, const int* axes) {
+                PassTableJob t{nbr, P.tab.get() + toff, V, base, zero_row, q, {}};
+                std::copy(axes, axes + q, t.axes);
+                jobs.push_back(t);
+            };
+            table(nF.get(), part.F, P.Z2, fa);
             toff += n;
             off[3 * i + 1] = (int)toff;
             if (p == 0)
-                launch_pass_table(nF.get(), V, part.F, P.Z2, q, ta, P.tab.get() + toff, s);
+                table(nF.get(), part.F, P.Z2, ta);
             else
-                launch_pass_table(nR.get(), V, part.R, P.Z2, q, ta, P.tab.get() + toff, s);
+                table(nR.get(), part.R, P.Z2, ta);
             toff += n;
             off[3 * i + 2] = (int)toff;
-            launch_pass_table(nX.get(), V, part.X, P.Z1, q, fa, P.tab.get() + toff, s);
+            table(nX.get(), part.X, P.Z1, fa);
             toff += n;
             P.vp2[p] = part.R + V;  // the parts are in decreasing pass count
             P.vp1[p] = part.X + V;
@@ -947,6 +958,7 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
         launch_slice_weights(lat.vtx.get(), lat.bary.get(), nullptr, 0, slice_alpha(d), N, d1, 0, gv.get(),
                              part.sw.get(), s);
     }
+    launch_pass_tables(jobs, s);
     // vertex rows: the zero rows stay zero (splats write vertex and partial rows, the
     // blur passes rows below the zero row)
     auto zeroed = [&](DevBuf<float>& b, size_t n) {
@@ -960,14 +972,14 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
     zeroed(P.B1, (size_t)(P.Z1 + 1) * L);
     // the all-ones input of every term (stacked, one value per pixel) through the plan's
     // splat and both chains; the reverse rows are the terms' K^T 1
-    zeroed(P.ones[0], (size_t)P.lo.rows);
+    zeroed(P.ones[0], (size_t)P.l2.rows);
     zeroed(P.ones[1], (size_t)P.Z2 + 1);
     zeroed(P.ones[2], (size_t)P.Z2 + 1);
     DevBuf<float> in1;
     in1.reserve((size_t)P.parts.size() * N);
     launch_fill(in1.get(), 1.f, (size_t)P.parts.size() * N, s);
-    splat_lists(P.lo, P.ent.get(), in1.get(), P.parts.size() * (size_t)N, 1, P.ones[0].get(), s);
-    combine_lists(P.lo, 1, P.ones[0].get(), s);
+    splat_lists(P.l2, P.ent.get(), in1.get(), P.parts.size() * (size_t)N, 1, P.ones[0].get(), s);
+    combine_lists(P.l2, 1, P.ones[0].get(), s);
     float* const obuf[2] = {P.ones[1].get(), P.ones[2].get()};
     kg_blur(P, false, P.ones[0].get(), obuf, 1, s);
     for (KgPart& part : P.parts) part.ones_rev = obuf[(part.passes - 1) & 1] + part.R;
@@ -1024,6 +1036,7 @@ void kernel_grad_group(dcrf_model& m, const KgPlan& P, const float* b, const flo
     const int T = (int)P.parts.size();
     float* pk = m.kgbuf.get();            // [T][N][2L]
     float* xb = pk + (size_t)2 * T * NL;  // [T][N][L]
+    float* lbl = xb + (size_t)T * NL;     // [T][N][L]
     bool any_x = false;
     SliceTable pst{};
     KgInputs in{};
@@ -1035,6 +1048,9 @@ void kernel_grad_group(dcrf_model& m, const KgPlan& P, const float* b, const flo
         pst.t[i] = SliceTerm{nullptr, nullptr, nullptr, 1, t.ckind, t.d_compat.get(), kw ? kw + k : nullptr, nullptr, L};
         in.norm[i] = t.norm.get();
         in.ntype[i] = t.ntype;
+        // x reads fa and lbl, but for AFTER
+        const bool need_fa = t.ntype != DCRF_NO_NORMALIZATION && t.ntype != DCRF_NORMALIZE_AFTER;
+        in.lbl[i] = need_fa ? lbl + (size_t)i * NL : nullptr;
     }
     launch_kg_prepare(Qt, b, m.ldv, in, N, L, pst, pk, s);
     splat_lists(P.l2, P.ent.get(), pk, (size_t)T * N, L2, P.S2.get(), s);
@@ -1060,7 +1076,7 @@ void kernel_grad_group(dcrf_model& m, const KgPlan& P, const float* b, const flo
             const int d1 = t.lat.d + 1;
             st.t[0] = SliceTerm{vtx, sw, need_fa ? rev_of(i) : nullptr, d1, -1, nullptr, nullptr, nullptr, L2};  // K^T a
             st.t[1] = SliceTerm{vtx, sw, need_fb ? fwd_of(i) + L : nullptr, d1, -1, nullptr, nullptr, nullptr, L2};  // K c
-            launch_kg_x(pk + (size_t)i * 2 * NL, t.norm.get(), N, L, st, t.ntype, x, s);
+            launch_kg_x(b, m.ldv, lbl + (size_t)i * NL, t.norm.get(), N, L, st, t.ntype, x, s);
         }
         splat_lists(P.l1, P.ent.get(), xb, (size_t)T * N, L, P.S1.get(), s);
         combine_lists(P.l1, L, P.S1.get(), s);
@@ -1222,7 +1238,7 @@ void blur_rows(dcrf_model& m, float* v0, float* v1, int Lv, bool transpose, hipS
 
 // The normalisers of all terms: norm = K 1 (pairwise.cpp:44), then the normalisation of
 // :46-61.  One filter of the all-ones input over every term's lattice, one float a row,
-// through the layout's run set and pass tables (so: the counts `so` for rows of one float).
+// through the layout's run set and pass tables (so: the counts of its sequential lists).
 void compute_norms(dcrf_model& m, const RunSet& rs, const SegPlan& so, hipStream_t s) {
     const int N = m.N(), T = (int)m.order.size(), V = m.V_total;
     struct Untimed {  // these launches are no part of the timed classes
@@ -1345,7 +1361,7 @@ void ensure_layout(dcrf_model& m) {
     m.tiled = false;
     SegPlan sp, so;
     if (m.tile_side && T) {
-        count_segments(rs, 0, 0, sp, s);
+        count_segments(rs, 0, 0, false, sp, s);
         std::vector<int> gs(rs.G + 1), ge(rs.G + 1), ts(NT + 1), te(NT + 1);
         copy_to_host(gs.data(), sp.gseg.get(), sizeof(int) * gs.size(), s);
         copy_to_host(ge.data(), rs.gebase.get(), sizeof(int) * ge.size(), s);
@@ -1370,10 +1386,11 @@ void ensure_layout(dcrf_model& m) {
     m.ldv = m.tiled ? L : padded_labels(L);
     if (T) {
         plan_segments(rs, m.ldv, !m.tiled, sp, s);
-        plan_segments(rs, 1, true, so, s);
+        plan_sequential(rs, so, s);
     }
     m.tl.clear();
     m.tl.resize(T);
+    std::vector<PassTableJob> jobs;
     for (int k : m.order) {  // what the normalisers need
         const TermLattice& lat = m.terms[k]->lat;
         const int d1 = lat.d + 1;
@@ -1382,9 +1399,10 @@ void ensure_layout(dcrf_model& m) {
         launch_remap_nbr(lat.nbr.get(), lay->nbr.get(), d1 * lat.V, m.vbase[k], V, s);
         if (m.pairs)  // forward passes walk axes 0..d, the transpose's d..0 (permutohedral.cpp:556)
             build_pass_tables(lay->nbr.get(), lat.V, lat.d, m.vbase[k], V, lay->pass_steps, lay->pass_off,
-                              lay->passF, lay->passT, s, step_limit[k]);
+                              lay->passF, lay->passT, step_limit[k], jobs);
         m.tl[k] = std::move(lay);
     }
+    launch_pass_tables(jobs, s);
     m.n_passes = m.pairs ? blur_launches(m) : 0;
     m.prefixP.assign(m.n_passes, 0);
     for (int p = 0; p < m.n_passes; p++)
@@ -1718,7 +1736,7 @@ void backward(dcrf_model& m, const float* dQ, float* dU, float* dcompat, float* 
         }
         size_t tmax = 1;
         for (const auto& P : m.kgplans) tmax = std::max(tmax, P->parts.size());
-        m.kgbuf.reserve(3 * tmax * NL);
+        m.kgbuf.reserve(4 * tmax * NL);
         if (dslow) m.kgdf.reserve((size_t)2 * N * dslow);
         pstride = kparam_partial_doubles(dmax);
         m.kpartial.reserve(pstride * T);

@@ -137,6 +137,16 @@ __device__ __forceinline__ const float* row_piece(const float* __restrict__ base
     return base + (size_t)row * ld + k0;
 }
 
+// s + w x, the product rounded as well (the filters' sums).  Fused multiply-adds have the
+// same errors on average, but every other rounding moves the kernel-parameter gradients
+// by their own error: those amplify the vertex rows' last bits a hundred times (1e-5 of
+// the result at 512x512x21).  The sums wait for the row gathers either way: 0.6 % of an inference at
+// 1024x768x21.
+__device__ __forceinline__ float add_product(float s, float w, float x) {
+    const float p = w * x;
+    return s + p;
+}
+
 // Value x of lane `lane` of the wave (every lane of the wave calls).
 __device__ __forceinline__ float wave_read(float x, int lane) {
     return __int_as_float(__builtin_amdgcn_ds_bpermute(lane << 2, __float_as_int(x)));
@@ -373,7 +383,7 @@ __device__ __forceinline__ void slice_piece(const SliceTerm& T, int p, int k0, i
     for (int j = 0; j < kMaxD1; j++)
         if (j < d1) {
 #pragma unroll
-            for (int r = 0; r < R; r++) m[r] = fmaf(w[j], x[j][r], m[r]);
+            for (int r = 0; r < R; r++) m[r] = add_product(m[r], w[j], x[j][r]);
         }
 }
 

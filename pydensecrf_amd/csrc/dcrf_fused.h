@@ -26,7 +26,7 @@ __device__ __forceinline__ void term_message(const SliceTerm& T, int k, const in
     for (int j = jb; j < je; j++) {
         const float w = __int_as_float(e[j].y);
 #pragma unroll
-        for (int r = 0; r < R; r++) raw[r] = fmaf(w, x[j][r], raw[r]);
+        for (int r = 0; r < R; r++) raw[r] = add_product(raw[r], w, x[j][r]);
     }
 #pragma unroll
     for (int r = 0; r < R; r++) m[r] = raw[r];

@@ -132,10 +132,11 @@ struct SegCounts {
     int partial, light, heavy, empty, pieces;
 };
 // The list sizes for per segments a splat wave (0: no in-wave runs) and perc lane groups a
-// recombination wave (0: two levels).
+// recombination wave (0: two levels, or one where split allows any number of partial rows).
 struct SegPlan {
-    int per = 0, perc = 0;
-    DevBuf<int> gseg, H, vcount, vfirst;
+    int per = 0, perc = 0, split = 0;
+    DevBuf<int> gseg, H;
+    DevBuf<int> vfirst;  // [V + 1] heads before each vertex
     DevBuf<SegCounts> vs;
     SegCounts host[2] = {};  // totals; [1].partial: the groups' segments
 };
@@ -150,7 +151,8 @@ struct SegLists {
 void build_run_set(const std::vector<const TermLattice*>& lats, const std::vector<int>& vbase, int n_tiles, int C,
                    RunSet& rs, hipStream_t s);
 // Queues the counting; P.host is valid after the stream has been synchronised.
-void count_segments(const RunSet& rs, int per, int perc, SegPlan& P, hipStream_t s);
+// sequential (with per = perc = 0): a vertex's segments are added one after another.
+void count_segments(const RunSet& rs, int per, int perc, bool sequential, SegPlan& P, hipStream_t s);
 // The lists, partial rows from row0 (after P's counts have arrived).
 void emit_segments(const RunSet& rs, const SegPlan& P, int row0, SegLists& L, hipStream_t s);
 
@@ -179,7 +181,7 @@ struct KgPlan {
     int gen = -1;  // the model's lattice generation the plan was built for
     int Z2 = 0, Z1 = 0, passes = 0;
     DevBuf<int2> ent;    // (stacked input row, barycentric weight bits) in segment order
-    SegLists l2, l1, lo;  // segment lists of the [a | c] and x layouts, and of the ones (paired rows)
+    SegLists l2, l1;  // segment lists of the paired rows ([a | c], the ones) and of the x rows
     std::vector<int> vp2, vp1;  // per pass: one past the last row it writes
     DevBuf<int> tab;            // the pass tables of all chains
     std::vector<std::vector<int>> tab_off;  // per pass: forward, reverse, x table of each part
@@ -370,9 +372,19 @@ void launch_blur(const float* src, float* dst, int v0, int Vp, int ldv, int L, c
 void launch_blur_pass(const float* src, float* dst, int v0, int Vp, int ldv, int L, const PassTable& pt,
                       hipStream_t s, int R = 0);
 // The table of a K-step pass (axes[0] first) of one term from its global neighbour
-// rows nbr [(d+1)][V].
-void launch_pass_table(const int2* nbr, int V, int vbase, int zero_row, int K, const int* axes, int* tab,
-                       hipStream_t s);
+// rows nbr [(d+1)][V]; many tables in one launch (each is a few microseconds' work: 25
+// launches a new lattice pair when every pass of every chain had its own).
+struct PassTableJob {
+    const int2* nbr;
+    int* tab;
+    int V, vbase, zero_row, K;
+    int axes[3];
+};
+struct PassTableJobs {
+    static constexpr size_t kMax = 32;
+    PassTableJob job[kMax];
+};
+void launch_pass_tables(const std::vector<PassTableJob>& jobs, hipStream_t s);
 // Mean-field update: E = -U - sum_k compat_k(slice_k); Q = softmax(E).  U may be null.
 // tmp1/tmp2 optional outputs (energy, last term's message).
 // Lv: floats of the vertex rows (padded_labels(L), or L); Q has rows of ldq floats, L or Lv.
@@ -483,14 +495,15 @@ void launch_set_compat(const float* raw, int ckind, int L, float* cw, hipStream_
 // AFTER), c = C (w Q_t) (times n for SYMMETRIC / BEFORE).  Qt and b have rows of ldq floats.
 struct KgInputs {
     const float* norm[DCRF_MAX_TERMS / 2];
+    float* lbl[DCRF_MAX_TERMS / 2];  // [N][L] C (w Q_t), or null
     int ntype[DCRF_MAX_TERMS / 2];
 };
 void launch_kg_prepare(const float* Qt, const float* b, int ldq, const KgInputs& in, int N, int L, const SliceTable& st,
                        float* P, hipStream_t s);
-// The normaliser-derivative input x of featureGradient for ntype from the term's rows
-// P, with fa sliced by st.t[0] and fb by st.t[1] (the same entries; null vals: not needed).
-void launch_kg_x(const float* P, const float* norm, int N, int L, const SliceTable& st, int ntype, float* x,
-                 hipStream_t s);
+// The normaliser-derivative input x of featureGradient for ntype (b rows of ldb floats),
+// with fa sliced by st.t[0] and fb by st.t[1] (the same entries; null vals: not needed).
+void launch_kg_x(const float* b, int ldb, const float* lbl, const float* norm, int N, int L, const SliceTable& st,
+                 int ntype, float* x, hipStream_t s);
 // Whether launch_kg_grad has a kernel for L labels and feature dimension d.
 bool kg_grad_fused(int L, int d);
 // The parameter gradient of fg = -G(x, 1) + G(a, c) (xr null: fg = G(a, c)) against

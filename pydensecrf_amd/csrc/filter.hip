@@ -153,7 +153,7 @@ __global__ void __launch_bounds__(1024) k_splat(const Chunk* __restrict__ chunks
                         if (i + u < b) {
                             const float wu = __int_as_float(e[u].y);
 #pragma unroll
-                            for (int r = 0; r < R; r++) acc[r] = fmaf(wu, xx[u][r], acc[r]);
+                            for (int r = 0; r < R; r++) acc[r] = add_product(acc[r], wu, xx[u][r]);
                         }
                     }
                 }
@@ -193,7 +193,7 @@ __global__ void __launch_bounds__(1024) k_splat(const Chunk* __restrict__ chunks
             if (i + u < ch.end) {
                 const float wu = __int_as_float(e[u].y);
 #pragma unroll
-                for (int r = 0; r < R; r++) acc[r] = fmaf(wu, xx[u][r], acc[r]);
+                for (int r = 0; r < R; r++) acc[r] = add_product(acc[r], wu, xx[u][r]);
             }
         }
     }
@@ -286,8 +286,7 @@ __global__ void __launch_bounds__(kWaveBlock) k_splat_split(const Chunk* __restr
 // the same bits).
 constexpr int kStage = 32;
 
-// FMA: k_splat's additions, else k_splat_split's.
-template <int R, bool FMA>
+template <int R>
 __global__ void __launch_bounds__(1024) k_splat_tiled(TiledSplat ts, const int2* __restrict__ ent,
                                                             const float* __restrict__ in, float* __restrict__ vals,
                                                             int ldv, int L, int S, int per, int q_max) {
@@ -348,14 +347,7 @@ __global__ void __launch_bounds__(1024) k_splat_tiled(TiledSplat ts, const int2*
         for (int r = 0; r < R; r++) acc[r] = 0.0f;
         auto add = [&](float ww, const float (&x)[R]) {
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                if (FMA) {
-                    acc[r] = fmaf(ww, x[r], acc[r]);
-                } else {
-                    const float prod = ww * x[r];
-                    acc[r] = acc[r] + prod;
-                }
-            }
+            for (int r = 0; r < R; r++) acc[r] = add_product(acc[r], ww, x[r]);
         };
         int i = b;
         for (; i + 4 <= e; i += 4) {
@@ -382,6 +374,9 @@ __global__ void __launch_bounds__(1024) k_splat_tiled(TiledSplat ts, const int2*
     }
 }
 
+// (Sequential lists have vertices of hundreds of partial rows, added one after another:
+// kLong loads in flight for those.  512x512x21: 16.1 -> 10.8 us.)
+constexpr int kLong = 16;
 template <bool WAVE, int R>
 __global__ void __launch_bounds__(1024) k_combine(const Combine* __restrict__ cb, int n, float* __restrict__ vals,
                                                   int ldv, int L, int S, int per) {
@@ -393,7 +388,17 @@ __global__ void __launch_bounds__(1024) k_combine(const Combine* __restrict__ cb
     float acc[R];
 #pragma unroll
     for (int r = 0; r < R; r++) acc[r] = 0.0f;
-    for (int i = 0; i < rc.count; i += kBatch) {  // count >= 2; loads clamped to the last row
+    int i = 0;
+    for (; i + kLong <= rc.count; i += kLong) {
+        float xx[kLong][R];
+#pragma unroll
+        for (int u = 0; u < kLong; u++) load_piece<R>(vals + (size_t)(rc.first + i + u) * ldv, k0, L, xx[u]);
+#pragma unroll
+        for (int u = 0; u < kLong; u++)
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[r] = acc[r] + xx[u][r];
+    }
+    for (; i < rc.count; i += kBatch) {  // count >= 2; loads clamped to the last row
         float xx[kBatch][R];
 #pragma unroll
         for (int u = 0; u < kBatch; u++)
@@ -620,11 +625,14 @@ __global__ void __launch_bounds__(1024) k_blur_pass(const float* __restrict__ sr
 
 // Pass table of one term: entry (i_K, .., i_1) of vertex v at v*3^K + sum i_j 3^(j-1),
 // expanding along axis ax[j-1] at level j (ax[K-1] first, the pass's last step).
-__global__ void k_pass_table(const int2* __restrict__ nbr, int V, int vbase, int zero_row, int K, int ax0, int ax1,
-                             int ax2, int* __restrict__ tab) {
+__global__ void k_pass_tables(PassTableJobs J) {
+    const PassTableJob& T = J.job[blockIdx.y];
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    const int V = T.V, vbase = T.vbase, zero_row = T.zero_row, K = T.K;
     if (v >= V) return;
-    const int ax[3] = {ax0, ax1, ax2};
+    const int2* __restrict__ nbr = T.nbr;
+    const int* ax = T.axes;
+    int* __restrict__ tab = T.tab;
     int cur[27], nxt[27];
     cur[0] = vbase + v;
     int n = 1;
@@ -832,15 +840,19 @@ __global__ void k_remap_nbr(const int* __restrict__ src, int2* __restrict__ dst,
     dst[i] = make_int2(a >= 0 ? a + vbase : zero_row, b >= 0 ? b + vbase : zero_row);
 }
 
+// The sorted entries' (pixel, weight) pairs of term `term` in the groups' order.  Bound: the
+// random reads of the weights, which stay inside a tile: each XCD takes one range of them.
+// 1024x768: 33 -> 24.5 us a launch.
 __global__ void k_entry_gather(const int* __restrict__ csr_e, int E, int d1, const float* __restrict__ bary,
                                const float* __restrict__ norm, int use_norm, const int* __restrict__ tile_ptr,
                                const int* __restrict__ gebase, int n_tiles, int T, int term, TileGeom g, int local,
                                int pix_off, int2* __restrict__ ent) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    const int j = xcd_block(blockIdx.x, gridDim.x) * kThreads + (int)threadIdx.x;
     if (j >= E) return;
     const int e = csr_e[j];
     const int p = e / d1;
-    const int t = last_le(tile_ptr, n_tiles, j);
+    int t = last_le(tile_ptr, n_tiles, __builtin_amdgcn_readfirstlane(j));  // one search a wave
+    if (j >= tile_ptr[t + 1]) t = last_le(tile_ptr, n_tiles, j);
     const int pos = gebase[t * T + term] + (j - tile_ptr[t]);
     const float b = bary[e];
     const float w = use_norm ? b * norm[p] : b;
@@ -987,22 +999,20 @@ void launch_splat_tiled(const TiledSplat& ts, const int2* ent, const float* in, 
     const int q_max = (ts.geom.side * ts.geom.side * L + 1) & ~1;  // the entry pairs start 8-byte aligned
     const int block = tiled_splat_block(lds, lds_cap);
     // dynamic LDS beyond the default launch limit must be granted per kernel
-    static size_t granted[10] = {};
+    static size_t granted[5] = {};
     auto grant = [&](const void* fn, int r) {
         if (lds > granted[r]) {
             DCRF_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
             granted[r] = lds;
         }
     };
-    const bool fma = splat_shape(L).K == 1;
-#define DCRF_TILED(R_, F_)                                                                                   \
-    case R_ * 2 + F_:                                                                                        \
-        grant(reinterpret_cast<const void*>(&k_splat_tiled<R_, F_>), R_ * 2 + F_);                            \
-        k_splat_tiled<R_, F_><<<ts.n_tiles, block, lds, s>>>(ts, ent, in, vals, ldv, L, sh.S, sh.per, q_max); \
+#define DCRF_TILED(R_)                                                                                   \
+    case R_:                                                                                             \
+        grant(reinterpret_cast<const void*>(&k_splat_tiled<R_>), R_);                                     \
+        k_splat_tiled<R_><<<ts.n_tiles, block, lds, s>>>(ts, ent, in, vals, ldv, L, sh.S, sh.per, q_max); \
         break;
-    switch (sh.R * 2 + (fma ? 1 : 0)) {
-        DCRF_TILED(1, 0) DCRF_TILED(2, 0) DCRF_TILED(3, 0) DCRF_TILED(4, 0)
-        DCRF_TILED(1, 1) DCRF_TILED(2, 1) DCRF_TILED(3, 1) DCRF_TILED(4, 1)
+    switch (sh.R) {
+        DCRF_TILED(1) DCRF_TILED(2) DCRF_TILED(3) DCRF_TILED(4)
         default: throw Error{DCRF_ERR_STATE, "no tiled splat kernel for this shape"};
     }
 #undef DCRF_TILED
@@ -1047,13 +1057,21 @@ void launch_blur_pass(const float* src, float* dst, int v0, int Vp, int ldv, int
     DCRF_DISPATCH(sh, k_blur_pass, blocks_for(Vp - v0, sh.items), 0, s, src, dst, v0, Vp, ldv, L, sh.S, sh.per, pt);
 }
 
-void launch_pass_table(const int2* nbr, int V, int vbase, int zero_row, int K, const int* axes, int* tab,
-                       hipStream_t s) {
-    if (V <= 0) return;
-    if (K < 1 || K > 3) throw Error{DCRF_ERR_STATE, "blur pass: 1 to 3 steps"};
-    k_pass_table<<<blocks_for(V), kThreads, 0, s>>>(nbr, V, vbase, zero_row, K, axes[0], K > 1 ? axes[1] : 0,
-                                                    K > 2 ? axes[2] : 0, tab);
-    DCRF_HIP_CHECK(hipGetLastError());
+void launch_pass_tables(const std::vector<PassTableJob>& jobs, hipStream_t s) {
+    constexpr size_t kMax = PassTableJobs::kMax;
+    for (size_t i0 = 0; i0 < jobs.size(); i0 += kMax) {
+        PassTableJobs J{};
+        const size_t n = std::min(kMax, jobs.size() - i0);
+        int V = 0;
+        for (size_t i = 0; i < n; i++) {
+            J.job[i] = jobs[i0 + i];
+            if (J.job[i].K < 1 || J.job[i].K > 3) throw Error{DCRF_ERR_STATE, "blur pass: 1 to 3 steps"};
+            V = std::max(V, J.job[i].V);
+        }
+        if (V <= 0) continue;
+        k_pass_tables<<<dim3(blocks_for(V), (unsigned)n), kThreads, 0, s>>>(J);
+        DCRF_HIP_CHECK(hipGetLastError());
+    }
 }
 
 bool fused_meanfield_ok(int L, int nterms, int d1_0, int d1_1) {

@@ -41,11 +41,12 @@ inline unsigned blocks_for(size_t n, int t = kThreads) { return (unsigned)((n + 
 // weighted Q_t (PairwisePotential::kernelGradient, pairwise.cpp:202-207; st.t[k] carries
 // the compatibility and the weight), and the row P[k N + p] = [a | c] (2L floats), a = b n
 // (SYMMETRIC, AFTER) or b, c = lbl n (SYMMETRIC, BEFORE) or lbl.  One splat and the two
-// blur orders of P give K a, K^T a, K c, K^T c.  Matrix weights with an LDS copy read the
+// blur orders of P give K a, K^T a, K c, K^T c.  lbl is stored where the caller gives a
+// buffer (the normaliser input x reads it).  Matrix weights with an LDS copy read the
 // pixel's messages as rows there in wave mode (msg; matrix_piece_rows).
-// Bound: memory, 2 rows read and 2 written per term and point.  One launch per term, with
-// lbl stored beside P and the messages passed by shuffles, took 2 x 29 us at 512x512x21
-// with two Matrix terms; this form 44 us.
+// Bound: memory, 2 rows read, and 3 written per term and point.  One launch per term, with
+// the messages passed by shuffles, took 2 x 29 us at 512x512x21 with two Matrix terms;
+// this form 50 us.
 template <bool WAVE, int R, bool CWL>
 __global__ void __launch_bounds__(1024) k_kg_prepare(const float* __restrict__ Qt, const float* __restrict__ b,
                                                      int ldq, KgInputs in, int N, int L, int S, int per,
@@ -103,32 +104,32 @@ __global__ void __launch_bounds__(1024) k_kg_prepare(const float* __restrict__ Q
             av[r] = na ? bv[r] * n : bv[r];
             cv[r] = nc ? c[r] * n : c[r];
         }
+        if (in.lbl[k]) store_piece<R>(in.lbl[k] + (size_t)p * L, G.k0, L, c);
         float* row = P + ((size_t)k * N + p) * 2 * L;
         store_piece<R>(row, G.k0, L, av);
         store_piece<R>(row + L, G.k0, L, cv);
     }
 }
 
-// The first argument x of featureGradient's norm-derivative term from fa = K^T a, fb = K c
-// and the point's row [a | c] of P, whose halves carry one factor n of the reference's
-// forms already:
-//   SYMMETRIC  x = (0.5 (b fb + fa lbl)) n^3 = (0.5 (a fb + fa c)) n^2   (pairwise.cpp:90-97)
-//   AFTER      x = (b fb) n^2 = (a fb) n                                 (:98-105)
-//   BEFORE     x = (fa lbl) n^2 = (fa c) n                               (:106-113)
+// The first argument x of featureGradient's norm-derivative term from fa = K^T a, fb = K c,
+// the point's b and lbl:
+//   SYMMETRIC  x = (0.5 (b fb + fa lbl)) n^3      (pairwise.cpp:90-97)
+//   AFTER      x = (b fb) n^2                     (:98-105)
+//   BEFORE     x = (fa lbl) n^2                   (:106-113)
 template <int R>
-__device__ __forceinline__ void kg_x_value(const float* __restrict__ prow, int k0, int L, float n, int ntype,
-                                           const float (&fa)[R], const float (&fb)[R], float (&v)[R]) {
-    float a[R] = {}, c[R] = {};
-    if (ntype != DCRF_NORMALIZE_BEFORE) load_piece<R>(prow, k0, L, a);
-    if (ntype != DCRF_NORMALIZE_AFTER) load_piece<R>(prow + L, k0, L, c);
+__device__ __forceinline__ void kg_x_value(const float* __restrict__ brow, const float* __restrict__ lrow, int k0,
+                                           int L, float n, int ntype, const float (&fa)[R], const float (&fb)[R],
+                                           float (&v)[R]) {
+    float bv[R] = {}, lv[R] = {};
+    const bool sym = ntype == DCRF_NORMALIZE_SYMMETRIC, after = ntype == DCRF_NORMALIZE_AFTER;
+    if (sym || after) load_piece<R>(brow, k0, L, bv);
+    if (!after) load_piece<R>(lrow, k0, L, lv);
+    const float n2 = n * n, n3 = n2 * n;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        if (ntype == DCRF_NORMALIZE_SYMMETRIC)
-            v[r] = 0.5f * fmaf(a[r], fb[r], fa[r] * c[r]) * (n * n);
-        else if (ntype == DCRF_NORMALIZE_AFTER)
-            v[r] = a[r] * fb[r] * n;
-        else
-            v[r] = fa[r] * c[r] * n;
+        const float p1 = bv[r] * fb[r], p2 = fa[r] * lv[r];
+        const float sum = p1 + p2;
+        v[r] = sym ? 0.5f * sum * n3 : after ? p1 * n2 : p2 * n2;
     }
 }
 
@@ -136,7 +137,8 @@ __device__ __forceinline__ void kg_x_value(const float* __restrict__ prow, int k
 // rows, from label L on) sliced in the same pass; a slice whose rows are null is not
 // needed by the normalisation type.  For the shapes that k_kg_x_rows does not cover.
 template <bool WAVE, int R>
-__global__ void __launch_bounds__(1024) k_kg_x(const float* __restrict__ P, const float* __restrict__ norm, int N,
+__global__ void __launch_bounds__(1024) k_kg_x(const float* __restrict__ b, int ldb, const float* __restrict__ lbl,
+                                               const float* __restrict__ norm, int N,
                                                int L, int S, int per, SliceTable st, int ntype,
                                                float* __restrict__ x) {
     LaneGroup<WAVE, R> G(L, S, per, nullptr);  // no group-wide operation here
@@ -145,7 +147,7 @@ __global__ void __launch_bounds__(1024) k_kg_x(const float* __restrict__ P, cons
     float fa[R] = {}, fb[R] = {}, v[R];
     if (st.t[0].vals) slice_piece<R>(st.t[0], p, G.k0, L, fa);
     if (st.t[1].vals) slice_piece<R>(st.t[1], p, G.k0, L, fb);
-    kg_x_value<R>(P + (size_t)p * 2 * L, G.k0, L, norm[p], ntype, fa, fb, v);
+    kg_x_value<R>(b + (size_t)p * ldb, lbl + (size_t)p * L, G.k0, L, norm[p], ntype, fa, fb, v);
     store_piece<R>(x + (size_t)p * L, G.k0, L, v);
 }
 
@@ -165,9 +167,10 @@ __device__ __forceinline__ void stage_done() {
 // The same for lane groups inside a wave and d = D: both slices use the lattice's entries
 // once, all 2 (D + 1) rows are in flight together.
 // Bound: the row gathers.  512x512x21: the form above took 38 us a term (mean of d = 2 and
-// 5), this one 19 (d = 2) and 27 us (d = 5).
+// 5), this one 21 (d = 2) and 31 us (d = 5).
 template <int R, int D>
-__global__ void __launch_bounds__(kWaveBlock) k_kg_x_rows(const float* __restrict__ P, const int* __restrict__ vtx,
+__global__ void __launch_bounds__(kWaveBlock) k_kg_x_rows(const float* __restrict__ b, int ldb,
+                                                          const float* __restrict__ lbl, const int* __restrict__ vtx,
                                                           const float* __restrict__ sw, const float* __restrict__ ra,
                                                           const float* __restrict__ rb, const float* __restrict__ norm,
                                                           int N, int L, int S, int per, int ntype,
@@ -196,11 +199,11 @@ __global__ void __launch_bounds__(kWaveBlock) k_kg_x_rows(const float* __restric
         const float w = ss[G.w][gp * D1 + q];
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            if (ra) fa[r] = fmaf(w, ua[q][r], fa[r]);
-            if (rb) fb[r] = fmaf(w, ub[q][r], fb[r]);
+            if (ra) fa[r] = add_product(fa[r], w, ua[q][r]);
+            if (rb) fb[r] = add_product(fb[r], w, ub[q][r]);
         }
     }
-    kg_x_value<R>(P + (size_t)p * L2, G.k0, L, norm[p], ntype, fa, fb, v);
+    kg_x_value<R>(b + (size_t)p * ldb, lbl + (size_t)p * L, G.k0, L, norm[p], ntype, fa, fb, v);
     if (G.on && G.g < np) store_piece<R>(x + (size_t)p * L, G.k0, L, v);
 }
 
@@ -291,171 +294,167 @@ struct KgGrad {
     int full;  // FULL_KERNEL: d*d parameters, else d
 };
 
-// t[q - 1] += sign * (sum over the lane's labels of c (u_q - u_0)), q = 1..D, u_q the
-// lane's piece of the point's vertex row q (rows of ld floats from vals).
-template <int R, int D>
-__device__ __forceinline__ void grad_dots(const float* __restrict__ vals, int ld, const int* v, int k0, int L,
-                                          const float (&c)[R], float (&t)[D]) {
-    float u0[R], u[D][R];
-    load_piece<R>(vals + (size_t)v[0] * ld + k0, 0, L, u0);
+// The point's elevated differences e_j of one label (the loop body of k_slice_grad) from
+// its d+1 vertex values: alpha u_q - alpha u_{q+1} in vertex order, rotated by select.
+template <int D>
+__device__ __forceinline__ void elevate(const float (&u)[D + 1], const int (&r0)[D + 1], const GradScale& gs,
+                                        float (&e)[D]) {
+    constexpr int D1 = D + 1;
+    float au[D1], diff[D1], ra[D1];
 #pragma unroll
-    for (int q = 1; q <= D; q++) load_piece<R>(vals + (size_t)v[q] * ld + k0, 0, L, u[q - 1]);
+    for (int q = 0; q < D1; q++) au[q] = gs.alpha * u[q];
 #pragma unroll
-    for (int q = 0; q < D; q++)
+    for (int q = 0; q < D1; q++) diff[q] = au[q] - au[q + 1 > D ? 0 : q + 1];
 #pragma unroll
-        for (int r = 0; r < R; r++) t[q] = fmaf(c[r], u[q][r] - u0[r], t[q]);
+    for (int j = 0; j < D1; j++) {
+        ra[j] = diff[0];
+#pragma unroll
+        for (int q = 1; q < D1; q++) ra[j] = r0[j] == q ? diff[q] : ra[j];
+    }
+    float sm = ra[0];
+#pragma unroll
+    for (int j = 1; j <= D; j++) {
+        const float jr = (float)j * ra[j];
+        const float d = sm - jr;
+        e[j - 1] = gs.sf[j - 1] * d;
+        sm = sm + ra[j];
+    }
+}
+
+// The lane's share of one direction of the slicing gradient for its R consecutive labels,
+// from the point's vertex rows (rows of ld floats from vals), paired with c: grad[j] sums
+// the lane's labels in order.  ONES: c is all ones.
+template <int R, int D, bool ONES>
+__device__ __forceinline__ void grad_share(const float* __restrict__ vals, int ld, const int (&v)[D + 1], int k0,
+                                           int L, const int (&r0)[D + 1], const float (&c)[R], const GradScale& gs,
+                                           float* grad) {
+    constexpr int D1 = D + 1;
+    float x[D1][R];
+#pragma unroll
+    for (int q = 0; q < D1; q++) load_piece<R>(vals + (size_t)v[q] * ld + k0, 0, L, x[q]);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        float u[D1], e[D];
+#pragma unroll
+        for (int q = 0; q < D1; q++) u[q] = x[q][r];
+        elevate<D>(u, r0, gs, e);
+#pragma unroll
+        for (int j = 0; j < D; j++) {
+            const float prod = ONES ? e[j] : c[r] * e[j];
+            grad[j] = r ? grad[j] + prod : 0.0f + prod;
+        }
+    }
 }
 
 // The whole per-point part of one term's kernel gradient in one pass, S lanes per point
 // and R labels per lane (S <= 64: lane groups inside one wave), d <= 6:
 //   g = G(a, c) = dir 0 (K a rows, paired with c) + dir 1 (K^T c rows, paired with a),
 //   r = G(x, 1) = dir 0 (K x rows, paired with ones) + dir 1 (K^T 1, paired with x),
-//   fg = -r + g (g alone without a normaliser term: x and its rows are not read).
-// A direction's share is linear in the products T_q = sum_k c_k u_q[k] of the paired row
-// with the point's vertex rows, and only differences of the T_q enter it: each lane
-// accumulates T_q - T_0 of all four directions over its labels (D values), the group adds
-// them (a pairwise tree towards its first lane), and the rotation by rank and the
-// elevation (k_slice_grad's, on alpha T) follow once per point, one lane each, for up to
-// 64 points of the wave's rounds together.  (Rotated and elevated per label, as
-// k_slice_grad does, the selections were most of the instructions: 90 us at 512x512x21
-// with d = 5 and 36 us with d = 2; this form 45 and 25 us, bound by the 3 (d + 1) row
-// gathers.)
+//   fg = -r + g (g alone without a normaliser term: x and its rows are not read),
+// each direction summed over the group's lanes (a pairwise tree towards the group's
+// first lane) before the two are added; the 4d lane shares go through one tree together.
+// Bound: instructions, most of them the selections of the rotation.  The differences are
+// taken before the selection (one select tree per axis instead of two), the all-ones
+// rows are elevated once per point instead of per label, and the entries are read once
+// per wave: 90 -> 65 us at 512x512x21 with d = 5; 36 us with d = 2, as before.  (Label sums
+// first, in double, and one rotation per point took 51 and 26 us and were left out: g and
+// r nearly cancel, and with any other rounding of the point's part the parameter gradients
+// land elsewhere within their 1e-5.)
 // The parameter products (pairwise.cpp:157-161), DIAG f[q(p)][j] fg[j], FULL fg[r]
-// f[q(p)][c] at c*d + r (column-major, like the reference), are added in double in a fixed
-// order: DIAG by each point's lane over the batches, then a tree over the lanes; FULL by
-// lane q of the wave for parameter q, over the batch's points in order.  At the end the
-// waves' sums are added in wave order, and the block adds them to partial[blockIdx.x][q]:
-// one row per block sums all reverse iterations, in iteration order.
+// f[q(p)][c] at c*d + r (column-major, like the reference), are added in double by one
+// lane per parameter.  Per round the group leaders leave fg and the point's feature row
+// in LDS, and lane q of the wave adds its product for the wave's points in point order,
+// over the block's `rounds` consecutive blocks' worth of points.  At the end the waves'
+// sums are added in wave order, and the block adds them to partial[blockIdx.x][q]: one
+// row per block sums all reverse iterations, in iteration order.  The label order of
+// each direction's sum differs from the reference's sequential one (float tolerance).
 template <int R, int D>
 __global__ void __launch_bounds__(kWaveBlock) k_kg_grad(const int* __restrict__ vtx, const int* __restrict__ rank,
                                                         KgGrad a, int N, int L, int S, int per, int rounds,
                                                         GradScale gs, double* __restrict__ partial) {
     constexpr int D1 = D + 1, W = kWaveBlock / 64;
-    __shared__ int sv[W][64 * D1];   // per wave: the round's vertices
-    __shared__ float tl[W][64][D];   // T_q - T_0 of the batch's points, then FULL: fg
-    __shared__ float ffl[W][64][D];  // FULL: the points' feature rows
+    __shared__ int sv[W][64 * D1], sr[W][64 * D1];  // per wave: the round's vertices and ranks
+    __shared__ float fgl[W][64][D];                 // fg of each group's point
+    __shared__ float ffl[W][64][D];                 // and the point's feature row
     __shared__ double wsum[W][D * D];
     const int np = a.full ? D * D : D;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     LaneGroup<true, R> G(L, S, per, nullptr);
     const int L2 = 2 * L;
+    const bool nx = a.xr != nullptr;
     // lane q < np: parameter q = (row, col) of the products fg[row] * f[col]
-    const int prow = lane % D, pcol = min(lane / D, D - 1);
-    double acc[D];  // FULL: acc[0]
-#pragma unroll
-    for (int j = 0; j < D; j++) acc[j] = 0.0;
+    const int prow = lane % D, pcol = a.full ? min(lane / D, D - 1) : prow;
+    double acc = 0.0;
     const int b0 = xcd_block(blockIdx.x, gridDim.x) * rounds;
-    const int batch = 64 / per;  // rounds whose points one lane each holds
-    const int pstep = W * per;   // from a round's points of the wave to the next round's
-    const int li = lane / per, lg = lane - li * per;
-    for (int i0 = 0; i0 < rounds; i0 += batch) {
-        const int nb = min(batch, rounds - i0);
-        const int pb = __builtin_amdgcn_readfirstlane(G.item_in(b0 + i0) - G.g);
-        for (int i = 0; i < nb; i++) {
-            const int p0 = pb + i * pstep, n = min(per, N - p0);
-            if (n <= 0) break;  // the wave's further rounds lie behind the last point too
-            stage_words(vtx + (size_t)p0 * D1, per * D1, n * D1, sv[w]);
-            stage_done();
-            const int gp = min(G.g, n - 1);
-            const size_t p = p0 + gp;
-            int v[D1];
+    for (int i = 0; i < rounds; i++) {
+        const int p0 = __builtin_amdgcn_readfirstlane(G.item_in(b0 + i) - G.g);
+        const int n = min(per, N - p0);  // the wave's points in this round
+        if (n <= 0) break;               // its further rounds lie behind the last point too
+        stage_words(vtx + (size_t)p0 * D1, per * D1, n * D1, sv[w]);
+        stage_words(rank + (size_t)p0 * D1, per * D1, n * D1, sr[w]);
+        stage_done();
+        const int gp = min(G.g, n - 1);  // (groups without a point repeat the last one's)
+        const size_t pp = p0 + gp;
+        const bool lead = G.on && G.g < n && G.l == 0;
+        int v[D1], r0[D1];
 #pragma unroll
-            for (int q = 0; q < D1; q++) v[q] = sv[w][gp * D1 + q];
-            float t[D], cv[R];
+        for (int q = 0; q < D1; q++) {
+            v[q] = sv[w][gp * D1 + q];
+            r0[q] = D - sr[w][gp * D1 + q];
+        }
+        // shares [dir 0 of G(a, c) | dir 1 | dir 0 of G(x, 1) | dir 1], d each; a
+        // direction's rows are loaded where its share is formed
+        float sh[4 * D], cv[R];
+        load_piece<R>(a.P + pp * L2 + L, G.k0, L, cv);
+        grad_share<R, D, false>(a.fwd, L2, v, G.k0, L, r0, cv, gs, sh);
+        load_piece<R>(a.P + pp * L2, G.k0, L, cv);
+        grad_share<R, D, false>(a.rev + L, L2, v, G.k0, L, r0, cv, gs, sh + D);
+        if (nx) {
+            grad_share<R, D, true>(a.xr, L, v, G.k0, L, r0, cv, gs, sh + 2 * D);
+            load_piece<R>(a.x + pp * L, G.k0, L, cv);
+            float u[D1], e[D];
 #pragma unroll
-            for (int q = 0; q < D; q++) t[q] = 0.0f;
-            if (a.xr) {
-                float u[R];
-                load_piece<R>(a.x + p * L, G.k0, L, cv);
-                float o[D1], xs = cv[0];
+            for (int q = 0; q < D1; q++) u[q] = a.ones[v[q]];
+            elevate<D>(u, r0, gs, e);
 #pragma unroll
-                for (int q = 0; q < D1; q++) o[q] = a.ones[v[q]];
+            for (int j = 0; j < D; j++) {
+                float s = 0.0f;
 #pragma unroll
-                for (int r = 1; r < R; r++) xs = xs + cv[r];
-#pragma unroll
-                for (int r = 0; r < R; r++) u[r] = 1.0f;
-                grad_dots<R, D>(a.xr, L, v, G.k0, L, u, t);
-#pragma unroll
-                for (int q = 0; q < D; q++) t[q] = -fmaf(xs, o[q + 1] - o[0], t[q]);
+                for (int r = 0; r < R; r++) s = add_product(s, cv[r], e[j]);
+                sh[3 * D + j] = s;
             }
-            load_piece<R>(a.P + p * L2 + L, G.k0, L, cv);
-            grad_dots<R, D>(a.fwd, L2, v, G.k0, L, cv, t);
-            load_piece<R>(a.P + p * L2, G.k0, L, cv);
-            grad_dots<R, D>(a.rev + L, L2, v, G.k0, L, cv, t);
-            for (int k = 1; k < S; k <<= 1) {
-                float y[D];
+        } else {
 #pragma unroll
-                for (int j = 0; j < D; j++) y[j] = wave_read(t[j], G.base + G.l + k);  // (wraps at 64)
-                if ((G.l & (2 * k - 1)) == 0 && G.l + k < S) {
+            for (int j = 2 * D; j < 4 * D; j++) sh[j] = 0.0f;
+        }
+        // the group's sums in its first lane (the tree of LaneGroup::all_sum)
+        for (int k = 1; k < S; k <<= 1) {
+            float y[4 * D];
 #pragma unroll
-                    for (int j = 0; j < D; j++) t[j] = t[j] + y[j];
-                }
+            for (int j = 0; j < 4 * D; j++) y[j] = wave_read(sh[j], G.base + G.l + k);  // (wraps at 64)
+            if ((G.l & (2 * k - 1)) == 0 && G.l + k < S) {
+#pragma unroll
+                for (int j = 0; j < 4 * D; j++) sh[j] = sh[j] + y[j];
             }
-            if (G.on && G.l == 0) {
+        }
+        if (lead) {
+            const int p = (int)pp;
+            const int inst = a.n_inst > 1 ? last_le(a.pix_base, a.n_inst, p) : 0;
+            const int fq = a.pad_base[inst] + (p - a.pix_base[inst]);
 #pragma unroll
-                for (int j = 0; j < D; j++) tl[w][i * per + G.g][j] = t[j];
+            for (int j = 0; j < D; j++) {
+                const float g = sh[j] + sh[D + j];
+                const float r = sh[2 * D + j] + sh[3 * D + j];
+                fgl[w][G.g][j] = nx ? -r + g : g;
+                ffl[w][G.g][j] = a.f[(size_t)fq * D + j];
             }
         }
         stage_done();
-        const int p = pb + li * pstep + lg;
-        const bool real = li < nb && p < N;  // a prefix of the wave's lanes
-        float fg[D], fv[D];
-#pragma unroll
-        for (int j = 0; j < D; j++) fg[j] = fv[j] = 0.0f;
-        if (real) {
-            const int inst = a.n_inst > 1 ? last_le(a.pix_base, a.n_inst, p) : 0;
-            const int fq = a.pad_base[inst] + (p - a.pix_base[inst]);
-            float T[D1];
-            T[0] = 0.0f;
-#pragma unroll
-            for (int j = 0; j < D; j++) {
-                fv[j] = a.f[(size_t)fq * D + j];
-                T[j + 1] = gs.alpha * tl[w][lane][j];
-            }
-            float ra[D1];
-#pragma unroll
-            for (int j = 0; j < D1; j++) {
-                const int r0 = D - rank[(size_t)p * D1 + j], r1 = r0 + 1 > D ? 0 : r0 + 1;
-                float x0 = T[0], x1 = T[0];
-#pragma unroll
-                for (int q = 1; q < D1; q++) {
-                    x0 = r0 == q ? T[q] : x0;
-                    x1 = r1 == q ? T[q] : x1;
-                }
-                ra[j] = x0 - x1;
-            }
-            float sm = ra[0];
-#pragma unroll
-            for (int j = 1; j <= D; j++) {
-                fg[j - 1] = gs.sf[j - 1] * (sm - (float)j * ra[j]);
-                sm = sm + ra[j];
-            }
-        }
-        if (!a.full) {
-#pragma unroll
-            for (int j = 0; j < D; j++) acc[j] += (double)fg[j] * (double)fv[j];
-        } else {
-            stage_done();  // every lane has read its T
-#pragma unroll
-            for (int j = 0; j < D; j++) {
-                tl[w][lane][j] = fg[j];
-                ffl[w][lane][j] = fv[j];
-            }
-            stage_done();
-            const int n = __popcll(__ballot(real));
-            for (int g = 0; g < n; g++) acc[0] += (double)tl[w][g][prow] * (double)ffl[w][g][pcol];
-        }
-        stage_done();  // (the next batch writes tl)
+        if (lane < np)
+            for (int g = 0; g < n; g++) acc += (double)fgl[w][g][prow] * (double)ffl[w][g][pcol];
+        stage_done();  // (the next round writes the rows)
     }
-    if (!a.full) {
-#pragma unroll
-        for (int j = 0; j < D; j++) {
-            for (int k = 32; k > 0; k >>= 1) acc[j] += __shfl_down(acc[j], k);
-            if (lane == 0) wsum[w][j] = acc[j];
-        }
-    } else if (lane < np) {
-        wsum[w][lane] = acc[0];
-    }
+    if (lane < np) wsum[w][lane] = acc;
     __syncthreads();
     for (int q = threadIdx.x; q < np; q += blockDim.x) {
         double s = 0.0;
@@ -602,14 +601,14 @@ void launch_kg_prepare(const float* Qt, const float* b, int ldq, const KgInputs&
                       ldq, in, N, L, sh.S, sh.per, st, cwf, P);
 }
 
-void launch_kg_x(const float* P, const float* norm, int N, int L, const SliceTable& st, int ntype, float* x,
+void launch_kg_x(const float* b, int ldb, const float* lbl, const float* norm, int N, int L, const SliceTable& st, int ntype, float* x,
                  hipStream_t s) {
     if (!N) return;
     const LaunchShape sh = shape_for(L);
     const int d = st.t[0].d1 - 1;
 #define DCRF_KGX(RR, DD)                                                                                         \
     case RR * 8 + DD:                                                                                            \
-        k_kg_x_rows<RR, DD><<<blocks_for(N, sh.items), kWaveBlock, 0, s>>>(P, st.t[0].vtx, st.t[0].sw,           \
+        k_kg_x_rows<RR, DD><<<blocks_for(N, sh.items), kWaveBlock, 0, s>>>(b, ldb, lbl, st.t[0].vtx, st.t[0].sw, \
                                                                            st.t[0].vals, st.t[1].vals, norm, N, \
                                                                            L, sh.S, sh.per, ntype, x);          \
         break;
@@ -626,7 +625,7 @@ void launch_kg_x(const float* P, const float* norm, int N, int L, const SliceTab
         return;
     }
 #undef DCRF_KGX
-    DCRF_DISPATCH(sh, k_kg_x, blocks_for(N, sh.items), 0, s, P, norm, N, L, sh.S, sh.per, st, ntype, x);
+    DCRF_DISPATCH(sh, k_kg_x, blocks_for(N, sh.items), 0, s, b, ldb, lbl, norm, N, L, sh.S, sh.per, st, ntype, x);
 }
 
 bool kg_grad_fused(int L, int d) { return d >= 1 && d <= 6 && shape_for(L).wave; }

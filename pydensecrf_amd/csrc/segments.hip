@@ -11,8 +11,8 @@
 //     (a head) carries the output row, the others out = -1;
 //   - a vertex with one head over all tiles is written directly, the others get partial
 //     rows, contiguous per vertex in list order, and an item in the recombination list.
-// (Without in-wave runs, for the LDS-tiled splat and lane groups wider than a wave, every
-// segment is a head and there are no fillers.)
+// (Without in-wave runs, for the LDS-tiled splat, lane groups wider than a wave and
+// sequential lists, every segment is a head and there are no fillers.)
 //
 // The host built these lists from downloaded runs before: at 1024x768 3.3 ms of a new
 // model's 14 ms went into its loops, and the lists into the uploads.  Here each stage is a
@@ -20,6 +20,7 @@
 // the lists.  The order of a vertex's partial rows is that of the stable sort by vertex,
 // i.e. list order, so the sums do not depend on anything but the runs.
 #include <cstring>
+#include <limits>
 
 #include <rocprim/rocprim.hpp>
 
@@ -76,21 +77,23 @@ __global__ void k_group_segments(const int* __restrict__ mbase, const int* __res
     n[g] = per ? (k + per - 1) / per * per : k;
 }
 
-// Heads of every run in vertex order, and their total per vertex (integers: any order).
-__global__ void k_heads(const int* __restrict__ sv, const int* __restrict__ si, int R, const int* __restrict__ rg,
-                        const int* __restrict__ mbase, const int* __restrict__ S, int per, int* __restrict__ h,
-                        int* __restrict__ vcount) {
+// Heads of every run in vertex order.
+__global__ void k_heads(const int* __restrict__ si, int R, const int* __restrict__ rg, const int* __restrict__ mbase,
+                        const int* __restrict__ S, int per, int* __restrict__ h) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= R) return;
     const int m = si[i];
-    const int n = run_heads(S[m] - S[mbase[rg[m]]], S[m + 1] - S[m], per);
-    h[i] = n;
-    atomicAdd(&vcount[sv[i]], n);
+    h[i] = run_heads(S[m] - S[mbase[rg[m]]], S[m + 1] - S[m], per);
 }
 
-__global__ void k_vertex_first(const int* __restrict__ sv, const int* __restrict__ H, int R, int* __restrict__ vfirst) {
+// Heads before every vertex: the first run of a vertex fills it in for its vertex and for
+// the ones without runs before it, thread R for those behind the last run's and for V.
+__global__ void k_vertex_first(const int* __restrict__ sv, const int* __restrict__ H, int R, int V,
+                               int* __restrict__ vfirst) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < R && (i == 0 || sv[i] != sv[i - 1])) vfirst[sv[i]] = H[i];
+    if (i > R) return;
+    const int last = i < R ? sv[i] : V, h = R ? H[i] : 0;
+    for (int v = i ? sv[i - 1] + 1 : 0; v <= last; v++) vfirst[v] = h;
 }
 
 // What a vertex contributes to the lists.
@@ -100,14 +103,14 @@ struct PlusCounts {
                          a.pieces + b.pieces};
     }
 };
-__global__ void k_vertex_counts(const int* __restrict__ vcount, int V, SegCounts* __restrict__ vc) {
+__global__ void k_vertex_counts(const int* __restrict__ vfirst, int V, int split, SegCounts* __restrict__ vc) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v > V) return;
-    const int n = v < V ? vcount[v] : 1;  // (one past the last: adds nothing)
+    const int n = v < V ? vfirst[v + 1] - vfirst[v] : 1;  // (one past the last: adds nothing)
     SegCounts c{0, 0, 0, 0, 0};
     c.partial = n > 1 ? n : 0;
-    c.light = n > 1 && n <= kCombineSplit;
-    c.heavy = n > kCombineSplit;
+    c.light = n > 1 && n <= split;
+    c.heavy = n > split;
     c.empty = n == 0;
     c.pieces = c.heavy ? (n + kCombineSplit - 1) / kCombineSplit : 0;
     vc[v] = c;
@@ -120,48 +123,53 @@ __global__ void k_totals(const SegCounts* __restrict__ vs, int V, const int* __r
     out[1] = SegCounts{gseg[G], 0, 0, 0, 0};
 }
 
-// One thread per run: its segments.
+// kRunLanes threads per run: its segments.  (One thread per run waited for the runs of
+// hundreds of segments that flat image regions have: 25 us at 512x512, now 5.6.)
+constexpr int kRunLanes = 8;
 __global__ void k_emit_runs(const int* __restrict__ sv, const int* __restrict__ si, int R, const int* __restrict__ rb,
                             const int* __restrict__ rl, const int* __restrict__ rg, const int* __restrict__ mbase,
                             const int* __restrict__ S, const int* __restrict__ gseg, const int* __restrict__ H,
-                            const int* __restrict__ vcount, const int* __restrict__ vfirst,
-                            const SegCounts* __restrict__ vs, int C, int per, int row0, Chunk* __restrict__ ch) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+                            const int* __restrict__ vfirst, const SegCounts* __restrict__ vs, int C, int per, int row0,
+                            Chunk* __restrict__ ch) {
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = (int)(t / kRunLanes);
     if (i >= R) return;
     const int v = sv[i], m = si[i], g = rg[m];
     const int o = S[m] - S[mbase[g]], k = S[m + 1] - S[m];
     const int beg = rb[m], end = beg + rl[m];
-    const bool direct = vcount[v] == 1;
-    int row = row0 + vs[v].partial + (H[i] - vfirst[v]);
+    const bool direct = vfirst[v + 1] - vfirst[v] == 1;
+    const int row = row0 + vs[v].partial + (H[i] - vfirst[v]);
     Chunk* out = ch + gseg[g] + o;
-    for (int j = 0; j < k; j++) {
+    for (int j = (int)(t % kRunLanes); j < k; j += kRunLanes) {
         const bool head = !per || j == 0 || (o + j) % per == 0;
-        out[j] = Chunk{v, beg + j * C, min(end, beg + (j + 1) * C), head ? (direct ? v : row++) : -1};
+        const int before = per ? (o + j) / per - o / per : j;  // heads before a head
+        out[j] = Chunk{v, beg + j * C, min(end, beg + (j + 1) * C), head ? (direct ? v : row + before) : -1};
     }
 }
 
 // One thread per vertex: its empty segment, or its recombination item(s).  perc: lane
 // groups a wave of the recombination (0: two levels, row2 the first second-level row).
-__global__ void k_emit_vertices(const int* __restrict__ vcount, const SegCounts* __restrict__ vs, int V, int E,
-                                int n_group_segs, int row0, int perc, int light_pad, int row2,
+__global__ void k_emit_vertices(const int* __restrict__ vfirst, const SegCounts* __restrict__ vs, int V, int E,
+                                int n_group_segs, int row0, int perc, int split, int light_pad,
+                                int row2,
                                 Chunk* __restrict__ ch, Combine* __restrict__ cb, Combine* __restrict__ cb2) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= V) return;
-    const int n = vcount[v];
+    const int n = vfirst[v + 1] - vfirst[v];
     const SegCounts c = vs[v];
     const int first = row0 + c.partial;
     if (n == 0) {
         ch[n_group_segs + c.empty] = Chunk{v, E, E, v};
-    } else if (n > 1 && n <= kCombineSplit) {
+    } else if (n > 1 && n <= split) {
         cb[c.light] = Combine{v, first, n, 0};
-    } else if (n > kCombineSplit && perc) {  // a whole wave: up to perc pieces side by side
+    } else if (n > split && perc) {  // a whole wave: up to perc pieces side by side
         const int pieces = min(perc, (n + kCombineSplit - 1) / kCombineSplit);
         for (int j = 0, off = 0; j < perc; j++) {
             const int q = j < pieces ? (n - off) / (pieces - j) : 0;
             cb[light_pad + c.heavy * perc + j] = Combine{v, first + off, q, pieces};
             off += q;
         }
-    } else if (n > kCombineSplit) {
+    } else if (n > split) {
         const int pieces = (n + kCombineSplit - 1) / kCombineSplit;
         for (int j = 0, off = 0; j < pieces; j++) {
             const int q = (n - off) / (pieces - j);
@@ -186,16 +194,6 @@ __global__ void k_emit_fillers(const int* __restrict__ mbase, const int* __restr
     }
     const int e = gebase[g + 1];
     for (int i = gseg[g] + S[mbase[g + 1]] - S[mbase[g]]; i < gseg[g + 1]; i++) ch[i] = Chunk{-1, e, e, -1};
-}
-
-__global__ void k_zero_int(int* p, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
-}
-void zero_int(int* p, size_t n, hipStream_t s) {
-    if (!n) return;
-    k_zero_int<<<blocks_for(n), kThreads, 0, s>>>(p, n);
-    DCRF_HIP_CHECK(hipGetLastError());
 }
 
 // out[0 .. n] = exclusive scan of in[0 .. n) and the total (in has n + 1 readable entries,
@@ -233,8 +231,6 @@ void build_run_set(const std::vector<const TermLattice*>& lats, const std::vecto
     ge.reserve(G + 1);
     rs.mbase.reserve(G + 1);
     rs.gebase.reserve(G + 1);
-    zero_int(gr.get() + G, 1, s);
-    zero_int(ge.get() + G, 1, s);
     for (int i = 0; i < T; i++) {
         k_group_counts<<<blocks_for(n_tiles), kThreads, 0, s>>>(lats[i]->tile_run.get(), lats[i]->tile_ptr.get(),
                                                                 n_tiles, T, i, gr.get(), ge.get());
@@ -245,7 +241,6 @@ void build_run_set(const std::vector<const TermLattice*>& lats, const std::vecto
     for (DevBuf<int>* b : {&rs.rv, &rs.rb, &rs.rl, &rs.rg, &rs.sv, &rs.si, &id}) b->reserve(R);
     ns.reserve(R + 1);
     rs.S.reserve(R + 1);
-    zero_int(ns.get() + R, 1, s);
     for (int i = 0; i < T; i++) {
         const TermLattice& l = *lats[i];
         if (!l.n_runs) continue;
@@ -269,38 +264,34 @@ void build_run_set(const std::vector<const TermLattice*>& lats, const std::vecto
                                              0, vbits, s));
 }
 
-void count_segments(const RunSet& rs, int per, int perc, SegPlan& P, hipStream_t s) {
+void count_segments(const RunSet& rs, int per, int perc, bool sequential, SegPlan& P, hipStream_t s) {
     P.per = per;
     P.perc = perc;
+    P.split = sequential ? std::numeric_limits<int>::max() : kCombineSplit;
     DevBuf<int> n, h;
     DevBuf<SegCounts> vc, tot;
     n.reserve(rs.G + 1);
-    zero_int(n.get() + rs.G, 1, s);
     P.gseg.reserve(rs.G + 1);
     if (rs.G) {
         k_group_segments<<<blocks_for(rs.G), kThreads, 0, s>>>(rs.mbase.get(), rs.S.get(), rs.G, per, n.get());
         DCRF_HIP_CHECK(hipGetLastError());
     }
     scan_int(n.get(), P.gseg.get(), rs.G, s);
-    P.vcount.reserve(rs.V);
-    P.vfirst.reserve(rs.V);
-    zero_int(P.vcount.get(), rs.V, s);
+    P.vfirst.reserve(rs.V + 1);
     h.reserve(rs.R + 1);
     P.H.reserve(rs.R + 1);
-    zero_int(h.get() + rs.R, 1, s);
     if (rs.R) {
-        k_heads<<<blocks_for(rs.R), kThreads, 0, s>>>(rs.sv.get(), rs.si.get(), rs.R, rs.rg.get(), rs.mbase.get(),
-                                                      rs.S.get(), per, h.get(), P.vcount.get());
+        k_heads<<<blocks_for(rs.R), kThreads, 0, s>>>(rs.si.get(), rs.R, rs.rg.get(), rs.mbase.get(), rs.S.get(),
+                                                      per, h.get());
         DCRF_HIP_CHECK(hipGetLastError());
     }
     scan_int(h.get(), P.H.get(), rs.R, s);
-    if (rs.R) {
-        k_vertex_first<<<blocks_for(rs.R), kThreads, 0, s>>>(rs.sv.get(), P.H.get(), rs.R, P.vfirst.get());
-        DCRF_HIP_CHECK(hipGetLastError());
-    }
+    k_vertex_first<<<blocks_for((size_t)rs.R + 1), kThreads, 0, s>>>(rs.sv.get(), P.H.get(), rs.R, rs.V,
+                                                                     P.vfirst.get());
+    DCRF_HIP_CHECK(hipGetLastError());
     vc.reserve(rs.V + 1);
     P.vs.reserve(rs.V + 1);
-    k_vertex_counts<<<blocks_for((size_t)rs.V + 1), kThreads, 0, s>>>(P.vcount.get(), rs.V, vc.get());
+    k_vertex_counts<<<blocks_for((size_t)rs.V + 1), kThreads, 0, s>>>(P.vfirst.get(), rs.V, P.split, vc.get());
     DCRF_HIP_CHECK(hipGetLastError());
     const SegCounts zero{0, 0, 0, 0, 0};
     size_t tb = 0;
@@ -328,15 +319,15 @@ void emit_segments(const RunSet& rs, const SegPlan& P, int row0, SegLists& L, hi
     L.cb.reserve(L.ncb);
     L.cb2.reserve(L.ncb2);
     if (rs.R) {
-        k_emit_runs<<<blocks_for(rs.R), kThreads, 0, s>>>(rs.sv.get(), rs.si.get(), rs.R, rs.rb.get(), rs.rl.get(),
+        k_emit_runs<<<blocks_for((size_t)rs.R * kRunLanes), kThreads, 0, s>>>(rs.sv.get(), rs.si.get(), rs.R, rs.rb.get(), rs.rl.get(),
                                                           rs.rg.get(), rs.mbase.get(), rs.S.get(), P.gseg.get(),
-                                                          P.H.get(), P.vcount.get(), P.vfirst.get(), P.vs.get(), rs.C,
+                                                          P.H.get(), P.vfirst.get(), P.vs.get(), rs.C,
                                                           P.per, row0, L.ch.get());
         DCRF_HIP_CHECK(hipGetLastError());
     }
     if (rs.V) {
-        k_emit_vertices<<<blocks_for(rs.V), kThreads, 0, s>>>(P.vcount.get(), P.vs.get(), rs.V, rs.E, n_group, row0,
-                                                              P.perc, light_pad, row2, L.ch.get(), L.cb.get(),
+        k_emit_vertices<<<blocks_for(rs.V), kThreads, 0, s>>>(P.vfirst.get(), P.vs.get(), rs.V, rs.E, n_group, row0,
+                                                              P.perc, P.split, light_pad, row2, L.ch.get(), L.cb.get(),
                                                               L.cb2.get());
         DCRF_HIP_CHECK(hipGetLastError());
     }

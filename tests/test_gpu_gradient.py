@@ -433,10 +433,9 @@ def test_unary_gradient_pending_slots(n, terms, L):
 
 
 @pytest.mark.parametrize("L,W,H", [(2, 1024, 513), (64, 203, 199), (21, 61, 1)])
-def test_kernel_gradient_batches(L, W, H):
-    """k_kg_grad holds the points of up to 64 / per rounds of a wave before it elevates
-    them: per = 64 points a round in several batches of one (L = 2: R = 2, one lane a
-    point; 2053 blocks of 256 points, 2 rounds), per = 4 (L = 64), and one round with a
+def test_kernel_gradient_rounds(L, W, H):
+    """k_kg_grad's rounds: 64 points a wave and round in two rounds (L = 2: one lane a point;
+    2053 blocks of 256 points), 4 points (L = 64, two rounds), and one round with a
     last wave that has fewer points than lane groups.  FULL kernels against the oracle
     (which adds their products in double); the DIAG gradient is the diagonal of the FULL
     one, up to the order of the additions in double and the rounding of the result."""
