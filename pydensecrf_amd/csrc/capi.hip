@@ -1384,6 +1384,8 @@ void ensure_layout(dcrf_model& m) {
     }
     // (the LDS-tiled splat stages unpadded rows)
     m.ldv = m.tiled ? L : padded_labels(L);
+    // a valid layout has the iterate's buffer: run_inference may allocate nothing
+    if (m.ldv != L) m.Qp.reserve((size_t)N * m.ldv);
     if (T) {
         plan_segments(rs, m.ldv, !m.tiled, sp, s);
         plan_sequential(rs, so, s);
@@ -1572,7 +1574,6 @@ void prepare(dcrf_model& m) {
     ensure_layout(m);
     const size_t n = (size_t)m.N() * m.L;
     m.Q.reserve(n);
-    if (m.ldv != m.L) m.Qp.reserve((size_t)m.N() * m.ldv);  // before any graph capture
     if (m.qblocks && !m.qblocks_ready && m.fused && !m.runs && !m.tiled && m.geo.is2d &&
         m.geo.n_inst == 1) {
         m.g_entB.reserve(m.E_total);
@@ -2255,6 +2256,8 @@ int dcrf_inference_device_noalloc(dcrf_model* m, int n_iter, const float* U_dev,
         require(!m->timing, "disable kernel timing for the allocation-free inference", DCRF_ERR_STATE);
         require(!m->tiled && !m->runs,
                 "the allocation-free inference runs the default splat and mean-field kernels only", DCRF_ERR_STATE);
+        require(m->ldv == m->L || m->Qp.n >= (size_t)m->N() * m->ldv, "the layout has no buffer for the padded iterate",
+                DCRF_ERR_STATE);
         require(U_dev || !m->has_unary || !m->unary_dirty,
                 "the unary changed since the last call: upload it with dcrf_inference_device first, or pass U_dev",
                 DCRF_ERR_STATE);
