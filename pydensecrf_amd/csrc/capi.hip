@@ -1301,6 +1301,23 @@ void compute_norms(dcrf_model& m, const RunSet& rs, const SegPlan& so, hipStream
     }
 }
 
+// Sets the stride of the gathered rows.  A training forward's Q_t were stored with the
+// stride of its time and a later backward reads them with the present one: they move along.
+void set_row_stride(dcrf_model& m, int ldv, hipStream_t s) {
+    if (ldv != m.ldv && m.train_n > 0) {
+        const int N = m.N(), L = m.L, n = m.train_n;
+        DevBuf<float> q;  // (layout: forward_train)
+        q.reserve((size_t)N * ((size_t)n * ldv + L));
+        // (the caller's stream wrote them)
+        DCRF_HIP_CHECK(hipDeviceSynchronize());
+        for (int t = 0; t <= n; t++)
+            launch_restride_rows(m.qcache.get() + (size_t)t * N * m.ldv, t < n ? m.ldv : L,
+                                 q.get() + (size_t)t * N * ldv, t < n ? ldv : L, N, L, s);
+        m.qcache = std::move(q);
+    }
+    m.ldv = ldv;
+}
+
 void ensure_layout(dcrf_model& m) {
     if (m.layout_valid) return;
     m.drop_graph();
@@ -1383,7 +1400,7 @@ void ensure_layout(dcrf_model& m) {
         }
     }
     // (the LDS-tiled splat stages unpadded rows)
-    m.ldv = m.tiled ? L : padded_labels(L);
+    set_row_stride(m, m.tiled ? L : padded_labels(L), s);
     // a valid layout has the iterate's buffer: run_inference may allocate nothing
     if (m.ldv != L) m.Qp.reserve((size_t)N * m.ldv);
     if (T) {
@@ -1588,7 +1605,7 @@ void prepare(dcrf_model& m) {
 // padding labels added.
 const float* splat_rows(dcrf_model& m, const float* Q, hipStream_t s) {
     if (m.ldv == m.L) return Q;
-    launch_pad_rows(Q, m.Qp.get(), m.N(), m.L, m.ldv, s);
+    launch_restride_rows(Q, m.L, m.Qp.get(), m.ldv, m.N(), m.L, s);
     return m.Qp.get();
 }
 

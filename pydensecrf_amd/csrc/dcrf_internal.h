@@ -433,8 +433,8 @@ void launch_interleave_slice(const int* vtx, const float* sw, int N, int d1, int
 void launch_slice_term(float* out, int N, int L, int Lv, const SliceTable& st, int which, hipStream_t s);
 // Q0 = softmax(-U), rows of ldq floats.
 void launch_softmax_neg(const float* U, float* Q, int ldq, int N, int L, int Lv, hipStream_t s);
-// out [N][Lv] = in [N][L] with zeros in the padding labels.
-void launch_pad_rows(const float* in, float* out, int N, int L, int Lv, hipStream_t s);
+// out [N][ldo] = in [N][ldi] (L labels each) with zeros in out's padding labels.
+void launch_restride_rows(const float* in, int ldi, float* out, int ldo, int N, int L, hipStream_t s);
 // KL divergence partial sums (one double per block, kl_blocks of them).
 int kl_blocks(int N, int Lv);
 void launch_kl(const float* Q, const float* U, int N, int L, int Lv, const SliceTable& st, double* partials,

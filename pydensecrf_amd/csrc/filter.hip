@@ -889,13 +889,15 @@ __global__ void k_argmax(const float* __restrict__ Q, int ldq, int N, int L, int
     out[p] = (int16_t)arg;
 }
 
-// out [N][Lv] = in [N][L], zeros in the padding labels.
-__global__ void k_pad_rows(const float* __restrict__ in, float* __restrict__ out, size_t n, int L, int Lv) {
+// out (rows of ldo floats) = in (rows of ldi), L labels and zeros in out's padding labels;
+// n floats of out.
+__global__ void k_restride_rows(const float* __restrict__ in, int ldi, float* __restrict__ out, int ldo, size_t n,
+                                int L) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const size_t p = i / Lv;
-    const int l = (int)(i - p * Lv);
-    out[i] = l < L ? in[p * L + l] : 0.0f;
+    const size_t p = i / ldo;
+    const int l = (int)(i - p * ldo);
+    out[i] = l < L ? in[p * ldi + l] : 0.0f;
 }
 
 // out[c][r] = in[r][c] for an rows x cols row-major input, 32x32 tiles through LDS.
@@ -928,10 +930,10 @@ void launch_argmax(const float* Q, int ldq, int N, int L, int16_t* out, hipStrea
     DCRF_HIP_CHECK(hipGetLastError());
 }
 
-void launch_pad_rows(const float* in, float* out, int N, int L, int Lv, hipStream_t s) {
-    const size_t n = (size_t)N * Lv;
+void launch_restride_rows(const float* in, int ldi, float* out, int ldo, int N, int L, hipStream_t s) {
+    const size_t n = (size_t)N * ldo;
     if (!n) return;
-    k_pad_rows<<<blocks_for(n), kThreads, 0, s>>>(in, out, n, L, Lv);
+    k_restride_rows<<<blocks_for(n), kThreads, 0, s>>>(in, ldi, out, ldo, n, L);
     DCRF_HIP_CHECK(hipGetLastError());
 }
 
