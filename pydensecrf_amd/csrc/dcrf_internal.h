@@ -34,12 +34,16 @@ struct Error {
     std::string msg;
 };
 void set_error(int code, const std::string& msg);
+// (The runtime keeps its last error until it is read: it is cleared with the throw, or
+// the launch check of a later call would report it once more.)
 #define DCRF_HIP_CHECK(expr)                                                              \
     do {                                                                                  \
         hipError_t e_ = (expr);                                                           \
-        if (e_ != hipSuccess)                                                             \
+        if (e_ != hipSuccess) {                                                           \
+            (void)hipGetLastError();                                                      \
             throw ::dcrf::Error{e_ == hipErrorOutOfMemory ? DCRF_ERR_MEMORY : DCRF_ERR_DEVICE, \
                                 std::string(#expr) + ": " + hipGetErrorString(e_)};      \
+        }                                                                                 \
     } while (0)
 
 // ---------------------------------------------------------------- device buffers

@@ -108,9 +108,11 @@ void* pool_alloc(size_t bytes) {
         release(P, dev);
         e = hipMalloc(&p, s);
     }
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
         throw Error{e == hipErrorOutOfMemory ? DCRF_ERR_MEMORY : DCRF_ERR_DEVICE,
                     std::string("hipMalloc: ") + hipGetErrorString(e)};
+    }
     P.live[p] = Block{s, dev};
     return p;
 }
