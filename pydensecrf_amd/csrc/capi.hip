@@ -1318,8 +1318,19 @@ void set_row_stride(dcrf_model& m, int ldv, hipStream_t s) {
     m.ldv = ldv;
 }
 
+void build_layout(dcrf_model& m);
+
 void ensure_layout(dcrf_model& m) {
     if (m.layout_valid) return;
+    try {
+        build_layout(m);
+    } catch (...) {
+        m.train_n = -1;  // (a backward reads the layout)
+        throw;
+    }
+}
+
+void build_layout(dcrf_model& m) {
     m.drop_graph();
     m.qblocks_ready = false;
     hipStream_t s = m.stream;
@@ -1659,6 +1670,7 @@ void forward_train(dcrf_model& m, int n_iter, const float* U, const float* compa
     const int N = m.N(), L = m.L, T = (int)m.terms.size();
     const int Lv = m.ldv;
     const size_t NL = (size_t)N * L, NLv = (size_t)N * Lv;  // Q_t (t < n): rows of ldv floats; Q_n: of L
+    m.train_n = -1;  // until the store is complete: a failed allocation below has lost the old one
     if (compat_raw) {
         size_t off = 0;
         for (auto& t : m.terms) {
