@@ -437,6 +437,7 @@ struct dcrf_model {
     // global filter layout
     bool layout_valid = false;
     int V_total = 0, rows0 = 0, E_total = 0, max_d = 0;
+    size_t noalloc_rows = 0;  // the rows that the allocation-free inference's limit counts
     std::vector<int> order, vbase;
     std::vector<int> prefixV;
     DevBuf<float> vals[2];
@@ -1301,6 +1302,25 @@ void compute_norms(dcrf_model& m, const RunSet& rs, const SegPlan& so, hipStream
     }
 }
 
+// The limit of the allocation-free inference counts the rows of a layout without padding
+// labels and with one lane group per segment, whatever the splat's form: the quad form has
+// more partial rows, padded rows of fewer lanes have fewer, and neither moves the line
+// between the models that the call takes and those it refuses.
+constexpr size_t kNoAllocRowBytes = (size_t)64 << 20;
+size_t noalloc_rows(const dcrf_model& m, const RunSet& rs, const SegPlan& sp, hipStream_t s) {
+    const LaunchShape sh = shape_for(m.L);
+    const int per = sh.wave ? sh.per : 0;
+    const size_t rows = (size_t)m.rows0 + m.V_total + 1;
+    if (m.tiled || !rs.T || (sp.per == per && sp.perc == per)) return rows;
+    // no layout has more partial and second-level rows than twice the segments
+    const size_t most = 2 * ((size_t)m.V_total + 1) + 2 * (size_t)sp.host[1].partial;
+    if (most * m.L * sizeof(float) <= kNoAllocRowBytes) return rows;
+    SegPlan p;
+    count_segments(rs, per, per, false, p, s);
+    DCRF_HIP_CHECK(hipStreamSynchronize(s));
+    return 2 * ((size_t)m.V_total + 1) + p.host[0].partial + (per ? 0 : p.host[0].pieces);
+}
+
 // Sets the stride of the gathered rows.  A training forward's Q_t were stored with the
 // stride of its time and a later backward reads them with the present one: they move along.
 void set_row_stride(dcrf_model& m, int ldv, hipStream_t s) {
@@ -1451,6 +1471,7 @@ void build_layout(dcrf_model& m) {
         m.rows0 = m.seg.rows;
         compute_norms(m, rs, so, s);
     }
+    m.noalloc_rows = noalloc_rows(m, rs, sp, s);
     m.tsplat = TiledSplat{m.seg.ch.get(), m.g_tile_seg.get(), m.g_tile_e.get(), NT, tg, e_max, s_max};
 
     m.vals[0].reserve((size_t)m.rows0 * m.ldv);
@@ -1887,9 +1908,8 @@ double objective_value(int kind, const std::vector<double>& OP, int L) {
 // device array per GPU instead of the model's buffers.  Host code must not use the
 // array's name as an address: the address comes from hipGetSymbolAddress, once per
 // device, and is kept in scratch_dev.
-// The limit counts rows of L floats; the array holds them padded (at most 8 floats for 5
-// labels) and the second buffer's alignment.
-constexpr size_t kNoAllocRowBytes = (size_t)64 << 20;
+// The limit (kNoAllocRowBytes) counts rows of L floats; the array holds them padded (at
+// most 8 floats for 5 labels) and the second buffer's alignment.
 constexpr size_t kNoAllocScratchBytes = kNoAllocRowBytes / 5 * 8 + 4096;
 constexpr int kMaxDevices = 64;
 static __device__ __align__(256) float scratch[kNoAllocScratchBytes / sizeof(float)];
@@ -2293,9 +2313,9 @@ int dcrf_inference_device_noalloc(dcrf_model* m, int n_iter, const float* U_dev,
         const size_t n0 = (size_t)m->rows0 * m->ldv, n1 = (size_t)(m->V_total + 1) * m->ldv;
         const size_t off1 = (n0 + 63) / 64 * 64;  // second buffer 256-byte aligned
         const size_t need = off1 + n1;
-        const size_t unpadded = ((size_t)m->rows0 + m->V_total + 1) * m->L * sizeof(float);
-        if (unpadded > kNoAllocRowBytes || need > kNoAllocScratchBytes / sizeof(float))
-            throw Error{DCRF_ERR_VALUE, "the model needs " + std::to_string(unpadded) +
+        const size_t bytes = m->noalloc_rows * m->L * sizeof(float);
+        if (bytes > kNoAllocRowBytes || need > kNoAllocScratchBytes / sizeof(float))
+            throw Error{DCRF_ERR_VALUE, "the model needs " + std::to_string(bytes) +
                                             " bytes of vertex rows; the allocation-free inference holds at most " +
                                             std::to_string(kNoAllocRowBytes) + " (use dcrf_inference_device)"};
         float* base = scratch_for_current_device();
