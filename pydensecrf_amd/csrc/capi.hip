@@ -957,7 +957,7 @@ void build_kg_plan(dcrf_model& m, std::vector<int> terms, KgPlan& P) {
         gv.reserve((size_t)N * d1);
         part.sw.reserve((size_t)N * d1);
         launch_slice_weights(lat.vtx.get(), lat.bary.get(), nullptr, 0, slice_alpha(d), N, d1, 0, gv.get(),
-                             part.sw.get(), s);
+                             part.sw.get(), nullptr, 0, 0, s);
     }
     launch_pass_tables(jobs, s);
     // vertex rows: the zero rows stay zero (splats write vertex and partial rows, the
@@ -1237,69 +1237,59 @@ void blur_rows(dcrf_model& m, float* v0, float* v1, int Lv, bool transpose, hipS
     }
 }
 
+// norm = N / sum(norm) per instance, in float (pairwise.cpp:46-53).
+void mean_norms(const dcrf_model& m, float* norm, hipStream_t s) {
+    const int N = m.N();
+    std::vector<float> h(N);
+    DCRF_HIP_CHECK(hipMemcpyAsync(h.data(), norm, sizeof(float) * N, hipMemcpyDeviceToHost, s));
+    DCRF_HIP_CHECK(hipStreamSynchronize(s));
+    for (int i = 0; i < m.geo.n_inst; i++) {
+        const int b = m.geo.pix_base[i], e = m.geo.pix_base[i + 1];
+        float mean = 0.f;
+        for (int p = b; p < e; p++) mean += h[p];
+        mean = (float)(e - b) / mean;
+        for (int p = b; p < e; p++) h[p] = mean;
+    }
+    DCRF_HIP_CHECK(hipMemcpyAsync(norm, h.data(), sizeof(float) * N, hipMemcpyHostToDevice, s));
+    DCRF_HIP_CHECK(hipStreamSynchronize(s));
+}
+
+NormTerm norm_term(const Term& t, const float* vals, int vbase, float* norm) {
+    const TermLattice& lat = t.lat;
+    return NormTerm{lat.vtx.get(), lat.bary.get(), vals, norm, slice_alpha(lat.d), lat.d + 1, vbase, t.ntype};
+}
+
 // The normalisers of all terms: norm = K 1 (pairwise.cpp:44), then the normalisation of
 // :46-61.  One filter of the all-ones input over every term's lattice, one float a row,
-// through the layout's run set and pass tables (so: the counts of its sequential lists).
-void compute_norms(dcrf_model& m, const RunSet& rs, const SegPlan& so, hipStream_t s) {
-    const int N = m.N(), T = (int)m.order.size(), V = m.V_total;
+// through the layout's run set and pass tables.
+//   A new small model is a chain of short launches (64x48: 94 with the two lattice builds),
+// so their number counts.  The sums need an order of their own (see plan_sequential), but
+// no segment list and no entries (splat_ones); with those, and a slice per term, a new
+// model took 127.  First inference of a new model, 10 iterations: 64x48x21 606 -> 444 us,
+// 320x213x21 740 -> 580, 1024x768x21 2090 -> 1870.
+void compute_norms(dcrf_model& m, const std::vector<const TermLattice*>& lats, const RunSet& rs, const SegPlan& sp,
+                   hipStream_t s) {
     struct Untimed {  // these launches are no part of the timed classes
         dcrf_model& m;
         bool was;
         explicit Untimed(dcrf_model& m_) : m(m_), was(m_.timing) { m.timing = false; }
         ~Untimed() { m.timing = was; }
     } untimed(m);
-    SegLists l;
-    emit_segments(rs, so, V + 1, l, s);
-    for (int i = 0; i < T; i++) {
-        const TermLattice& lat = m.terms[m.order[i]]->lat;
-        const int d1 = lat.d + 1;
-        launch_entry_gather(lat.csr_e.get(), N * d1, d1, lat.bary.get(), nullptr, 0, lat.tile_ptr.get(),
-                            rs.gebase.get(), rs.NT, T, i, nullptr, m.g_entF.get(), s);
-    }
-    DevBuf<float> ones, v0, v1;
-    ones.reserve(N);
-    v0.reserve(l.rows);
+    const int V = m.V_total;
+    DevBuf<float> v0, v1;
+    v0.reserve((size_t)V + 1);
     v1.reserve((size_t)V + 1);
-    launch_fill(ones.get(), 1.f, N, s);
-    launch_fill(v0.get(), 0.f, l.rows, s);
-    launch_fill(v1.get(), 0.f, (size_t)V + 1, s);
-    splat_lists(l, m.g_entF.get(), ones.get(), N, 1, v0.get(), s);
-    combine_lists(l, 1, v0.get(), s);
+    splat_ones(lats, rs, sp, v0.get(), v1.get(), s);
     blur_rows(m, v0.get(), v1.get(), 1, false, s);
-    DevBuf<int> gv;
-    DevBuf<float> sw;
+    NormTerms nt{};
     for (int k : m.order) {
         Term& t = *m.terms[k];
-        const TermLattice& lat = t.lat;
-        const int d1 = lat.d + 1;
-        gv.reserve((size_t)N * d1);
-        sw.reserve((size_t)N * d1);
-        launch_slice_weights(lat.vtx.get(), lat.bary.get(), nullptr, 0, slice_alpha(lat.d), N, d1, m.vbase[k], gv.get(),
-                             sw.get(), s);
-        SliceTable st{};
-        st.nterms = 1;
-        st.t[0] = SliceTerm{gv.get(), sw.get(), result_parity(m, k) ? v1.get() : v0.get(), d1, -1, nullptr, nullptr,
-                            nullptr, 1};
-        t.norm.reserve(N);
-        launch_slice_term(t.norm.get(), N, 1, 1, st, 0, s);
-        if (t.ntype != DCRF_NO_NORMALIZATION) {
-            launch_norm_finish(t.norm.get(), N, t.ntype, s);
-            continue;
-        }
-        // mean_norm = N / sum(norm) per instance, in float (pairwise.cpp:46-53)
-        std::vector<float> h(N);
-        DCRF_HIP_CHECK(hipMemcpyAsync(h.data(), t.norm.get(), sizeof(float) * N, hipMemcpyDeviceToHost, s));
-        DCRF_HIP_CHECK(hipStreamSynchronize(s));
-        for (int i = 0; i < m.geo.n_inst; i++) {
-            const int b = m.geo.pix_base[i], e = m.geo.pix_base[i + 1];
-            float mean = 0.f;
-            for (int p = b; p < e; p++) mean += h[p];
-            mean = (float)(e - b) / mean;
-            for (int p = b; p < e; p++) h[p] = mean;
-        }
-        DCRF_HIP_CHECK(hipMemcpyAsync(t.norm.get(), h.data(), sizeof(float) * N, hipMemcpyHostToDevice, s));
-        DCRF_HIP_CHECK(hipStreamSynchronize(s));
+        t.norm.reserve(m.N());
+        nt.t[nt.T++] = norm_term(t, result_parity(m, k) ? v1.get() : v0.get(), m.vbase[k], t.norm.get());
     }
+    launch_norms(nt, m.N(), s);
+    for (int k : m.order)
+        if (m.terms[k]->ntype == DCRF_NO_NORMALIZATION) mean_norms(m, m.terms[k]->norm.get(), s);
 }
 
 // The limit of the allocation-free inference counts the rows of a layout without padding
@@ -1393,8 +1383,8 @@ void build_layout(dcrf_model& m) {
     // levels.  Block-mode shapes and the tiled splat have no in-wave runs.
     const int NT = m.tiles.n_tiles();
     RunSet rs;
+    std::vector<const TermLattice*> lats;
     {
-        std::vector<const TermLattice*> lats;
         std::vector<int> vb;
         for (int k : m.order) {
             lats.push_back(&m.terms[k]->lat);
@@ -1407,7 +1397,7 @@ void build_layout(dcrf_model& m) {
     const TileGeom tg = tile_geom(m);
     int e_max = 0, s_max = 0;
     m.tiled = false;
-    SegPlan sp, so;
+    SegPlan sp;
     if (m.tile_side && T) {
         count_segments(rs, 0, 0, false, sp, s);
         std::vector<int> gs(rs.G + 1), ge(rs.G + 1), ts(NT + 1), te(NT + 1);
@@ -1434,14 +1424,11 @@ void build_layout(dcrf_model& m) {
     set_row_stride(m, m.tiled ? L : padded_labels(L), s);
     // a valid layout has the iterate's buffer: run_inference may allocate nothing
     if (m.ldv != L) m.Qp.reserve((size_t)N * m.ldv);
-    if (T) {
-        plan_segments(rs, m.ldv, !m.tiled, sp, s);
-        plan_sequential(rs, so, s);
-    }
+    if (T) plan_segments(rs, m.ldv, !m.tiled, sp, s);
     m.tl.clear();
     m.tl.resize(T);
     std::vector<PassTableJob> jobs;
-    for (int k : m.order) {  // what the normalisers need
+    for (int k : m.order) {  // what the normalisers' filter needs
         const TermLattice& lat = m.terms[k]->lat;
         const int d1 = lat.d + 1;
         auto lay = std::make_unique<TermLayout>();
@@ -1469,7 +1456,7 @@ void build_layout(dcrf_model& m) {
     if (T) {
         emit_segments(rs, sp, V + 1, m.seg, s);
         m.rows0 = m.seg.rows;
-        compute_norms(m, rs, so, s);
+        compute_norms(m, lats, rs, sp, s);
     }
     m.noalloc_rows = noalloc_rows(m, rs, sp, s);
     m.tsplat = TiledSplat{m.seg.ch.get(), m.g_tile_seg.get(), m.g_tile_e.get(), NT, tg, e_max, s_max};
@@ -1478,6 +1465,18 @@ void build_layout(dcrf_model& m) {
     m.vals[1].reserve((size_t)(V + 1) * m.ldv);
     launch_fill(m.vals[0].get(), 0.f, (size_t)m.rows0 * m.ldv, s);
     launch_fill(m.vals[1].get(), 0.f, (size_t)(V + 1) * m.ldv, s);
+    // interleaved slice pairs for the fused mean-field kernel, in term order
+    m.runs = false;
+    m.slcT_valid = false;
+    m.fused = m.mf_mode != 1 &&
+              fused_meanfield_ok(L, T, T > 0 ? m.terms[0]->lat.d + 1 : 0, T > 1 ? m.terms[1]->lat.d + 1 : 0);
+    int ds = 0;
+    std::vector<int> slc_off(T);
+    for (int k = 0; k < T; k++) {
+        slc_off[k] = ds;
+        ds += m.terms[k]->lat.d + 1;
+    }
+    if (m.fused) m.g_slc.reserve((size_t)N * ds);
     for (int i = 0; i < T; i++) {
         const int k = m.order[i];
         Term& t = *m.terms[k];
@@ -1494,30 +1493,16 @@ void build_layout(dcrf_model& m) {
         lay.swF.reserve(Ek);
         const float alpha = slice_alpha(lat.d);
         launch_slice_weights(lat.vtx.get(), lat.bary.get(), t.norm.get(), post_norm(t.ntype, false), alpha, N, d1,
-                             m.vbase[k], lay.vtx.get(), lay.swF.get(), s);
+                             m.vbase[k], lay.vtx.get(), lay.swF.get(), m.fused ? m.g_slc.get() : nullptr, ds,
+                             slc_off[k], s);
         if (!m.all_symmetric) {
             lay.swT.reserve(Ek);
             launch_slice_weights(lat.vtx.get(), lat.bary.get(), t.norm.get(), post_norm(t.ntype, true), alpha, N, d1,
-                                 m.vbase[k], lay.vtx.get(), lay.swT.get(), s);
+                                 m.vbase[k], lay.vtx.get(), lay.swT.get(), nullptr, 0, 0, s);
         }
     }
-    // interleaved slice pairs for the fused mean-field kernel
-    m.runs = false;
-    m.slcT_valid = false;
-    m.fused = m.mf_mode != 1 &&
-              fused_meanfield_ok(L, T, T > 0 ? m.terms[0]->lat.d + 1 : 0, T > 1 ? m.terms[1]->lat.d + 1 : 0);
     if (m.fused) {
-        int ds = 0;
-        for (int k = 0; k < T; k++) ds += m.terms[k]->lat.d + 1;
-        m.g_slc.reserve((size_t)N * ds);
-        int off = 0;
-        for (int k = 0; k < T; k++) {
-            const int d1 = m.terms[k]->lat.d + 1;
-            launch_interleave_slice(m.tl[k]->vtx.get(), m.tl[k]->swF.get(), N, d1, ds, off, m.g_slc.get(), s);
-            off += d1;
-        }
         // pixel runs (on request): entry j reads vals[result_parity] of its term
-        m.runs = false;
         if (m.mf_mode == 3 && m.V_total < (1 << 30)) {
             unsigned par = 0;
             int j = 0;

@@ -153,6 +153,12 @@ __device__ __forceinline__ float wave_read(float x, int lane) {
 }
 __device__ __forceinline__ int wave_read(int x, int lane) { return __builtin_amdgcn_ds_bpermute(lane << 2, x); }
 
+// x of lane J of the quad.
+template <int J>
+__device__ __forceinline__ float quad_value(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), J * 0x55, 0xf, 0xf, true));
+}
+
 template <bool WAVE, int R>
 struct LaneGroup {
     int L, S, g, l, k0, base, t, per;

@@ -131,6 +131,7 @@ struct RunSet {
     DevBuf<int> rv, rb, rl, rg;  // [R] vertex, first entry, entries, group
     DevBuf<int> S;               // [R + 1] segments before each run
     DevBuf<int> sv, si;          // [R] the runs sorted by vertex: vertex, merged index
+    DevBuf<int> vrun;            // [V + 1] first run of each vertex in that order
 };
 struct SegCounts {
     int partial, light, heavy, empty, pieces;
@@ -139,8 +140,8 @@ struct SegCounts {
 // recombination wave (0: two levels, or one where split allows any number of partial rows).
 struct SegPlan {
     int per = 0, perc = 0, split = 0;
-    DevBuf<int> gseg, H;
-    DevBuf<int> vfirst;  // [V + 1] heads before each vertex
+    DevBuf<int> gseg;
+    DevBuf<int2> H;  // [R + 1] heads and segments before each run in vertex order
     DevBuf<SegCounts> vs;
     SegCounts host[2] = {};  // totals; [1].partial: the groups' segments
 };
@@ -159,6 +160,10 @@ void build_run_set(const std::vector<const TermLattice*>& lats, const std::vecto
 void count_segments(const RunSet& rs, int per, int perc, bool sequential, SegPlan& P, hipStream_t s);
 // The lists, partial rows from row0 (after P's counts have arrived).
 void emit_segments(const RunSet& rs, const SegPlan& P, int row0, SegLists& L, hipStream_t s);
+// Splat of the all-ones input to one float a vertex (v0), the segments of a vertex one after
+// another (of any plan P: its lists are not needed); row V of v0 and v1 becomes zero.
+void splat_ones(const std::vector<const TermLattice*>& lats, const RunSet& rs, const SegPlan& P, float* v0, float* v1,
+                hipStream_t s);
 
 // The lattice filters of the kernel-parameter gradient (the lattice_.compute and
 // Permutohedral::gradient calls of DenseKernel::featureGradient, pairwise.cpp:88-114,
@@ -443,8 +448,20 @@ void launch_restride_rows(const float* in, int ldi, float* out, int ldo, int N, 
 int kl_blocks(int N, int Lv);
 void launch_kl(const float* Q, const float* U, int N, int L, int Lv, const SliceTable& st, double* partials,
                hipStream_t s);
-// norm = f(K*1) per the normalisation type, from the sliced values (L = 1).
-void launch_norm_finish(float* norm, int N, int ntype, hipStream_t s);
+// norm = f(K 1) per the normalisation type (NO_NORMALIZATION: K 1 itself), sliced from
+// vals (one float a vertex, this term's from row vbase on).
+struct NormTerm {
+    const int* vtx;
+    const float *bary, *vals;
+    float* norm;
+    float alpha;
+    int d1, vbase, ntype;
+};
+struct NormTerms {
+    int T;
+    NormTerm t[DCRF_MAX_TERMS];
+};
+void launch_norms(const NormTerms& terms, int N, hipStream_t s);
 void launch_fill(float* p, float v, size_t n, hipStream_t s);
 // out[c][r] = in[r][c] (in is rows x cols row-major).
 void launch_transpose(const float* in, float* out, int rows, int cols, hipStream_t s);
@@ -578,8 +595,10 @@ void launch_remap_nbr(const int* src, int2* dst, int n, int vbase, int zero_row,
 void launch_entry_gather(const int* csr_e, int E, int d1, const float* bary, const float* norm, int use_norm,
                          const int* tile_ptr, const int* gebase, int n_tiles, int T, int i, const TileGeom* local,
                          int2* ent_out, hipStream_t s, int pix_off = 0);
+// slc (may be null): the same as (vertex, weight bits) pairs, ds a pixel, this term's from
+// off on.
 void launch_slice_weights(const int* vtx, const float* bary, const float* norm, int use_norm,
-                          float alpha, int N, int d1, int vbase, int* gvtx, float* sw,
+                          float alpha, int N, int d1, int vbase, int* gvtx, float* sw, int2* slc, int ds, int off,
                           hipStream_t s);
 
 }  // namespace dcrf

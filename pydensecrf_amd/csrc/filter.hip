@@ -213,11 +213,6 @@ __global__ void __launch_bounds__(1024) k_splat(const Chunk* __restrict__ chunks
 // k_splat, in groups of S quads.
 constexpr int kSplitBatch = 8;
 
-template <int J>
-__device__ __forceinline__ float quad_value(float x) {  // x of lane J of the quad
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), J * 0x55, 0xf, 0xf, true));
-}
-
 template <int R, bool NARROW>
 __global__ void __launch_bounds__(kWaveBlock) k_splat_split(const Chunk* __restrict__ chunks, int n,
                                                             const int2* __restrict__ ent, const float* __restrict__ in,
@@ -824,12 +819,23 @@ __global__ void __launch_bounds__(1024) k_kl(const float* __restrict__ Q, const 
 }
 
 // DenseKernel::initLattice normalisers (pairwise.cpp:54-61), in double like the reference.
-__global__ void k_norm_finish(float* norm, int N, int ntype) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const double x = (double)norm[i] + 1e-20;
-    if (ntype == DCRF_NORMALIZE_SYMMETRIC) norm[i] = (float)(1.0 / sqrt(x));
-    else if (ntype == DCRF_NORMALIZE_BEFORE || ntype == DCRF_NORMALIZE_AFTER) norm[i] = (float)(1.0 / x);
+// The normalisers of every term (blockIdx.y) from the filtered all-ones rows: slice, then
+// the normalisation (pairwise.cpp:44-61).
+__global__ void k_norms(NormTerms M, int N) {
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= N) return;
+    const NormTerm& T = M.t[blockIdx.y];
+    const int* __restrict__ vt = T.vtx + (size_t)p * T.d1;
+    const float* __restrict__ bary = T.bary + (size_t)p * T.d1;
+    float x = 0.0f;
+#pragma unroll 4
+    for (int j = 0; j < T.d1; j++) x = add_product(x, bary[j] * T.alpha, T.vals[vt[j] + T.vbase]);
+    const double y = (double)x + 1e-20;
+    if (T.ntype == DCRF_NORMALIZE_SYMMETRIC)
+        x = (float)(1.0 / sqrt(y));
+    else if (T.ntype == DCRF_NORMALIZE_BEFORE || T.ntype == DCRF_NORMALIZE_AFTER)
+        x = (float)(1.0 / y);
+    T.norm[p] = x;
 }
 
 __global__ void k_remap_nbr(const int* __restrict__ src, int2* __restrict__ dst, int n, int vbase,
@@ -861,13 +867,17 @@ __global__ void k_entry_gather(const int* __restrict__ csr_e, int E, int d1, con
 
 __global__ void k_slice_weights(const int* __restrict__ vtx, const float* __restrict__ bary,
                                 const float* __restrict__ norm, int use_norm, float alpha, int N, int d1,
-                                int vbase, int* __restrict__ gvtx, float* __restrict__ sw) {
+                                int vbase, int* __restrict__ gvtx, float* __restrict__ sw, int2* __restrict__ slc,
+                                int ds, int off) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)N * d1) return;
-    const int p = (int)(i / d1);
-    gvtx[i] = vtx[i] + vbase;
+    const size_t p = i / d1;
+    const int v = vtx[i] + vbase;
     const float wa = bary[i] * alpha;
-    sw[i] = use_norm ? wa * norm[p] : wa;
+    const float w = use_norm ? wa * norm[p] : wa;
+    gvtx[i] = v;
+    sw[i] = w;
+    if (slc) slc[p * ds + off + (i - p * d1)] = make_int2(v, __float_as_int(w));
 }
 
 // DenseCRF::currentMap (densecrf.cpp:202-211): out[p] = the first label of the largest
@@ -1158,8 +1168,9 @@ void launch_kl(const float* Q, const float* U, int N, int L, int Lv, const Slice
                       partials);
 }
 
-void launch_norm_finish(float* norm, int N, int ntype, hipStream_t s) {
-    k_norm_finish<<<blocks_for(N), kThreads, 0, s>>>(norm, N, ntype);
+void launch_norms(const NormTerms& terms, int N, hipStream_t s) {
+    if (!N || !terms.T) return;
+    k_norms<<<dim3(blocks_for(N), terms.T), kThreads, 0, s>>>(terms, N);
     DCRF_HIP_CHECK(hipGetLastError());
 }
 
@@ -1180,10 +1191,10 @@ void launch_entry_gather(const int* csr_e, int E, int d1, const float* bary, con
 }
 
 void launch_slice_weights(const int* vtx, const float* bary, const float* norm, int use_norm, float alpha, int N,
-                          int d1, int vbase, int* gvtx, float* sw, hipStream_t s) {
+                          int d1, int vbase, int* gvtx, float* sw, int2* slc, int ds, int off, hipStream_t s) {
     if (!N) return;
     k_slice_weights<<<blocks_for((size_t)N * d1), kThreads, 0, s>>>(vtx, bary, norm, use_norm, alpha, N, d1, vbase,
-                                                                    gvtx, sw);
+                                                                    gvtx, sw, slc, ds, off);
     DCRF_HIP_CHECK(hipGetLastError());
 }
 
