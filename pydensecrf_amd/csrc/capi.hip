@@ -1292,6 +1292,35 @@ void compute_norms(dcrf_model& m, const std::vector<const TermLattice*>& lats, c
         if (m.terms[k]->ntype == DCRF_NO_NORMALIZATION) mean_norms(m, m.terms[k]->norm.get(), s);
 }
 
+// One term's normaliser without a layout (dcrf_get_lattice): the same sums.
+void term_norm(const dcrf_model& m, const Term& t, DevBuf<float>& norm) {
+    const TermLattice& lat = t.lat;
+    const int V = lat.V, d1 = lat.d + 1;
+    hipStream_t s = m.stream;
+    RunSet rs;
+    SegPlan sp;
+    build_run_set({&lat}, {0}, lat.n_tiles, m.chunk(), rs, s);
+    count_segments(rs, 0, 0, true, sp, s);
+    DevBuf<float> v[2];
+    for (DevBuf<float>& b : v) b.reserve((size_t)V + 1);
+    splat_ones({&lat}, rs, sp, v[0].get(), v[1].get(), s);
+    DevBuf<int2> nbr;
+    nbr.reserve((size_t)d1 * V);
+    launch_remap_nbr(lat.nbr.get(), nbr.get(), d1 * V, 0, V, s);
+    BlurTable bt{};
+    bt.nterms = 1;
+    bt.t[0] = BlurTerm{0, V, lat.d, nbr.get()};
+    for (int step = 0; step < d1; step++)
+        launch_blur(v[step & 1].get(), v[(step + 1) & 1].get(), 0, V, 1, 1, bt, step, 0, s);
+    norm.reserve(m.N());
+    NormTerms nt{};
+    nt.T = 1;
+    nt.t[0] = norm_term(t, v[d1 & 1].get(), 0, norm.get());
+    launch_norms(nt, m.N(), s);
+    if (t.ntype == DCRF_NO_NORMALIZATION) mean_norms(m, norm.get(), s);
+    DCRF_HIP_CHECK(hipStreamSynchronize(s));
+}
+
 // The limit of the allocation-free inference counts the rows of a layout without padding
 // labels and with one lane group per segment, whatever the splat's form: the quad form has
 // more partial rows, padded rows of fewer lanes have fewer, and neither moves the line
@@ -2791,14 +2820,12 @@ int dcrf_term_instance_vertices(const dcrf_model* m, int term, int inst, int* V)
     });
 }
 
-int dcrf_get_lattice(const dcrf_model* cm, int term, int inst, int* offset, int* rank, float* bary, int* nbr,
+int dcrf_get_lattice(const dcrf_model* m, int term, int inst, int* offset, int* rank, float* bary, int* nbr,
                      int16_t* keys, float* norm) {
     return guard([&] {
-        dcrf_model* m = const_cast<dcrf_model*>(cm);  // the normalisers come with the (cached) layout
         require(m != nullptr, "null model");
         require(term >= 0 && term < (int)m->terms.size(), "pairwise term index out of range");
         require(inst >= 0 && inst < m->geo.n_inst, "instance index out of range");
-        if (norm) ensure_layout(*m);
         const Term& t = *m->terms[term];
         const TermLattice& lat = t.lat;
         const int d1 = lat.d + 1;
@@ -2824,7 +2851,12 @@ int dcrf_get_lattice(const dcrf_model* cm, int term, int inst, int* offset, int*
         if (keys)
             DCRF_HIP_CHECK(hipMemcpy(keys, lat.keys.get() + (size_t)vb * lat.d, sizeof(int16_t) * (size_t)Vi * lat.d,
                                      hipMemcpyDeviceToHost));
-        if (norm) DCRF_HIP_CHECK(hipMemcpy(norm, t.norm.get() + pb, sizeof(float) * Ni, hipMemcpyDeviceToHost));
+        if (norm) {
+            DevBuf<float> own;  // the layout, which holds the normalisers, is not built for them
+            if (!m->layout_valid) term_norm(*m, t, own);
+            const float* src = m->layout_valid ? t.norm.get() : own.get();
+            DCRF_HIP_CHECK(hipMemcpy(norm, src + pb, sizeof(float) * Ni, hipMemcpyDeviceToHost));
+        }
     });
 }
 
