@@ -334,8 +334,8 @@ struct LaunchShape {
     int S;      // lanes per item, ceil(L / R)
 };
 int choose_labels_per_lane(int L);
-// Floats of a gathered row (vertex rows, Q between iterations) of L labels: L where three or
-// four labels per lane divide it (or all fit one lane), else L rounded up to 4.
+// Floats of a gathered row (vertex rows, Q between iterations) of L labels: L, or L rounded
+// up to 4 where neither three nor four labels per lane divide it (see the rule).
 int padded_labels(int L);
 // The splat's: K lanes share each lane position of a segment's row (kSplitLanes for rows of
 // one or two lanes, else 1), per segments per wave.

@@ -35,15 +35,24 @@ int choose_labels_per_lane(int L) {
     return 1;
 }
 
-// Rows of L floats that neither 4 nor 3 divides took one or two labels per lane: at 19
+// Rows of L floats that neither 4 nor 3 divides take one or two labels per lane: at 19
 // labels 19 lanes and 3 rows per wave instruction, each with its own addresses and
-// weights.  Padded to 20, five lanes of four labels and 12 rows: 1021x511x19, 10
-// iterations, 1745 -> 1006 us.  Three labels per lane stay: 21 labels padded to 24 (6
-// lanes for 7, aligned 16-byte pieces, but 14 % more bytes in every gathered row) measured
-// 1514 against 1464 us at 1024x768, 10 iterations.
+// weights.  Padded to 20, five lanes of four labels and 12 rows.  10 iterations, unpadded ->
+// padded, us (training forward and backward: the same ratios):
+//   one label per lane    5       7       11      13      17      25      61      257
+//     320x213          310/297 316/290 359/340 349/322 383/355 458/381 707/447 12357/2311
+//     1024x768        1005/761 1152/767 1559/1000 1793/998 2096/1242 2962/1702 6201/3354
+//   two labels per lane   10      14      22      26      34      130
+//     320x213          317/344 330/323 395/367 412/374 458/402 1684/1032
+//     1024x768         969/994 1173/1004 1873/1395 2259/1727 3024/2193
+// 10 labels lose at every size (a fifth more bytes in every row; 64x48: 209 -> 240), the
+// next, 14, gain from 320x213 on: the line for two labels per lane is there.  At 64x48,
+// where launches count, the padded form is up to 12 % slower (11 labels), the same from 65
+// labels on.  Three labels per lane stay: 21 labels padded to 24 (6 lanes for 7, aligned
+// 16-byte pieces, but 14 % more bytes) measured 1514 against 1464 us at 1024x768.
 int padded_labels(int L) {
     const int R = choose_labels_per_lane(L);
-    return L >= 5 && R < 3 ? (L + 3) & ~3 : L;
+    return (R == 1 && L >= 5) || (R == 2 && L >= 14) ? (L + 3) & ~3 : L;
 }
 
 // Rows of one or two lanes (up to 8 labels) take the quad form of the splat
