@@ -510,9 +510,11 @@ __device__ __forceinline__ void matrix_piece_rows(const float* __restrict__ w, i
 
 // y[r] / s for the lane's values, s the same for all of them: one reciprocal (Newton's
 // step on the hardware's approximation), then per value the product and one residual
-// correction (Markstein), which gives the rounded quotient for the softmax's operands
-// (0 <= y <= 1 <= s <= DCRF_MAX_LABELS; NaNs pass through).  Three full divisions took a
-// tenth of the fused mean-field kernel's instructions.
+// correction (Markstein).  For the softmax's operands (0 <= y <= 1 <= s <= DCRF_MAX_LABELS)
+// that is the rounded quotient where y >= 2^-100 and within one unit in the last place
+// below, where the residual is not exact any more (300,000 operands of each range, the
+// reciprocal up to one unit off, in host arithmetic); NaNs pass through.  Three full
+// divisions took a tenth of the fused mean-field kernel's instructions.
 template <int R>
 __device__ __forceinline__ void divide_all(const float (&y)[R], float s, float (&q)[R]) {
     float rc = __builtin_amdgcn_rcpf(s);
