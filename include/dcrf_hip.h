@@ -147,10 +147,10 @@ int dcrf_launch_graph(dcrf_model *m, void *stream);
 /* dcrf_inference_device without any device allocation, for callers that cannot
  * allocate (code under hipGraph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  No counterpart in the reference.  The filter's vertex rows live in one
- * static device array of 64 MiB per GPU (held until the process ends) instead of the
+ * static device array per GPU (102 MiB, held until the process ends) instead of the
  * model's buffers; the model must have run dcrf_inference_device (or dcrf_inference)
- * once, so that its layout and unary are on the device, and its vertex rows must fit
- * the array (DCRF_ERR_VALUE otherwise).  Every call on one GPU shares that array, which
+ * once, so that its layout and unary are on the device, and its vertex rows must be at
+ * most 64 MiB, counted without padding labels (DCRF_ERR_VALUE otherwise).  Every call on one GPU shares that array, which
  * keeps the last call's contents: calls that overlap on one GPU race.  Same kernels and
  * results as dcrf_inference_device. */
 int dcrf_inference_device_noalloc(dcrf_model *m, int n_iterations, const float *U_dev, float *Q_dev,

@@ -827,7 +827,8 @@ void kg_blur(const KgPlan& P, bool x, const float* src, float* const buf[2], int
 
 // Fill plan P for the model terms `terms` (at most DCRF_MAX_TERMS / 2; P's device
 // buffers are reused where they are large enough): the layouts of KgPlan, the merged
-// segment and entry lists (the x layout's lists derived on the device), the pass tables
+// segment and entry lists (those of the paired rows mapped from the x layout's on the
+// device), the pass tables
 // of every chain, and per term the slice weights and the all-ones input splatted and
 // blurred in reverse order (one value per vertex, through the plan's own launches: the
 // same segments, sums and pass order as a filter of that term alone).
@@ -1000,7 +1001,7 @@ void ensure_kg_plans(dcrf_model& m) {
     for (int k = 0; k < (int)m.terms.size(); k++) {
         const Term& t = *m.terms[k];
         if (!t.num_kparams()) continue;
-        // (at most one partial row per entry, and per 16 of those a second-level row)
+        // (sequential lists: at most one partial row per segment, no second level)
         const long long ek = N * (t.lat.d + 1), rk = 2LL * t.lat.V + ek / std::max(1, m.chunk()) + t.lat.n_runs;
         if (!g.empty() && ((int)g.size() == DCRF_MAX_TERMS / 2 || e + ek > lim || rows + rk + 1 > lim ||
                            (long long)(g.size() + 1) * N > lim)) {
@@ -1540,9 +1541,8 @@ void build_layout(dcrf_model& m) {
                 for (int q = 0; q < d1; q++, j++)
                     if (result_parity(m, k)) par |= 1u << j;
             }
-            // rectangles of 2 waves' pixels per row x 16 rows (18 x 16 at 21 labels)
-            // rectangles two waves of pixels wide, at most run_rows high and at most
-            // 24 KiB of slice pairs
+            // rectangles two waves of pixels wide (18 at 21 labels), at most run_rows
+            // high and at most 24 KiB of slice pairs
             const int TW = 2 * shape_for(L).per;
             const int TH = std::max(1, std::min(m.run_rows, (24 * 1024) / (TW * ds * 8)));
             build_run_slice(m.geo, m.geod, m.g_slc.get(), ds, par, TW, TH, m.rslice, s);

@@ -93,13 +93,14 @@ void copy_to_device(void* dst, const void* src, size_t n, hipStream_t s);
 
 // ---------------------------------------------------------------- lattice of one term
 struct Chunk {
-    int v;    // vertex (term-local, later global)
+    int v;    // vertex row; -1: a filler, which pads a wave
     int beg;  // first entry
     int end;  // one past the last entry
-    int out;  // output row: >= 0 vertex row; < 0 partial row -(r+1) (term-local)
+    int out;  // row written (the vertex's or a partial one); -1: none, the sum joins the
+              // segment before it in the wave (a filler: nothing)
 };
 struct Combine {
-    int v;      // vertex
+    int v;      // row written: the vertex's, or a second-level one
     int first;  // first partial row
     int count;  // number of partial rows
     int pad;    // one-launch lists: 0 for a whole vertex, else its number of pieces

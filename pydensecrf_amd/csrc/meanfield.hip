@@ -15,11 +15,12 @@ namespace {
 inline unsigned blocks_for(size_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
 // Mean-field update for models of one or two terms with d+1 = D0 (and D1) lattice
-// (3, 6: images; 4 and 5: volumes with intensity, where the generic kernels took 45 us
-// (mean-field) and 62 us (adjoint) per launch on 1.5 M voxels with 4 labels)
 // entries per pixel: slc holds every pixel's (vertex, weight bits) pairs of both terms
 // side by side, so all D0 + D1 vertex rows are gathered after one dependent load.  Same
 // arithmetic, in the same order, as k_meanfield.
+//   3 and 6 entries are images; 4 and 5 volumes with intensity, where the generic kernels
+// took 45 us (mean-field) and 62 us (adjoint) per launch on 1.5 M voxels with 4 labels,
+// and these 32 and 48.
 template <int R, int D0, int D1, bool CWL, bool NARROW>
 __global__ void __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(R <= 3 ? 8 : 7)))  // <= 64 (72) VGPRs
 k_meanfield_fused(const float* __restrict__ U, float* __restrict__ Q, int ldq, int N, int L, int S, int per,

@@ -16,8 +16,8 @@
 //
 // The host built these lists from downloaded runs before: at 1024x768 3.3 ms of a new
 // model's 14 ms went into its loops, and the lists into the uploads.  Here each stage is a
-// scan or one thread per run, vertex or group; the host reads one set of counts to size
-// the lists.  The order of a vertex's partial rows is that of the stable sort by vertex,
+// scan or one thread per run, vertex or group, the stages that do not wait for each other
+// in one launch; the host reads one set of counts to size the lists.  The order of a vertex's partial rows is that of the stable sort by vertex,
 // i.e. list order, so the sums do not depend on anything but the runs.
 #include <cstring>
 #include <limits>
@@ -226,6 +226,9 @@ __global__ void k_emit(Emit A) {
 // the sums of a sequential list, without its lists and entries.  Segments in vertex order
 // (H[].y), a quad per segment: its lanes load every fourth weight and add all of them in
 // entry order (quad_value), like the splat of few labels.
+// Bound: the random reads of the weights, in vertex order (52 us at 1024x768, 8 at 512x512;
+// the entries in tile order and a list splat: 2 x 24 + 19 us).  One range of segments per XCD
+// took 62 us: the terms' vertices differ in entries, so the ranges differ in work.
 struct OnesTerms {
     int T;
     struct {
