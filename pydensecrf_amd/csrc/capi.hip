@@ -776,8 +776,9 @@ void plan_segments(const RunSet& rs, int Lr, bool runs, SegPlan& P, hipStream_t 
     count_segments(rs, sh.wave && runs ? splat_shape(Lr).per : 0, sh.wave ? sh.per : 0, false, P, s);
 }
 
-// The same for the filters of the normalisers and of the kernel-parameter gradient: every
-// vertex's segments in one sequence, whatever the row length and the other terms.  The
+// The same for the filters of the kernel-parameter gradient: every vertex's segments in one
+// sequence, whatever the row length and the other terms (the normalisers' sums have that
+// order too, splat_ones).  The
 // parameter gradient amplifies the last bits of its vertex rows and of the normalisers a
 // hundred times (two orders of summation differ by 1e-5 of the result at 512x512x21), so
 // these sums keep one order; it costs 11 us a recombination there against in-wave runs

@@ -17,8 +17,9 @@
 // The host built these lists from downloaded runs before: at 1024x768 3.3 ms of a new
 // model's 14 ms went into its loops, and the lists into the uploads.  Here each stage is a
 // scan or one thread per run, vertex or group, the stages that do not wait for each other
-// in one launch; the host reads one set of counts to size the lists.  The order of a vertex's partial rows is that of the stable sort by vertex,
-// i.e. list order, so the sums do not depend on anything but the runs.
+// in one launch; the host reads one set of counts to size the lists.  The order of a
+// vertex's partial rows is that of the stable sort by vertex, i.e. list order, so the sums
+// do not depend on anything but the runs.
 #include <cstring>
 #include <limits>
 
